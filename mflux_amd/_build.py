@@ -259,8 +259,11 @@ OPS_PATH = os.path.join(CSRC, "libmfq_torch.so")
 
 
 def build_torch_ops(verbose: bool = False) -> str:
-    """Compiles csrc/torch_ops.cpp (the torch.ops.mfq registrations, host C++
-    only) against this interpreter's torch and links it to libmfq.so."""
+    """Compiles csrc/torch_ops.cpp (the torch.ops.mfq registrations) and
+    csrc/py_calls.cpp (the module calls as Python C functions), host C++ only,
+    against this interpreter's torch and links them to libmfq.so."""
+    import sysconfig
+
     from torch.utils import cpp_extension
 
     torch_lib = cpp_extension.library_paths()[0]
@@ -268,11 +271,12 @@ def build_torch_ops(verbose: bool = False) -> str:
     tmp = OPS_PATH + ".tmp"
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            "-D_GLIBCXX_USE_CXX11_ABI=1", *[f"-I{p}" for p in cpp_extension.include_paths()], f"-I{rocm}/include",
-           os.path.join(CSRC, "torch_ops.cpp"), "-o", tmp, f"-L{CSRC}", "-lmfq", f"-L{torch_lib}", "-ltorch",
-           "-ltorch_cpu", "-lc10", "-ltorch_hip", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+           f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, "torch_ops.cpp"), os.path.join(CSRC, "py_calls.cpp"),
+           "-o", tmp, f"-L{CSRC}", "-lmfq", f"-L{torch_lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+           "-ltorch_hip", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"g++ failed on torch_ops.cpp:\n{res.stdout}\n{res.stderr}")
+        raise RuntimeError(f"g++ failed on torch_ops.cpp / py_calls.cpp:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, OPS_PATH)
     if verbose:
         print(f"built {OPS_PATH}")

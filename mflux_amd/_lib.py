@@ -95,6 +95,27 @@ def ops():
     return _ops
 
 
+_native = None
+
+
+def native():
+    """The Python C functions of csrc/py_calls.cpp, which live in the same library
+    as the ops: ``linear``, ``silu_linear`` and ``epilogue_linear`` take the
+    ordinary call of a quantized linear straight to the C ABI and return None
+    for anything else."""
+    global _native
+    if _native is None:
+        import importlib.machinery
+        import importlib.util
+
+        ops()
+        loader = importlib.machinery.ExtensionFileLoader("libmfq_torch", OPS_PATH)
+        spec = importlib.util.spec_from_file_location("libmfq_torch", OPS_PATH, loader=loader)
+        _native = importlib.util.module_from_spec(spec)
+        loader.exec_module(_native)
+    return _native
+
+
 def check(fn: str, status: int) -> None:
     if status != 0:
         raise MfqError(fn, status, load().mfq_strerror(status).decode())

@@ -221,6 +221,10 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     """``x @ dequantize(w).T`` (``transpose=True``) or ``x @ dequantize(w)``; see
     ``_quantized_matmul_forward``.  Differentiable with respect to ``x`` and
     ``bias``; ``low_rank`` (inference only) is described there."""
+    if transpose and low_rank is None and mode == "affine":
+        y = _lib.native().linear(x, w, scales, biases, bias, group_size, bits)
+        if y is not None:
+            return y
     _check_mode("quantized_matmul", mode)
     _check_group_bits("quantized_matmul", group_size, bits)
     if not transpose:
@@ -357,6 +361,10 @@ def silu_quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor
     product to ``x``'s dtype.  Not differentiable in its fused form: with
     gradients enabled on ``x`` or ``bias`` the composed form runs.
     """
+    if mode == "affine":
+        y = _lib.native().silu_linear(x, w, scales, biases, bias, group_size, bits)
+        if y is not None:
+            return y
     _check_mode("quantized_matmul", mode)
     _check_group_bits("quantized_matmul", group_size, bits)
     needs_grad = torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad))
@@ -464,6 +472,11 @@ def quantized_matmul_epilogue(x: torch.Tensor, w: torch.Tensor, scales: torch.Te
     Every step rounds to ``x``'s dtype as the separate operations do.  Inference
     only (no autograd through the fused form: with gradients enabled on an input
     the composed form runs)."""
+    if mode == "affine":
+        y = _lib.native().epilogue_linear(x, w, scales, biases, bias, group_size, bits, EPILOGUES.get(epilogue, 0), gate,
+                                          residual, act_from)
+        if y is not None:
+            return y
     _check_mode("quantized_matmul", mode)
     _check_group_bits("quantized_matmul", group_size, bits)
     if epilogue not in EPILOGUES:

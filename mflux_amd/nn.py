@@ -124,20 +124,28 @@ class QuantizedLinear(torch.nn.Module):
         self._prepared_key = self._weights_key() if self._prepared is not None else None
         return self._prepared is not None
 
+    def _operands(self):
+        # straight from the buffers: an attribute of a module that is not in its __dict__ costs a Python-level lookup
+        b = self._buffers
+        try:
+            return b["weight"], b["scales"], b["biases"], b["bias"] if "bias" in b else self.bias
+        except KeyError:  # a tensor that someone registered as a parameter
+            return self.weight, self.scales, self.biases, self.bias
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if (getattr(self, "_prepared", None) is not None and x.dtype == self.scales.dtype and x.shape[-1] > 0
+        if (self.__dict__.get("_prepared") is not None and x.dtype == self.scales.dtype and x.shape[-1] > 0
                 and x.numel() // x.shape[-1] >= self.PREPARED_MIN_ROWS and not (torch.is_grad_enabled() and x.requires_grad)):
             if not self._prepared_is_current():
                 self.prepare()
             if self._prepared is not None:
                 return core.quantized_matmul_prepared(x, self._prepared, self.output_dims, self.bias)
-        return core.quantized_matmul(x, self.weight, self.scales, self.biases, transpose=True,
-                                     group_size=self.group_size, bits=self.bits, mode=self.mode, bias=self.bias)
+        weight, scales, biases, bias = self._operands()
+        return core.quantized_matmul(x, weight, scales, biases, True, self.group_size, self.bits, self.mode, bias=bias)
 
     def silu_forward(self, x: torch.Tensor) -> torch.Tensor:
         """``self(silu(x))``, the activation inside the matvec kernel when ``x`` is one row."""
-        return core.silu_quantized_matmul(x, self.weight, self.scales, self.biases, group_size=self.group_size,
-                                          bits=self.bits, mode=self.mode, bias=self.bias)
+        weight, scales, biases, bias = self._operands()
+        return core.silu_quantized_matmul(x, weight, scales, biases, self.group_size, self.bits, self.mode, bias=bias)
 
     @classmethod
     def from_linear(cls, linear_layer: torch.nn.Module, group_size: int | None = None, bits: int | None = None,
@@ -190,7 +198,7 @@ def silu_linear(layer: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
 def _linear_parts(layer: torch.nn.Module, fn: str):
     if not isinstance(layer, QuantizedLinear):
         raise ValueError(f"[{fn}] expected a QuantizedLinear, got {type(layer).__name__}")
-    return layer.weight, layer.scales, layer.biases
+    return layer._operands()
 
 
 def layer_norm_modulate(x: torch.Tensor, scale: torch.Tensor | None = None, shift: torch.Tensor | None = None,
@@ -212,9 +220,9 @@ def gelu_linear(layer: torch.nn.Module, x: torch.Tensor, act_from: int = 0) -> t
     if not isinstance(layer, QuantizedLinear):
         y = layer(x)
         return torch.cat([y[..., :act_from], core.gelu_approx(y[..., act_from:])], dim=-1) if act_from else core.gelu_approx(y)
-    w, s, b = _linear_parts(layer, "gelu_linear")
+    w, s, b, bias = _linear_parts(layer, "gelu_linear")
     return core.quantized_matmul_epilogue(x, w, s, b, epilogue="gelu", group_size=layer.group_size, bits=layer.bits,
-                                          mode=layer.mode, bias=layer.bias, act_from=act_from)
+                                          mode=layer.mode, bias=bias, act_from=act_from)
 
 
 def gate_residual_linear(layer: torch.nn.Module, x: torch.Tensor, gate: torch.Tensor,
@@ -228,7 +236,7 @@ def gate_residual_linear(layer: torch.nn.Module, x: torch.Tensor, gate: torch.Te
     ``gate`` of shape ``[B, N]`` or ``[B, 1, N]`` next to ``x`` of ``[B, S, K]``
     runs the kernel once per batch entry, each with its own vector.  A float
     layer gets the composed form."""
-    N = layer.output_dims if isinstance(layer, QuantizedLinear) else layer.weight.shape[0]
+    N = layer.weight.shape[0]
     if gate.numel() != N:
         B = x.shape[0] if x.ndim >= 3 else 0
         if B and gate.numel() == B * N and tuple(gate.shape) in ((B, N), (B, 1, N)) and residual.shape[0] == B:
@@ -238,9 +246,9 @@ def gate_residual_linear(layer: torch.nn.Module, x: torch.Tensor, gate: torch.Te
                          f"[B, 1, {N}] next to x of [B, S, K]; got {tuple(gate.shape)} for x of {tuple(x.shape)}")
     if not isinstance(layer, QuantizedLinear):
         return residual + gate.reshape(-1) * layer(x)
-    w, s, b = _linear_parts(layer, "gate_residual_linear")
+    w, s, b, bias = _linear_parts(layer, "gate_residual_linear")
     return core.quantized_matmul_epilogue(x, w, s, b, epilogue="gate_residual", group_size=layer.group_size,
-                                          bits=layer.bits, mode=layer.mode, bias=layer.bias, gate=gate,
+                                          bits=layer.bits, mode=layer.mode, bias=bias, gate=gate,
                                           residual=residual)
 
 
@@ -286,9 +294,9 @@ def swiglu_linear(stacked: QuantizedLinear, x: torch.Tensor) -> torch.Tensor:
     """``silu(w1 x) * w3 x`` for ``stacked = stack_gate_up(w1, w3)``: one GEMM over
     both projections whose epilogue writes the ``[..., N / 2]`` product, instead
     of two GEMMs and three element-wise passes."""
-    w, s, b = _linear_parts(stacked, "swiglu_linear")
+    w, s, b, bias = _linear_parts(stacked, "swiglu_linear")
     return core.quantized_matmul_epilogue(x, w, s, b, epilogue="swiglu", group_size=stacked.group_size,
-                                          bits=stacked.bits, mode=stacked.mode, bias=stacked.bias)
+                                          bits=stacked.bits, mode=stacked.mode, bias=bias)
 
 
 def concat_quantized(layers: list[QuantizedLinear], share_storage: bool = False) -> QuantizedLinear:
