@@ -20,6 +20,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../include/mfq.h"
 
@@ -69,6 +70,7 @@ struct Linear {
 
   bool check() {
     if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled()) return false;
+    if (torch::jit::tracer::isTracing()) return false;  // a trace would keep this call's result as a constant
     if (!plain(x) || !plain(wq) || !plain(scales) || !plain(biases) || (bias.defined() && !plain(bias))) return false;
     if (c10::GradMode::is_enabled() && (x.requires_grad() || (bias.defined() && bias.requires_grad()))) return false;
     const at::ScalarType t = scales.scalar_type();

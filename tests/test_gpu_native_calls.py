@@ -67,6 +67,14 @@ def test_everything_else_is_left_to_the_general_route():
 
     with Mode():
         assert n.linear(x, w, s, b, bias, 64, 8) is None
+    answers = []
+
+    def traced(t):
+        answers.append(n.linear(t, w, s, b, bias, 64, 8))
+        return t + 1
+
+    torch.jit.trace(traced, x, check_trace=False)
+    assert answers == [None]
     with pytest.raises(ValueError, match="does not match"):
         layer(x[:, :192])
     # autograd still sees the call
