@@ -323,8 +323,8 @@ int mfq_qmm_t_static(const void* x, int x_dtype, int64_t M, int64_t K, const uin
  * mfq_qmm_t does for M <= 4.  Arguments as for mfq_qmm_t.
  * MFQ_EUNSUPPORTED when no fused kernel takes the shape (bits other than 4
  * and 8; M = 1 with rows of more than 6 KiB of 8-bit or 3 KiB of 4-bit codes;
- * M = 2..4 outside what the eight-rows kernels (K = 1024, 2048, 3072 or 4096,
- * group size 64, N a multiple of 8) and the four-rows kernel (K <= 4096, N a
+ * M = 2..4 outside what the eight-rows kernels (K = 256, 1024, 2048, 2560,
+ * 3072, 3840, 4096 or 6144, group size 64, N a multiple of 8) and the four-rows kernel (K <= 4096, N a
  * multiple of 4, rows of 1, 2, 3, 4, 6, 8, 12 or 16 times 256 bytes) take;
  * M > 4): apply the activation separately and call mfq_qmm_t.
  */

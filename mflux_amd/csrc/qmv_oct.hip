@@ -1,6 +1,6 @@
-// Quantized matvec for one to four activation rows on gfx950, eight weight rows
+// Quantized matvec for one to sixteen activation rows on gfx950, eight weight rows
 // at a time on the int8 matrix-core instruction:
-//   y[0:M, n] = x[0:M] . dequant(W[n]) (+ bias),  M <= 4, 8-bit codes, groups of 64.
+//   y[0:M, n] = x[0:M] . dequant(W[n]) (+ bias),  8-bit codes, groups of 64.
 // The adaLN modulation call of every DiT block
 // (src/mflux/models/flux/model/flux_transformer/ada_layer_norm_zero.py:12,
 // src/mflux/models/qwen/model/qwen_transformer/qwen_transformer_block.py:36-37).
@@ -18,7 +18,8 @@
 //     high bytes in row 2 m, low bytes in row 2 m + 1.  Of D, column j's rows
 //     0..7 (j even) or 8..15 (j odd) are the products that belong together; the
 //     others pair a half of the weights with the other half of x and are dropped.
-//     Up to four activation rows cost what one does.
+//     Up to four activation rows cost what one does; five to eight take a second
+//     instruction on the same B operand, and more than eight a second workgroup.
 //   - a code enters as the signed byte code - 128 (one XOR per word); a half step
 //     is one group of 64 codes, so per instruction and lane, with Sx the sum of xq
 //     over the group's 64 k,
@@ -32,9 +33,13 @@
 // three blocks in flight in three register sets, all unconditional so that every
 // wait leaves exactly the younger loads in flight.  The eight partial sums of a
 // block meet in LDS at the end of the run, where each thread adds up one output.
+// Bound by HBM, and from five rows on by the image of x in front of the first block:
+// 3072 -> 18432 takes 11.4 us with one row, 13.3 with eight (24.8 on the kernel that
+// dequantises, whose error against float64 is 1.6e-3 where this one's is 1.4e-5).
+// Rows whose steps do not come in eights are split over ten wavefronts (K = 2560, 3840).
 #include <type_traits>
 
-#include "common.h"
+#include "qmv_oct_common.h"
 
 namespace mfq {
 namespace {
@@ -43,7 +48,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kOctRows = 8;       // weight rows per block
-constexpr int kOctWaves = 8;      // wavefronts per workgroup: eighths of K
 constexpr int kOctSets = 3;       // blocks in flight per wavefront
 constexpr int kOctMaxBlocks = 12;  // blocks per workgroup (their partial sums wait in LDS)
 constexpr int kOctLongRun = 9;    // blocks per workgroup when a compute unit's share exceeds that
@@ -79,17 +83,18 @@ struct ScaleWindow {
   uint32_t d[kSteps];  // dword s: the scales (or biases) of the two halves of step s
 };
 
-// kSteps: 128-byte steps per wavefront and row (K = 1024 kSteps); kM: activation rows the image is built for
-// (1, 2 or 4; M = 3 runs as 4 with its last row repeated)
-template <typename T, int kSteps, int kM, bool kSilu>
-__global__ __launch_bounds__(64 * kOctWaves) void qmv_oct_kernel(
+// K = 128 kWaves kSteps, kSteps 128-byte steps per wavefront and row; kM: activation rows the image is built for
+// (1, 2, 4 or 8; other M run as the next of these with their last row repeated)
+template <typename T, int kWaves, int kSteps, int kM, bool kSilu>
+__global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
     const uint16_t* __restrict__ biases, const uint16_t* __restrict__ bias, void* __restrict__ y, int y_is_f32, int M,
     int N, int blocks_per_wg) {
-  constexpr int K = 128 * kOctWaves * kSteps;
+  constexpr int K = 128 * kWaves * kSteps;
   constexpr int kSlice = 128 * kSteps;       // bytes (= codes) per row and wavefront
   constexpr int kGroups = K / 64;
   constexpr int kPitch = kSlice + 16;        // image rows in LDS
+  constexpr int kPasses = kM > 4 ? 2 : 1;    // fours of activation rows
   constexpr int kImageRows = 2 * kM;
   constexpr int kImageBytes = ((kImageRows * kPitch + kM * 2 * kSteps * 4) + 255) & ~255;  // + the sums of xq
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -99,20 +104,29 @@ __global__ __launch_bounds__(64 * kOctWaves) void qmv_oct_kernel(
   const int n8 = j >> 1, h = j & 1;
   char* image = lds + wave * kImageBytes;
   float* sums = reinterpret_cast<float*>(image + kImageRows * kPitch);
-  float2* partials = reinterpret_cast<float2*>(lds + kOctWaves * kImageBytes);  // [block][wavefront][lane]
+  float2* partials = reinterpret_cast<float2*>(lds + kWaves * kImageBytes);  // [block][wavefront][pass][kSlots]
+  constexpr int kSlots = kM > 4 ? 32 : 64;   // every lane's pair, or the useful half of the lanes' (2 j + q % 2)
+  int run = blockIdx.x;
+  if constexpr (kM > 4) {  // more than eight activation rows: eight to a workgroup
+    const int m0 = oct_run_and_first_row<kM>(M, run);
+    x += (size_t)m0 * K;
+    y = static_cast<char*>(y) + (size_t)m0 * N * (y_is_f32 ? 4 : 2);
+    M = min(kM, M - m0);
+  }
 
   const int n_blocks_all = N / kOctRows;
-  const int blk_first = blockIdx.x * blocks_per_wg;
+  const int blk_first = run * blocks_per_wg;
+  if (kM > 4 && blk_first >= n_blocks_all) return;  // (runs are dealt out in eights)
   const int n_blocks = min(blocks_per_wg, n_blocks_all - blk_first);
   const int blk_last = blk_first + n_blocks - 1;
 
   // the output this thread will add up at the end (block, weight row, activation row), and its layer bias:
   // requested now, with everything else, so that nothing is fetched behind the last barrier
-  constexpr int kOuts = (kOctMaxBlocks * kOctRows * 4 + 64 * kOctWaves - 1) / (64 * kOctWaves);
+  constexpr int kOuts = (kOctMaxBlocks * kOctRows * (kM > 4 ? kM : 4) + 64 * kWaves - 1) / (64 * kWaves);
   uint16_t out_bias[kOuts];
 #pragma unroll
   for (int i = 0; i < kOuts; ++i) {
-    const int o = (int)threadIdx.x + i * 64 * kOctWaves;
+    const int o = (int)threadIdx.x + i * 64 * kWaves;
     const int64_t row = (int64_t)(blk_first + min(o / M / kOctRows, n_blocks - 1)) * kOctRows + (o / M) % kOctRows;
     out_bias[i] = (bias ? bias : scales)[row];
   }
@@ -185,60 +199,74 @@ __global__ __launch_bounds__(64 * kOctWaves) void qmv_oct_kernel(
     }
   }
   // (LDS written and read by this wavefront only: program order holds)
-  // this lane's A operands: image row j % 8 over half j / 8 of every step (image rows past 2 kM: any row, their
-  // results are never read)
-  i32x4 xa[kSteps];
-  {
-    const char* arow = image + (j & 7 & (kImageRows - 1)) * kPitch + 64 * (j >> 3) + 16 * q;
+  // this lane's A operands, pass p: image row 8 p + j % 8 over half j / 8 of every step (image rows past 2 kM: any
+  // row, their results are never read)
+  i32x4 xa[kPasses][kSteps];
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) xa[s] = *reinterpret_cast<const i32x4*>(arow + 128 * s);
+  for (int p = 0; p < kPasses; ++p) {
+    const char* arow = image + (8 * p + (j & 7 & (kImageRows - 1))) * kPitch + 64 * (j >> 3) + 16 * q;
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) xa[p][s] = *reinterpret_cast<const i32x4*>(arow + 128 * s);
   }
   // results: register r of lane (j, q) is A's row 4 q + r against column j.  Of use where q / 2 == j % 2:
-  // activation rows 2 (q % 2) (registers 0, 1: high, low bytes) and 2 (q % 2) + 1 (registers 2, 3)
+  // activation rows 4 p + 2 (q % 2) (registers 0, 1: high, low bytes) and 4 p + 2 (q % 2) + 1 (registers 2, 3)
   constexpr bool kTwo = kM > 1;  // one activation row: registers 2 and 3 hold nothing of use
-  const int m_a = (2 * (q & 1)) & (kM - 1), m_b = (2 * (q & 1) + 1) & (kM - 1);
   // the sums of xq over this lane's half steps: as float for the bias term, and 128 times them as integers
   // (a code enters the matrix instruction as code - 128; adding 128 sum(xq) to its result gives sum(xq code))
-  float sx_a[kSteps], sx_b[kSteps];
-  int sx128_a[kSteps], sx128_b[kSteps];
+  float sx_a[kPasses][kSteps], sx_b[kPasses][kSteps], us_a[kPasses], us_b[kPasses];
+  int sx128_a[kPasses][kSteps], sx128_b[kPasses][kSteps];
 #pragma unroll
-  for (int s = 0; s < kSteps; ++s) {
-    sx_a[s] = sums[m_a * 2 * kSteps + 2 * s + h];
-    sx_b[s] = kTwo ? sums[m_b * 2 * kSteps + 2 * s + h] : 0.f;
-    sx128_a[s] = 128 * (int)sx_a[s];
-    sx128_b[s] = 128 * (int)sx_b[s];
-  }
-  float us_a = unscale_m[0], us_b = unscale_m[kM > 1 ? 1 : 0];
+  for (int p = 0; p < kPasses; ++p) {
+    const int m_a = (4 * p + 2 * (q & 1)) & (kM - 1), m_b = (4 * p + 2 * (q & 1) + 1) & (kM - 1);
 #pragma unroll
-  for (int m = 2; m < kM; ++m) {
-    us_a = m_a == m ? unscale_m[m] : us_a;
-    us_b = m_b == m ? unscale_m[m] : us_b;
+    for (int s = 0; s < kSteps; ++s) {
+      sx_a[p][s] = sums[m_a * 2 * kSteps + 2 * s + h];
+      sx_b[p][s] = kTwo ? sums[m_b * 2 * kSteps + 2 * s + h] : 0.f;
+      sx128_a[p][s] = 128 * (int)sx_a[p][s];
+      sx128_b[p][s] = 128 * (int)sx_b[p][s];
+    }
+    us_a[p] = unscale_m[4 * p];
+    us_b[p] = unscale_m[4 * p + (kTwo ? 1 : 0)];
+    if constexpr (kM > 2) {
+      us_a[p] = (q & 1) ? unscale_m[4 * p + 2] : us_a[p];
+      us_b[p] = (q & 1) ? unscale_m[4 * p + 3] : us_b[p];
+    }
   }
 
 #pragma unroll
   for (int t = 1; t < kOctSets; ++t) issue(t, blk_first + t);
   auto consume = [&](int set, int slot) __attribute__((always_inline)) {
-    float acc_a = 0.f, acc_b = 0.f;
+    float acc_a[kPasses], acc_b[kPasses];
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) acc_a[p] = 0.f, acc_b[p] = 0.f;
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
       i32x4 wb;
 #pragma unroll
       for (int k = 0; k < 4; ++k) wb[k] = (int)(wv[set][s][k] ^ 0x80808080u);  // code - 128 as signed bytes
-      const i32x4 zero = {0, 0, 0, 0};
-      const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[s], wb, zero, 0, 0, 0);
       const float sc = T::to_f32((uint16_t)(h ? sw[set].d[s] >> 16 : sw[set].d[s]));
       const float bi = T::to_f32((uint16_t)(h ? bw[set].d[s] >> 16 : bw[set].d[s]));
-      // sum(xq code) over the half step's group, exact: high and low bytes of xq joined as integers
-      const int da = d[0] * 256 + d[1] + sx128_a[s];
-      acc_a = __builtin_fmaf(sc, (float)da, acc_a);
-      acc_a = __builtin_fmaf(bi, sx_a[s], acc_a);
-      if constexpr (kTwo) {
-        const int db = d[2] * 256 + d[3] + sx128_b[s];
-        acc_b = __builtin_fmaf(sc, (float)db, acc_b);
-        acc_b = __builtin_fmaf(bi, sx_b[s], acc_b);
+#pragma unroll
+      for (int p = 0; p < kPasses; ++p) {
+        const i32x4 zero = {0, 0, 0, 0};
+        const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[p][s], wb, zero, 0, 0, 0);
+        // sum(xq code) over the half step's group, exact: high and low bytes of xq joined as integers
+        const int da = d[0] * 256 + d[1] + sx128_a[p][s];
+        acc_a[p] = __builtin_fmaf(sc, (float)da, acc_a[p]);
+        acc_a[p] = __builtin_fmaf(bi, sx_a[p][s], acc_a[p]);
+        if constexpr (kTwo) {
+          const int db = d[2] * 256 + d[3] + sx128_b[p][s];
+          acc_b[p] = __builtin_fmaf(sc, (float)db, acc_b[p]);
+          acc_b[p] = __builtin_fmaf(bi, sx_b[p][s], acc_b[p]);
+        }
       }
     }
-    partials[(slot * kOctWaves + wave) * 64 + lane] = make_float2(acc_a * us_a, acc_b * us_b);
+    if (kSlots == 64 || (q >> 1) == h) {
+      const int u = kSlots == 64 ? lane : 2 * j + (q & 1);
+#pragma unroll
+      for (int p = 0; p < kPasses; ++p)
+        partials[((slot * kWaves + wave) * kPasses + p) * kSlots + u] = make_float2(acc_a[p] * us_a[p], acc_b[p] * us_b[p]);
+    }
   };
 
   // Three blocks per trip, one per register set, and between the arithmetic of two blocks the requests for the
@@ -265,19 +293,25 @@ __global__ __launch_bounds__(64 * kOctWaves) void qmv_oct_kernel(
   // ---- one output per thread: block, weight row, activation row; 8 eighths x 2 halves of partial sums --------
 #pragma unroll
   for (int i = 0; i < kOuts; ++i) {
-    const int o = (int)threadIdx.x + i * 64 * kOctWaves;
+    const int o = (int)threadIdx.x + i * 64 * kWaves;
     const int out_m = o % M, out_row8 = (o / M) % kOctRows, out_blk = o / M / kOctRows;
     if (out_blk >= n_blocks) break;
     const int64_t out_row = (int64_t)(blk_first + out_blk) * kOctRows + out_row8;
     float v = 0.f;
 #pragma unroll
-    for (int w = 0; w < kOctWaves; ++w)
+    for (int w = 0; w < kWaves; ++w)
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
-        const int src = (2 * out_row8 + hh) + 16 * (2 * hh + (out_m >> 1));
-        const float2 p = partials[(out_blk * kOctWaves + w) * 64 + src];
+        const int src_j = 2 * out_row8 + hh, pair = (out_m >> 1) & 1;
+        const int src = kSlots == 64 ? src_j + 16 * (2 * hh + pair) : 2 * src_j + pair;
+        const float2 p = partials[((out_blk * kWaves + w) * kPasses + (out_m >> 2)) * kSlots + src];
         v += (out_m & 1) ? p.y : p.x;
       }
+    // more than four rows: an infinity in x is an infinity of the weight's sign in y, as the kernel that
+    // dequantises gives it (the rows that meet no infinity or NaN never come here)
+    if constexpr (kM > 4) {
+      if (v != v) v = oct_plain_dot<T, 8>(x + (size_t)out_m * K, wq, scales, biases, out_row, K);
+    }
     const float bias_v = T::to_f32(out_bias[i]);
     if (y_is_f32) {
       reinterpret_cast<float*>(y)[(int64_t)out_m * N + out_row] = bias ? v + bias_v : v;
@@ -289,58 +323,54 @@ __global__ __launch_bounds__(64 * kOctWaves) void qmv_oct_kernel(
   }
 }
 
-template <typename T, int kSteps, int kM, bool kSilu>
+template <typename T, int kWaves, int kSteps, int kM, bool kSilu>
 int launch_oct(const void* x, int64_t M, const uint32_t* wq, const void* scales, const void* biases, const void* bias,
                int64_t N, void* y, int y_dtype, hipStream_t stream) {
-  auto kernel = qmv_oct_kernel<T, kSteps, kM, kSilu>;
+  auto kernel = qmv_oct_kernel<T, kWaves, kSteps, kM, kSilu>;
   constexpr int kImageBytes = ((2 * kM * (128 * kSteps + 16) + kM * 2 * kSteps * 4) + 255) & ~255;
-  constexpr int kLdsMax = kOctWaves * kImageBytes + (kOctMaxBlocks + 1) * kOctWaves * 512;
+  constexpr int kPerBlock = kWaves * 512;  // partial sums: 64 pairs per wavefront, or two passes of 32
   static PerDeviceInt configured;
-  if (!raise_lds_limit(configured, reinterpret_cast<const void*>(kernel), kLdsMax)) return MFQ_ELAUNCH;
-  // One workgroup per compute unit while that is at most kOctMaxBlocks blocks each; longer weights in runs of
-  // kOctLongRun blocks to as many workgroups as that takes (several resident per unit: a run's last loads and
-  // its adding-up overlap the next run's first requests).
-  const int64_t blocks = N / kOctRows;
-  const int64_t cus = compute_units();
-  int64_t per_wg = (blocks + cus - 1) / cus;
-  if (per_wg > kOctMaxBlocks) per_wg = kOctLongRun;
-  const int64_t n_wg = (blocks + per_wg - 1) / per_wg;
-  const int lds = kOctWaves * kImageBytes + ((int)per_wg + 1) * kOctWaves * 512;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)n_wg), dim3(64 * kOctWaves), lds, stream, (const uint16_t*)x, wq,
-                     (const uint16_t*)scales, (const uint16_t*)biases, (const uint16_t*)bias, y,
-                     (int)(y_dtype == MFQ_F32), (int)M, (int)N, (int)per_wg);
-  return hipGetLastError() == hipSuccess ? MFQ_OK : MFQ_ELAUNCH;
+  return launch_oct_runs<kWaves, kM>(kernel, configured, kWaves * kImageBytes, kPerBlock, kOctRows, kOctMaxBlocks,
+                                     kOctLongRun, x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
 }
 
-template <typename T, int kSteps, bool kSilu>
+// Activation rows the image is built for: 1, 2, 4 or 8, fours and eights with their last rows repeated.
+template <typename T, int kWaves, int kSteps, bool kSilu>
 int launch_oct_rows(const void* x, int64_t M, const uint32_t* wq, const void* scales, const void* biases,
                     const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream) {
-  if (M == 1) return launch_oct<T, kSteps, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-  if (M == 2) return launch_oct<T, kSteps, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-  return launch_oct<T, kSteps, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  if (M == 1) return launch_oct<T, kWaves, kSteps, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  if (M == 2) return launch_oct<T, kWaves, kSteps, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  if (M <= 4) return launch_oct<T, kWaves, kSteps, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  if constexpr (!kSilu)
+    return launch_oct<T, kWaves, kSteps, 8, false>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  return MFQ_EUNSUPPORTED;
 }
 
+// The split of K: wavefronts times 128-byte steps of each.
 template <typename T, bool kSilu>
 int launch_oct_steps(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* scales, const void* biases,
                      const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream) {
-  switch (K / (128 * kOctWaves)) {
-    case 1: return launch_oct_rows<T, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 2: return launch_oct_rows<T, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 3: return launch_oct_rows<T, 3, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 4: return launch_oct_rows<T, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  switch (K) {
+    case 256: return launch_oct_rows<T, 2, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 1024: return launch_oct_rows<T, 8, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 2048: return launch_oct_rows<T, 8, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 2560: return launch_oct_rows<T, 10, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 3072: return launch_oct_rows<T, 8, 3, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 3840: return launch_oct_rows<T, 10, 3, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 4096: return launch_oct_rows<T, 8, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 6144: return launch_oct_rows<T, 8, 6, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     default: return MFQ_EUNSUPPORTED;
   }
 }
 
 }  // namespace
 
-// Shapes this kernel takes: 8-bit codes in groups of 64, one to four activation rows, K of 1024, 2048, 3072
-// or 4096 (an eighth of a row is whole 128-byte steps), whole eights of weight rows, x and the weights
-// 16-byte aligned, scales and biases 4-byte aligned.
+// Shapes this kernel takes: 8-bit codes in groups of 64, up to sixteen activation rows, the K that
+// launch_oct_steps splits, whole eights of weight rows, x and the weights 16-byte aligned, scales and biases
+// 4-byte aligned.
 bool qmv_oct_covers(int64_t M, int64_t K, int64_t N, int gs, int bits, const void* x, const void* scales,
                     const void* biases) {
-  if (!(bits == 8 && gs == 64 && M >= 1 && M <= 4 && K % (128 * kOctWaves) == 0 && K >= 128 * kOctWaves && K <= 4096 && N % kOctRows == 0))
-    return false;
+  if (!(bits == 8 && gs == 64 && oct_takes(M, K, bits) && N % kOctRows == 0)) return false;
   return aligned16(x) && ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 3u) == 0;
 }
 

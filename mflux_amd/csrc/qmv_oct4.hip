@@ -1,7 +1,7 @@
-// Quantized matvec for one to four activation rows and 4-bit codes on gfx950,
+// Quantized matvec for one to sixteen activation rows and 4-bit codes on gfx950,
 // eight weight rows at a time on the int8 matrix-core instruction: the scheme
 // of qmv_oct.hip (which see) for packed nibbles,
-//   y[0:M, n] = x[0:M] . dequant(W[n]) (+ bias),  M <= 4, groups of 64.
+//   y[0:M, n] = x[0:M] . dequant(W[n]) (+ bias),  groups of 64.
 // The adaLN modulation call of every DiT block of a 4-bit model
 // (src/mflux/models/qwen/model/qwen_transformer/qwen_transformer_block.py:36-37,
 // src/mflux/models/flux/model/flux_transformer/ada_layer_norm_zero.py:12).
@@ -21,12 +21,13 @@
 // nothing is offset:
 //     d = 256 D_high + D_low      (int32, exactly sum(xq code) over the group)
 //     acc += scale * d + bias * sum(xq)
-// Three and four activation rows take a second pair of instructions on the same
-// B operands.  Work layout, register sets, the meeting of the wavefronts'
-// partial sums at the end: qmv_oct.hip's, with K split over kWaves4 wavefronts.
+// Every further two activation rows (up to eight; more take a second workgroup) are
+// another pair of instructions on the same B operands: 3072 -> 18432 takes 7.4 us with
+// one row, 8.6 with four, 11.4 with eight (31.2 on the kernel that dequantises).  Work layout, register sets, the meeting of the wavefronts'
+// partial sums at the end: qmv_oct.hip's, with K split over kWaves wavefronts.
 #include <type_traits>
 
-#include "common.h"
+#include "qmv_oct_common.h"
 
 namespace mfq {
 namespace {
@@ -70,7 +71,7 @@ struct ScaleWindow4 {
 };
 
 // kWaves: wavefronts per workgroup, each with kSteps 128-byte steps of every row (K = 256 kWaves kSteps codes);
-// kM: activation rows the image is built for (1, 2 or 4; M = 3 runs as 4 with its last row repeated)
+// kM: activation rows the image is built for (1, 2, 4 or 8; other M run as the next of these with their last row repeated)
 template <typename T, int kWaves, int kSteps, int kM, bool kSilu>
 __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
@@ -80,7 +81,7 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
   constexpr int kRowBytes = K / 2;
   constexpr int kSlice = 128 * kSteps;       // bytes per row and wavefront: 2 kSlice codes
   constexpr int kGroups = K / 64;
-  constexpr int kPasses = kM > 2 ? 2 : 1;    // pairs of activation rows
+  constexpr int kPasses = kM > 2 ? kM / 2 : 1;  // pairs of activation rows
   constexpr int kImageRows = 2 * kM;         // (activation row, high / low byte)
   constexpr int kPitch = 2 * kSlice + 32;    // an image row: kSlice bytes of even k, kSlice of odd k
   constexpr int kImageBytes = ((kImageRows * kPitch + kM * 4 * kSteps * 4) + 255) & ~255;  // + the sums of xq
@@ -91,16 +92,25 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
   const int n8 = j >> 1, h = j & 1;
   char* image = lds + wave * kImageBytes;
   float* sums = reinterpret_cast<float*>(image + kImageRows * kPitch);  // [activation row][group of the slice]
-  float2* partials = reinterpret_cast<float2*>(lds + kWaves * kImageBytes);  // [block][wavefront][pass][lane]
+  float2* partials = reinterpret_cast<float2*>(lds + kWaves * kImageBytes);  // [block][wavefront][pass][kSlots]
+  constexpr int kSlots = kM > 4 ? 32 : 64;   // every lane's pair, or the useful half of the lanes' (2 j + q % 2)
+  int run = blockIdx.x;
+  if constexpr (kM > 4) {  // more than eight activation rows: eight to a workgroup
+    const int m0 = oct_run_and_first_row<kM>(M, run);
+    x += (size_t)m0 * K;
+    y = static_cast<char*>(y) + (size_t)m0 * N * (y_is_f32 ? 4 : 2);
+    M = min(kM, M - m0);
+  }
 
   const int n_blocks_all = N / kRows4;
-  const int blk_first = blockIdx.x * blocks_per_wg;
+  const int blk_first = run * blocks_per_wg;
+  if (kM > 4 && blk_first >= n_blocks_all) return;  // (runs are dealt out in eights)
   const int n_blocks = min(blocks_per_wg, n_blocks_all - blk_first);
   const int blk_last = blk_first + n_blocks - 1;
 
   // the outputs this thread will add up at the end (block, weight row, activation row), and their layer bias:
   // requested now, with everything else, so that nothing is fetched behind the last barrier
-  constexpr int kOuts = (kMaxBlocks4 * kRows4 * 4 + 64 * kWaves - 1) / (64 * kWaves);
+  constexpr int kOuts = (kMaxBlocks4 * kRows4 * (kM > 4 ? kM : 4) + 64 * kWaves - 1) / (64 * kWaves);
   uint16_t out_bias[kOuts];
 #pragma unroll
   for (int i = 0; i < kOuts; ++i) {
@@ -250,9 +260,12 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
         }
       }
     }
+    if (kSlots == 64 || (q >> 1) == h) {
+      const int u = kSlots == 64 ? lane : 2 * j + g;
 #pragma unroll
-    for (int p = 0; p < kPasses; ++p)
-      partials[((slot * kWaves + wave) * kPasses + p) * 64 + lane] = make_float2(acc_a[p] * us_a[p], acc_b[p] * us_b[p]);
+      for (int p = 0; p < kPasses; ++p)
+        partials[((slot * kWaves + wave) * kPasses + p) * kSlots + u] = make_float2(acc_a[p] * us_a[p], acc_b[p] * us_b[p]);
+    }
   };
 
   // Three blocks per trip, one per register set, and between the arithmetic of two blocks the requests for the
@@ -287,10 +300,14 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
     for (int w = 0; w < kWaves; ++w)
 #pragma unroll
       for (int hg = 0; hg < 4; ++hg) {  // half hg / 2, group hg % 2: lane (2 row + half, 2 half + group)
-        const int src = (2 * out_row8 + (hg >> 1)) + 16 * hg;
-        const float2 p = partials[((out_blk * kWaves + w) * kPasses + (out_m >> 1)) * 64 + src];
+        const int src_j = 2 * out_row8 + (hg >> 1);
+        const int src = kSlots == 64 ? src_j + 16 * hg : 2 * src_j + (hg & 1);
+        const float2 p = partials[((out_blk * kWaves + w) * kPasses + (out_m >> 1)) * kSlots + src];
         v += (out_m & 1) ? p.y : p.x;
       }
+    if constexpr (kM > 4) {  // as in the 8-bit kernel: what an infinity or NaN in x makes of y
+      if (v != v) v = oct_plain_dot<T, 4>(x + (size_t)out_m * K, wq, scales, biases, out_row, K);
+    }
     const float bias_v = T::to_f32(out_bias[i]);
     if (y_is_f32) {
       reinterpret_cast<float*>(y)[(int64_t)out_m * N + out_row] = bias ? v + bias_v : v;
@@ -306,26 +323,11 @@ template <typename T, int kWaves, int kSteps, int kM, bool kSilu>
 int launch_oct4(const void* x, int64_t M, const uint32_t* wq, const void* scales, const void* biases, const void* bias,
                 int64_t N, void* y, int y_dtype, hipStream_t stream) {
   auto kernel = qmv_oct4_kernel<T, kWaves, kSteps, kM, kSilu>;
-  constexpr int kPasses = kM > 2 ? 2 : 1;
   constexpr int kImageBytes = ((2 * kM * (256 * kSteps + 32) + kM * 4 * kSteps * 4) + 255) & ~255;
-  constexpr int kPerBlock = kWaves * kPasses * 512;
-  constexpr int kLdsWanted = kWaves * kImageBytes + (kMaxBlocks4 + 1) * kPerBlock;
-  constexpr int kLdsMax = kLdsWanted < 160 * 1024 ? kLdsWanted : 160 * 1024;
+  constexpr int kPerBlock = kWaves * (kM > 4 ? kM / 2 * 256 : kM > 2 ? 1024 : 512);
   static PerDeviceInt configured;
-  if (!raise_lds_limit(configured, reinterpret_cast<const void*>(kernel), kLdsMax)) return MFQ_ELAUNCH;
-  // one workgroup per compute unit while that is at most kMaxBlocks4 blocks each; longer weights in runs of
-  // kLongRun4 blocks to as many workgroups as that takes
-  const int64_t blocks = N / kRows4;
-  const int64_t cus = compute_units();
-  int64_t per_wg = (blocks + cus - 1) / cus;
-  if (per_wg > kMaxBlocks4) per_wg = kLongRun4;
-  while (kWaves * kImageBytes + ((int)per_wg + 1) * kPerBlock > kLdsMax) --per_wg;  // (many wavefronts, four rows)
-  const int64_t n_wg = (blocks + per_wg - 1) / per_wg;
-  const int lds = kWaves * kImageBytes + ((int)per_wg + 1) * kPerBlock;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)n_wg), dim3(64 * kWaves), lds, stream, (const uint16_t*)x, wq,
-                     (const uint16_t*)scales, (const uint16_t*)biases, (const uint16_t*)bias, y,
-                     (int)(y_dtype == MFQ_F32), (int)M, (int)N, (int)per_wg);
-  return hipGetLastError() == hipSuccess ? MFQ_OK : MFQ_ELAUNCH;
+  return launch_oct_runs<kWaves, kM>(kernel, configured, kWaves * kImageBytes, kPerBlock, kRows4, kMaxBlocks4, kLongRun4,
+                                     x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
 }
 
 template <typename T, int kWaves, int kSteps, bool kSilu>
@@ -333,7 +335,10 @@ int launch_oct4_rows(const void* x, int64_t M, const uint32_t* wq, const void* s
                      const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream) {
   if (M == 1) return launch_oct4<T, kWaves, kSteps, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
   if (M == 2) return launch_oct4<T, kWaves, kSteps, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-  return launch_oct4<T, kWaves, kSteps, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  if (M <= 4) return launch_oct4<T, kWaves, kSteps, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  if constexpr (!kSilu)
+    return launch_oct4<T, kWaves, kSteps, 8, false>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  return MFQ_EUNSUPPORTED;
 }
 
 template <typename T, bool kSilu>
@@ -341,22 +346,26 @@ int launch_oct4_k(const void* x, int64_t M, int64_t K, const uint32_t* wq, const
                   const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream) {
   // (K = 3072, twelve steps to a row: six wavefronts of two measured ahead of four of three and twelve of one)
   switch (K) {
+    case 256: return launch_oct4_rows<T, 1, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     case 1024: return launch_oct4_rows<T, 4, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     case 2048: return launch_oct4_rows<T, 8, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 2560: return launch_oct4_rows<T, 5, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     case 3072: return launch_oct4_rows<T, 6, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 3840: return launch_oct4_rows<T, 5, 3, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     case 4096: return launch_oct4_rows<T, 8, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 6144: return launch_oct4_rows<T, 8, 3, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     default: return MFQ_EUNSUPPORTED;
   }
 }
 
 }  // namespace
 
-// Shapes this kernel takes: 4-bit codes in groups of 64, one to four activation rows, K of 1024, 2048, 3072
-// or 4096, whole eights of weight rows, x and the weights 16-byte aligned, scales and biases 4-byte aligned.
+// Shapes this kernel takes: 4-bit codes in groups of 64, up to sixteen activation rows, the K that
+// launch_oct4_k splits, whole eights of weight rows, x and the weights 16-byte aligned, scales and biases
+// 4-byte aligned.
 bool qmv_oct4_covers(int64_t M, int64_t K, int64_t N, int gs, int bits, const void* x, const void* scales,
                      const void* biases) {
-  if (!(bits == 4 && gs == 64 && M >= 1 && M <= 4 && (K == 1024 || K == 2048 || K == 3072 || K == 4096) &&
-        N % kRows4 == 0))
+  if (!(bits == 4 && gs == 64 && oct_takes(M, K, bits) && N % kRows4 == 0))
     return false;
   return aligned16(x) && ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 3u) == 0;
 }

@@ -1,0 +1,91 @@
+// What the two eight-rows matvec kernels (qmv_oct.hip, qmv_oct4.hip) share on the host and off their main path.
+#pragma once
+#include "common.h"
+
+namespace mfq {
+
+// The calls the kernels take: row lengths they are built for, up to sixteen activation rows.  Measured against the
+// kernels that take these calls otherwise (us, stream of launches on cold weights):
+//   one row: K = 1024 .. 4096 in steps of 1024 (11.4 on 3072 -> 18432 at 8 bits); on the other row lengths the
+//     one-row kernel of qmv_dot.hip is level or ahead (2560 -> 15360 at 8 bits 9.1 against 9.7, 3840 -> 23040 at 4 bits
+//     10.1 against 10.9) unless a quarter or more of its KiB-sized loads lies past the row's end (256 -> 15360 at 8 bits
+//     4.6 against 3.5 here, 2560 -> 15360 at 4 bits 7.3 against 6.2);
+//   two to four: everywhere (6144 -> 36864 at 8 bits 63.5 -> 38.6, 256 -> 15360 at 4 bits 10.8 -> 3.9);
+//   five and more, against the kernel that dequantises (qmv.hip): 3072 -> 18432 at 8 bits, five rows 19.5 -> 13.3,
+//     sixteen 37.4 -> 25.4; at 4 bits 23.4 -> 11.2 and 60.2 -> 21.6.  Rows of 256 8-bit codes: that kernel
+//     is ahead up to eight rows (4.8 against 5.7), behind from nine (7.7 against 6.5).
+inline bool oct_takes(int64_t M, int64_t K, int bits) {
+  if (M < 1 || M > 16) return false;
+  const bool even = K == 1024 || K == 2048 || K == 3072 || K == 4096;
+  if (!even && K != 256 && K != 2560 && K != 3840 && K != 6144) return false;
+  if (M == 1) {
+    const int64_t bytes = K * bits / 8, loads = (bytes + 1023) / 1024;
+    return even || 4 * bytes <= 3 * 1024 * loads;
+  }
+  return !(K == 256 && bits == 8 && M > 4 && M <= 8);
+}
+
+// Workgroup -> run of weight rows and first activation row.  With two eights of activation rows the two workgroups
+// of a run are eight apart in the grid, on one XCD and at one time, so the second finds the weights in a cache.
+template <int kM>
+__device__ inline int oct_run_and_first_row(int M, int& run) {
+  if (M <= kM) return 0;
+  const int second = (run >> 3) & 1;
+  run = ((run >> 4) << 3) + (run & 7);
+  return second * kM;
+}
+
+// x . dequant(W[row]) one k after the other on the weights rounded to the 16-bit type: what an output is whose row
+// of x holds an infinity or a NaN, which the integer image cannot.
+template <typename T, int BITS>
+__device__ __attribute__((noinline)) float oct_plain_dot(const uint16_t* x, const uint32_t* wq, const uint16_t* scales,
+                                                         const uint16_t* biases, int64_t row, int K) {
+  constexpr int kPerWord = 32 / BITS;
+  const uint32_t* w = wq + row * (K / kPerWord);
+  float v = 0.f;
+#pragma unroll 1
+  for (int k = 0; k < K; ++k) {
+    const int64_t grp = row * (K / 64) + k / 64;
+    const uint32_t code = (w[k / kPerWord] >> (BITS * (k % kPerWord))) & ((1u << BITS) - 1);
+    const float wv = __builtin_fmaf((float)code, T::to_f32(scales[grp]), T::to_f32(biases[grp]));
+    v = __builtin_fmaf(T::to_f32(x[k]), T::to_f32(T::from_f32(wv)), v);
+  }
+  return v;
+}
+
+// Launches either kernel on contiguous runs of blocks of weight rows.  kM: activation rows of the instantiation.
+template <int kWaves, int kM, typename Kernel>
+int launch_oct_runs(Kernel kernel, PerDeviceInt& configured, int image_bytes, int per_block, int rows, int max_blocks,
+                    int long_run, const void* x, int64_t M, const uint32_t* wq, const void* scales, const void* biases,
+                    const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream) {
+  const int wanted = image_bytes + (max_blocks + 1) * per_block;
+  const int lds_max = wanted < 160 * 1024 ? wanted : 160 * 1024;
+  if (!raise_lds_limit(configured, reinterpret_cast<const void*>(kernel), lds_max)) return MFQ_ELAUNCH;
+  const int64_t blocks = N / rows;
+  // workgroups resident at once: one per compute unit, several where a workgroup is only one or two wavefronts
+  const int64_t places = (int64_t)compute_units() * (kWaves <= 2 ? 8 / kWaves : 1);
+  const int64_t groups = kM > 4 ? (M + kM - 1) / kM : 1;
+  const int64_t fit = (lds_max - image_bytes) / per_block - 1;
+  int64_t per_wg = (blocks * groups + places - 1) / places;
+  if (kM > 4) {
+    // as many equal rounds of workgroups as the room for partial sums asks for
+    const int64_t most = fit < max_blocks ? fit : max_blocks;
+    const int64_t rounds = (per_wg + most - 1) / most;
+    per_wg = (blocks * groups + places * rounds - 1) / (places * rounds);
+  } else {
+    // One workgroup per compute unit while that is at most max_blocks blocks each; longer weights in runs of
+    // long_run blocks to as many workgroups as that takes (several resident per unit: a run's last loads and
+    // its adding-up overlap the next run's first requests).
+    if (per_wg > max_blocks) per_wg = long_run;
+    if (per_wg > fit) per_wg = fit;
+  }
+  int64_t n_wg = (blocks + per_wg - 1) / per_wg;
+  if (groups > 1) n_wg = (n_wg + 7) / 8 * 8 * groups;  // pairs of workgroups, eight runs at a time
+  const int lds = image_bytes + ((int)per_wg + 1) * per_block;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)n_wg), dim3(64 * kWaves), lds, stream, (const uint16_t*)x,
+                     wq, (const uint16_t*)scales, (const uint16_t*)biases, (const uint16_t*)bias, y,
+                     (int)(y_dtype == MFQ_F32), (int)M, (int)N, (int)per_wg);
+  return hipGetLastError() == hipSuccess ? MFQ_OK : MFQ_ELAUNCH;
+}
+
+}  // namespace mfq

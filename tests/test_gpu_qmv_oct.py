@@ -129,3 +129,47 @@ def test_oct_unit_weight_is_exact(oracle):
     xf = o.bf16_bits_to_f32(x).astype(np.float64)
     # 15-bit fixed point of each eighth of a row: 2^-15 of the eighth's largest magnitude
     assert np.all(np.abs(got - xf) <= 2.0 ** -14 * np.abs(xf).max())
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("K", [256, 1024, 2560, 3072, 3840, 4096, 6144])
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+def test_oct_row_lengths_and_eights_of_rows(oracle, K, M, bits):
+    """Every split of K over the wavefronts, one image of eight activation rows
+    and two of them (the second with one row and with eight)."""
+    o = oracle
+    args = _case(o, 64, M, K, 8 * 261, bits)
+    _assert_close(_run(o, *args, bits), _ref(o, *args, bits))
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("N", [8, 8 * 255, 8 * 256 * 11, 8 * 256 * 13 + 8])
+def test_oct_run_lengths_of_eight_rows(oracle, N, bits):
+    """Runs of one block, and past what the partial sums of a workgroup hold (two rounds of workgroups)."""
+    o = oracle
+    args = _case(o, 65, 7, 1024, N, bits)
+    _assert_close(_run(o, *args, bits), _ref(o, *args, bits))
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+def test_oct_infinity_and_nan_stay_in_their_rows(oracle, bits):
+    """More than four rows: an infinity in x gives what the product with the
+    dequantised weights gives (its own sign times the weight's), a NaN gives
+    NaN, and the other rows are what they are without either."""
+    import mflux_amd
+
+    torch.manual_seed(66)
+    M, K, N = 6, 3072, 8 * 40
+    w = (torch.randn(N, K, device="cuda") * 0.02).bfloat16()
+    wq, s, b = mflux_amd.quantize(w, 64, bits)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    clean = mflux_amd.quantized_matmul(x, wq, s, b, group_size=64, bits=bits)
+    x[1, 700] = float("inf")
+    x[4, 3] = float("nan")
+    y = mflux_amd.quantized_matmul(x, wq, s, b, group_size=64, bits=bits)
+    # (in float32: a weight that is zero only after the product's own rounding is not zero to the fma of a matmul)
+    column = mflux_amd.dequantize(wq, s, b, 64, bits, dtype=torch.float32)[:, 700]
+    torch.testing.assert_close(y[1].float(), column * float("inf"), rtol=0, atol=0, equal_nan=True)
+    assert bool(torch.isnan(y[4]).all())
+    keep = [0, 2, 3, 5]
+    assert torch.equal(y[keep], clean[keep])
