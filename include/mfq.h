@@ -333,6 +333,13 @@ int mfq_qmv_silu(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_
                  int group_size, int bits, void* y, int y_dtype, void* stream);
 
 /*
+ * y[i] = x[i] * sigmoid(x[i]), i < n, on 16-bit values, with the sigmoid and the
+ * product each rounded to dtype (the nn.silu in front of mfq_qmm_t for the calls
+ * mfq_qmv_silu does not take).  x and y 16-byte aligned; in place is allowed.
+ */
+int mfq_silu(const void* x, int dtype, int64_t n, void* y, void* stream);
+
+/*
  * A quantized linear layer with LoRA adapters on it in one call:
  *   y = x @ dequantize(wq, scales, biases)^T + t @ bs^T (+ bias).
  * Replaces the body of LoRALinear.__call__

@@ -356,8 +356,9 @@ def silu_quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor
 
     For one to four rows of 16-bit ``x`` against 4- or 8-bit weights the
     activation runs inside the matvec kernel, where the rows are converted
-    anyway (``mfq_qmv_silu``); for any other call it is :func:`silu`, an elementwise
-    pass, in front of :func:`quantized_matmul`.  Both round the sigmoid and the
+    anyway (``mfq_qmv_silu``), for five to sixteen it is one launch in front of it
+    (``mfq_silu``, the values of :func:`silu`); for any other call it is :func:`silu`, an
+    elementwise pass, in front of :func:`quantized_matmul`.  Both round the sigmoid and the
     product to ``x``'s dtype.  Not differentiable in its fused form: with
     gradients enabled on ``x`` or ``bias`` the composed form runs.
     """

@@ -133,13 +133,21 @@ PyObject* silu_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Linear p;
   if (n != 7 || !p.parse(args)) Py_RETURN_NONE;
-  if (p.M > 4 || (p.bits != 4 && p.bits != 8)) Py_RETURN_NONE;
+  if (p.M > 16 || (p.bits != 4 && p.bits != 8)) Py_RETURN_NONE;
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(p.x.device());
-  Tensor y = p.out(p.N);
+  Tensor y = p.out(p.N), s;
+  if (p.M > 4) s = p.out(p.K);  // five rows and more: the activation in a launch of its own
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  rc = mfq_qmv_silu(p.x.data_ptr(), p.dtype, p.M, p.K, p.codes(), p.scales.data_ptr(), p.biases.data_ptr(), p.dtype,
-                    p.bias_ptr(), p.N, (int)p.gs, (int)p.bits, y.data_ptr(), p.dtype, p.stream());
+  if (p.M > 4) {
+    rc = mfq_silu(p.x.data_ptr(), p.dtype, p.M * p.K, s.data_ptr(), p.stream());
+    if (rc == MFQ_OK)
+      rc = mfq_qmm_t(s.data_ptr(), p.dtype, p.M, p.K, p.codes(), p.scales.data_ptr(), p.biases.data_ptr(), p.dtype,
+                     p.bias_ptr(), p.N, (int)p.gs, (int)p.bits, y.data_ptr(), p.dtype, p.stream());
+  } else {
+    rc = mfq_qmv_silu(p.x.data_ptr(), p.dtype, p.M, p.K, p.codes(), p.scales.data_ptr(), p.biases.data_ptr(), p.dtype,
+                      p.bias_ptr(), p.N, (int)p.gs, (int)p.bits, y.data_ptr(), p.dtype, p.stream());
+  }
   Py_END_ALLOW_THREADS
   return result(rc, y);
   END_HANDLE_TH_ERRORS

@@ -223,3 +223,36 @@ def test_modulation_linears_of_several_blocks_as_one_call(oracle):
     for part, ref, layer in zip(parts, alone, layers):
         assert torch.equal(part, ref)
         assert torch.equal(qnn.silu_linear(layer, temb), ref)     # the layers still work, now as views of the bank
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n", [1, 7, 8, 511, 513, 1 << 16])
+def test_silu_pass_is_the_two_operations_bit_for_bit(dtype, n):
+    """mfq_silu against ``x * sigmoid(x)`` as torch's two operations, over all 2^16
+    values and with a last piece that is not whole."""
+    import mflux_amd
+    from mflux_amd import _lib
+
+    x = torch.arange(1 << 16, dtype=torch.int32, device="cuda").to(torch.int16).view(dtype)[-n:].clone()
+    y = torch.full((n + 8,), 7.0, device="cuda", dtype=dtype)
+    code = _lib.BF16 if dtype == torch.bfloat16 else _lib.F16
+    rc = _lib.load().mfq_silu(x.data_ptr(), code, n, y.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    want = mflux_amd.silu(x)
+    nan = torch.isnan(want)
+    assert torch.equal(torch.isnan(y[:n]), nan)
+    assert torch.equal(y[:n].view(torch.int16)[~nan], want.view(torch.int16)[~nan])
+    assert bool((y[n:] == 7).all())
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M", [5, 8, 16])
+def test_silu_matvec_five_rows_and_more_is_the_composition(bits, M):
+    import mflux_amd
+
+    torch.manual_seed(37)
+    w = (torch.randn(520, 2560, device="cuda") * 0.02).bfloat16()
+    packed = mflux_amd.quantize(w, 64, bits)
+    x = torch.randn(M, 2560, device="cuda").bfloat16()
+    y = mflux_amd.silu_quantized_matmul(x, *packed, group_size=64, bits=bits)
+    assert torch.equal(y, mflux_amd.quantized_matmul(mflux_amd.silu(x), *packed, group_size=64, bits=bits))
