@@ -118,6 +118,90 @@ def _packed_for(owner: torch.nn.Module, loras: list[LoRALinear], dtype: torch.dt
     return cache[1]
 
 
+class _LoRALinearFunction(torch.autograd.Function):
+    """``base(x) + scale * (x @ A) @ B`` for training: the update rides in the base
+    GEMM (``low_rank``), where the composition writes and reads the ``[M, N]``
+    product three times more (a rank-16 matmul, the scaling, the add: 65 us of a
+    step of 410 at 1536 rows, 3072 -> 12288), and backward scales the ``[M, R]``
+    product of the gradient instead of the gradient.  One rounding where the
+    composition has four."""
+
+    @staticmethod
+    def forward(ctx, x, lora_a, lora_b, w, scales, biases, bias, scale, group_size, bits):
+        t = torch.matmul(x.reshape(-1, x.shape[-1]), lora_a)
+        ctx.save_for_backward(x, lora_a, lora_b, w, scales, biases, t)
+        ctx.meta = (scale, group_size, bits)
+        bs = lora_b if scale == 1.0 else (scale * lora_b.float()).to(lora_b.dtype)
+        return core.quantized_matmul(x, w, scales, biases, True, group_size, bits, bias=bias,
+                                     low_rank=(_padded(t).reshape(*x.shape[:-1], -1), _padded(bs.t()).contiguous()))
+
+    @staticmethod
+    def backward(ctx, grad_y):
+        x, lora_a, lora_b, w, scales, biases, t = ctx.saved_tensors
+        scale, group_size, bits = ctx.meta
+        x2, g = x.reshape(-1, x.shape[-1]), grad_y.reshape(-1, grad_y.shape[-1])
+        twice = torch.is_grad_enabled()  # create_graph: everything below in operations that differentiate again
+        grad_x = grad_a = grad_b = gt = None
+        if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
+            gt = torch.matmul(g, lora_b.t())
+            if scale != 1.0:
+                gt = scale * gt
+        if ctx.needs_input_grad[1]:
+            grad_a = torch.matmul(x2.t(), gt)
+        if ctx.needs_input_grad[2]:
+            grad_b = torch.matmul((torch.matmul(x2, lora_a) if twice else t).t(), g)
+            if scale != 1.0:
+                grad_b = scale * grad_b
+        if ctx.needs_input_grad[0]:
+            grad_x = core._matmul_untransposed(grad_y, w, scales, biases, group_size, bits)
+            if twice:
+                grad_x = grad_x + torch.matmul(gt, lora_a.t()).reshape(grad_x.shape)
+            else:
+                _lib.ops().low_rank_add_(grad_x.view(x2.shape), _padded(gt).contiguous(), _padded(lora_a).contiguous())
+        return grad_x, grad_a, grad_b, None, None, None, None, None, None, None
+
+
+def _padded(t: torch.Tensor) -> torch.Tensor:
+    """Zero columns up to a multiple of the step the kernels take the rank in."""
+    pad = -t.shape[1] % _RANK_STEP
+    return torch.nn.functional.pad(t, (0, pad)) if pad else t
+
+
+_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+_GLOBAL_HOOKS = ("_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks",
+                 "_global_backward_pre_hooks")
+
+
+def _trains_in_one(base: torch.nn.Module, lora: LoRALinear, x: torch.Tensor) -> bool:
+    """Whether a call with gradients is what ``_LoRALinearFunction`` computes: plain
+    16-bit HIP tensors of one type against a plain ``QuantizedLinear`` whose own
+    call nobody watches (hooks) or replaces, with more than 16 rows (below them the
+    update is a launch of its own anyway), and none of the transforms that need
+    the composition's own operations (tracing, functorch, forward mode, autocast)."""
+    if type(base) is not QuantizedLinear or base.mode != "affine" or base.__dict__.get("_prepared") is not None:
+        return False
+    if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.device == x.device and t.dtype == x.dtype
+               for t in (x, lora.lora_A, lora.lora_B, base.scales, base.biases)):
+        return False
+    if x.dtype not in (torch.bfloat16, torch.float16) or type(lora.scale) not in (int, float):
+        return False
+    K, N, rank = base.input_dims, base.output_dims, lora.lora_A.shape[-1]
+    if (x.shape[-1:] != (K,) or x.numel() <= 16 * K or lora.lora_A.shape != (K, rank) or lora.lora_B.shape != (rank, N)
+            or not 1 <= rank <= 1024 or base.weight.ndim != 2 or base.weight.device != x.device):
+        return False
+    if base.bias is not None and (base.bias.requires_grad or base.bias.dtype != x.dtype or base.bias.device != x.device):
+        return False
+    if base.scales.requires_grad or base.biases.requires_grad:
+        return False
+    if "forward" in base.__dict__ or any(getattr(base, h) for h in _HOOKS):
+        return False
+    if any(getattr(torch.nn.modules.module, h, None) for h in _GLOBAL_HOOKS):
+        return False
+    return not (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
 def _forward(owner: torch.nn.Module, base: torch.nn.Module, loras: list[LoRALinear], x: torch.Tensor) -> torch.Tensor:
     if not loras:
         return base(x)
@@ -127,6 +211,10 @@ def _forward(owner: torch.nn.Module, base: torch.nn.Module, loras: list[LoRALine
     fused = (isinstance(base, QuantizedLinear) and x.is_cuda and not needs_grad and rank <= 1024
              and base.scales.dtype in (torch.bfloat16, torch.float16) and x.numel() > 0)
     if not fused:
+        if needs_grad and len(loras) == 1 and _trains_in_one(base, loras[0], x):
+            lora = loras[0]
+            return _LoRALinearFunction.apply(x, lora.lora_A, lora.lora_B, base.weight, base.scales, base.biases, base.bias,
+                                             float(lora.scale), base.group_size, base.bits)
         return _composed(base, loras, x)
     compute = base.scales.dtype
     a_cat, af, bs = _packed_for(owner, loras, compute)

@@ -318,3 +318,69 @@ def test_bake_with_requantize_folds_the_adapters_into_the_codes(bits):
         baked = q(x).double()
     err = (baked - wrapped).abs().max() / wrapped.abs().max()
     assert err < (0.15 if bits == 4 else 0.02)
+
+
+@pytest.mark.parametrize("M,K,N,rank,bits,scale", [
+    (17, 256, 192, 4, 4, 1.0), (300, 512, 768, 16, 8, 0.5), (130, 1024, 520, 24, 6, -2.0), (1100, 3072, 256, 8, 4, 1.0)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_training_step_against_float64(M, K, N, rank, bits, scale, bias):
+    """Output and gradients of a trainable adapter on a quantized base: ranks that
+    are padded, either side of the row counts where the base GEMMs change, odd
+    bits, scales other than one.  Every result is rounded to bfloat16 once or
+    twice (2^-9 each) on sums of products of rounded factors: 1e-2 of its norm."""
+    import mflux_amd
+    from mflux_amd import lora, nn
+
+    torch.manual_seed(91)
+    lin = torch.nn.Linear(K, N, bias=bias, device="cuda", dtype=torch.bfloat16)
+    layer = lora.LoRALinear.from_linear(nn.QuantizedLinear.from_linear(lin, 64, bits), r=rank, scale=scale)
+    layer.lora_B.data.normal_(std=0.02)
+    x = torch.randn(2, (M + 1) // 2, K, device="cuda").bfloat16().requires_grad_(True)
+    g = torch.randn(*x.shape[:-1], N, device="cuda").bfloat16()
+    assert lora._trains_in_one(layer.linear, layer, x)
+    got = [layer(x)]
+    got += torch.autograd.grad(got[0], (x, layer.lora_A, layer.lora_B), g)
+    q = layer.linear
+    w = mflux_amd.dequantize(q.weight, q.scales, q.biases, 64, bits, dtype=torch.float32).double()
+    x64, a64, b64 = (t.detach().double().requires_grad_(True) for t in (x, layer.lora_A, layer.lora_B))
+    y64 = x64 @ w.t() + scale * ((x64 @ a64) @ b64) + (q.bias.double() if bias else 0)
+    want = [y64, *torch.autograd.grad(y64, (x64, a64, b64), g.double())]
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and a.dtype == torch.bfloat16
+        assert float((a.detach().double() - b.detach()).norm() / b.detach().norm()) < 1e-2
+
+
+def test_training_calls_that_keep_the_composition():
+    """Hooks on the base, autocast, forward mode, a transform, few rows, another
+    adapter type: the composition, which serves them; and a second derivative of
+    the one-call form is the composition's."""
+    from mflux_amd import lora, nn
+
+    torch.manual_seed(92)
+    lin = torch.nn.Linear(256, 128, device="cuda", dtype=torch.bfloat16)
+    layer = lora.LoRALinear.from_linear(nn.QuantizedLinear.from_linear(lin, 64, 8), r=16, scale=0.5)
+    layer.lora_B.data.normal_(std=0.02)
+    x = torch.randn(64, 256, device="cuda").bfloat16().requires_grad_(True)
+    takes = lambda v=x: lora._trains_in_one(layer.linear, layer, v)
+    assert takes() and not takes(x[:16]) and not takes(x.float())
+    seen = []
+    handle = layer.linear.register_forward_hook(lambda m, i, o: seen.append(o))
+    assert not takes()
+    layer(x)
+    assert len(seen) == 1
+    handle.remove()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not takes()
+    with torch.autograd.forward_ad.dual_level():
+        assert not takes()
+    inside = []
+    torch.func.vmap(lambda v: inside.append(takes()) or v)(torch.zeros(2, device="cuda"))
+    assert inside == [False] and takes()
+
+    def second(y):
+        (ga,) = torch.autograd.grad(y.float().square().sum(), layer.lora_A, create_graph=True)
+        return torch.autograd.grad(ga.float().square().sum(), (layer.lora_A, layer.lora_B))
+
+    # (the base takes no part in a second derivative: neither form differentiates its untransposed product)
+    for a, b in zip(second(layer(x)), second(lora._composed(layer.linear, [layer], x))):
+        assert float((a.double() - b.double()).norm() / b.double().norm()) < 3e-2
