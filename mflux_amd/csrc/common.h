@@ -409,6 +409,8 @@ int launch_qmm_mid(const void* x, int dtype, int64_t M, int64_t K, const uint32_
                    const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
                    void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank = LowRank(),
                    Epilogue epi = Epilogue());
+// what launch_qmm_mid is estimated to take (groups of 64)
+float qmm_mid_estimate_us(int64_t M, int64_t N, int64_t K);
 size_t qmm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs);
 // the same kernel for 3, 5 and 6 bits (any M above one row; K % 32 == 0)
 int launch_qmm_mid_stream(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,

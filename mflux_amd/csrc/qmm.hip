@@ -1125,10 +1125,25 @@ int launch_qmm_epilogue(const void* x, int dtype, int64_t M, int64_t K, const ui
 #else
 // Shapes whose 256 x 256 tiles would leave more than half of the compute units
 // idle go to the 128-column-tile kernel, except many rows against a long K,
-// where cutting K between 256 x 256 tiles measures about a tenth faster.
+// where cutting K between 256 x 256 tiles measures about a tenth faster -- unless
+// that cut still leaves half of the units idle (it needs equal ranges: 600 rows x
+// 18944 -> 3584 196 us, 132 on the other kernel).  Below 1024 rows a shape with
+// more tiles goes there too where its rows fill 128-row tiles and rounds of
+// workgroups much better: 320 rows x 3584 -> 37888 150 us on 296 tiles of 256 x 256
+// (one round and 40 tiles cut in two), 129 on 888 of 128 x 128; 600 rows x 3072 ->
+// 12288 70 against 62.  The estimate of this kernel: 1.68 us per k step and round.
 bool use_mid_kernel(int64_t M, int64_t N, int64_t K) {
-  const bool few_tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * 2 <= compute_units();
-  return few_tiles && !(M > 512 && K >= 8192);
+  const int64_t cus = compute_units();
+  const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  if (tiles * 2 <= cus) {
+    if (!(M > 512 && K >= 8192)) return true;
+    return M < 1024 && K % BK == 0 && N * K < (int64_t)1 << 31 && tiles * plan_tail(M, N, K, period_of(64), (int)cus).splits * 2 < cus;
+  }
+  if (M >= 1024 || M * K >= (int64_t)1 << 31 || N * K >= (int64_t)1 << 31) return false;  // (what that kernel addresses)
+  const float step_us = 1.68f * (float)((K + BK - 1) / BK);
+  const int64_t rest = tiles % cus;
+  const float tail = rest == 0 ? 0.f : rest * 2 > cus ? step_us : 0.5f * step_us + 10.f;
+  return qmm_mid_estimate_us(M, N, K) < 0.9f * (step_us * (float)(tiles / cus) + tail);
 }
 
 #ifndef MFQ_ODD_FRAG_ROWS

@@ -66,7 +66,7 @@ template <typename T, int GS, int BITS, bool kFast, int kWavesM>
 __global__ __launch_bounds__(threads_of(kWavesM), 2) void qmm_mid_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
     const uint16_t* __restrict__ biases, const uint16_t* __restrict__ bias, void* __restrict__ y, int y_is_f32, int M,
-    int N, int K, int tiles_m, int tiles_n, int steps, const uint16_t* __restrict__ lr_t,
+    int N, int K, int tiles_m, int tiles_n, int base_steps, int n_long, const uint16_t* __restrict__ lr_t,
     const uint16_t* __restrict__ lr_bs, int lr_rank, Epilogue epi) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   using vec8 = typename T::vec8;
@@ -102,7 +102,9 @@ __global__ __launch_bounds__(threads_of(kWavesM), 2) void qmm_mid_kernel(
   }
   const int m0 = (tile % tiles_m) * TM;
   const int n0 = (tile / tiles_m) * TN;
-  const int kb = split * steps * TK;  // first k of the item
+  // the first n_long k ranges are one scale period longer than the others
+  const int steps = base_steps + (split < n_long ? kPer : 0);
+  const int kb = (split * base_steps + min(split, n_long) * kPer) * TK;  // first k of the item
   char* y_item = static_cast<char*>(y) + (size_t)split * M * N * 4;  // split > 0 only with float32 planes
 
   // global offsets (bytes; they fit 32 bits, checked by the launcher)
@@ -352,30 +354,45 @@ __global__ __launch_bounds__(threads_of(kWavesM), 2) void qmm_mid_kernel(
 
 struct MidPlan {
   int splits;
-  int steps;  // k steps per range
+  int steps;   // k steps per range
+  int n_long;  // the first n_long ranges are one scale period longer
+  int waves_m;
+  float us;    // what the call is estimated to take
 };
 
 inline int period_of(int gs) { return 4 * gs / TK; }
 
-// Up to 128 activation rows: 128-row tiles, two workgroups of four wavefronts
-// per compute unit.  More: 256-row tiles (every dequantised weight then serves
-// twice the matrix work), one workgroup of eight wavefronts per compute unit.
-inline int waves_m_of(int64_t M) { return M <= 128 ? 2 : 4; }
-
-// K is cut into equal ranges of whole scale periods (at least 8 k steps each)
-// while the work items are fewer than the compute units and the cut keeps them
-// within what runs at once.
-inline MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int period, int cus) {
+// Tile height and K cut by estimated time.  K is cut into ranges of whole scale periods, at least 8 k steps each and
+// equal to within one period (ranges of exactly equal length left K = 18944, 37 x 8 steps, at two ranges for 56 tiles:
+// 320 rows x 18944 -> 3584 took 116 us with 112 of 256 compute units at work), as long as all items run at once.
+// Measured per k step: 0.87 us for a 256-row tile (one workgroup of eight wavefronts per compute unit); for 128-row tiles
+// 0.62 us with one to a unit and 1.1 with two (the same matrix work as one 256-row tile, every code dequantised
+// twice).  128-row tiles win where they fill rounds that 256-row ones leave half empty (320 rows, 2560 -> 4096: 96
+// tiles x 5 ranges against 64 x 2).  A cut costs a launch and its float32 planes, written at 5 and read at 7 bytes/ps.
+inline MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int period, int cus, bool may_cut = true) {
   const int steps = (int)((K + TK - 1) / TK);  // K % 64 == 32: the last step is half empty
-  const int waves_m = waves_m_of(M);
-  const int tm = tile_m(waves_m);
-  const int64_t tiles = ((M + tm - 1) / tm) * ((N + TN - 1) / TN);
-  const int64_t slots = waves_m == 2 ? 2 * (int64_t)cus : cus;
-  MidPlan plan{1, steps};
-  if (K % TK || steps % period != 0) return plan;
-  for (int s = 2; s <= steps / 8 && tiles * plan.splits < cus && tiles * s <= slots; ++s)
-    if (steps % s == 0 && (steps / s) % period == 0) plan = MidPlan{s, steps / s};
-  return plan;
+  if (K % TK || steps % period != 0) may_cut = false;
+  const int periods = steps / period;
+  const float plane_us = (float)M * (float)N * 4.f * (1.f / 5e6f + 1.f / 7e6f);
+  MidPlan best{0, 0, 0, 0, 0.f};
+  for (const int waves_m : {4, 2}) {
+    if (M <= 128 && waves_m == 4) continue;
+    const int64_t tiles = ((M + tile_m(waves_m) - 1) / tile_m(waves_m)) * ((N + TN - 1) / TN);
+    const int64_t slots = waves_m == 2 ? 2 * (int64_t)cus : cus;
+    for (int s = 1; s == 1 || (may_cut && tiles * s <= slots && (periods / s) * period >= 8); ++s) {
+      const int64_t items = tiles * s, rest = items % slots;
+      const int longest = s == 1 ? steps : (periods + s - 1) / s * period;
+      const float full = waves_m == 2 ? 1.1f : 0.87f;
+      const float last = rest == 0 ? 0.f : (waves_m == 2 && rest <= cus) ? 0.62f : full;
+      float us = (float)longest * (full * (float)(items / slots) + last);
+      if (s > 1) us += 2.5f + (float)s * plane_us;
+      // (the estimate is good to some 5 %: the higher tile, and the coarser cut, unless it is further off)
+      if (best.splits == 0 || us < (best.waves_m == waves_m ? 0.98f : 0.95f) * best.us)
+        best = s == 1 ? MidPlan{1, steps, 0, waves_m, us}
+                      : MidPlan{s, periods / s * period, periods % s, waves_m, us};
+    }
+  }
+  return best;
 }
 
 template <typename T, int GS, int BITS, bool kFast, int kWavesM>
@@ -392,7 +409,7 @@ int launch_kernel(const void* x, int64_t M, int64_t K, const uint32_t* wq, const
   hipLaunchKernelGGL(kernel, dim3((unsigned)n_items), dim3(threads_of(kWavesM)), kLds, stream, (const uint16_t*)x, wq,
                      (const uint16_t*)scales, (const uint16_t*)biases, (const uint16_t*)bias, y,
                      (int)(y_dtype == MFQ_F32), (int)M, (int)N, (int)K, tiles_m, tiles_n, plan.steps,
-                     (const uint16_t*)lr.t, (const uint16_t*)lr.bs, lr.R, epi);
+                     plan.n_long, (const uint16_t*)lr.t, (const uint16_t*)lr.bs, lr.R, epi);
   return hipGetLastError() == hipSuccess ? MFQ_OK : MFQ_ELAUNCH;
 }
 
@@ -400,7 +417,7 @@ template <typename T, int GS, int BITS, bool kFast>
 int launch_tile(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* scales, const void* biases,
                 const void* bias, int64_t N, void* y, int y_dtype, MidPlan plan, hipStream_t stream, LowRank lr,
                 Epilogue epi) {
-  if (waves_m_of(M) == 2)
+  if (plan.waves_m == 2)
     return launch_kernel<T, GS, BITS, kFast, 2>(x, M, K, wq, scales, biases, bias, N, y, y_dtype, plan, stream, lr, epi);
   return launch_kernel<T, GS, BITS, kFast, 4>(x, M, K, wq, scales, biases, bias, N, y, y_dtype, plan, stream, lr, epi);
 }
@@ -412,14 +429,13 @@ int launch_one(const void* x, int64_t M, int64_t K, const uint32_t* wq, const vo
   const int64_t steps = (K + TK - 1) / TK;
   constexpr int kPer = 4 * GS / TK;
   const bool aligned8 = ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 7u) == 0;
+  const MidPlan whole = plan_mid(M, N, K, kPer, compute_units(), false);
   if (!(K % TK == 0 && steps % kPer == 0 && aligned8))
-    return launch_tile<T, GS, BITS, false>(x, M, K, wq, scales, biases, bias, N, y, y_dtype, MidPlan{1, (int)steps},
-                                           stream, lr, epi);
+    return launch_tile<T, GS, BITS, false>(x, M, K, wq, scales, biases, bias, N, y, y_dtype, whole, stream, lr, epi);
   const MidPlan plan = plan_mid(M, N, K, kPer, compute_units());
   const size_t need = (size_t)plan.splits * M * N * sizeof(float);
   if (plan.splits == 1 || !workspace || workspace_bytes < need || !aligned16(workspace))
-    return launch_tile<T, GS, BITS, true>(x, M, K, wq, scales, biases, bias, N, y, y_dtype, MidPlan{1, (int)steps},
-                                          stream, lr, epi);
+    return launch_tile<T, GS, BITS, true>(x, M, K, wq, scales, biases, bias, N, y, y_dtype, whole, stream, lr, epi);
   // K cut into ranges: float32 planes, and the second kernel applies bias and epilogue
   if (int rc = launch_tile<T, GS, BITS, true>(x, M, K, wq, scales, biases, nullptr, N, workspace, MFQ_F32, plan,
                                               stream, lr, Epilogue()))
@@ -473,6 +489,8 @@ size_t qmm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs) {
   const MidPlan plan = plan_mid(M, N, K, period_of(gs), compute_units());
   return plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
 }
+
+float qmm_mid_estimate_us(int64_t M, int64_t N, int64_t K) { return plan_mid(M, N, K, period_of(64), compute_units()).us; }
 
 int launch_qmm_mid(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                    const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
