@@ -364,16 +364,17 @@ inline int period_of(int gs) { return 4 * gs / TK; }
 
 // Tile height and K cut by estimated time.  K is cut into ranges of whole scale periods, at least 8 k steps each and
 // equal to within one period (ranges of exactly equal length left K = 18944, 37 x 8 steps, at two ranges for 56 tiles:
-// 320 rows x 18944 -> 3584 took 116 us with 112 of 256 compute units at work), as long as all items run at once.
+// 256 rows x 18944 -> 3584 took 116 us with 56 of 256 compute units at work, now 52), as long as all items run at once.
 // Measured per k step: 0.87 us for a 256-row tile (one workgroup of eight wavefronts per compute unit); for 128-row tiles
-// 0.62 us with one to a unit and 1.1 with two (the same matrix work as one 256-row tile, every code dequantised
+// 0.62-0.70 us with one to a unit and 1.1 with two (the same matrix work as one 256-row tile, every code dequantised
 // twice).  128-row tiles win where they fill rounds that 256-row ones leave half empty (320 rows, 2560 -> 4096: 96
-// tiles x 5 ranges against 64 x 2).  A cut costs a launch and its float32 planes, written at 5 and read at 7 bytes/ps.
+// tiles x 5 ranges against 64 x 2).  A cut costs a launch and its float32 planes, written at 4 and read at 6
+// bytes/ps (with less, 512 rows x 3840 -> 3840 took four ranges at 32.6 us instead of three at 30.2).
 inline MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int period, int cus, bool may_cut = true) {
   const int steps = (int)((K + TK - 1) / TK);  // K % 64 == 32: the last step is half empty
   if (K % TK || steps % period != 0) may_cut = false;
   const int periods = steps / period;
-  const float plane_us = (float)M * (float)N * 4.f * (1.f / 5e6f + 1.f / 7e6f);
+  const float plane_us = (float)M * (float)N * 4.f * (1.f / 4e6f + 1.f / 6e6f);
   MidPlan best{0, 0, 0, 0, 0.f};
   for (const int waves_m : {4, 2}) {
     if (M <= 128 && waves_m == 4) continue;
@@ -383,11 +384,11 @@ inline MidPlan plan_mid(int64_t M, int64_t N, int64_t K, int period, int cus, bo
       const int64_t items = tiles * s, rest = items % slots;
       const int longest = s == 1 ? steps : (periods + s - 1) / s * period;
       const float full = waves_m == 2 ? 1.1f : 0.87f;
-      const float last = rest == 0 ? 0.f : (waves_m == 2 && rest <= cus) ? 0.62f : full;
+      const float last = rest == 0 ? 0.f : (waves_m == 2 && rest <= cus) ? 0.68f : full;
       float us = (float)longest * (full * (float)(items / slots) + last);
       if (s > 1) us += 2.5f + (float)s * plane_us;
-      // (the estimate is good to some 5 %: the higher tile, and the coarser cut, unless it is further off)
-      if (best.splits == 0 || us < (best.waves_m == waves_m ? 0.98f : 0.95f) * best.us)
+      // (the estimate is good to some 5 to 8 %: the higher tile, and the coarser cut, unless it is further off)
+      if (best.splits == 0 || us < (best.waves_m == waves_m ? 0.98f : 0.92f) * best.us)
         best = s == 1 ? MidPlan{1, steps, 0, waves_m, us}
                       : MidPlan{s, periods / s * period, periods % s, waves_m, us};
     }
