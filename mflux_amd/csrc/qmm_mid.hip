@@ -94,7 +94,7 @@ __global__ __launch_bounds__(threads_of(kWavesM), 2) void qmm_mid_kernel(
   // XCDs; item b is mapped so that an XCD walks a contiguous run of the tile
   // sequence (tile row fastest), sharing x tiles and weight tiles in its L2.
   const int n_tiles = tiles_m * tiles_n;
-  const int split = blockIdx.x / n_tiles;
+  const int split = __builtin_amdgcn_readfirstlane((int)blockIdx.x / n_tiles);  // in a scalar: the step counts follow from it
   int tile = blockIdx.x - split * n_tiles;
   {
     const int per_xcd = n_tiles / 8;
