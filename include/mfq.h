@@ -131,14 +131,16 @@ int mfq_dequantize_rows(const uint32_t* wq, const void* scales, const void* bias
  * GEMM kernels (128-column tiles while 256 x 256 tiles would leave more than
  * half of the compute units idle, 256 x 256 tiles otherwise).  3, 5 and 6 bits:
  * one activation row of up to 8192 elements has its own kernel, everything
- * else runs on the 128-column-tile GEMM.  For M > 4 the
+ * else runs on the 128-column-tile GEMM.  For M > 16 the
  * dequantised weights are rounded once to x_dtype and sums are float32.  For
- * M <= 4 (4 and 8 bits; shapes the integer kernels take) every row of x
+ * M <= 16 (4 and 8 bits; shapes the integer kernels take) every row of x
  * becomes 15-bit fixed point (one power of two per row brings its largest
  * magnitude under 2^14: an error of 2^-15 of that magnitude per element, exact
  * for small integers and one-hot rows), the integer products with the raw
  * codes are exact, and scale and bias are applied to their sums in float32; an
- * infinity or NaN in a row of x makes every output of that row NaN.
+ * infinity or NaN in a row of x makes every output of that row NaN for
+ * M = 1 and, at K of 1024 to 4096 in steps of 1024, for M <= 4, and gives
+ * what the dequantised weights give for the others.
  */
 int mfq_qmm_t(const void* x, int x_dtype, int64_t M, int64_t K,
               const uint32_t* wq, const void* scales, const void* biases,

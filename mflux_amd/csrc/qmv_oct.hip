@@ -307,10 +307,10 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
         const float2 p = partials[((out_blk * kWaves + w) * kPasses + (out_m >> 2)) * kSlots + src];
         v += (out_m & 1) ? p.y : p.x;
       }
-    // more than four rows: an infinity in x is an infinity of the weight's sign in y, as the kernel that
-    // dequantises gives it (the rows that meet no infinity or NaN never come here)
-    if constexpr (kM > 4) {
-      if (v != v) v = oct_plain_dot<T, 8>(x + (size_t)out_m * K, wq, scales, biases, out_row, K);
+    // an infinity in x is an infinity of the weight's sign in y, as the kernels that dequantise give it (the rows
+    // that meet no infinity or NaN never come here)
+    if constexpr (oct_keeps_infinities(kM, K, 8)) {
+      if (v != v) v = oct_plain_dot<T, 8, kSilu>(x + (size_t)out_m * K, wq, scales, biases, out_row, K);
     }
     const float bias_v = T::to_f32(out_bias[i]);
     if (y_is_f32) {

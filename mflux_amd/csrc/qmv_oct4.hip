@@ -305,8 +305,8 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
         const float2 p = partials[((out_blk * kWaves + w) * kPasses + (out_m >> 1)) * kSlots + src];
         v += (out_m & 1) ? p.y : p.x;
       }
-    if constexpr (kM > 4) {  // as in the 8-bit kernel: what an infinity or NaN in x makes of y
-      if (v != v) v = oct_plain_dot<T, 4>(x + (size_t)out_m * K, wq, scales, biases, out_row, K);
+    if constexpr (oct_keeps_infinities(kM, K, 4)) {  // as in the 8-bit kernel: what an infinity or NaN in x makes of y
+      if (v != v) v = oct_plain_dot<T, 4, kSilu>(x + (size_t)out_m * K, wq, scales, biases, out_row, K);
     }
     const float bias_v = T::to_f32(out_bias[i]);
     if (y_is_f32) {

@@ -37,7 +37,7 @@ __device__ inline int oct_run_and_first_row(int M, int& run) {
 
 // x . dequant(W[row]) one k after the other on the weights rounded to the 16-bit type: what an output is whose row
 // of x holds an infinity or a NaN, which the integer image cannot.
-template <typename T, int BITS>
+template <typename T, int BITS, bool kSilu>
 __device__ __attribute__((noinline)) float oct_plain_dot(const uint16_t* x, const uint32_t* wq, const uint16_t* scales,
                                                          const uint16_t* biases, int64_t row, int K) {
   constexpr int kPerWord = 32 / BITS;
@@ -48,9 +48,16 @@ __device__ __attribute__((noinline)) float oct_plain_dot(const uint16_t* x, cons
     const int64_t grp = row * (K / 64) + k / 64;
     const uint32_t code = (w[k / kPerWord] >> (BITS * (k % kPerWord))) & ((1u << BITS) - 1);
     const float wv = __builtin_fmaf((float)code, T::to_f32(scales[grp]), T::to_f32(biases[grp]));
-    v = __builtin_fmaf(T::to_f32(x[k]), T::to_f32(T::from_f32(wv)), v);
+    const uint16_t xv = kSilu ? (uint16_t)silu_pair<T>(x[k]) : x[k];
+    v = __builtin_fmaf(T::to_f32(xv), T::to_f32(T::from_f32(wv)), v);
   }
   return v;
+}
+
+// Which instantiations do so: the calls that came from kernels on dequantised weights (more than four rows; two to
+// four on row lengths the four-rows kernel does not take).  The others' rows become NaN, as the integer kernels' do.
+constexpr bool oct_keeps_infinities(int m, int K, int bits) {
+  return m > 4 || (m > 1 && (K % 1024 != 0 || K > 4096) && !(bits == 8 && K == 256));
 }
 
 // Launches either kernel on contiguous runs of blocks of weight rows.  kM: activation rows of the instantiation.

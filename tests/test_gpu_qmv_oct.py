@@ -173,3 +173,22 @@ def test_oct_infinity_and_nan_stay_in_their_rows(oracle, bits):
     assert bool(torch.isnan(y[4]).all())
     keep = [0, 2, 3, 5]
     assert torch.equal(y[keep], clean[keep])
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("K", [2560, 3840, 6144])
+@pytest.mark.parametrize("silu", [False, True])
+def test_oct_infinity_of_two_rows_on_the_other_row_lengths(oracle, K, bits, silu):
+    """Two to four rows on row lengths that are no multiple of 1024, or above 4096: the same."""
+    import mflux_amd
+
+    torch.manual_seed(67)
+    w = (torch.randn(8 * 20, K, device="cuda") * 0.02).bfloat16()
+    wq, s, b = mflux_amd.quantize(w, 64, bits)
+    x = torch.randn(3, K, device="cuda").bfloat16()
+    x[1, 600] = float("inf")
+    f = mflux_amd.silu_quantized_matmul if silu else mflux_amd.quantized_matmul
+    y = f(x, wq, s, b, group_size=64, bits=bits)
+    column = mflux_amd.dequantize(wq, s, b, 64, bits, dtype=torch.float32)[:, 600]
+    torch.testing.assert_close(y[1].float(), column * float("inf"), rtol=0, atol=0, equal_nan=True)
+    assert bool(torch.isfinite(y[[0, 2]]).all())
