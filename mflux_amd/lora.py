@@ -122,9 +122,9 @@ class _LoRALinearFunction(torch.autograd.Function):
     """``base(x) + scale * (x @ A) @ B`` for training: the update rides in the base
     GEMM (``low_rank``), where the composition writes and reads the ``[M, N]``
     product three times more (a rank-16 matmul, the scaling, the add: 65 us of a
-    step of 410 at 1536 rows, 3072 -> 12288), and backward scales the ``[M, R]``
-    product of the gradient instead of the gradient.  One rounding where the
-    composition has four."""
+    step of 410 at 1536 rows, 3072 -> 12288), and backward in bfloat16 scales the
+    ``[M, R]`` product of the gradient instead of the gradient.  One rounding where
+    the composition has four."""
 
     @staticmethod
     def forward(ctx, x, lora_a, lora_b, w, scales, biases, bias, scale, group_size, bits):
@@ -141,6 +141,11 @@ class _LoRALinearFunction(torch.autograd.Function):
         scale, group_size, bits = ctx.meta
         x2, g = x.reshape(-1, x.shape[-1]), grad_y.reshape(-1, grad_y.shape[-1])
         twice = torch.is_grad_enabled()  # create_graph: everything below in operations that differentiate again
+        # float16: the gradient is scaled before anything is summed over it, as the composition does.  A product of the
+        # unscaled one leaves the type's range at 65504 |scale| of the true gradient, and a scaled-down lora_B of a
+        # young adapter its normal numbers; bfloat16 has float32's range, and the [M, R] products are scaled instead.
+        if scale != 1.0 and g.dtype == torch.float16:
+            g, scale = scale * g, 1.0
         grad_x = grad_a = grad_b = gt = None
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
             gt = torch.matmul(g, lora_b.t())

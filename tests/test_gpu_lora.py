@@ -350,6 +350,31 @@ def test_training_step_against_float64(M, K, N, rank, bits, scale, bias):
         assert float((a.detach().double() - b.detach()).norm() / b.detach().norm()) < 1e-2
 
 
+@pytest.mark.parametrize("scale", [0.05, 8.0])
+def test_float16_training_gradients_are_finite_where_the_composition_is(scale):
+    """Loss-scaled float16 training runs its gradients near 65504: the sums over a
+    gradient must hold the scale already, as in the composition.  3000 sqrt(1536)
+    |t| passes 65504 for scale 0.05 before the scale is applied and is 20 times
+    smaller after it.  Tolerance: both forms round the same float16 products, in
+    another order (2^-11 each, four of them)."""
+    from mflux_amd import lora, nn
+
+    torch.manual_seed(93)
+    lin = torch.nn.Linear(512, 512, bias=False, device="cuda", dtype=torch.float16)
+    layer = lora.LoRALinear.from_linear(nn.QuantizedLinear.from_linear(lin, 64, 4), r=16, scale=scale)
+    layer.lora_A.data.normal_(std=0.02)
+    layer.lora_B.data.normal_(std=0.02)
+    x = torch.randn(1536, 512, device="cuda").half().requires_grad_(True)
+    g = torch.randn(1536, 512, device="cuda").mul_(3000 if scale < 1 else 20).half()
+    assert lora._trains_in_one(layer.linear, layer, x)
+    inputs = (x, layer.lora_A, layer.lora_B)
+    got = torch.autograd.grad(layer(x), inputs, g)
+    want = torch.autograd.grad(lora._composed(layer.linear, [layer], x), inputs, g)
+    for a, b in zip(got, want):
+        assert bool(torch.isfinite(b).all()) and bool(torch.isfinite(a).all())
+        assert float((a.double() - b.double()).norm() / b.double().norm()) < 4 * 2.0 ** -11
+
+
 def test_training_calls_that_keep_the_composition():
     """Hooks on the base, autocast, forward mode, a transform, few rows, another
     adapter type: the composition, which serves them; and a second derivative of
