@@ -133,7 +133,7 @@ class _LoRALinearFunction(torch.autograd.Function):
         ctx.meta = (scale, group_size, bits)
         bs = lora_b if scale == 1.0 else (scale * lora_b.float()).to(lora_b.dtype)
         return core.quantized_matmul(x, w, scales, biases, True, group_size, bits, bias=bias,
-                                     low_rank=(_padded(t).reshape(*x.shape[:-1], -1), _padded(bs.t()).contiguous()))
+                                     low_rank=(_operand(t).reshape(*x.shape[:-1], -1), _operand(bs.t())))
 
     @staticmethod
     def backward(ctx, grad_y):
@@ -162,14 +162,17 @@ class _LoRALinearFunction(torch.autograd.Function):
             if twice:
                 grad_x = grad_x + torch.matmul(gt, lora_a.t()).reshape(grad_x.shape)
             else:
-                _lib.ops().low_rank_add_(grad_x.view(x2.shape), _padded(gt).contiguous(), _padded(lora_a).contiguous())
+                _lib.ops().low_rank_add_(grad_x.view(x2.shape), _operand(gt), _operand(lora_a))
         return grad_x, grad_a, grad_b, None, None, None, None, None, None, None
 
 
-def _padded(t: torch.Tensor) -> torch.Tensor:
-    """Zero columns up to a multiple of the step the kernels take the rank in."""
+def _operand(t: torch.Tensor) -> torch.Tensor:
+    """A factor as the kernels take it: zero columns up to a multiple of the step
+    they take the rank in, contiguous, 16-byte aligned (a parameter may be a view
+    of a flat buffer at any offset)."""
     pad = -t.shape[1] % _RANK_STEP
-    return torch.nn.functional.pad(t, (0, pad)) if pad else t
+    t = (torch.nn.functional.pad(t, (0, pad)) if pad else t).contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 _HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")

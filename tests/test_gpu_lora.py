@@ -375,6 +375,33 @@ def test_float16_training_gradients_are_finite_where_the_composition_is(scale):
         assert float((a.double() - b.double()).norm() / b.double().norm()) < 4 * 2.0 ** -11
 
 
+@pytest.mark.parametrize("rank,N", [(16, 512), (16, 1), (24, 64)])
+def test_training_factors_at_any_address(rank, N):
+    """Factors that are views of a flat parameter buffer at an odd offset, which the
+    kernels' 16-byte loads cannot take as they are: the gradients of aligned
+    copies, bit for bit (a rank that is a multiple of 16 is not padded, and one
+    output feature makes lora_B's transpose contiguous as it is)."""
+    from mflux_amd import lora, nn
+
+    torch.manual_seed(94)
+    lin = torch.nn.Linear(256, N, bias=False, device="cuda", dtype=torch.bfloat16)
+    layer = lora.LoRALinear.from_linear(nn.QuantizedLinear.from_linear(lin, 64, 4), r=rank, scale=1.0)
+    layer.lora_B.data.normal_(std=0.02)
+    x = torch.randn(64, 256, device="cuda").bfloat16().requires_grad_(True)
+    g = torch.randn(64, N, device="cuda").bfloat16()
+    step = lambda: torch.autograd.grad(layer(x), (x, layer.lora_A, layer.lora_B), g)
+    want = step()
+    for name in ("lora_A", "lora_B"):
+        p = getattr(layer, name)
+        flat = torch.empty(p.numel() + 1, device="cuda", dtype=p.dtype)
+        flat[1:] = p.detach().reshape(-1)
+        setattr(layer, name, torch.nn.Parameter(flat[1:].view(p.shape)))
+    assert layer.lora_A.data_ptr() % 16 and layer.lora_B.data_ptr() % 16
+    assert lora._trains_in_one(layer.linear, layer, x)
+    for a, b in zip(step(), want):
+        assert torch.equal(a, b)
+
+
 def test_training_calls_that_keep_the_composition():
     """Hooks on the base, autocast, forward mode, a transform, few rows, another
     adapter type: the composition, which serves them; and a second derivative of
