@@ -127,20 +127,28 @@ int mfq_dequantize_rows(const uint32_t* wq, const void* scales, const void* bias
  *   biases  [N, K/group_size]      sb_dtype
  *   bias    [N] or NULL            sb_dtype
  *   y       [M, N]                 y_dtype (sb_dtype or MFQ_F32)
- * M <= 16 runs the HBM-bound dequant-GEMV kernel, larger M one of two MFMA
- * GEMM kernels (128-column tiles while 256 x 256 tiles would leave more than
- * half of the compute units idle, 256 x 256 tiles otherwise).  3, 5 and 6 bits:
- * one activation row of up to 8192 elements has its own kernel, everything
- * else runs on the 128-column-tile GEMM.  For M > 16 the
- * dequantised weights are rounded once to x_dtype and sums are float32.  For
- * M <= 16 (4 and 8 bits; shapes the integer kernels take) every row of x
- * becomes 15-bit fixed point (one power of two per row brings its largest
- * magnitude under 2^14: an error of 2^-15 of that magnitude per element, exact
- * for small integers and one-hot rows), the integer products with the raw
- * codes are exact, and scale and bias are applied to their sums in float32; an
- * infinity or NaN in a row of x makes every output of that row NaN for
- * M = 1 and, at K of 1024 to 4096 in steps of 1024, for M <= 4, and gives
- * what the dequantised weights give for the others.
+ * M <= 16 runs the HBM-bound matvec kernels, larger M one of two MFMA GEMM
+ * kernels: 128-column tiles while 256 x 256 tiles would leave more than half of
+ * the compute units idle (unless K is long enough to be cut between those
+ * tiles), and below 1024 rows where an estimate of both finds them faster;
+ * 256 x 256 tiles otherwise.  3, 5 and 6 bits: one activation row of up to 8192
+ * elements has its own kernel, everything else runs on the 128-column-tile GEMM.
+ * Sums are float32, on dequantised weights rounded once to x_dtype -- except in
+ * the integer matvec kernels of 4 and 8 bits, where x becomes fixed point (one
+ * power of two per row, or per part of a row that a wavefront multiplies, from
+ * its largest magnitude), the integer products with the raw codes are exact, and
+ * scale and bias are applied to their sums in float32:
+ *   M = 1, rows of up to 6 KiB of 8-bit or 3 KiB of 4-bit codes; M = 2..4 on the
+ *     four-rows kernel and, in groups of 64, at K = 1024, 2048, 3072 and 4096 and
+ *     at K = 256 with 8 bits: 15 bits, an error per element of 2^-14 of that
+ *     magnitude at most, none for small integers and one-hot rows; an infinity
+ *     or NaN in a row of x makes every output of that row NaN;
+ *   M = 2..4 at K = 2560, 3840 and 6144 and at K = 256 with 4 bits, and M = 5..16
+ *     at K = 2048, 2560, 3072, 3840, 4096 and 6144 and, with 4 bits, 256 and 1024
+ *     (groups of 64, N a multiple of 8): 23 bits, 2^-23 of it, as a float32 sum
+ *     over it would round.
+ * Everywhere but in the 15-bit kernels an infinity or NaN in x gives what the
+ * dequantised weights give for it.
  */
 int mfq_qmm_t(const void* x, int x_dtype, int64_t M, int64_t K,
               const uint32_t* wq, const void* scales, const void* biases,

@@ -210,6 +210,27 @@ __device__ inline void split4(uint32_t p0, uint32_t p1, float mult, uint32_t& hi
   hi = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, t23), __builtin_bit_cast(uint32_t, t01), 0x07050301u);
 }
 
+// The same in 23 bits, as far as a float32 sum over the part reaches below its largest element (half a unit is at most
+// 2^-23 of it).  The largest value three signed bytes hold is 0x7f7f7f: magnitudes that round up past it take the next
+// power of two.  ldexp instead of a factor: the exponents of tiny bfloat16 rows lie outside float32's.
+template <typename T>
+__device__ inline int wide_exponent(int amax_bits);
+template <>
+__device__ inline int wide_exponent<BF16>(int amax_bits) { return 23 - (((amax_bits + 1) >> 7) - 127 + 1); }
+template <>
+__device__ inline int wide_exponent<F16>(int amax_bits) { return 23 - (((amax_bits + 8) >> 10) - 15 + 1); }
+
+// xq = 65536 h + 256 m + l, m and l read as signed: xq + 0x8080 has h on top, and m and l with their top bits flipped.
+template <typename T>
+__device__ inline void split4_wide(uint32_t p0, uint32_t p1, int e, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  const auto image = [&](float v) { return (uint32_t)((int)__builtin_rintf(__builtin_amdgcn_ldexpf(v, e)) + 0x8080); };
+  const uint32_t t0 = image(lo_f32<T>(p0)), t1 = image(hi_f32<T>(p0)), t2 = image(lo_f32<T>(p1)), t3 = image(hi_f32<T>(p1));
+  const uint32_t t01 = __builtin_amdgcn_perm(t1, t0, 0x05010400u), t23 = __builtin_amdgcn_perm(t3, t2, 0x05010400u);
+  lo = __builtin_amdgcn_perm(t23, t01, 0x05040100u) ^ 0x80808080u;
+  mid = __builtin_amdgcn_perm(t23, t01, 0x07060302u) ^ 0x80808080u;
+  hi = __builtin_amdgcn_perm(t1, t0, 0x0c0c0602u) | __builtin_amdgcn_perm(t3, t2, 0x06020c0cu);
+}
+
 // SiLU of a pair of 16-bit floats as MLX's nn.silu computes it on that type,
 // x * sigmoid(x) with the sigmoid rounded to the type before the product
 // (src/mflux/models/flux/model/flux_transformer/ada_layer_norm_zero.py:12 feeds
@@ -331,7 +352,7 @@ bool qmv_quad_covers(int64_t M, int64_t K, int64_t N, int gs, int bits, const vo
 int launch_qmv_quad(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                     const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
                     hipStream_t stream, bool silu = false);
-// one to sixteen activation rows (four with `silu`), 8-bit codes: eight weight rows at a time on the int8 16x16x64
+// one to sixteen activation rows (four with `silu`, and at rows of up to 1024 codes), 8-bit codes: eight weight rows at a time on the int8 16x16x64
 // matrix instruction, K split over the wavefronts of a workgroup (qmv_oct_covers() says whether it takes a shape)
 bool qmv_oct_covers(int64_t M, int64_t K, int64_t N, int gs, int bits, const void* x, const void* scales,
                     const void* biases);

@@ -18,8 +18,7 @@
 //     high bytes in row 2 m, low bytes in row 2 m + 1.  Of D, column j's rows
 //     0..7 (j even) or 8..15 (j odd) are the products that belong together; the
 //     others pair a half of the weights with the other half of x and are dropped.
-//     Up to four activation rows cost what one does; five to eight take a second
-//     instruction on the same B operand, and more than eight a second workgroup.
+//     Up to four activation rows cost what one does.
 //   - a code enters as the signed byte code - 128 (one XOR per word); a half step
 //     is one group of 64 codes, so per instruction and lane, with Sx the sum of xq
 //     over the group's 64 k,
@@ -33,9 +32,15 @@
 // three blocks in flight in three register sets, all unconditional so that every
 // wait leaves exactly the younger loads in flight.  The eight partial sums of a
 // block meet in LDS at the end of the run, where each thread adds up one output.
+// Calls that multiplied x as it is before (oct_wide(): more than four rows, two to four on
+// some row lengths) keep three bytes of it, 23 bits: A's rows 4 i .. 4 i + 2 are the bytes
+// of one activation row, two rows to an instruction, high and lower bytes are summed apart
+// as integers and joined in float32.
 // Bound by HBM, and from five rows on by the image of x in front of the first block:
-// 3072 -> 18432 takes 11.4 us with one row, 13.3 with eight (24.8 on the kernel that
-// dequantises, whose error against float64 is 1.6e-3 where this one's is 1.4e-5).
+// 3072 -> 18432 takes 11.4 us with one row, 14.7 with eight (24.5 on the kernel that
+// dequantises).  Distance from float64 of a float32 output, rows with one element in 128
+// at 300 times the others: 2e-7 of the norm with three bytes, 3.4e-4 with two; with the
+// rounded weights of the kernels that dequantise 1.6e-3 in bfloat16, 2e-4 in float16.
 // Rows whose steps do not come in eights are split over ten wavefronts (K = 2560, 3840).
 #include <type_traits>
 
@@ -84,8 +89,9 @@ struct ScaleWindow {
 };
 
 // K = 128 kWaves kSteps, kSteps 128-byte steps per wavefront and row; kM: activation rows the image is built for
-// (1, 2, 4 or 8; other M run as the next of these with their last row repeated)
-template <typename T, int kWaves, int kSteps, int kM, bool kSilu>
+// (1, 2, 4 or 8; other M run as the next of these with their last row repeated, more than kM on several workgroups).
+// kWide: three bytes per element of x instead of two.
+template <typename T, int kWaves, int kSteps, int kM, bool kWide, bool kSilu>
 __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
     const uint16_t* __restrict__ biases, const uint16_t* __restrict__ bias, void* __restrict__ y, int y_is_f32, int M,
@@ -94,20 +100,21 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
   constexpr int kSlice = 128 * kSteps;       // bytes (= codes) per row and wavefront
   constexpr int kGroups = K / 64;
   constexpr int kPitch = kSlice + 16;        // image rows in LDS
-  constexpr int kPasses = kM > 4 ? 2 : 1;    // fours of activation rows
-  constexpr int kImageRows = 2 * kM;
-  constexpr int kImageBytes = ((kImageRows * kPitch + kM * 2 * kSteps * 4) + 255) & ~255;  // + the sums of xq
+  constexpr int kBytes = kWide ? 3 : 2;
+  constexpr int kPasses = kWide ? kM / 2 : 1;  // instructions per step: two activation rows each, or up to four
+  constexpr int kImageRows = kBytes * kM;
+  constexpr int kImageBytes = oct_image_bytes(kWide, kM, 8, kPitch, 2 * kSteps);
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int j = lane & 15, q = lane >> 4;
   const int n8 = j >> 1, h = j & 1;
   char* image = lds + wave * kImageBytes;
-  float* sums = reinterpret_cast<float*>(image + kImageRows * kPitch);
-  float2* partials = reinterpret_cast<float2*>(lds + kWaves * kImageBytes);  // [block][wavefront][pass][kSlots]
-  constexpr int kSlots = kM > 4 ? 32 : 64;   // every lane's pair, or the useful half of the lanes' (2 j + q % 2)
+  int2* sums = reinterpret_cast<int2*>(image + kImageRows * kPitch);  // of xq: high bytes, the rest (narrow: all)
+  float* partials = reinterpret_cast<float*>(lds + kWaves * kImageBytes);  // [block][wavefront][oct_partials()]
+  constexpr int kPartials = oct_partials(kWide, kM, 8);
   int run = blockIdx.x;
-  if constexpr (kM > 4) {  // more than eight activation rows: eight to a workgroup
+  if constexpr (kWide) {
     const int m0 = oct_run_and_first_row<kM>(M, run);
     x += (size_t)m0 * K;
     y = static_cast<char*>(y) + (size_t)m0 * N * (y_is_f32 ? 4 : 2);
@@ -116,7 +123,7 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
 
   const int n_blocks_all = N / kOctRows;
   const int blk_first = run * blocks_per_wg;
-  if (kM > 4 && blk_first >= n_blocks_all) return;  // (runs are dealt out in eights)
+  if (kWide && blk_first >= n_blocks_all) return;  // (runs are dealt out in eights)
   const int n_blocks = min(blocks_per_wg, n_blocks_all - blk_first);
   const int blk_last = blk_first + n_blocks - 1;
 
@@ -164,7 +171,7 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
   // ---- the integer image of this wavefront's eighth of x ------------------------------------------------
   // One power of two per activation row and eighth of K: the eighths' sums are scaled back before they meet,
   // so the wavefronts need not agree on it and nobody waits for anybody here.
-  float unscale_m[kM];
+  float unscale_m[kM];  // narrow: the factor, wide: the exponent
 #pragma unroll
   for (int m = 0; m < kM; ++m) {
     int amax = 0;
@@ -177,59 +184,83 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
       amax = max(amax, max(mag_bits(raw[m][t].x), mag_bits(raw[m][t].y)));
     }
     amax = oct_wave_max(amax);
-    const int e = scale_exponent<T>(amax);
-    const float mult = pow2(e);
     // an infinity or NaN anywhere in a row of x: every output of that row is NaN (through this eighth's sums)
-    unscale_m[m] = not_finite<T>(amax) ? __builtin_nanf("") : pow2(-e);
+    const int e = kWide ? wide_exponent<T>(amax) : scale_exponent<T>(amax);
+    const float mult = kWide ? 0.f : pow2(e);
+    unscale_m[m] = not_finite<T>(amax) ? __builtin_nanf("") : kWide ? __builtin_amdgcn_ldexpf(1.f, -e) : pow2(-e);
 #pragma unroll
     for (int t = 0; t < kChunks; ++t) {
       const int c = lane + 64 * t;
       const bool in = c < 32 * kSteps;
-      uint32_t hi, lo;
-      split4<T>(raw[m][t].x, raw[m][t].y, mult, hi, lo);
+      uint32_t hi, mid = 0, lo;
+      if constexpr (kWide)
+        split4_wide<T>(raw[m][t].x, raw[m][t].y, e, hi, mid, lo);
+      else
+        split4<T>(raw[m][t].x, raw[m][t].y, mult, hi, lo);
       if (in) {
-        *reinterpret_cast<uint32_t*>(image + (2 * m) * kPitch + 4 * c) = hi;
-        *reinterpret_cast<uint32_t*>(image + (2 * m + 1) * kPitch + 4 * c) = lo;
+        uint32_t* row = reinterpret_cast<uint32_t*>(image + kBytes * m * kPitch + 4 * c);
+        row[0] = hi;
+        if constexpr (kWide) row[kPitch / 4] = mid;
+        row[(kBytes - 1) * (kPitch / 4)] = lo;
       }
       // the sum of xq over a half step's 64 k: its 16 chunks are the 16 lanes of a row of lanes
-      const int part = __builtin_amdgcn_sdot4((int)hi, 0x01010101, 0, false) * 256 +
-                       __builtin_amdgcn_sdot4((int)lo, 0x01010101, 0, false);
-      const int total = oct_row16_sum(in ? part : 0);
-      if (j == 0 && in) sums[m * 2 * kSteps + (c >> 4)] = (float)total;
+      const int dot_hi = __builtin_amdgcn_sdot4((int)hi, 0x01010101, 0, false);
+      const int dot_lo = __builtin_amdgcn_sdot4((int)lo, 0x01010101, 0, false);
+      const int dot_mid = kWide ? __builtin_amdgcn_sdot4((int)mid, 0x01010101, 0, false) : dot_hi;
+      const int rest = oct_row16_sum(in ? dot_mid * 256 + dot_lo : 0);
+      const int high = kWide ? oct_row16_sum(in ? dot_hi : 0) : 0;
+      if (j == 0 && in) sums[m * 2 * kSteps + (c >> 4)] = make_int2(high, rest);
     }
   }
   // (LDS written and read by this wavefront only: program order holds)
-  // this lane's A operands, pass p: image row 8 p + j % 8 over half j / 8 of every step (image rows past 2 kM: any
-  // row, their results are never read)
+  // this lane's A operands, pass p.  Two bytes: image row j % 8 over half j / 8 of every step (image rows past 2 kM:
+  // any row, their results are never read).  Three: activation row 2 p + (j % 8) / 4, byte j % 4 (the fourth: the
+  // third again, never read).
   i32x4 xa[kPasses][kSteps];
 #pragma unroll
   for (int p = 0; p < kPasses; ++p) {
-    const char* arow = image + (8 * p + (j & 7 & (kImageRows - 1))) * kPitch + 64 * (j >> 3) + 16 * q;
+    const int r = kWide ? 3 * (2 * p + ((j >> 2) & 1)) + min(j & 3, 2) : j & 7 & (kImageRows - 1);
+    const char* arow = image + r * kPitch + 64 * (j >> 3) + 16 * q;
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) xa[p][s] = *reinterpret_cast<const i32x4*>(arow + 128 * s);
   }
-  // results: register r of lane (j, q) is A's row 4 q + r against column j.  Of use where q / 2 == j % 2:
-  // activation rows 4 p + 2 (q % 2) (registers 0, 1: high, low bytes) and 4 p + 2 (q % 2) + 1 (registers 2, 3)
-  constexpr bool kTwo = kM > 1;  // one activation row: registers 2 and 3 hold nothing of use
+  // results: register r of lane (j, q) is A's row 4 q + r against column j.  Of use where q / 2 == j % 2.  Two bytes:
+  // activation rows 2 (q % 2) (registers 0, 1: high, low bytes) and 2 (q % 2) + 1 (registers 2, 3); three:
+  // activation row 2 p + q % 2 (registers 0, 1, 2).
+  constexpr bool kTwo = !kWide && kM > 1;  // one activation row: registers 2 and 3 hold nothing of use
   // the sums of xq over this lane's half steps: as float for the bias term, and 128 times them as integers
   // (a code enters the matrix instruction as code - 128; adding 128 sum(xq) to its result gives sum(xq code))
   float sx_a[kPasses][kSteps], sx_b[kPasses][kSteps], us_a[kPasses], us_b[kPasses];
-  int sx128_a[kPasses][kSteps], sx128_b[kPasses][kSteps];
+  int sx128_a[kPasses][kSteps], sx128_b[kPasses][kSteps];  // wide: of the lower bytes, of the high ones
 #pragma unroll
   for (int p = 0; p < kPasses; ++p) {
-    const int m_a = (4 * p + 2 * (q & 1)) & (kM - 1), m_b = (4 * p + 2 * (q & 1) + 1) & (kM - 1);
+    if constexpr (kWide) {
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      sx_a[p][s] = sums[m_a * 2 * kSteps + 2 * s + h];
-      sx_b[p][s] = kTwo ? sums[m_b * 2 * kSteps + 2 * s + h] : 0.f;
-      sx128_a[p][s] = 128 * (int)sx_a[p][s];
-      sx128_b[p][s] = 128 * (int)sx_b[p][s];
-    }
-    us_a[p] = unscale_m[4 * p];
-    us_b[p] = unscale_m[4 * p + (kTwo ? 1 : 0)];
-    if constexpr (kM > 2) {
-      us_a[p] = (q & 1) ? unscale_m[4 * p + 2] : us_a[p];
-      us_b[p] = (q & 1) ? unscale_m[4 * p + 3] : us_b[p];
+      for (int s = 0; s < kSteps; ++s) {
+        const int2 sum = sums[(2 * p + (q & 1)) * 2 * kSteps + 2 * s + h];
+        sx_a[p][s] = (float)(sum.x * 65536 + sum.y);  // 64 elements below 2^23
+        sx128_a[p][s] = 128 * sum.y;
+        sx128_b[p][s] = 128 * sum.x;
+      }
+      us_a[p] = unscale_m[2 * p];
+      us_a[p] = (q & 1) ? unscale_m[2 * p + 1] : us_a[p];
+    } else {
+      const int m_a = (2 * (q & 1)) & (kM - 1), m_b = (2 * (q & 1) + 1) & (kM - 1);
+#pragma unroll
+      for (int s = 0; s < kSteps; ++s) {
+        const int sum_a = sums[m_a * 2 * kSteps + 2 * s + h].y;
+        const int sum_b = kTwo ? sums[m_b * 2 * kSteps + 2 * s + h].y : 0;
+        sx_a[p][s] = (float)sum_a;
+        sx_b[p][s] = (float)sum_b;
+        sx128_a[p][s] = 128 * sum_a;
+        sx128_b[p][s] = 128 * sum_b;
+      }
+      us_a[p] = unscale_m[0];
+      us_b[p] = unscale_m[kTwo ? 1 : 0];
+      if constexpr (kM > 2) {
+        us_a[p] = (q & 1) ? unscale_m[2] : us_a[p];
+        us_b[p] = (q & 1) ? unscale_m[3] : us_b[p];
+      }
     }
   }
 
@@ -250,22 +281,32 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
       for (int p = 0; p < kPasses; ++p) {
         const i32x4 zero = {0, 0, 0, 0};
         const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[p][s], wb, zero, 0, 0, 0);
-        // sum(xq code) over the half step's group, exact: high and low bytes of xq joined as integers
-        const int da = d[0] * 256 + d[1] + sx128_a[p][s];
-        acc_a[p] = __builtin_fmaf(sc, (float)da, acc_a[p]);
-        acc_a[p] = __builtin_fmaf(bi, sx_a[p][s], acc_a[p]);
-        if constexpr (kTwo) {
-          const int db = d[2] * 256 + d[3] + sx128_b[p][s];
-          acc_b[p] = __builtin_fmaf(sc, (float)db, acc_b[p]);
-          acc_b[p] = __builtin_fmaf(bi, sx_b[p][s], acc_b[p]);
+        if constexpr (kWide) {
+          // sum(xq code) over the half step's group: high and lower bytes exact, joined in float32
+          const int dl = d[1] * 256 + d[2] + sx128_a[p][s], dh = d[0] + sx128_b[p][s];
+          acc_a[p] = __builtin_fmaf(sc, __builtin_fmaf(65536.f, (float)dh, (float)dl), acc_a[p]);
+          acc_a[p] = __builtin_fmaf(bi, sx_a[p][s], acc_a[p]);
+        } else {
+          // sum(xq code) over the half step's group, exact: high and low bytes of xq joined as integers
+          const int da = d[0] * 256 + d[1] + sx128_a[p][s];
+          acc_a[p] = __builtin_fmaf(sc, (float)da, acc_a[p]);
+          acc_a[p] = __builtin_fmaf(bi, sx_a[p][s], acc_a[p]);
+          if constexpr (kTwo) {
+            const int db = d[2] * 256 + d[3] + sx128_b[p][s];
+            acc_b[p] = __builtin_fmaf(sc, (float)db, acc_b[p]);
+            acc_b[p] = __builtin_fmaf(bi, sx_b[p][s], acc_b[p]);
+          }
         }
       }
     }
-    if (kSlots == 64 || (q >> 1) == h) {
-      const int u = kSlots == 64 ? lane : 2 * j + (q & 1);
+    float* dst = partials + (slot * kWaves + wave) * kPartials;
+    if constexpr (kWide) {
+      if ((q >> 1) == h) {  // the useful half of the lanes, one value per pass
 #pragma unroll
-      for (int p = 0; p < kPasses; ++p)
-        partials[((slot * kWaves + wave) * kPasses + p) * kSlots + u] = make_float2(acc_a[p] * us_a[p], acc_b[p] * us_b[p]);
+        for (int p = 0; p < kPasses; ++p) dst[32 * p + 2 * j + (q & 1)] = acc_a[p] * us_a[p];
+      }
+    } else {
+      reinterpret_cast<float2*>(dst)[lane] = make_float2(acc_a[0] * us_a[0], acc_b[0] * us_b[0]);
     }
   };
 
@@ -295,27 +336,30 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
   for (int i = 0; i < kOuts; ++i) {
     const int o = (int)threadIdx.x + i * 64 * kWaves;
     const int out_m = o % M, out_row8 = (o / M) % kOctRows, out_blk = o / M / kOctRows;
-    if (out_blk >= n_blocks) break;
+    const bool mine = out_blk < n_blocks;
     const int64_t out_row = (int64_t)(blk_first + out_blk) * kOctRows + out_row8;
     float v = 0.f;
+    if (mine) {
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w)
+      for (int w = 0; w < kWaves; ++w)
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const int src_j = 2 * out_row8 + hh, pair = (out_m >> 1) & 1;
-        const int src = kSlots == 64 ? src_j + 16 * (2 * hh + pair) : 2 * src_j + pair;
-        const float2 p = partials[((out_blk * kWaves + w) * kPasses + (out_m >> 2)) * kSlots + src];
-        v += (out_m & 1) ? p.y : p.x;
-      }
-    // an infinity in x is an infinity of the weight's sign in y, as the kernels that dequantise give it (the rows
-    // that meet no infinity or NaN never come here)
-    if constexpr (oct_keeps_infinities(kM, K, 8)) {
-      if (v != v) v = oct_plain_dot<T, 8, kSilu>(x + (size_t)out_m * K, wq, scales, biases, out_row, K);
+        for (int hh = 0; hh < 2; ++hh) {
+          const int src_j = 2 * out_row8 + hh;
+          const float* src = partials + (out_blk * kWaves + w) * kPartials;
+          if constexpr (kWide) {
+            v += src[32 * (out_m >> 1) + 2 * src_j + (out_m & 1)];
+          } else {
+            const float2 p = reinterpret_cast<const float2*>(src)[src_j + 16 * (2 * hh + (out_m >> 1))];
+            v += (out_m & 1) ? p.y : p.x;
+          }
+        }
     }
+    // an infinity in x is an infinity of the weight's sign in y, as the kernels that dequantise give it
+    if constexpr (kWide) v = oct_keep_infinities<T, 8, kSilu>(mine, v, x, wq, scales, biases, out_m, out_row, K, lane);
     const float bias_v = T::to_f32(out_bias[i]);
-    if (y_is_f32) {
+    if (mine && y_is_f32) {
       reinterpret_cast<float*>(y)[(int64_t)out_m * N + out_row] = bias ? v + bias_v : v;
-    } else {
+    } else if (mine) {
       const uint16_t h0 = T::from_f32(v);
       const uint16_t h1 = T::from_f32(T::to_f32(h0) + bias_v);  // second rounding, as a separate add would do
       reinterpret_cast<uint16_t*>(y)[(int64_t)out_m * N + out_row] = bias ? h1 : h0;
@@ -323,42 +367,45 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
   }
 }
 
-template <typename T, int kWaves, int kSteps, int kM, bool kSilu>
+template <typename T, int kWaves, int kSteps, int kM, bool kWide, bool kSilu>
 int launch_oct(const void* x, int64_t M, const uint32_t* wq, const void* scales, const void* biases, const void* bias,
                int64_t N, void* y, int y_dtype, hipStream_t stream) {
-  auto kernel = qmv_oct_kernel<T, kWaves, kSteps, kM, kSilu>;
-  constexpr int kImageBytes = ((2 * kM * (128 * kSteps + 16) + kM * 2 * kSteps * 4) + 255) & ~255;
-  constexpr int kPerBlock = kWaves * 512;  // partial sums: 64 pairs per wavefront, or two passes of 32
+  auto kernel = qmv_oct_kernel<T, kWaves, kSteps, kM, kWide, kSilu>;
+  constexpr int kImageBytes = oct_image_bytes(kWide, kM, 8, 128 * kSteps + 16, 2 * kSteps);
+  constexpr int kPerBlock = kWaves * oct_partials(kWide, kM, 8) * 4;
   static PerDeviceInt configured;
   return launch_oct_runs<kWaves, kM>(kernel, configured, kWaves * kImageBytes, kPerBlock, kOctRows, kOctMaxBlocks,
                                      kOctLongRun, x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
 }
 
-// Activation rows the image is built for: 1, 2, 4 or 8, fours and eights with their last rows repeated.
-template <typename T, int kWaves, int kSteps, bool kSilu>
+// Activation rows the image is built for: 1, 2, 4 or kMost (0: four at most), the last two with their last rows repeated.
+template <typename T, int kWaves, int kSteps, int kMost, bool kSilu>
 int launch_oct_rows(const void* x, int64_t M, const uint32_t* wq, const void* scales, const void* biases,
                     const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream) {
-  if (M == 1) return launch_oct<T, kWaves, kSteps, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-  if (M == 2) return launch_oct<T, kWaves, kSteps, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-  if (M <= 4) return launch_oct<T, kWaves, kSteps, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-  if constexpr (!kSilu)
-    return launch_oct<T, kWaves, kSteps, 8, false>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  constexpr int K = 128 * kWaves * kSteps;
+  if (M == 1) return launch_oct<T, kWaves, kSteps, 1, false, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  constexpr bool kWide = oct_wide(2, K, 8);
+  if (M == 2) return launch_oct<T, kWaves, kSteps, 2, kWide, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  if (M <= 4) return launch_oct<T, kWaves, kSteps, 4, kWide, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  if constexpr (!kSilu && kMost > 0)
+    return launch_oct<T, kWaves, kSteps, kMost, true, false>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
   return MFQ_EUNSUPPORTED;
 }
 
-// The split of K: wavefronts times 128-byte steps of each.
+// The split of K: wavefronts times 128-byte steps of each, and the rows a workgroup takes of more than four: eight where
+// their image fits the registers (10 x 3: 168 of them, 78 us of spills instead of 31), 0 where oct_takes() ends at four.
 template <typename T, bool kSilu>
 int launch_oct_steps(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* scales, const void* biases,
                      const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream) {
   switch (K) {
-    case 256: return launch_oct_rows<T, 2, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 1024: return launch_oct_rows<T, 8, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 2048: return launch_oct_rows<T, 8, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 2560: return launch_oct_rows<T, 10, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 3072: return launch_oct_rows<T, 8, 3, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 3840: return launch_oct_rows<T, 10, 3, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 4096: return launch_oct_rows<T, 8, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 6144: return launch_oct_rows<T, 8, 6, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 256: return launch_oct_rows<T, 2, 1, 0, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 1024: return launch_oct_rows<T, 8, 1, 0, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 2048: return launch_oct_rows<T, 8, 2, 8, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 2560: return launch_oct_rows<T, 10, 2, 8, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 3072: return launch_oct_rows<T, 8, 3, 8, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 3840: return launch_oct_rows<T, 10, 3, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 4096: return launch_oct_rows<T, 8, 4, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 6144: return launch_oct_rows<T, 8, 6, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     default: return MFQ_EUNSUPPORTED;
   }
 }

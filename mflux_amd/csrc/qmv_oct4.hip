@@ -21,10 +21,14 @@
 // nothing is offset:
 //     d = 256 D_high + D_low      (int32, exactly sum(xq code) over the group)
 //     acc += scale * d + bias * sum(xq)
-// Every further two activation rows (up to eight; more take a second workgroup) are
-// another pair of instructions on the same B operands: 3072 -> 18432 takes 7.4 us with
-// one row, 8.6 with four, 11.4 with eight (31.2 on the kernel that dequantises).  Work layout, register sets, the meeting of the wavefronts'
-// partial sums at the end: qmv_oct.hip's, with K split over kWaves wavefronts.
+// Rows three and four are another pair of instructions on the same B operands.  Calls
+// that multiplied x as it is before (oct_wide()) keep three bytes of it: A's row
+// 8 h + 4 g + l is byte l of ONE activation row, and d = 65536 D_high + 256 D_mid + D_low
+// is put together in float32.  More than four activation rows take a workgroup to every
+// four.  3072 -> 18432 takes 7.4 us with one row, 8.4 with four, 17 with eight, where
+// the vector instructions of the bytes are as long as the loads (31 on the kernel that
+// dequantises).  Work layout, register sets, the meeting of the wavefronts' partial sums
+// at the end: qmv_oct.hip's, with K split over kWaves wavefronts.
 #include <type_traits>
 
 #include "qmv_oct_common.h"
@@ -71,8 +75,9 @@ struct ScaleWindow4 {
 };
 
 // kWaves: wavefronts per workgroup, each with kSteps 128-byte steps of every row (K = 256 kWaves kSteps codes);
-// kM: activation rows the image is built for (1, 2, 4 or 8; other M run as the next of these with their last row repeated)
-template <typename T, int kWaves, int kSteps, int kM, bool kSilu>
+// kM: activation rows the image is built for (1, 2, 4 or 8; other M run as the next of these with their last row repeated, more than
+// kM on several workgroups).  kWide: three bytes per element of x instead of two.
+template <typename T, int kWaves, int kSteps, int kM, bool kWide, bool kSilu>
 __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
     const uint16_t* __restrict__ biases, const uint16_t* __restrict__ bias, void* __restrict__ y, int y_is_f32, int M,
@@ -81,10 +86,11 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
   constexpr int kRowBytes = K / 2;
   constexpr int kSlice = 128 * kSteps;       // bytes per row and wavefront: 2 kSlice codes
   constexpr int kGroups = K / 64;
-  constexpr int kPasses = kM > 2 ? kM / 2 : 1;  // pairs of activation rows
-  constexpr int kImageRows = 2 * kM;         // (activation row, high / low byte)
+  constexpr int kBytes = kWide ? 3 : 2;
+  constexpr int kPasses = kWide ? kM : kM > 2 ? kM / 2 : 1;  // pairs of instructions per step: one activation row each, or two
+  constexpr int kImageRows = kBytes * kM;    // (activation row, byte from the top)
   constexpr int kPitch = 2 * kSlice + 32;    // an image row: kSlice bytes of even k, kSlice of odd k
-  constexpr int kImageBytes = ((kImageRows * kPitch + kM * 4 * kSteps * 4) + 255) & ~255;  // + the sums of xq
+  constexpr int kImageBytes = oct_image_bytes(kWide, kM, 4, kPitch, 4 * kSteps);
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -92,10 +98,10 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
   const int n8 = j >> 1, h = j & 1;
   char* image = lds + wave * kImageBytes;
   float* sums = reinterpret_cast<float*>(image + kImageRows * kPitch);  // [activation row][group of the slice]
-  float2* partials = reinterpret_cast<float2*>(lds + kWaves * kImageBytes);  // [block][wavefront][pass][kSlots]
-  constexpr int kSlots = kM > 4 ? 32 : 64;   // every lane's pair, or the useful half of the lanes' (2 j + q % 2)
+  float* partials = reinterpret_cast<float*>(lds + kWaves * kImageBytes);  // [block][wavefront][oct_partials()]
+  constexpr int kPartials = oct_partials(kWide, kM, 4);
   int run = blockIdx.x;
-  if constexpr (kM > 4) {  // more than eight activation rows: eight to a workgroup
+  if constexpr (kWide) {
     const int m0 = oct_run_and_first_row<kM>(M, run);
     x += (size_t)m0 * K;
     y = static_cast<char*>(y) + (size_t)m0 * N * (y_is_f32 ? 4 : 2);
@@ -104,7 +110,7 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
 
   const int n_blocks_all = N / kRows4;
   const int blk_first = run * blocks_per_wg;
-  if (kM > 4 && blk_first >= n_blocks_all) return;  // (runs are dealt out in eights)
+  if (kWide && blk_first >= n_blocks_all) return;  // (runs are dealt out in eights)
   const int n_blocks = min(blocks_per_wg, n_blocks_all - blk_first);
   const int blk_last = blk_first + n_blocks - 1;
 
@@ -161,10 +167,10 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
         amax = max(amax, mag_bits(raw[m][t][i]));
       }
     amax = oct4_wave_max(amax);
-    const int e = scale_exponent<T>(amax);
-    const float mult = pow2(e);
     // an infinity or NaN anywhere in a row of x: every output of that row is NaN (through this part's sums)
-    unscale_m[m] = not_finite<T>(amax) ? __builtin_nanf("") : pow2(-e);
+    const int e = kWide ? wide_exponent<T>(amax) : scale_exponent<T>(amax);
+    const float mult = kWide ? 0.f : pow2(e);
+    unscale_m[m] = not_finite<T>(amax) ? __builtin_nanf("") : kWide ? __builtin_amdgcn_ldexpf(1.f, -e) : pow2(-e);
 #pragma unroll
     for (int t = 0; t < kChunks; ++t) {
       const int c = lane + 64 * t;
@@ -173,35 +179,48 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
       const u32x4 r = raw[m][t];
       const uint32_t ev0 = (r[0] & 0xffffu) | (r[1] << 16), ev1 = (r[2] & 0xffffu) | (r[3] << 16);
       const uint32_t od0 = (r[0] >> 16) | (r[1] & 0xffff0000u), od1 = (r[2] >> 16) | (r[3] & 0xffff0000u);
-      uint32_t hi_e, lo_e, hi_o, lo_o;
-      split4<T>(ev0, ev1, mult, hi_e, lo_e);
-      split4<T>(od0, od1, mult, hi_o, lo_o);
-      if (in) {
-        *reinterpret_cast<uint32_t*>(image + (2 * m) * kPitch + 4 * c) = hi_e;
-        *reinterpret_cast<uint32_t*>(image + (2 * m) * kPitch + kSlice + 16 + 4 * c) = hi_o;
-        *reinterpret_cast<uint32_t*>(image + (2 * m + 1) * kPitch + 4 * c) = lo_e;
-        *reinterpret_cast<uint32_t*>(image + (2 * m + 1) * kPitch + kSlice + 16 + 4 * c) = lo_o;
+      uint32_t hi_e, mid_e = 0, lo_e, hi_o, mid_o = 0, lo_o;
+      if constexpr (kWide) {
+        split4_wide<T>(ev0, ev1, e, hi_e, mid_e, lo_e);
+        split4_wide<T>(od0, od1, e, hi_o, mid_o, lo_o);
+      } else {
+        split4<T>(ev0, ev1, mult, hi_e, lo_e);
+        split4<T>(od0, od1, mult, hi_o, lo_o);
       }
-      // the sum of xq over a group's 64 k: its 8 chunks are 8 neighbouring lanes
-      const int part = (__builtin_amdgcn_sdot4((int)hi_e, 0x01010101, 0, false) +
-                        __builtin_amdgcn_sdot4((int)hi_o, 0x01010101, 0, false)) * 256 +
-                       __builtin_amdgcn_sdot4((int)lo_e, 0x01010101, 0, false) +
-                       __builtin_amdgcn_sdot4((int)lo_o, 0x01010101, 0, false);
+      if (in) {
+        char* even = image + kBytes * m * kPitch + 4 * c;
+        char* odd = even + kSlice + 16;
+        *reinterpret_cast<uint32_t*>(even) = hi_e;
+        *reinterpret_cast<uint32_t*>(odd) = hi_o;
+        if constexpr (kWide) {
+          *reinterpret_cast<uint32_t*>(even + kPitch) = mid_e;
+          *reinterpret_cast<uint32_t*>(odd + kPitch) = mid_o;
+        }
+        *reinterpret_cast<uint32_t*>(even + (kBytes - 1) * kPitch) = lo_e;
+        *reinterpret_cast<uint32_t*>(odd + (kBytes - 1) * kPitch) = lo_o;
+      }
+      // the sum of xq over a group's 64 k (below 2^29): its 8 chunks are 8 neighbouring lanes
+      const auto sum4 = [](uint32_t a, uint32_t b) __attribute__((always_inline)) {
+        return __builtin_amdgcn_sdot4((int)a, 0x01010101, 0, false) + __builtin_amdgcn_sdot4((int)b, 0x01010101, 0, false);
+      };
+      int part = sum4(hi_e, hi_o) * 256;
+      if constexpr (kWide) part = (part + sum4(mid_e, mid_o)) * 256;
+      part += sum4(lo_e, lo_o);
       const int total = oct4_sum8(in ? part : 0);
       if ((lane & 7) == 0 && in) sums[m * 4 * kSteps + (c >> 3)] = (float)total;
     }
   }
   // (LDS written and read by this wavefront only: program order holds)
-  // this lane's A operands, pass p: A's row j = 8 h' + 4 g + 2 (m % 2) + l -- activation row 2 p + (j / 2) % 2,
-  // byte l = j % 2, over half h' = j / 8 of every step, zero unless this lane's k (pieces 2 g, 2 g + 1 of the
-  // half: q / 2 == g) belong to group g = (j / 4) % 2
+  // this lane's A operands, pass p: A's row j = 8 h' + 4 g + r over half h' = j / 8 of every step, zero unless this
+  // lane's k (pieces 2 g, 2 g + 1 of the half: q / 2 == g) belong to group g = (j / 4) % 2.  Two bytes: r = 2 (m % 2) + l
+  // is byte l of activation row m = 2 p + r / 2; three: byte r of activation row p (r = 3: byte 2 again, never read)
   i32x4 xa_e[kPasses][kSteps], xa_o[kPasses][kSteps];
   {
     const bool mine = (q >> 1) == ((j >> 2) & 1);
 #pragma unroll
     for (int p = 0; p < kPasses; ++p) {
-      const int m = (2 * p + ((j >> 1) & 1)) & (kM - 1);
-      const char* arow = image + (2 * m + (j & 1)) * kPitch + 64 * (j >> 3) + 16 * q;
+      const int row = kWide ? 3 * p + min(j & 3, 2) : 2 * ((2 * p + ((j >> 1) & 1)) & (kM - 1)) + (j & 1);
+      const char* arow = image + row * kPitch + 64 * (j >> 3) + 16 * q;
 #pragma unroll
       for (int s = 0; s < kSteps; ++s) {
         const i32x4 zero = {0, 0, 0, 0};
@@ -211,13 +230,14 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
     }
   }
   // results: register r of lane (j, q) is A's row 4 q + r against column j.  Of use where q / 2 == j % 2: group
-  // g = q % 2 of the column's half, activation rows 2 p (registers 0, 1: high, low bytes) and 2 p + 1 (2, 3)
-  constexpr bool kTwo = kM > 1;  // one activation row: registers 2 and 3 hold nothing of use
+  // g = q % 2 of the column's half.  Two bytes: activation rows 2 p (registers 0, 1: high, low bytes) and 2 p + 1
+  // (2, 3); three: activation row p (0, 1, 2)
+  constexpr bool kTwo = !kWide && kM > 1;  // one activation row: registers 2 and 3 hold nothing of use
   const int g = q & 1;
   float sx_a[kPasses][kSteps], sx_b[kPasses][kSteps], us_a[kPasses], us_b[kPasses];
 #pragma unroll
   for (int p = 0; p < kPasses; ++p) {
-    const int m_a = (2 * p) & (kM - 1), m_b = (2 * p + 1) & (kM - 1);
+    const int m_a = kWide ? p : (2 * p) & (kM - 1), m_b = (2 * p + 1) & (kM - 1);
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
       sx_a[p][s] = sums[m_a * 4 * kSteps + 4 * s + 2 * h + g];
@@ -251,20 +271,31 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
         const i32x4 zero = {0, 0, 0, 0};
         i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa_e[p][s], ev, zero, 0, 0, 0);
         d = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa_o[p][s], od, d, 0, 0, 0);
-        // sum(xq code) over the group, exact: high and low bytes of xq joined as integers
-        acc_a[p] = __builtin_fmaf(sc, (float)(d[0] * 256 + d[1]), acc_a[p]);
-        acc_a[p] = __builtin_fmaf(bi, sx_a[p][s], acc_a[p]);
-        if constexpr (kTwo) {
-          acc_b[p] = __builtin_fmaf(sc, (float)(d[2] * 256 + d[3]), acc_b[p]);
-          acc_b[p] = __builtin_fmaf(bi, sx_b[p][s], acc_b[p]);
+        if constexpr (kWide) {
+          // sum(xq code) over the group: high and lower bytes exact, joined in float32
+          acc_a[p] = __builtin_fmaf(sc, __builtin_fmaf(65536.f, (float)d[0], (float)(d[1] * 256 + d[2])), acc_a[p]);
+          acc_a[p] = __builtin_fmaf(bi, sx_a[p][s], acc_a[p]);
+        } else {
+          // sum(xq code) over the group, exact: high and low bytes of xq joined as integers
+          acc_a[p] = __builtin_fmaf(sc, (float)(d[0] * 256 + d[1]), acc_a[p]);
+          acc_a[p] = __builtin_fmaf(bi, sx_a[p][s], acc_a[p]);
+          if constexpr (kTwo) {
+            acc_b[p] = __builtin_fmaf(sc, (float)(d[2] * 256 + d[3]), acc_b[p]);
+            acc_b[p] = __builtin_fmaf(bi, sx_b[p][s], acc_b[p]);
+          }
         }
       }
     }
-    if (kSlots == 64 || (q >> 1) == h) {
-      const int u = kSlots == 64 ? lane : 2 * j + g;
+    float* dst = partials + (slot * kWaves + wave) * kPartials;
+    if constexpr (kWide) {
+      if ((q >> 1) == h) {  // the useful half of the lanes
+#pragma unroll
+        for (int p = 0; p < kPasses; ++p) dst[32 * p + 2 * j + g] = acc_a[p] * us_a[p];
+      }
+    } else {
 #pragma unroll
       for (int p = 0; p < kPasses; ++p)
-        partials[((slot * kWaves + wave) * kPasses + p) * kSlots + u] = make_float2(acc_a[p] * us_a[p], acc_b[p] * us_b[p]);
+        reinterpret_cast<float2*>(dst)[64 * p + lane] = make_float2(acc_a[p] * us_a[p], acc_b[p] * us_b[p]);
     }
   };
 
@@ -293,25 +324,30 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
   for (int i = 0; i < kOuts; ++i) {
     const int o = (int)threadIdx.x + i * 64 * kWaves;
     const int out_m = o % M, out_row8 = (o / M) % kRows4, out_blk = o / M / kRows4;
-    if (out_blk >= n_blocks) break;
+    const bool mine = out_blk < n_blocks;
     const int64_t out_row = (int64_t)(blk_first + out_blk) * kRows4 + out_row8;
     float v = 0.f;
+    if (mine) {
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w)
+      for (int w = 0; w < kWaves; ++w)
 #pragma unroll
-      for (int hg = 0; hg < 4; ++hg) {  // half hg / 2, group hg % 2: lane (2 row + half, 2 half + group)
-        const int src_j = 2 * out_row8 + (hg >> 1);
-        const int src = kSlots == 64 ? src_j + 16 * hg : 2 * src_j + (hg & 1);
-        const float2 p = partials[((out_blk * kWaves + w) * kPasses + (out_m >> 1)) * kSlots + src];
-        v += (out_m & 1) ? p.y : p.x;
-      }
-    if constexpr (oct_keeps_infinities(kM, K, 4)) {  // as in the 8-bit kernel: what an infinity or NaN in x makes of y
-      if (v != v) v = oct_plain_dot<T, 4, kSilu>(x + (size_t)out_m * K, wq, scales, biases, out_row, K);
+        for (int hg = 0; hg < 4; ++hg) {  // half hg / 2, group hg % 2: lane (2 row + half, 2 half + group)
+          const int src_j = 2 * out_row8 + (hg >> 1);
+          const float* src = partials + (out_blk * kWaves + w) * kPartials;
+          if constexpr (kWide) {
+            v += src[32 * out_m + 2 * src_j + (hg & 1)];
+          } else {
+            const float2 p = reinterpret_cast<const float2*>(src)[64 * (out_m >> 1) + src_j + 16 * hg];
+            v += (out_m & 1) ? p.y : p.x;
+          }
+        }
     }
+    // an infinity in x is an infinity of the weight's sign in y, as the kernels that dequantise give it
+    if constexpr (kWide) v = oct_keep_infinities<T, 4, kSilu>(mine, v, x, wq, scales, biases, out_m, out_row, K, lane);
     const float bias_v = T::to_f32(out_bias[i]);
-    if (y_is_f32) {
+    if (mine && y_is_f32) {
       reinterpret_cast<float*>(y)[(int64_t)out_m * N + out_row] = bias ? v + bias_v : v;
-    } else {
+    } else if (mine) {
       const uint16_t h0 = T::from_f32(v);
       const uint16_t h1 = T::from_f32(T::to_f32(h0) + bias_v);  // second rounding, as a separate add would do
       reinterpret_cast<uint16_t*>(y)[(int64_t)out_m * N + out_row] = bias ? h1 : h0;
@@ -319,25 +355,30 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
   }
 }
 
-template <typename T, int kWaves, int kSteps, int kM, bool kSilu>
+template <typename T, int kWaves, int kSteps, int kM, bool kWide, bool kSilu>
 int launch_oct4(const void* x, int64_t M, const uint32_t* wq, const void* scales, const void* biases, const void* bias,
                 int64_t N, void* y, int y_dtype, hipStream_t stream) {
-  auto kernel = qmv_oct4_kernel<T, kWaves, kSteps, kM, kSilu>;
-  constexpr int kImageBytes = ((2 * kM * (256 * kSteps + 32) + kM * 4 * kSteps * 4) + 255) & ~255;
-  constexpr int kPerBlock = kWaves * (kM > 4 ? kM / 2 * 256 : kM > 2 ? 1024 : 512);
+  auto kernel = qmv_oct4_kernel<T, kWaves, kSteps, kM, kWide, kSilu>;
+  constexpr int kImageBytes = oct_image_bytes(kWide, kM, 4, 256 * kSteps + 32, 4 * kSteps);
+  constexpr int kPerBlock = kWaves * oct_partials(kWide, kM, 4) * 4;
   static PerDeviceInt configured;
   return launch_oct_runs<kWaves, kM>(kernel, configured, kWaves * kImageBytes, kPerBlock, kRows4, kMaxBlocks4, kLongRun4,
                                      x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
 }
 
+// Activation rows the image is built for: 1, 2 or 4, fours with their last row repeated.  More than four rows: a
+// workgroup to every four (eight to one, with a register image twice as large, measured behind on every row length:
+// 256 -> 15360 14.0 against 6.6 us, 3072 -> 18432, where it spills, 35 against 17).
 template <typename T, int kWaves, int kSteps, bool kSilu>
 int launch_oct4_rows(const void* x, int64_t M, const uint32_t* wq, const void* scales, const void* biases,
                      const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream) {
-  if (M == 1) return launch_oct4<T, kWaves, kSteps, 1, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-  if (M == 2) return launch_oct4<T, kWaves, kSteps, 2, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-  if (M <= 4) return launch_oct4<T, kWaves, kSteps, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  constexpr int K = 256 * kWaves * kSteps;
+  if (M == 1) return launch_oct4<T, kWaves, kSteps, 1, false, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  constexpr bool kWide = oct_wide(2, K, 4);
+  if (M == 2) return launch_oct4<T, kWaves, kSteps, 2, kWide, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+  if (M <= 4) return launch_oct4<T, kWaves, kSteps, 4, kWide, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
   if constexpr (!kSilu)
-    return launch_oct4<T, kWaves, kSteps, 8, false>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    return launch_oct4<T, kWaves, kSteps, 4, true, false>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
   return MFQ_EUNSUPPORTED;
 }
 

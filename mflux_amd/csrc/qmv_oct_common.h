@@ -10,10 +10,10 @@ namespace mfq {
 //     one-row kernel of qmv_dot.hip is level or ahead (2560 -> 15360 at 8 bits 9.1 against 9.7, 3840 -> 23040 at 4 bits
 //     10.1 against 10.9) unless a quarter or more of its KiB-sized loads lies past the row's end (256 -> 15360 at 8 bits
 //     4.6 against 3.5 here, 2560 -> 15360 at 4 bits 7.3 against 6.2);
-//   two to four: everywhere (6144 -> 36864 at 8 bits 63.5 -> 38.6, 256 -> 15360 at 4 bits 10.8 -> 3.9);
-//   five and more, against the kernel that dequantises (qmv.hip): 3072 -> 18432 at 8 bits, five rows 19.5 -> 13.3,
-//     sixteen 37.4 -> 25.4; at 4 bits 23.4 -> 11.2 and 60.2 -> 21.6.  Rows of 256 8-bit codes: that kernel
-//     is ahead up to eight rows (4.8 against 5.7), behind from nine (7.7 against 6.5).
+//   two to four: everywhere (6144 -> 36864 at 8 bits 67 -> 40, 256 -> 15360 at 4 bits 11.4 -> 5.9);
+//   five and more, against the kernel that dequantises (qmv.hip): 3072 -> 18432 at 8 bits, five rows 19.7 -> 14.4,
+//     sixteen 36.5 -> 25.8; at 4 bits 23.6 -> 17.0 and 59.9 -> 27.7.  8-bit rows of up to 1024 codes stay there: the
+//     image of x in front of the first block is most of so short a call (1024 -> 6144, five rows 5.4 there, 6.5 here).
 inline bool oct_takes(int64_t M, int64_t K, int bits) {
   if (M < 1 || M > 16) return false;
   const bool even = K == 1024 || K == 2048 || K == 3072 || K == 4096;
@@ -22,17 +22,38 @@ inline bool oct_takes(int64_t M, int64_t K, int bits) {
     const int64_t bytes = K * bits / 8, loads = (bytes + 1023) / 1024;
     return even || 4 * bytes <= 3 * 1024 * loads;
   }
-  return !(K == 256 && bits == 8 && M > 4 && M <= 8);
+  return M <= 4 || bits == 4 || K > 1024;
 }
 
-// Workgroup -> run of weight rows and first activation row.  With two eights of activation rows the two workgroups
-// of a run are eight apart in the grid, on one XCD and at one time, so the second finds the weights in a cache.
+// Whether a call of m rows keeps three bytes of an element of x: the calls that came from kernels on dequantised
+// weights (more than four rows; two to four on row lengths the four-rows kernel does not take), which multiplied x as
+// it is.  With two bytes, float16 rows with one element in 128 at 300 times the others were 3.4e-4 of the norm from
+// float64, 2.0e-4 in those kernels and 2e-7 with three.  The other calls keep the two bytes (15-bit fixed point) of
+// the integer kernels they came from.
+constexpr bool oct_wide(int64_t m, int64_t K, int bits) {
+  return m > 4 || (m > 1 && (K % 1024 != 0 || K > 4096) && !(bits == 8 && K == 256));
+}
+
+// LDS of a wavefront's image of x: its rows and, for every `sums_per_row` groups of 64 k of each, the sum of xq.
+constexpr int oct_image_bytes(bool wide, int m, int bits, int pitch, int sums_per_row) {
+  return ((wide ? 3 : 2) * m * pitch + m * sums_per_row * (bits == 8 ? 8 : 4) + 255) & ~255;
+}
+
+// Floats of partial sums per block and wavefront.  Two bytes: a pair per lane and instruction (8 bits: up to four rows
+// an instruction, 4 bits: two).  Three: one per lane of the useful half (8 bits: two rows an instruction, 4 bits: one).
+constexpr int oct_partials(bool wide, int m, int bits) {
+  if (wide) return 32 * (bits == 8 ? m / 2 : m);
+  return bits == 4 && m > 2 ? 256 : 128;
+}
+
+// Workgroup -> run of weight rows and first activation row.  With more than kM activation rows the workgroups of a run
+// are eight apart in the grid, on one XCD and at one time, so that all but the first find the weights in a cache.
 template <int kM>
 __device__ inline int oct_run_and_first_row(int M, int& run) {
   if (M <= kM) return 0;
-  const int second = (run >> 3) & 1;
-  run = ((run >> 4) << 3) + (run & 7);
-  return second * kM;
+  const int groups = (M + kM - 1) / kM, eight = run >> 3;
+  run = (eight / groups << 3) + (run & 7);
+  return eight % groups * kM;
 }
 
 // x . dequant(W[row]) one k after the other on the weights rounded to the 16-bit type: what an output is whose row
@@ -53,11 +74,12 @@ __device__ __attribute__((noinline)) float oct_plain_dot(const uint16_t* x, cons
   }
   return v;
 }
-
-// Which instantiations do so: the calls that came from kernels on dequantised weights (more than four rows; two to
-// four on row lengths the four-rows kernel does not take).  The others' rows become NaN, as the integer kernels' do.
-constexpr bool oct_keeps_infinities(int m, int K, int bits) {
-  return m > 4 || (m > 1 && (K % 1024 != 0 || K > 4096) && !(bits == 8 && K == 256));
+template <typename T, int BITS, bool kSilu>
+__device__ inline float oct_keep_infinities(bool mine, float v, const uint16_t* x, const uint32_t* wq,
+                                            const uint16_t* scales, const uint16_t* biases, int out_m, int64_t out_row,
+                                            int K, int lane) {
+  if (mine && v != v) v = oct_plain_dot<T, BITS, kSilu>(x + (size_t)out_m * K, wq, scales, biases, out_row, K);
+  return v;
 }
 
 // Launches either kernel on contiguous runs of blocks of weight rows.  kM: activation rows of the instantiation.
@@ -71,10 +93,10 @@ int launch_oct_runs(Kernel kernel, PerDeviceInt& configured, int image_bytes, in
   const int64_t blocks = N / rows;
   // workgroups resident at once: one per compute unit, several where a workgroup is only one or two wavefronts
   const int64_t places = (int64_t)compute_units() * (kWaves <= 2 ? 8 / kWaves : 1);
-  const int64_t groups = kM > 4 ? (M + kM - 1) / kM : 1;
+  const int64_t groups = (M + kM - 1) / kM;
   const int64_t fit = (lds_max - image_bytes) / per_block - 1;
   int64_t per_wg = (blocks * groups + places - 1) / places;
-  if (kM > 4) {
+  if (kM > 4 || groups > 1) {
     // as many equal rounds of workgroups as the room for partial sums asks for
     const int64_t most = fit < max_blocks ? fit : max_blocks;
     const int64_t rounds = (per_wg + most - 1) / most;
@@ -87,7 +109,7 @@ int launch_oct_runs(Kernel kernel, PerDeviceInt& configured, int image_bytes, in
     if (per_wg > fit) per_wg = fit;
   }
   int64_t n_wg = (blocks + per_wg - 1) / per_wg;
-  if (groups > 1) n_wg = (n_wg + 7) / 8 * 8 * groups;  // pairs of workgroups, eight runs at a time
+  if (groups > 1) n_wg = (n_wg + 7) / 8 * 8 * groups;  // the groups of eight runs at a time
   const int lds = image_bytes + ((int)per_wg + 1) * per_block;
   hipLaunchKernelGGL(kernel, dim3((unsigned)n_wg), dim3(64 * kWaves), lds, stream, (const uint16_t*)x,
                      wq, (const uint16_t*)scales, (const uint16_t*)biases, (const uint16_t*)bias, y,

@@ -1,8 +1,8 @@
 """GPU parity: the matvec kernels that take eight weight rows at a time on the
 int8 matrix instruction (csrc/qmv_oct.hip for 8-bit codes, csrc/qmv_oct4.hip
-for 4-bit codes: groups of 64, one to four activation rows, K of 1024 .. 4096
-in steps of 1024, N a multiple of 8) against the float64 oracle on MLX-format
-operands, through the C ABI.
+for 4-bit codes: groups of 64, one to sixteen activation rows, K of 256, 1024,
+2048, 2560, 3072, 3840, 4096 and 6144, N a multiple of 8) against the float64
+oracle on MLX-format operands, through the C ABI.
 
 Tolerance of this path: max |y - y_ref| <= 1e-2 * max|y_ref row| per output
 row; the cases with float32 output show how far inside it the kernel is.
@@ -132,11 +132,11 @@ def test_oct_unit_weight_is_exact(oracle):
 
 
 @pytest.mark.parametrize("bits", [8, 4])
-@pytest.mark.parametrize("K", [256, 1024, 2560, 3072, 3840, 4096, 6144])
+@pytest.mark.parametrize("K", [256, 1024, 2048, 2560, 3072, 3840, 4096, 6144])
 @pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
 def test_oct_row_lengths_and_eights_of_rows(oracle, K, M, bits):
-    """Every split of K over the wavefronts, one image of eight activation rows
-    and two of them (the second with one row and with eight)."""
+    """Every split of K over the wavefronts, and activation rows on two, three and
+    four workgroups of four or one and two of eight (the last with one row and full)."""
     o = oracle
     args = _case(o, 64, M, K, 8 * 261, bits)
     _assert_close(_run(o, *args, bits), _ref(o, *args, bits))
@@ -144,34 +144,36 @@ def test_oct_row_lengths_and_eights_of_rows(oracle, K, M, bits):
 
 @pytest.mark.parametrize("bits", [8, 4])
 @pytest.mark.parametrize("N", [8, 8 * 255, 8 * 256 * 11, 8 * 256 * 13 + 8])
-def test_oct_run_lengths_of_eight_rows(oracle, N, bits):
+@pytest.mark.parametrize("M", [7, 16])
+def test_oct_run_lengths_of_eight_rows(oracle, N, bits, M):
     """Runs of one block, and past what the partial sums of a workgroup hold (two rounds of workgroups)."""
     o = oracle
-    args = _case(o, 65, 7, 1024, N, bits)
+    args = _case(o, 65, M, 1024 if bits == 4 else 2048, N, bits)
     _assert_close(_run(o, *args, bits), _ref(o, *args, bits))
 
 
 @pytest.mark.parametrize("bits", [8, 4])
-def test_oct_infinity_and_nan_stay_in_their_rows(oracle, bits):
+@pytest.mark.parametrize("M,inf,nan", [(6, 1, 4), (16, 12, 15)])
+def test_oct_infinity_and_nan_stay_in_their_rows(oracle, bits, M, inf, nan):
     """More than four rows: an infinity in x gives what the product with the
     dequantised weights gives (its own sign times the weight's), a NaN gives
     NaN, and the other rows are what they are without either."""
     import mflux_amd
 
     torch.manual_seed(66)
-    M, K, N = 6, 3072, 8 * 40
+    K, N = 3072, 8 * 40
     w = (torch.randn(N, K, device="cuda") * 0.02).bfloat16()
     wq, s, b = mflux_amd.quantize(w, 64, bits)
     x = torch.randn(M, K, device="cuda").bfloat16()
     clean = mflux_amd.quantized_matmul(x, wq, s, b, group_size=64, bits=bits)
-    x[1, 700] = float("inf")
-    x[4, 3] = float("nan")
+    x[inf, 700] = float("inf")
+    x[nan, 3] = float("nan")
     y = mflux_amd.quantized_matmul(x, wq, s, b, group_size=64, bits=bits)
     # (in float32: a weight that is zero only after the product's own rounding is not zero to the fma of a matmul)
     column = mflux_amd.dequantize(wq, s, b, 64, bits, dtype=torch.float32)[:, 700]
-    torch.testing.assert_close(y[1].float(), column * float("inf"), rtol=0, atol=0, equal_nan=True)
-    assert bool(torch.isnan(y[4]).all())
-    keep = [0, 2, 3, 5]
+    torch.testing.assert_close(y[inf].float(), column * float("inf"), rtol=0, atol=0, equal_nan=True)
+    assert bool(torch.isnan(y[nan]).all())
+    keep = [m for m in range(M) if m not in (inf, nan)]
     assert torch.equal(y[keep], clean[keep])
 
 
@@ -192,3 +194,55 @@ def test_oct_infinity_of_two_rows_on_the_other_row_lengths(oracle, K, bits, silu
     column = mflux_amd.dequantize(wq, s, b, 64, bits, dtype=torch.float32)[:, 600]
     torch.testing.assert_close(y[1].float(), column * float("inf"), rtol=0, atol=0, equal_nan=True)
     assert bool(torch.isfinite(y[[0, 2]]).all())
+
+
+@pytest.mark.parametrize("K,bits,nan", [(256, 8, True), (256, 4, False), (512, 8, True), (512, 4, True), (1024, 8, True)])
+@pytest.mark.parametrize("M", [2, 4])
+def test_infinity_of_two_to_four_rows(oracle, K, bits, nan, M):
+    """An infinity makes its row NaN in the kernels that hold x in 15 bits, and gives
+    the dequantised weights' infinities in the others."""
+    import mflux_amd
+
+    torch.manual_seed(68)
+    packed = mflux_amd.quantize((torch.randn(8 * 20, K, device="cuda") * 0.02).bfloat16(), 64, bits)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    x[1, 100] = float("inf")
+    y = mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=bits)
+    if nan:
+        assert bool(torch.isnan(y[1]).all())
+    else:
+        column = mflux_amd.dequantize(*packed, 64, bits, dtype=torch.float32)[:, 100]
+        torch.testing.assert_close(y[1].float(), column * float("inf"), rtol=0, atol=0, equal_nan=True)
+    assert bool(torch.isfinite(y[[m for m in range(M) if m != 1]]).all())
+
+
+# K, M, bits of the calls whose rows enter as 23-bit fixed point (the kernels that took them before kept x in
+# its 16-bit type)
+_WIDE = [(K, M, bits) for bits in (4, 8) for K in (256, 1024, 2048, 2560, 3072, 3840, 4096, 6144)
+         for M in (2, 4, 5, 8, 9, 16)
+         if M > 4 and (bits == 4 or K > 1024) or M <= 4 and (K in (2560, 3840, 6144) or (K, bits) == (256, 4))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,M,bits", _WIDE)
+def test_oct_rows_with_outliers_in_float32(K, M, bits, dtype):
+    """One element of every 128 at 300 times the others: the float32 output against
+    float64.  An element enters with an error of 2^-23 of its part's largest at
+    most, as a float32 sum over it would round; 0.6 * 2^-23 * sqrt(128) in the
+    2-norm of a sum that this largest dominates, plus a float32 rounding for
+    each of the partial sums: 2^-18.  (With 15 bits it was 2^-11.5, with weights
+    rounded to 16 bits 2^-9 and 2^-12.)"""
+    import mflux_amd
+
+    torch.manual_seed(70)
+    N = 8 * 33
+    packed = mflux_amd.quantize((torch.randn(N, K, device="cuda") * 0.02).to(dtype), 64, bits)
+    x = torch.randn(M, K, device="cuda")
+    x[:, 5::128] = x[:, 5::128].sign() * 300
+    x = x.to(dtype)
+    y = mflux_amd.quantized_matmul(x.float(), *packed, group_size=64, bits=bits)
+    assert y.dtype == torch.float32 and y.shape == (M, N)
+    ref = x.double() @ mflux_amd.dequantize(*packed, 64, bits, dtype=torch.float32).double().t()
+    # (dequantize rounds in float32 only: 2^-24 of a weight)
+    for m in range(M):
+        assert float((y[m].double() - ref[m]).norm() / ref[m].norm()) <= 2.0 ** -18, m
