@@ -56,29 +56,44 @@ __device__ inline int oct_run_and_first_row(int M, int& run) {
   return eight % groups * kM;
 }
 
-// x . dequant(W[row]) one k after the other on the weights rounded to the 16-bit type: what an output is whose row
-// of x holds an infinity or a NaN, which the integer image cannot.
+// x . dequant(W[row]) on the weights rounded to the 16-bit type: what an output is whose row of x holds an infinity or
+// a NaN, which the integer image cannot.  Called by whole wavefronts: a lane takes every 64th word of codes.
 template <typename T, int BITS, bool kSilu>
 __device__ __attribute__((noinline)) float oct_plain_dot(const uint16_t* x, const uint32_t* wq, const uint16_t* scales,
-                                                         const uint16_t* biases, int64_t row, int K) {
+                                                         const uint16_t* biases, int64_t row, int K, int lane) {
   constexpr int kPerWord = 32 / BITS;
-  const uint32_t* w = wq + row * (K / kPerWord);
+  typedef uint32_t xwords __attribute__((ext_vector_type(kPerWord / 2)));
   float v = 0.f;
-#pragma unroll 1
-  for (int k = 0; k < K; ++k) {
-    const int64_t grp = row * (K / 64) + k / 64;
-    const uint32_t code = (w[k / kPerWord] >> (BITS * (k % kPerWord))) & ((1u << BITS) - 1);
-    const float wv = __builtin_fmaf((float)code, T::to_f32(scales[grp]), T::to_f32(biases[grp]));
-    const uint16_t xv = kSilu ? (uint16_t)silu_pair<T>(x[k]) : x[k];
-    v = __builtin_fmaf(T::to_f32(xv), T::to_f32(T::from_f32(wv)), v);
+#pragma unroll 4
+  for (int k = kPerWord * lane; k < K; k += kPerWord * kWave) {
+    const uint32_t codes = wq[(row * K + k) / kPerWord];
+    const float sc = T::to_f32(scales[(row * K + k) / 64]), bi = T::to_f32(biases[(row * K + k) / 64]);
+    const xwords xv = *reinterpret_cast<const xwords*>(x + k);
+#pragma unroll
+    for (int i = 0; i < kPerWord; ++i) {
+      const float wv = __builtin_fmaf((float)((codes >> (BITS * i)) & ((1u << BITS) - 1)), sc, bi);
+      const uint32_t pair = kSilu ? silu_pair<T>(xv[i / 2]) : xv[i / 2];
+      v = __builtin_fmaf(T::to_f32((uint16_t)(i & 1 ? pair >> 16 : pair)), T::to_f32(T::from_f32(wv)), v);
+    }
   }
+#pragma unroll
+  for (int i = kWave / 2; i > 0; i /= 2) v += __shfl_xor(v, i);
   return v;
 }
+// v, or where it is NaN on a lane whose output is `mine` the above.  The wavefront walks such rows one after the other:
+// with a lane to each, 3072 -> 18432 at 8 bits with an infinity in one row of eight took 778 us (24 without).
 template <typename T, int BITS, bool kSilu>
 __device__ inline float oct_keep_infinities(bool mine, float v, const uint16_t* x, const uint32_t* wq,
                                             const uint16_t* scales, const uint16_t* biases, int out_m, int64_t out_row,
                                             int K, int lane) {
-  if (mine && v != v) v = oct_plain_dot<T, BITS, kSilu>(x + (size_t)out_m * K, wq, scales, biases, out_row, K);
+  uint64_t left = __ballot(mine && v != v);
+  while (left) {
+    const int of = __builtin_ctzll(left);
+    left &= left - 1;
+    const int m = __builtin_amdgcn_readlane(out_m, of), row = __builtin_amdgcn_readlane((int)out_row, of);
+    const float dot = oct_plain_dot<T, BITS, kSilu>(x + (size_t)m * K, wq, scales, biases, row, K, lane);
+    if (lane == of) v = dot;
+  }
   return v;
 }
 

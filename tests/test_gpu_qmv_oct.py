@@ -246,3 +246,31 @@ def test_oct_rows_with_outliers_in_float32(K, M, bits, dtype):
     # (dequantize rounds in float32 only: 2^-24 of a weight)
     for m in range(M):
         assert float((y[m].double() - ref[m]).norm() / ref[m].norm()) <= 2.0 ** -18, m
+
+
+@pytest.mark.parametrize("K,N,M,bits", [(3072, 18432, 8, 8), (3072, 9216, 5, 4), (6144, 36864, 3, 8)])
+def test_oct_time_with_an_infinity(K, N, M, bits):
+    """A row with an infinity is walked again on the dequantised weights, by whole
+    wavefronts: some times the finite call, not the 32 to 50 of a lane to each row."""
+    import mflux_amd
+
+    packed = mflux_amd.quantize((torch.randn(N, K, device="cuda") * 0.02).bfloat16(), 64, bits)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+
+    def us(x):
+        f = lambda: mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=bits)
+        f()
+        best = 1e9
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(10):
+                f()
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 100)
+        return best
+
+    finite = us(x)
+    x[1, 3] = float("inf")
+    assert us(x) < 15 * finite
