@@ -250,6 +250,18 @@ __device__ inline uint32_t silu_pair(uint32_t pair) {
   return out;
 }
 
+// x * sigmoid(x) of a 16-bit float as torch's two operations give it, bit for bit (expf and a division in float32, the
+// sigmoid and the product each rounded to the type).  silu_pair's sigmoid rounds the other way now and then.
+template <typename T>
+__device__ inline uint16_t silu_exact(uint16_t x) {
+  const float v = T::to_f32(x);
+  return T::from_f32(v * T::to_f32(T::from_f32(1.f / (1.f + expf(-v)))));
+}
+template <typename T>
+__device__ inline uint32_t silu_exact_pair(uint32_t pair) {
+  return silu_exact<T>((uint16_t)pair) | (uint32_t)silu_exact<T>((uint16_t)(pair >> 16)) << 16;
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Launch parameters that depend on the device (compute units, resident

@@ -178,8 +178,8 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
 #pragma unroll
     for (int t = 0; t < kChunks; ++t) {
       if constexpr (kSilu) {
-        raw[m][t].x = silu_pair<T>(raw[m][t].x);
-        raw[m][t].y = silu_pair<T>(raw[m][t].y);
+        raw[m][t].x = oct_silu<T, kWide>(raw[m][t].x);
+        raw[m][t].y = oct_silu<T, kWide>(raw[m][t].y);
       }
       amax = max(amax, max(mag_bits(raw[m][t].x), mag_bits(raw[m][t].y)));
     }

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
     for (int t = 0; t < kChunks; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        if constexpr (kSilu) raw[m][t][i] = silu_pair<T>(raw[m][t][i]);
+        if constexpr (kSilu) raw[m][t][i] = oct_silu<T, kWide>(raw[m][t][i]);
         amax = max(amax, mag_bits(raw[m][t][i]));
       }
     amax = oct4_wave_max(amax);

@@ -256,3 +256,23 @@ def test_silu_matvec_five_rows_and_more_is_the_composition(bits, M):
     x = torch.randn(M, 2560, device="cuda").bfloat16()
     y = mflux_amd.silu_quantized_matmul(x, *packed, group_size=64, bits=bits)
     assert torch.equal(y, mflux_amd.quantized_matmul(mflux_amd.silu(x), *packed, group_size=64, bits=bits))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,bits", [(256, 4), (2560, 4), (2560, 8), (3840, 4), (3840, 8), (6144, 4), (6144, 8)])
+@pytest.mark.parametrize("M", [2, 3, 4])
+def test_silu_matvec_two_to_four_rows_on_the_other_row_lengths_is_the_composition(K, bits, M, dtype):
+    """Row lengths of the eight-rows kernels that the four-rows kernel does not take: the separate
+    activation's values (torch's sigmoid and product), bit for bit."""
+    import mflux_amd
+
+    torch.manual_seed(38)
+    w = (torch.randn(520, K, device="cuda") * 0.02).to(dtype)
+    packed = mflux_amd.quantize(w, 64, bits)
+    # every value up to 60000 in order of its bits, so that the values of a row are of one size
+    every = torch.arange(1 << 16, dtype=torch.int32, device="cuda").to(torch.int16).view(dtype)
+    every = every[every.float().abs() < 60000]
+    every = torch.cat([every, every[: -every.numel() % (M * K)]])
+    for x in every.reshape(-1, M, K):
+        y = mflux_amd.silu_quantized_matmul(x, *packed, group_size=64, bits=bits)
+        assert torch.equal(y, mflux_amd.quantized_matmul(mflux_amd.silu(x), *packed, group_size=64, bits=bits))
