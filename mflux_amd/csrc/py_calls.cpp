@@ -9,7 +9,9 @@
 // plain contiguous HIP tensors of one 16-bit type that need no gradient, with
 // nothing intercepting torch calls -- straight to the C ABI of include/mfq.h,
 // and return None for every other case, malformed calls included: the caller
-// then goes through core.py, which handles it or words the error.
+// then goes through core.py, which handles it or words the error.  Whatever can
+// throw (allocations, looking up a pointer or the stream) happens with the
+// interpreter's lock held; without it there is only the C call.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -99,12 +101,22 @@ struct Linear {
     return at::empty(shape, x.options().requires_grad(false));
   }
   Tensor workspace(size_t bytes) const { return at::empty({(int64_t)bytes}, x.options().dtype(at::kByte).requires_grad(false)); }
-  const uint32_t* codes() const { return static_cast<const uint32_t*>(wq.data_ptr()); }
-  const void* bias_ptr() const { return bias.defined() ? bias.data_ptr() : nullptr; }
-  void* stream() const { return c10::hip::getCurrentHIPStream(x.get_device()).stream(); }
+  // where the operands are, for reading only (a copy-on-write tensor stays one)
+  struct Pointers {
+    const void *x, *scales, *biases, *bias;
+    const uint32_t* wq;
+    void* stream;
+  };
+  Pointers pointers() const {
+    return {x.const_data_ptr(), scales.const_data_ptr(), biases.const_data_ptr(),
+            bias.defined() ? bias.const_data_ptr() : nullptr, static_cast<const uint32_t*>(wq.const_data_ptr()),
+            c10::hip::getCurrentHIPStream(x.get_device()).stream()};
+  }
 };
 
-PyObject* result(int rc, const Tensor& y) {
+// y, or None where another route may take the call; a launch that failed is not issued a second time
+PyObject* result(const char* fn, int rc, const Tensor& y) {
+  TORCH_CHECK(rc != MFQ_ELAUNCH, fn, " failed: ", mfq_strerror(rc), " (status ", rc, ")");
   if (rc != MFQ_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(y);
 }
@@ -118,13 +130,14 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Tensor y = p.out(p.N), ws;
   const size_t ws_bytes = mfq_qmm_t_workspace_bytes(p.M, p.K, p.N, (int)p.gs, (int)p.bits);
   if (ws_bytes) ws = p.workspace(ws_bytes);
+  const Linear::Pointers in = p.pointers();
+  void *y_p = y.data_ptr(), *ws_p = ws_bytes ? ws.data_ptr() : nullptr;
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  rc = mfq_qmm_t_ws(p.x.data_ptr(), p.dtype, p.M, p.K, p.codes(), p.scales.data_ptr(), p.biases.data_ptr(), p.dtype,
-                    p.bias_ptr(), p.N, (int)p.gs, (int)p.bits, y.data_ptr(), p.dtype,
-                    ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, p.stream());
+  rc = mfq_qmm_t_ws(in.x, p.dtype, p.M, p.K, in.wq, in.scales, in.biases, p.dtype, in.bias, p.N, (int)p.gs, (int)p.bits,
+                    y_p, p.dtype, ws_p, ws_bytes, in.stream);
   Py_END_ALLOW_THREADS
-  return result(rc, y);
+  return result("mfq_qmm_t_ws", rc, y);
   END_HANDLE_TH_ERRORS
 }
 
@@ -137,19 +150,21 @@ PyObject* silu_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(p.x.device());
   Tensor y = p.out(p.N), s;
   if (p.M > 4) s = p.out(p.K);  // five rows and more: the activation in a launch of its own
+  const Linear::Pointers in = p.pointers();
+  void *y_p = y.data_ptr(), *s_p = p.M > 4 ? s.data_ptr() : nullptr;
   int rc;
   Py_BEGIN_ALLOW_THREADS
   if (p.M > 4) {
-    rc = mfq_silu(p.x.data_ptr(), p.dtype, p.M * p.K, s.data_ptr(), p.stream());
+    rc = mfq_silu(in.x, p.dtype, p.M * p.K, s_p, in.stream);
     if (rc == MFQ_OK)
-      rc = mfq_qmm_t(s.data_ptr(), p.dtype, p.M, p.K, p.codes(), p.scales.data_ptr(), p.biases.data_ptr(), p.dtype,
-                     p.bias_ptr(), p.N, (int)p.gs, (int)p.bits, y.data_ptr(), p.dtype, p.stream());
+      rc = mfq_qmm_t(s_p, p.dtype, p.M, p.K, in.wq, in.scales, in.biases, p.dtype, in.bias, p.N, (int)p.gs, (int)p.bits,
+                     y_p, p.dtype, in.stream);
   } else {
-    rc = mfq_qmv_silu(p.x.data_ptr(), p.dtype, p.M, p.K, p.codes(), p.scales.data_ptr(), p.biases.data_ptr(), p.dtype,
-                      p.bias_ptr(), p.N, (int)p.gs, (int)p.bits, y.data_ptr(), p.dtype, p.stream());
+    rc = mfq_qmv_silu(in.x, p.dtype, p.M, p.K, in.wq, in.scales, in.biases, p.dtype, in.bias, p.N, (int)p.gs,
+                      (int)p.bits, y_p, p.dtype, in.stream);
   }
   Py_END_ALLOW_THREADS
-  return result(rc, y);
+  return result(p.M > 4 ? "mfq_silu, mfq_qmm_t" : "mfq_qmv_silu", rc, y);
   END_HANDLE_TH_ERRORS
 }
 
@@ -174,8 +189,8 @@ PyObject* epilogue_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
         residual.numel() != p.M * p.N || residual.size(-1) != p.N ||
         !residual.sizes().slice(0, residual.dim() - 1).equals(p.x.sizes().slice(0, p.x.dim() - 1)))
       Py_RETURN_NONE;
-    gate_p = gate.data_ptr();
-    residual_p = residual.data_ptr();
+    gate_p = gate.const_data_ptr();
+    residual_p = residual.const_data_ptr();
   } else if (epilogue == MFQ_EPILOGUE_SWIGLU) {
     if (p.N % 64) Py_RETURN_NONE;
   } else if (epilogue != MFQ_EPILOGUE_GELU || act_from < 0 || act_from > p.N || act_from % 8) {
@@ -185,13 +200,15 @@ PyObject* epilogue_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Tensor y = p.out(epilogue == MFQ_EPILOGUE_SWIGLU ? p.N / 2 : p.N), ws;
   const size_t ws_bytes = mfq_qmm_t_workspace_bytes(p.M, p.K, p.N, (int)p.gs, (int)p.bits);
   if (ws_bytes) ws = p.workspace(ws_bytes);
+  const Linear::Pointers in = p.pointers();
+  void *y_p = y.data_ptr(), *ws_p = ws_bytes ? ws.data_ptr() : nullptr;
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  rc = mfq_qmm_t_epilogue(p.x.data_ptr(), p.dtype, p.M, p.K, p.codes(), p.scales.data_ptr(), p.biases.data_ptr(),
-                          p.dtype, p.bias_ptr(), p.N, (int)p.gs, (int)p.bits, (int)epilogue, gate_p, residual_p,
-                          act_from, y.data_ptr(), p.dtype, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, p.stream());
+  rc = mfq_qmm_t_epilogue(in.x, p.dtype, p.M, p.K, in.wq, in.scales, in.biases, p.dtype, in.bias, p.N, (int)p.gs,
+                          (int)p.bits, (int)epilogue, gate_p, residual_p, act_from, y_p, p.dtype, ws_p, ws_bytes,
+                          in.stream);
   Py_END_ALLOW_THREADS
-  return result(rc, y);
+  return result("mfq_qmm_t_epilogue", rc, y);
   END_HANDLE_TH_ERRORS
 }
 

@@ -81,3 +81,36 @@ def test_everything_else_is_left_to_the_general_route():
     xg = x.clone().requires_grad_(True)
     layer(xg).sum().backward()
     assert xg.grad is not None
+
+
+def test_inputs_are_only_read():
+    """A lazily cloned (copy-on-write) input stays one: only the output is written."""
+    from mflux_amd import _lib
+
+    layer = _layer(256, 192, 8)
+    w = layer._operands()
+    n = _lib.native()
+    for M in (1, 6, 40):
+        x = torch.randn(M, 256, device="cuda", dtype=torch.bfloat16)
+        lazy = torch._lazy_clone(x)
+        res, gate = torch.randn(M, 192, device="cuda", dtype=x.dtype), torch.randn(192, device="cuda", dtype=x.dtype)
+        lazy_res = torch._lazy_clone(res)
+        assert torch.equal(n.linear(lazy, *w, 64, 8), n.linear(x, *w, 64, 8))
+        if M <= 16:
+            n.silu_linear(lazy, *w, 64, 8)
+        else:
+            n.epilogue_linear(lazy, *w, 64, 8, _lib.EPILOGUE_GATE_RESIDUAL, gate, lazy_res, 0)
+        assert torch._C._is_cow_tensor(lazy) and torch._C._is_cow_tensor(lazy_res)
+
+
+@pytest.mark.parametrize("epilogue,act_from", [("gelu", 0), ("gelu", 72), ("swiglu", 0)])
+@pytest.mark.parametrize("bits", [4, 6, 8])
+def test_epilogues_same_bits_as_the_operator(epilogue, act_from, bits):
+    from mflux_amd import _lib, core
+
+    layer = _layer(256, 192, bits)
+    x = torch.randn(2, 20, 256, device="cuda", dtype=torch.bfloat16)
+    w = layer._operands()
+    got = _lib.native().epilogue_linear(x, *w, 64, bits, core.EPILOGUES[epilogue], None, None, act_from)
+    ref, ok = _lib.ops().qmm_t_epilogue(x.reshape(-1, 256), *w, 64, bits, core.EPILOGUES[epilogue], None, None, act_from)
+    assert ok and got.shape == (2, 20, ref.shape[-1]) and torch.equal(got, ref.reshape(got.shape))
