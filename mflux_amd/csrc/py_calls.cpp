@@ -11,12 +11,14 @@
 // and return None for every other case, malformed calls included: the caller
 // then goes through core.py, which handles it or words the error.  Whatever can
 // throw (allocations, looking up a pointer or the stream) happens with the
-// interpreter's lock held; without it there is only the C call.
+// interpreter's lock held; without it there is only the C call.  A profiler sees
+// the operator that the call stands for.
 #include <Python.h>
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <ATen/record_function.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -101,6 +103,8 @@ struct Linear {
     return at::empty(shape, x.options().requires_grad(false));
   }
   Tensor workspace(size_t bytes) const { return at::empty({(int64_t)bytes}, x.options().dtype(at::kByte).requires_grad(false)); }
+  std::vector<c10::IValue> inputs() const { return {x, wq, scales, biases, bias, gs, bits}; }  // for a profiler
+
   // where the operands are, for reading only (a copy-on-write tensor stays one)
   struct Pointers {
     const void *x, *scales, *biases, *bias;
@@ -126,7 +130,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Linear p;
   if (n != 7 || !p.parse(args)) Py_RETURN_NONE;
-  const c10::hip::HIPGuardMasqueradingAsCUDA guard(p.x.device());
+  RECORD_FUNCTION("mfq::qmm_t", p.inputs());
+  const c10::hip::HIPGuardMasqueradingAsCUDA on_device(p.x.device());
   Tensor y = p.out(p.N), ws;
   const size_t ws_bytes = mfq_qmm_t_workspace_bytes(p.M, p.K, p.N, (int)p.gs, (int)p.bits);
   if (ws_bytes) ws = p.workspace(ws_bytes);
@@ -147,7 +152,8 @@ PyObject* silu_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Linear p;
   if (n != 7 || !p.parse(args)) Py_RETURN_NONE;
   if (p.M > 16 || (p.bits != 4 && p.bits != 8)) Py_RETURN_NONE;
-  const c10::hip::HIPGuardMasqueradingAsCUDA guard(p.x.device());
+  RECORD_FUNCTION(p.M > 4 ? "mfq::qmm_t" : "mfq::qmv_silu", p.inputs());
+  const c10::hip::HIPGuardMasqueradingAsCUDA on_device(p.x.device());
   Tensor y = p.out(p.N), s;
   if (p.M > 4) s = p.out(p.K);  // five rows and more: the activation in a launch of its own
   const Linear::Pointers in = p.pointers();
@@ -196,7 +202,8 @@ PyObject* epilogue_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   } else if (epilogue != MFQ_EPILOGUE_GELU || act_from < 0 || act_from > p.N || act_from % 8) {
     Py_RETURN_NONE;
   }
-  const c10::hip::HIPGuardMasqueradingAsCUDA guard(p.x.device());
+  RECORD_FUNCTION("mfq::qmm_t_epilogue", p.inputs());
+  const c10::hip::HIPGuardMasqueradingAsCUDA on_device(p.x.device());
   Tensor y = p.out(epilogue == MFQ_EPILOGUE_SWIGLU ? p.N / 2 : p.N), ws;
   const size_t ws_bytes = mfq_qmm_t_workspace_bytes(p.M, p.K, p.N, (int)p.gs, (int)p.bits);
   if (ws_bytes) ws = p.workspace(ws_bytes);

@@ -103,6 +103,23 @@ def test_inputs_are_only_read():
         assert torch._C._is_cow_tensor(lazy) and torch._C._is_cow_tensor(lazy_res)
 
 
+def test_profiler_lists_the_calls():
+    """A torch profile of module calls names the operators, as when they go through the dispatcher."""
+    from torch.profiler import ProfilerActivity, profile
+
+    import mflux_amd
+    from mflux_amd import nn
+
+    layer = _layer(256, 192, 8)
+    x = torch.randn(40, 256, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad(), profile(activities=[ProfilerActivity.CPU]) as prof:
+        layer(x)
+        nn.silu_linear(layer, x[:1])
+        nn.gelu_linear(layer, x)
+    names = {e.name for e in prof.events()}
+    assert {"mfq::qmm_t", "mfq::qmv_silu", "mfq::qmm_t_epilogue"} <= names
+
+
 @pytest.mark.parametrize("epilogue,act_from", [("gelu", 0), ("gelu", 72), ("swiglu", 0)])
 @pytest.mark.parametrize("bits", [4, 6, 8])
 def test_epilogues_same_bits_as_the_operator(epilogue, act_from, bits):
