@@ -99,6 +99,13 @@ def ops():
 _native = None
 
 
+class _NotBuilt:
+    """Stands in for the C functions where the libraries are not built: every call takes the
+    general route, which words argument errors first and then says what is missing."""
+
+    linear = silu_linear = epilogue_linear = staticmethod(lambda *args: None)
+
+
 def native():
     """The Python C functions of csrc/py_calls.cpp, which live in the same library
     as the ops: ``linear``, ``silu_linear`` and ``epilogue_linear`` take the
@@ -109,6 +116,8 @@ def native():
         import importlib.machinery
         import importlib.util
 
+        if not (os.path.exists(LIB_PATH) and os.path.exists(OPS_PATH)):
+            return _NotBuilt
         ops()
         loader = importlib.machinery.ExtensionFileLoader("libmfq_torch", OPS_PATH)
         spec = importlib.util.spec_from_file_location("libmfq_torch", OPS_PATH, loader=loader)

@@ -45,6 +45,27 @@ def test_no_cpu_fallback():
         mflux_amd.dequantize(wq, s, s)
 
 
+def test_argument_errors_without_the_built_libraries(monkeypatch):
+    """Arguments are checked, and worded, before a library is looked for."""
+    from mflux_amd import _lib
+
+    for name in ("_lib", "_ops", "_native"):
+        monkeypatch.setattr(_lib, name, None)
+    for name in ("LIB_PATH", "OPS_PATH"):
+        monkeypatch.setattr(_lib, name, "/nowhere/" + name)
+    wq = torch.zeros(8, 16, dtype=torch.uint32)
+    s = torch.zeros(8, 2, dtype=torch.bfloat16)
+    x = torch.zeros(2, 128, dtype=torch.bfloat16)
+    for f in (mflux_amd.quantized_matmul, mflux_amd.silu_quantized_matmul,
+              lambda *a, **k: mflux_amd.core.quantized_matmul_epilogue(*a, epilogue="gelu", **k)):
+        with pytest.raises(ValueError, match="incompatible"):
+            f(x, wq, s, s, bits=8)
+        with pytest.raises(ValueError, match="group size 48 is not supported"):
+            f(x, wq, s, s, group_size=48)
+    with pytest.raises(RuntimeError, match="no CPU fallback"):
+        mflux_amd.quantized_matmul(x, wq, s, s)
+
+
 def test_quantized_matmul_shape_errors():
     wq = torch.zeros(8, 16, dtype=torch.uint32)
     s = torch.zeros(8, 2, dtype=torch.bfloat16)
