@@ -133,7 +133,7 @@ int mfq_dequantize_rows(const uint32_t* wq, const void* scales, const void* bias
  * tiles), and below 1024 rows where an estimate of both finds them faster;
  * 256 x 256 tiles otherwise.  3, 5 and 6 bits: one activation row of up to 8192
  * elements has its own kernel, everything else runs on the 128-column-tile GEMM.
- * Sums are float32, on dequantised weights rounded once to x_dtype -- except in
+ * Sums are float32, on dequantised weights rounded at most once, to x_dtype -- except in
  * the integer matvec kernels of 4 and 8 bits, where x becomes fixed point (one
  * power of two per row, or per part of a row that a wavefront multiplies, from
  * its largest magnitude), the integer products with the raw codes are exact, and
@@ -334,9 +334,11 @@ int mfq_qmm_t_static(const void* x, int x_dtype, int64_t M, int64_t K, const uin
  * MFQ_EUNSUPPORTED when no fused kernel takes the shape (bits other than 4
  * and 8; M = 1 with rows of more than 6 KiB of 8-bit or 3 KiB of 4-bit codes;
  * M = 2..4 outside what the eight-rows kernels (K = 256, 1024, 2048, 2560,
- * 3072, 3840, 4096 or 6144, group size 64, N a multiple of 8) and the four-rows kernel (K <= 4096, N a
- * multiple of 4, rows of 1, 2, 3, 4, 6, 8, 12 or 16 times 256 bytes) take;
- * M > 4): apply the activation separately and call mfq_qmm_t.
+ * 3072, 3840, 4096 or 6144, group size 64, N a multiple of 8) and the four-rows
+ * kernel (K <= 4096, N a multiple of 4, rows of 1, 2, 3, 4, 6, 8, 12 or 16
+ * times 256 bytes) take; M > 4): apply the activation separately and call
+ * mfq_qmm_t.  The sigmoid is hardware exponential and reciprocal, rounded to the
+ * type (where x enters in 23 bits: mfq_silu's values).
  */
 int mfq_qmv_silu(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq,
                  const void* scales, const void* biases, int sb_dtype, const void* bias, int64_t N,

@@ -8,9 +8,10 @@ quantized ``nn.Linear`` call such as
 src/mflux/models/flux/model/flux_transformer/single_transformer_block.py:53,57.
 
 Tensors are torch tensors on a HIP device; torch only provides the device
-memory and the stream, the arithmetic is libmfq's hand-written kernels, reached
-through the ``torch.ops.mfq`` ops of csrc/torch_ops.cpp (a thin C++ layer over
-the C ABI of include/mfq.h).
+memory and the stream, the arithmetic is libmfq's hand-written kernels.  The
+ordinary call of a quantized linear reaches the C ABI of include/mfq.h through
+the C functions of csrc/py_calls.cpp, everything else through the
+``torch.ops.mfq`` ops of csrc/torch_ops.cpp.
 """
 from __future__ import annotations
 

@@ -364,8 +364,9 @@ bool qmv_quad_covers(int64_t M, int64_t K, int64_t N, int gs, int bits, const vo
 int launch_qmv_quad(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                     const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
                     hipStream_t stream, bool silu = false);
-// one to sixteen activation rows (four with `silu`, and at rows of up to 1024 codes), 8-bit codes: eight weight rows at a time on the int8 16x16x64
-// matrix instruction, K split over the wavefronts of a workgroup (qmv_oct_covers() says whether it takes a shape)
+// one to sixteen activation rows (four with `silu`, and with weight rows of up to 1024 codes), 8-bit codes: eight weight
+// rows at a time on the int8 16x16x64 matrix instruction, K split over the wavefronts of a workgroup
+// (qmv_oct_covers() says whether it takes a shape)
 bool qmv_oct_covers(int64_t M, int64_t K, int64_t N, int gs, int bits, const void* x, const void* scales,
                     const void* biases);
 int launch_qmv_oct(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
@@ -392,8 +393,9 @@ int launch_qmm_epilogue(const void* x, int dtype, int64_t M, int64_t K, const ui
                         void* workspace, size_t workspace_bytes, hipStream_t stream, Epilogue epi);
 // y[M, N] += t @ bs^T, rounded to y's type (dtype: the type of t, bs and a 16-bit y)
 int launch_low_rank_add(int dtype, LowRank low_rank, int64_t M, int64_t N, void* y, int y_dtype, hipStream_t stream);
-// t[M, R] = x[M, K] @ A[K, R], A in fragment order ([R/16][K/32][4][16][8]); 16-bit type `dtype`; R % 16 == 0, K % 32 == 0
+// y[i] = silu(x[i]), the sigmoid and the product each rounded to the 16-bit type
 int launch_silu(const void* x, int dtype, int64_t n, void* y, hipStream_t stream);
+// t[M, R] = x[M, K] @ A[K, R], A in fragment order ([R/16][K/32][4][16][8]); 16-bit type `dtype`; R % 16 == 0, K % 32 == 0
 int launch_low_rank_down(const void* x, int dtype, int64_t M, int64_t K, const void* at, int64_t R, void* t,
                          hipStream_t stream);
 // what a caller should bring (the K split's planes, or the scratch copy of the two-kernel path where that is

@@ -55,7 +55,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // group covers all 64 banks.  The lanes of a matrix fragment (row lane % 16, column 2 (lane / 16) + pass) put two
 // columns that differ in bit 1 into a group, so the rows 0-3, 12-15 and the rows 4-11 need column masks that are
 // each closed under an XOR with 2: i -> (i2, i0, i2 ^ i1).  With plain bits 1..3, as for the 32-row fragments of
-// qmm.hip, every fragment read met a two-way conflict (126 instead of 248 bytes per clock and compute unit).
+// qmm.hip, every fragment read met a two-way conflict (126 instead of 248 bytes per clock and compute unit for the reads
+// by themselves; the calls, which are bound elsewhere, are level).
 __host__ __device__ inline int swz_mask(int row) {
   const int i = (row >> 1) & 7;
   return (i & 4) | ((i & 1) << 1) | ((i >> 2) ^ ((i >> 1) & 1));
@@ -345,7 +346,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
       woff[j] = nb * (uint32_t)steps_total * (uint32_t)kBlockBytes + (uint32_t)lane * 16u;
     }
     // lane l of a direct load lands in LDS at 16 l past the load's base: row l / 8 of the wavefront's eight,
-    // 16-byte slot l % 8, which in the swizzled tile holds the row's piece (l % 8) ^ ((row / 2) % 8)
+    // 16-byte slot l % 8, which in the swizzled tile holds the row's piece (l % 8) ^ swz_mask(row)
     const uint32_t piece = (uint32_t)((t & 7) ^ swz_mask(t >> 3));  // 32 i rows further on: the same
 #pragma unroll
     for (int i = 0; i < 8; ++i)

@@ -11,9 +11,9 @@ Around a ``QuantizedLinear`` base on the GPU, at inference, the whole layer is
 one call of the quantized matmul: the adapters' down-projections are
 concatenated into one ``[K, R]`` matrix (one small library GEMM gives ``t = x @ A``),
 the scaled up-projections into one ``[N, R]`` matrix, and the kernel treats
-them as ``R`` more ``k`` of the same product.  When gradients are needed, or
-the base is not quantized, the layer is the reference's composition of
-separate matmuls.
+them as ``R`` more ``k`` of the same product.  With gradients one adapter on a
+quantized base keeps that form (``_LoRALinearFunction``); anything else, and a
+base that is not quantized, is the reference's composition of separate matmuls.
 """
 from __future__ import annotations
 
