@@ -216,13 +216,20 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
   // this lane's A operands, pass p.  Two bytes: image row j % 8 over half j / 8 of every step (image rows past 2 kM:
   // any row, their results are never read).  Three: activation row 2 p + (j % 8) / 4, byte j % 4 (the fourth: the
   // third again, never read).
-  i32x4 xa[kPasses][kSteps];
+  // They stay in registers up to twelve of them (each four); otherwise every block reads them again, four times its
+  // weights' bytes, a third of what the LDS delivers in the time the weights take (4096 -> 24576, eight rows: 25.8 us,
+  // 29.0 on two workgroups of four).
+  constexpr bool kHeld = kPasses * kSteps <= 12;
+  const int arow = (kWide ? 3 * ((j >> 2) & 1) + min(j & 3, 2) : j & 7 & (kImageRows - 1)) * kPitch + 64 * (j >> 3) + 16 * q;
+  i32x4 xa[kHeld ? kPasses : 1][kHeld ? kSteps : 1];
+  const auto a_operand = [&](int p, int s) __attribute__((always_inline)) {
+    return *reinterpret_cast<const i32x4*>(image + arow + 6 * p * kPitch + 128 * s);
+  };
+  if constexpr (kHeld) {
 #pragma unroll
-  for (int p = 0; p < kPasses; ++p) {
-    const int r = kWide ? 3 * (2 * p + ((j >> 2) & 1)) + min(j & 3, 2) : j & 7 & (kImageRows - 1);
-    const char* arow = image + r * kPitch + 64 * (j >> 3) + 16 * q;
+    for (int p = 0; p < kPasses; ++p)
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) xa[p][s] = *reinterpret_cast<const i32x4*>(arow + 128 * s);
+      for (int s = 0; s < kSteps; ++s) xa[p][s] = a_operand(p, s);
   }
   // results: register r of lane (j, q) is A's row 4 q + r against column j.  Of use where q / 2 == j % 2.  Two bytes:
   // activation rows 2 (q % 2) (registers 0, 1: high, low bytes) and 2 (q % 2) + 1 (registers 2, 3); three:
@@ -280,7 +287,10 @@ __global__ __launch_bounds__(64 * kWaves) void qmv_oct_kernel(
 #pragma unroll
       for (int p = 0; p < kPasses; ++p) {
         const i32x4 zero = {0, 0, 0, 0};
-        const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[p][s], wb, zero, 0, 0, 0);
+        i32x4 a;
+        if constexpr (kHeld) a = xa[p][s];
+        else a = a_operand(p, s);
+        const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, wb, zero, 0, 0, 0);
         if constexpr (kWide) {
           // sum(xq code) over the half step's group: high and lower bytes exact, joined in float32
           const int dl = d[1] * 256 + d[2] + sx128_a[p][s], dh = d[0] + sx128_b[p][s];
@@ -393,7 +403,8 @@ int launch_oct_rows(const void* x, int64_t M, const uint32_t* wq, const void* sc
 }
 
 // The split of K: wavefronts times 128-byte steps of each, and the rows a workgroup takes of more than four: eight where
-// their image fits the registers (10 x 3: 168 of them, 78 us of spills instead of 31), 0 where oct_takes() ends at four.
+// that fits (10 x 3: 168 registers to a wavefront, 78 us of spills instead of 31, and no less from LDS; 8 x 6: no room in
+// LDS for more than two blocks' sums), 0 where oct_takes() ends at four.
 template <typename T, bool kSilu>
 int launch_oct_steps(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* scales, const void* biases,
                      const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream) {
@@ -404,7 +415,7 @@ int launch_oct_steps(const void* x, int64_t M, int64_t K, const uint32_t* wq, co
     case 2560: return launch_oct_rows<T, 10, 2, 8, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     case 3072: return launch_oct_rows<T, 8, 3, 8, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     case 3840: return launch_oct_rows<T, 10, 3, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
-    case 4096: return launch_oct_rows<T, 8, 4, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    case 4096: return launch_oct_rows<T, 8, 4, 8, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     case 6144: return launch_oct_rows<T, 8, 6, 4, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
     default: return MFQ_EUNSUPPORTED;
   }

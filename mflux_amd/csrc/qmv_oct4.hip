@@ -25,7 +25,7 @@
 // that multiplied x as it is before (oct_wide()) keep three bytes of it: A's row
 // 8 h + 4 g + l is byte l of ONE activation row, and d = 65536 D_high + 256 D_mid + D_low
 // is put together in float32.  More than four activation rows take a workgroup to every
-// four.  3072 -> 18432 takes 7.4 us with one row, 8.4 with four, 17 with eight, where
+// three or four.  3072 -> 18432 takes 7.4 us with one row, 8.4 with four, 17 with eight, where
 // the vector instructions of the bytes are as long as the loads (31 on the kernel that
 // dequantises).  Work layout, register sets, the meeting of the wavefronts' partial sums
 // at the end: qmv_oct.hip's, with K split over kWaves wavefronts.
@@ -75,7 +75,7 @@ struct ScaleWindow4 {
 };
 
 // kWaves: wavefronts per workgroup, each with kSteps 128-byte steps of every row (K = 256 kWaves kSteps codes);
-// kM: activation rows the image is built for (1, 2, 4 or 8; other M run as the next of these with their last row repeated, more than
+// kM: activation rows the image is built for (1, 2, 3 or 4; other M run as the next of these with their last row repeated, more than
 // kM on several workgroups).  kWide: three bytes per element of x instead of two.
 template <typename T, int kWaves, int kSteps, int kM, bool kWide, bool kSilu>
 __global__ __launch_bounds__(64 * kWaves) void qmv_oct4_kernel(
@@ -367,8 +367,9 @@ int launch_oct4(const void* x, int64_t M, const uint32_t* wq, const void* scales
 }
 
 // Activation rows the image is built for: 1, 2 or 4, fours with their last row repeated.  More than four rows: a
-// workgroup to every four (eight to one, with a register image twice as large, measured behind on every row length:
-// 256 -> 15360 14.0 against 6.6 us, 3072 -> 18432, where it spills, 35 against 17).
+// workgroup to every four, or to every three where that makes no more of them (five rows of 3072 -> 18432: 14.8 us, 17.7
+// in fours).  Eight to one, with a register image twice as large, measured behind on every row length: 256 -> 15360 14.0
+// against 6.6 us, 3072 -> 18432, where it spills, 35 against 17.
 template <typename T, int kWaves, int kSteps, bool kSilu>
 int launch_oct4_rows(const void* x, int64_t M, const uint32_t* wq, const void* scales, const void* biases,
                      const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream) {
@@ -378,7 +379,9 @@ int launch_oct4_rows(const void* x, int64_t M, const uint32_t* wq, const void* s
   if (M == 2) return launch_oct4<T, kWaves, kSteps, 2, kWide, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
   if (M <= 4) return launch_oct4<T, kWaves, kSteps, 4, kWide, kSilu>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
   if constexpr (!kSilu)
-    return launch_oct4<T, kWaves, kSteps, 4, true, false>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
+    return (M + 2) / 3 == (M + 3) / 4
+               ? launch_oct4<T, kWaves, kSteps, 3, true, false>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream)
+               : launch_oct4<T, kWaves, kSteps, 4, true, false>(x, M, wq, scales, biases, bias, N, y, y_dtype, stream);
   return MFQ_EUNSUPPORTED;
 }
 

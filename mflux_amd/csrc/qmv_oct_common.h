@@ -12,7 +12,7 @@ namespace mfq {
 //     4.6 against 3.5 here, 2560 -> 15360 at 4 bits 7.3 against 6.2);
 //   two to four: everywhere (6144 -> 36864 at 8 bits 67 -> 40, 256 -> 15360 at 4 bits 11.4 -> 5.9);
 //   five and more, against the kernel that dequantises (qmv.hip): 3072 -> 18432 at 8 bits, five rows 19.7 -> 14.4,
-//     sixteen 36.5 -> 25.8; at 4 bits 23.6 -> 17.0 and 59.9 -> 27.7.  8-bit rows of up to 1024 codes stay there: the
+//     sixteen 36.5 -> 25.8; at 4 bits 23.6 -> 14.8 and 59.9 -> 27.7.  8-bit rows of up to 1024 codes stay there: the
 //     image of x in front of the first block is most of so short a call (1024 -> 6144, five rows 5.4 there, 6.5 here).
 inline bool oct_takes(int64_t M, int64_t K, int bits) {
   if (M < 1 || M > 16) return false;
