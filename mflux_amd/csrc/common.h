@@ -90,17 +90,32 @@ __device__ inline float hi_f32(uint32_t p) { return T::to_f32((uint16_t)(p >> 16
 // byte j of a word as float (selects v_cvt_f32_ubyte{j})
 __device__ inline float ubyte_f32(uint32_t w, int j) { return (float)((w >> (8 * j)) & 0xffu); }
 
+// Two 4-bit codes in neighbouring bytes (the low two of `w`, or with kHigh the high two) as floats, in one instruction:
+// a byte n = 0 .. 15 read as an 8-bit e4m3 float is n 2^-9 (denormal up to 7, exponent 1 from 8 on), so the conversion
+// of a pair of those, scaled by 2^9, gives n exactly.  v_cvt_f32_ubyte converts one byte in the same time (8 cycles of a
+// lone wavefront, 4.4 of several), and every vector instruction more than two per matrix instruction is paid for in
+// full (an iteration of 4 v_mfma_16x16x32 with 8, 12, 16 vector instructions: 28.6, 36.2, 43.6 ns).  With a conversion
+// for every code, and the bit-field extract the compiler put in front of each, 320 rows x 3584 -> 37888 -> 3584 took
+// 210.5 us on the 128-column-tile kernel, 203.9 with pairs.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+template <bool kHigh>
+__device__ inline f32x2 nibble_pair_f32(uint32_t w) {
+  return __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w, 512.0f, kHigh);
+}
+
 // Dequantise 8 consecutive codes into 8 packed 16-bit elements:
 // value = fma(code, scale, bias) in float32, rounded once to T.
 template <typename T>
 __device__ inline uint4 dequant8_w4(uint32_t word, float s, float b) {
   const uint32_t even = word & 0x0f0f0f0fu;         // codes 0,2,4,6 in bytes 0..3
   const uint32_t odd = (word >> 4) & 0x0f0f0f0fu;   // codes 1,3,5,7
+  const f32x2 e0 = nibble_pair_f32<false>(even), o0 = nibble_pair_f32<false>(odd);
+  const f32x2 e1 = nibble_pair_f32<true>(even), o1 = nibble_pair_f32<true>(odd);
   uint4 r;
-  r.x = T::pack2(__builtin_fmaf(ubyte_f32(even, 0), s, b), __builtin_fmaf(ubyte_f32(odd, 0), s, b));
-  r.y = T::pack2(__builtin_fmaf(ubyte_f32(even, 1), s, b), __builtin_fmaf(ubyte_f32(odd, 1), s, b));
-  r.z = T::pack2(__builtin_fmaf(ubyte_f32(even, 2), s, b), __builtin_fmaf(ubyte_f32(odd, 2), s, b));
-  r.w = T::pack2(__builtin_fmaf(ubyte_f32(even, 3), s, b), __builtin_fmaf(ubyte_f32(odd, 3), s, b));
+  r.x = T::pack2(__builtin_fmaf(e0[0], s, b), __builtin_fmaf(o0[0], s, b));
+  r.y = T::pack2(__builtin_fmaf(e0[1], s, b), __builtin_fmaf(o0[1], s, b));
+  r.z = T::pack2(__builtin_fmaf(e1[0], s, b), __builtin_fmaf(o1[0], s, b));
+  r.w = T::pack2(__builtin_fmaf(e1[1], s, b), __builtin_fmaf(o1[1], s, b));
   return r;
 }
 
