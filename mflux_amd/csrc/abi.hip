@@ -97,7 +97,9 @@ size_t mfq_qmm_t_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size
   if (bits != 4 && bits != 8) {
     if (M <= 1) return 0;
     if (mfq::prefer_frag_path(M, N, K, group_size, bits)) return mfq::qmm_workspace_bytes(M, N, K, group_size, bits);
-    return mfq::qmm_mid_workspace_bytes(M, N, K, group_size);
+    const size_t planes = mfq::qmm_mid_workspace_bytes(M, N, K, group_size);
+    const size_t slice = mfq::qmm_slice_workspace_bytes(M, N, K, group_size, bits);
+    return planes > slice ? planes : slice;
   }
   if (M <= 16) return 0;
   return mfq::qmm_workspace_bytes(M, N, K, group_size, bits);
@@ -123,7 +125,7 @@ int mfq_qmm_t_static(const void* x, int x_dtype, int64_t M, int64_t K, const uin
   if (int rc = check_common(group_size, bits)) return rc;
   size_t need = mfq_qmm_t_workspace_bytes(M, K, N, group_size, bits);
   // a scratch copy of the weights that does not fit is done without (the fused kernel); the planes of a K split are not
-  if (need > kScratchBytes && (bits == 4 || bits == 8) && M > 16) need = mfq::qmm_min_workspace_bytes(M, N, K, group_size);
+  if (need > kScratchBytes && (bits == 4 || bits == 8) && M > 16) need = mfq::qmm_min_workspace_bytes(M, N, K, group_size, bits);
   if (need > kScratchBytes) return MFQ_ESCRATCH;
   void* ws = nullptr;
   if (need) {

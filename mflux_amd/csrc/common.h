@@ -416,7 +416,7 @@ int launch_low_rank_down(const void* x, int dtype, int64_t M, int64_t K, const v
 // what a caller should bring (the K split's planes, or the scratch copy of the two-kernel path where that is
 // preferred) and what the call cannot do without (the planes only)
 size_t qmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits);
-size_t qmm_min_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs);
+size_t qmm_min_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits);
 // the two-kernel path (qmm_frag.hip): dequantize once into a 16-bit copy in fragment order, then a GEMM on
 // 16x16x32 matrix instructions; 4 and 8 bits, 16-bit y of x's type, a low-rank update or an epilogue as
 // launch_qmm / launch_qmm_epilogue.
@@ -459,8 +459,15 @@ int launch_qmm_mid(const void* x, int dtype, int64_t M, int64_t K, const uint32_
                    const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
                    void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank = LowRank(),
                    Epilogue epi = Epilogue());
-// what launch_qmm_mid is estimated to take (groups of 64)
-float qmm_mid_estimate_us(int64_t M, int64_t N, int64_t K);
+// what launch_qmm_mid is estimated to take
+float qmm_mid_estimate_us(int64_t M, int64_t N, int64_t K, int gs);
+// 64- or 32-row tiles with K whole, for shapes with too few of the 128-column tiles (qmm_slice.hip): all bit widths.
+// MFQ_EUNSUPPORTED where that is not estimated to be the faster, or the alignment is wrong; workspace as launch_qmm_mid's
+int launch_qmm_slice(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
+                     const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
+                     void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank = LowRank(),
+                     Epilogue epi = Epilogue());
+size_t qmm_slice_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits);
 size_t qmm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs);
 // the same kernel for 3, 5 and 6 bits (any M above one row; K % 32 == 0)
 int launch_qmm_mid_stream(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,

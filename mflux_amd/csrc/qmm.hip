@@ -1146,7 +1146,7 @@ bool use_mid_kernel(int64_t M, int64_t N, int64_t K) {
   const float step_us = 1.68f * (float)((K + BK - 1) / BK);
   const int64_t rest = tiles % cus;
   const float tail = rest == 0 ? 0.f : rest * 2 > cus ? step_us : 0.5f * step_us + 10.f;
-  return qmm_mid_estimate_us(M, N, K) < 0.9f * (step_us * (float)(tiles / cus) + tail);
+  return qmm_mid_estimate_us(M, N, K, 64) < 0.9f * (step_us * (float)(tiles / cus) + tail);
 }
 
 #ifndef MFQ_ODD_FRAG_ROWS
@@ -1164,14 +1164,17 @@ bool prefer_frag_path(int64_t M, int64_t N, int64_t K, int gs, int bits) {
   return M >= least_rows && qmm_frag_shape_ok(M, N, K, bits) && !use_mid_kernel(M, N, K);
 }
 
-size_t qmm_min_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs) {
+size_t qmm_min_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits) {
   if (K % BK) return 0;
-  if (use_mid_kernel(M, N, K)) return qmm_mid_workspace_bytes(M, N, K, gs);
-  return tail_plane_bytes(M, N, plan_tail(M, N, K, period_of(gs), compute_units()));
+  const size_t planes = use_mid_kernel(M, N, K) ? qmm_mid_workspace_bytes(M, N, K, gs)
+                                                : tail_plane_bytes(M, N, plan_tail(M, N, K, period_of(gs), compute_units()));
+  // (not the smaller of the two: a misaligned operand or an epilogue may still send the call to the other kernels)
+  const size_t slice = qmm_slice_workspace_bytes(M, N, K, gs, bits);
+  return planes > slice ? planes : slice;
 }
 
 size_t qmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits) {
-  const size_t planes = qmm_min_workspace_bytes(M, N, K, gs);
+  const size_t planes = qmm_min_workspace_bytes(M, N, K, gs, bits);
   return prefer_frag_path(M, N, K, gs, bits) ? qmm_frag_copy_bytes(N, K) + planes : planes;
 }
 
@@ -1256,6 +1259,10 @@ int launch_qmm_n_ws(const void* x, int dtype, int64_t M, int64_t N, const uint32
 int launch_qmm(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
                void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank, Epilogue epi) {
+  if (const int rc = launch_qmm_slice(x, dtype, M, K, wq, scales, biases, bias, N, gs, bits, y, y_dtype, workspace,
+                                      workspace_bytes, stream, low_rank, epi);
+      rc != MFQ_EUNSUPPORTED)
+    return rc;
   if (use_mid_kernel(M, N, K))
     return launch_qmm_mid(x, dtype, M, K, wq, scales, biases, bias, N, gs, bits, y, y_dtype, workspace,
                           workspace_bytes, stream, low_rank, epi);

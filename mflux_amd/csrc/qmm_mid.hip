@@ -496,7 +496,7 @@ size_t qmm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs) {
   return plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
 }
 
-float qmm_mid_estimate_us(int64_t M, int64_t N, int64_t K) { return plan_mid(M, N, K, period_of(64), compute_units()).us; }
+float qmm_mid_estimate_us(int64_t M, int64_t N, int64_t K, int gs) { return plan_mid(M, N, K, period_of(gs), compute_units()).us; }
 
 int launch_qmm_mid(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                    const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
@@ -509,6 +509,12 @@ int launch_qmm_mid(const void* x, int dtype, int64_t M, int64_t K, const uint32_
   if (epi.kind != kEpiNone && (y_dtype == MFQ_F32 || N % 8)) return MFQ_EUNSUPPORTED;
   // 32-bit byte offsets into x, the packed weight and the scales
   if (M * K >= (int64_t)1 << 31 || N * K >= (int64_t)1 << 31) return MFQ_EUNSUPPORTED;
+#ifdef MFQ_MID_STREAM
+  if (const int rc = launch_qmm_slice(x, dtype, M, K, wq, scales, biases, bias, N, gs, bits, y, y_dtype, workspace,
+                                      workspace_bytes, stream, low_rank, epi);
+      rc != MFQ_EUNSUPPORTED)
+    return rc;
+#endif
   if (dtype == MFQ_BF16)
     return launch_gs<BF16>(x, M, K, wq, scales, biases, bias, N, gs, bits, y, y_dtype, workspace, workspace_bytes,
                            stream, low_rank, epi);
