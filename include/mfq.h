@@ -234,6 +234,19 @@ int mfq_qmm_n_ws(const void* x, int x_dtype, int64_t M, int64_t N, const uint32_
                  void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * The input gradient of a layer with a LoRA adapter on it,
+ *   y[M, K] = x[M, N] @ dequantize(wq[N, K]) + t[M, rank] @ bs[K, rank]^T:
+ * mfq_qmm_n_ws with the update's operands as in mfq_qmm_t_low_rank (t = x @ lora_B^T,
+ * scaled, and bs = lora_A).  Where the two-kernel path runs the update is `rank`
+ * more k of its float32 sums and rounded with them; elsewhere it is added to the
+ * rounded product (mfq_low_rank_add).  rank == 0: mfq_qmm_n_ws.
+ */
+int mfq_qmm_n_low_rank(const void* x, int x_dtype, int64_t M, int64_t N, const uint32_t* wq, const void* scales,
+                       const void* biases, int sb_dtype, int64_t K, int group_size, int bits, const void* t,
+                       const void* bs, int64_t rank, void* y, int y_dtype, void* workspace, size_t workspace_bytes,
+                       void* stream);
+
+/*
  * mfq_qmm_t with an optional float32 workspace.  Has no counterpart in the
  * reference (MLX allocates inside its ops).  Shapes whose output tiles do not
  * fill the GPU's compute units -- the text-stream linears of the double

@@ -149,7 +149,7 @@ def dequantize_rows(w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
     return out.reshape(*indices.shape, K)
 
 
-def _matmul_untransposed(x, w, scales, biases, group_size, bits):
+def _matmul_untransposed(x, w, scales, biases, group_size, bits, low_rank=None):
     """``x @ dequantize(w)`` (``w`` packed ``[N, K*bits/32]``, ``x`` ``[..., N]``): the
     product MLX computes for ``transpose=False``, which is what the gradient of a
     quantized linear with respect to its input needs when a LoRA is trained on a
@@ -157,7 +157,8 @@ def _matmul_untransposed(x, w, scales, biases, group_size, bits):
     wraps ``nn.QuantizedLinear`` in a trainable ``LoRALinear``).  One kernel
     (``mfq_qmm_n``): the weight tile is dequantised and transposed on its way
     into LDS; float32 ``x`` is rounded to the dtype of ``scales`` as for
-    ``transpose=True``."""
+    ``transpose=True``.  ``low_rank``: ``(t [M, R], bs [K, R])`` in that dtype, as
+    the kernels take them; ``t @ bs.T`` is added to the product."""
     _check_packed("quantized_matmul", w, scales, biases, group_size, bits)
     if w.ndim != 2:
         raise NotImplementedError("[quantized_matmul] batched weights are not implemented in this build")
@@ -186,7 +187,7 @@ def _matmul_untransposed(x, w, scales, biases, group_size, bits):
         biases = torch.cat([biases, biases.new_zeros((pad, biases.shape[1]))])
     if x2.shape[0] == 0:
         return torch.empty((*lead, K), dtype=out_dtype, device=x.device)
-    y, ok = _lib.ops().qmm_n(x2.contiguous(), w, scales, biases, group_size, bits, out_dtype)
+    y, ok = _lib.ops().qmm_n(x2.contiguous(), w, scales, biases, group_size, bits, out_dtype, *(low_rank or (None, None)))
     if not ok:
         raise NotImplementedError(f"[quantized_matmul] no kernel for x {tuple(x.shape)} against a weight of "
                                   f"{N} x {K} with transpose=False (an operand exceeds 2 GiB)")

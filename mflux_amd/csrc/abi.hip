@@ -269,7 +269,24 @@ size_t mfq_qmm_n_workspace_bytes(int64_t M, int64_t N, int64_t K, int group_size
 int mfq_qmm_n_ws(const void* x, int x_dtype, int64_t M, int64_t N, const uint32_t* wq, const void* scales,
                  const void* biases, int sb_dtype, int64_t K, int group_size, int bits, void* y, int y_dtype,
                  void* workspace, size_t workspace_bytes, void* stream) {
+  return mfq_qmm_n_low_rank(x, x_dtype, M, N, wq, scales, biases, sb_dtype, K, group_size, bits, nullptr, nullptr, 0, y,
+                            y_dtype, workspace, workspace_bytes, stream);
+}
+
+int mfq_qmm_n_low_rank(const void* x, int x_dtype, int64_t M, int64_t N, const uint32_t* wq, const void* scales,
+                       const void* biases, int sb_dtype, int64_t K, int group_size, int bits, const void* t,
+                       const void* bs, int64_t rank, void* y, int y_dtype, void* workspace, size_t workspace_bytes,
+                       void* stream) {
   if (int rc = check_common(group_size, bits)) return rc;
+  if (rank < 0 || rank > 1024 || rank % 16) return MFQ_ESHAPE;
+  if (rank && (!t || !bs)) return MFQ_ENULL;
+  if (rank && (!mfq::aligned16(t) || !mfq::aligned16(bs))) return MFQ_EALIGN;
+  mfq::LowRank low_rank;
+  if (rank) {
+    low_rank.t = t;
+    low_rank.bs = bs;
+    low_rank.R = (int)rank;
+  }
   if (!is16(x_dtype) || x_dtype != sb_dtype) return MFQ_EDTYPE;
   if (y_dtype != sb_dtype && y_dtype != MFQ_F32) return MFQ_EDTYPE;
   if (M <= 0 || N <= 0 || K <= 0 || K % group_size) return MFQ_ESHAPE;
@@ -277,7 +294,7 @@ int mfq_qmm_n_ws(const void* x, int x_dtype, int64_t M, int64_t N, const uint32_
   if (!x || !wq || !scales || !biases || !y) return MFQ_ENULL;
   if (!mfq::aligned16(x) || !mfq::aligned16(wq) || !mfq::aligned16(y)) return MFQ_EALIGN;
   return mfq::launch_qmm_n_ws(x, x_dtype, M, N, wq, scales, biases, K, group_size, bits, y, y_dtype, workspace,
-                              workspace_bytes, (hipStream_t)stream);
+                              workspace_bytes, (hipStream_t)stream, low_rank);
 }
 
 int mfq_qmv_silu(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,

@@ -1242,18 +1242,21 @@ size_t qmm_n_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits) 
 
 int launch_qmm_n_ws(const void* x, int dtype, int64_t M, int64_t N, const uint32_t* wq, const void* scales,
                     const void* biases, int64_t K, int gs, int bits, void* y, int y_dtype, void* workspace,
-                    size_t workspace_bytes, hipStream_t stream) {
+                    size_t workspace_bytes, hipStream_t stream, LowRank low_rank) {
+  // (32-bit offsets into the update's operands)
   if (y_dtype == dtype && workspace && aligned16(workspace) && prefer_frag_n(M, N, K, bits) &&
-      workspace_bytes >= qmm_frag_copy_bytes(K, N)) {
+      workspace_bytes >= qmm_frag_copy_bytes(K, N) && (M + BM) * low_rank.R < (int64_t)1 << 31 &&
+      (K + BN) * low_rank.R < (int64_t)1 << 31) {
     const int64_t tiles = ((M + BM - 1) / BM) * ((K + BN - 1) / BN);
     TailPlan plan = plan_tail(M, K, N, 2, compute_units());
     if (plan.splits > 1 && workspace_bytes < qmm_frag_copy_bytes(K, N) + tail_plane_bytes(M, K, plan))
       plan = TailPlan{(int)tiles, 1};
     float* planes = reinterpret_cast<float*>(static_cast<char*>(workspace) + qmm_frag_copy_bytes(K, N));
     return launch_qmm_frag_n(x, dtype, M, N, wq, scales, biases, K, gs, bits, y, workspace, planes, plan.n_whole,
-                             plan.splits, stream);
+                             plan.splits, stream, low_rank);
   }
-  return launch_qmm_n(x, dtype, M, N, wq, scales, biases, K, gs, bits, y, y_dtype, stream);
+  const int rc = launch_qmm_n(x, dtype, M, N, wq, scales, biases, K, gs, bits, y, y_dtype, stream);
+  return rc ? rc : launch_low_rank_add(dtype, low_rank, M, K, y, y_dtype, stream);
 }
 
 int launch_qmm(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,

@@ -1027,13 +1027,13 @@ bool qmm_frag_n_shape_ok(int64_t M, int64_t N, int64_t K, int bits) {
 
 int launch_qmm_frag_n(const void* x, int dtype, int64_t M, int64_t N, const uint32_t* wq, const void* scales,
                       const void* biases, int64_t K, int gs, int bits, void* y, void* workspace, float* planes,
-                      int n_whole, int splits, hipStream_t stream) {
+                      int n_whole, int splits, hipStream_t stream, LowRank low_rank) {
   if (!qmm_frag_n_shape_ok(M, N, K, bits)) return MFQ_EUNSUPPORTED;
   int rc = MFQ_EDTYPE;
   if (dtype == MFQ_BF16) rc = launch_dequant_t<BF16>(wq, scales, biases, gs, bits, workspace, N, K, stream);
   if (dtype == MFQ_F16) rc = launch_dequant_t<F16>(wq, scales, biases, gs, bits, workspace, N, K, stream);
   if (rc) return rc;
-  return launch_qmm_frag_gemm(x, dtype, M, N, workspace, nullptr, K, y, planes, n_whole, splits, stream, LowRank(),
+  return launch_qmm_frag_gemm(x, dtype, M, N, workspace, nullptr, K, y, planes, n_whole, splits, stream, low_rank,
                               Epilogue());
 }
 

@@ -188,9 +188,10 @@ std::tuple<Tensor, bool> qmm_t_epilogue(const Tensor& x, const Tensor& wq, const
   return {y, true};
 }
 
-// y[M, K] = x[M, N] @ dequantize(wq[N, K]); `ok` is false when N is not a multiple of 8
+// y[M, K] = x[M, N] @ dequantize(wq[N, K]) (+ t @ bs^T); `ok` is false when N is not a multiple of 8
 std::tuple<Tensor, bool> qmm_n(const Tensor& x, const Tensor& wq, const Tensor& scales, const Tensor& biases,
-                               int64_t group_size, int64_t bits, at::ScalarType out_dtype) {
+                               int64_t group_size, int64_t bits, at::ScalarType out_dtype,
+                               const c10::optional<Tensor>& lr_t, const c10::optional<Tensor>& lr_bs) {
   check_packed(wq, scales, biases);
   TORCH_CHECK(x.dim() == 2 && x.is_contiguous() && x.device() == wq.device() && x.size(1) == wq.size(0) &&
                   x.scalar_type() == scales.scalar_type(),
@@ -200,14 +201,27 @@ std::tuple<Tensor, bool> qmm_n(const Tensor& x, const Tensor& wq, const Tensor& 
   Tensor y = at::empty({M, K}, x.options().dtype(out_dtype));
   if (M == 0) return {y, true};
   const int sb = dtype_code(scales.scalar_type(), "scales");
+  const void *t = nullptr, *bs = nullptr;
+  int64_t rank = 0;
+  if (lr_t.has_value() || lr_bs.has_value()) {
+    TORCH_CHECK(lr_t.has_value() && lr_bs.has_value(), "mfq::qmm_n: the low-rank update needs both t and bs");
+    TORCH_CHECK(lr_t->dim() == 2 && lr_bs->dim() == 2 && lr_t->size(0) == M && lr_bs->size(0) == K &&
+                    lr_t->size(1) == lr_bs->size(1) && lr_t->scalar_type() == x.scalar_type() &&
+                    lr_bs->scalar_type() == x.scalar_type() && lr_t->is_contiguous() && lr_bs->is_contiguous() &&
+                    lr_t->device() == x.device() && lr_bs->device() == x.device(),
+                "mfq::qmm_n: the low-rank update is t [M, R], bs [K, R], contiguous, in x's dtype");
+    rank = lr_bs->size(1);
+    t = lr_t->data_ptr();
+    bs = lr_bs->data_ptr();
+  }
   // the transposed 16-bit copy of the two-kernel path (and the planes of its K cut), where that is used
   const size_t ws_bytes = mfq_qmm_n_workspace_bytes(M, N, K, (int)group_size, (int)bits);
   Tensor ws;
   if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
-  const int rc = mfq_qmm_n_ws(x.data_ptr(), sb, M, N, static_cast<const uint32_t*>(wq.data_ptr()), scales.data_ptr(),
-                              biases.data_ptr(), sb, K, (int)group_size, (int)bits, y.data_ptr(),
-                              dtype_code(out_dtype, "the output"), ws_bytes ? ws.data_ptr() : nullptr, ws_bytes,
-                              stream_of(x));
+  const int rc = mfq_qmm_n_low_rank(x.data_ptr(), sb, M, N, static_cast<const uint32_t*>(wq.data_ptr()),
+                                    scales.data_ptr(), biases.data_ptr(), sb, K, (int)group_size, (int)bits, t, bs, rank,
+                                    y.data_ptr(), dtype_code(out_dtype, "the output"),
+                                    ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, stream_of(x));
   if (rc == MFQ_EUNSUPPORTED) return {y, false};
   check_status("mfq_qmm_n", rc);
   return {y, true};
@@ -291,7 +305,7 @@ TORCH_LIBRARY(mfq, m) {
   m.def("dequantize_rows(Tensor wq, Tensor scales, Tensor biases, Tensor indices, int group_size, int bits, ScalarType out_dtype) -> Tensor");
   m.def("qmm_t(Tensor x, Tensor wq, Tensor scales, Tensor biases, Tensor? bias, int group_size, int bits, ScalarType out_dtype, Tensor? lr_t, Tensor? lr_bs) -> (Tensor, bool)");
   m.def("qmm_t_epilogue(Tensor x, Tensor wq, Tensor scales, Tensor biases, Tensor? bias, int group_size, int bits, int epilogue, Tensor? gate, Tensor? residual, int act_from) -> (Tensor, bool)");
-  m.def("qmm_n(Tensor x, Tensor wq, Tensor scales, Tensor biases, int group_size, int bits, ScalarType out_dtype) -> (Tensor, bool)");
+  m.def("qmm_n(Tensor x, Tensor wq, Tensor scales, Tensor biases, int group_size, int bits, ScalarType out_dtype, Tensor? lr_t=None, Tensor? lr_bs=None) -> (Tensor, bool)");
   m.def("qmv_silu(Tensor x, Tensor wq, Tensor scales, Tensor biases, Tensor? bias, int group_size, int bits) -> (Tensor, bool)");
   m.def("layer_norm_modulate(Tensor x, Tensor? scale, Tensor? shift, float eps) -> (Tensor, bool)");
   m.def("low_rank_add_(Tensor(a!) y, Tensor t, Tensor bs) -> ()");

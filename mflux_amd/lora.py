@@ -158,11 +158,10 @@ class _LoRALinearFunction(torch.autograd.Function):
             if scale != 1.0:
                 grad_b = scale * grad_b
         if ctx.needs_input_grad[0]:
-            grad_x = core._matmul_untransposed(grad_y, w, scales, biases, group_size, bits)
+            update = None if twice else (_operand(gt), _operand(lora_a))
+            grad_x = core._matmul_untransposed(grad_y, w, scales, biases, group_size, bits, update)
             if twice:
                 grad_x = grad_x + torch.matmul(gt, lora_a.t()).reshape(grad_x.shape)
-            else:
-                _lib.ops().low_rank_add_(grad_x.view(x2.shape), _operand(gt), _operand(lora_a))
         return grad_x, grad_a, grad_b, None, None, None, None, None, None, None
 
 

@@ -436,3 +436,26 @@ def test_training_calls_that_keep_the_composition():
     # (the base takes no part in a second derivative: neither form differentiates its untransposed product)
     for a, b in zip(second(layer(x)), second(lora._composed(layer.linear, [layer], x))):
         assert float((a.double() - b.double()).norm() / b.double().norm()) < 3e-2
+
+
+# rows on either side of the two-kernel path (1024), with and without a K cut there; ranks of half a step, and of several
+@pytest.mark.parametrize("M,N,K", [(100, 256, 320), (1030, 1024, 520), (1536, 12288, 3072)])
+@pytest.mark.parametrize("rank,bits,dtype", [(16, 4, torch.bfloat16), (48, 8, torch.float16)])
+def test_untransposed_product_with_update(M, N, K, rank, bits, dtype):
+    """x @ W + t @ bs^T against float64 on the weights rounded once: the update is part of the float32 sums (one rounding
+    of the result, at most 2^-8 or 2^-11 of it) or added to the rounded product (two)."""
+    import mflux_amd
+    from mflux_amd import _lib
+
+    K -= K % 64
+    gen = torch.Generator(device="cuda").manual_seed(91)
+    packed = mflux_amd.quantize((torch.randn(N, K, generator=gen, device="cuda") * 0.02).to(dtype), 64, bits)
+    x = torch.randn(M, N, generator=gen, device="cuda").to(dtype)
+    t = torch.randn(M, rank, generator=gen, device="cuda").to(dtype)
+    bs = (torch.randn(K, rank, generator=gen, device="cuda") * 0.1).to(dtype)
+    y, ok = _lib.ops().qmm_n(x, *packed, 64, bits, dtype, t, bs)
+    assert ok
+    w_hat = mflux_amd.dequantize(*packed, 64, bits, dtype=torch.float32).to(dtype).double()
+    ref = x.double() @ w_hat + t.double() @ bs.double().t()
+    bound = (2 * 2.0 ** (-8 if dtype == torch.bfloat16 else -11) + 2.0 ** -12) * ref.abs().amax(dim=1)
+    assert bool(((y.double() - ref).abs().amax(dim=1) <= bound).all())
