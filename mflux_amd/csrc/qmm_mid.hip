@@ -113,7 +113,8 @@ __global__ __launch_bounds__(threads_of(kWavesM), 2) void qmm_mid_kernel(
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     xoff[i] = ((uint32_t)min(m0 + (t >> 3) + kXPass * i, M - 1) * (uint32_t)K + 8u * (t & 7)) * 2u;
-  const bool deq = t < kDeqThreads;             // uniform per wavefront
+  // (uniform per wavefront; spelt out where every thread does: left to the compiler it was a branch in every quarter step)
+  const bool deq = kDeqThreads == kThreads || t < kDeqThreads;
   const int td = t % kDeqThreads;               // the other threads request what thread td does and drop it
   const int f = td / kParts, part = td % kParts;  // this thread's feature of the tile and part of the k step
   const int hh = part * kCodes / 32;            // which half of the step (the group, for groups of 32)
