@@ -469,6 +469,17 @@ int launch_qmm_slice(const void* x, int dtype, int64_t M, int64_t K, const uint3
                      void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank = LowRank(),
                      Epilogue epi = Epilogue());
 size_t qmm_slice_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits);
+// what launch_qmm_slice is estimated to take, 0 where it does not take the shape
+float qmm_slice_estimate_us(int64_t M, int64_t N, int64_t K, int gs, int bits);
+// 128 x 256 tiles that dequantise into registers (qmm_wide.hip): 4 and 8 bits, K % 256 == 0, up to 1024 rows.
+// MFQ_EUNSUPPORTED where that is not estimated to be the faster, or the alignment is wrong; workspace as launch_qmm_mid's
+int launch_qmm_wide(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
+                    const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
+                    void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank = LowRank(),
+                    Epilogue epi = Epilogue());
+size_t qmm_wide_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits);
+// what launch_qmm is estimated to take at 4 and 8 bits without launch_qmm_wide (below 1024 rows)
+float qmm_others_estimate_us(int64_t M, int64_t N, int64_t K, int gs, int bits);
 size_t qmm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs);
 // the same kernel for 3, 5 and 6 bits (any M above one row; K % 32 == 0)
 int launch_qmm_mid_stream(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,

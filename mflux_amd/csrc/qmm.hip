@@ -25,6 +25,7 @@
 //     and costs a third of the kernel's time.
 //   - the k order inside a step is permuted (lane half h covers k 32h..32h+31)
 //     identically for both operands, which the dot product does not notice.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -1123,6 +1124,14 @@ int launch_qmm_epilogue(const void* x, int dtype, int64_t M, int64_t K, const ui
                       stream, LowRank(), epi);
 }
 #else
+// the 256 x 256-tile kernel, measured: 1.68 us per k step and round
+static float tiles_estimate_us(int64_t tiles, int64_t K) {
+  const int64_t cus = compute_units(), rest = tiles % cus;
+  const float step_us = 1.68f * (float)((K + BK - 1) / BK);
+  const float tail = rest == 0 ? 0.f : rest * 2 > cus ? step_us : 0.5f * step_us + 10.f;
+  return step_us * (float)(tiles / cus) + tail;
+}
+
 // Shapes whose 256 x 256 tiles would leave more than half of the compute units
 // idle go to the 128-column-tile kernel, except many rows against a long K,
 // where cutting K between 256 x 256 tiles measures about a tenth faster -- unless
@@ -1131,7 +1140,7 @@ int launch_qmm_epilogue(const void* x, int dtype, int64_t M, int64_t K, const ui
 // more tiles goes there too where its rows fill 128-row tiles and rounds of
 // workgroups much better: 320 rows x 3584 -> 37888 150 us on 296 tiles of 256 x 256
 // (one round and 40 tiles cut in two), 129 on 888 of 128 x 128; 600 rows x 3072 ->
-// 12288 70 against 62.  The estimate of this kernel: 1.68 us per k step and round.
+// 12288 70 against 62.
 // Both rules take groups of 64 for all.  Groups of 32 can be cut more often (18944 -> 3584, four ranges instead of two),
 // which this kernel gains by and the rule does not see: there 513 .. 768 rows are 8 to 10 % faster on the other kernel,
 // 900 rows 155 us against 144.
@@ -1143,10 +1152,18 @@ bool use_mid_kernel(int64_t M, int64_t N, int64_t K) {
     return M < 1024 && K % BK == 0 && N * K < (int64_t)1 << 31 && tiles * plan_tail(M, N, K, period_of(64), (int)cus).splits * 2 < cus;
   }
   if (M >= 1024 || M * K >= (int64_t)1 << 31 || N * K >= (int64_t)1 << 31) return false;  // (what that kernel addresses)
-  const float step_us = 1.68f * (float)((K + BK - 1) / BK);
-  const int64_t rest = tiles % cus;
-  const float tail = rest == 0 ? 0.f : rest * 2 > cus ? step_us : 0.5f * step_us + 10.f;
-  return qmm_mid_estimate_us(M, N, K, 64) < 0.9f * (step_us * (float)(tiles / cus) + tail);
+  return qmm_mid_estimate_us(M, N, K, 64) < 0.9f * tiles_estimate_us(tiles, K);
+}
+
+// (5 us: the launches and the first bytes, which the two estimates leave out; a cut tail as plan_tail() prices it)
+float qmm_others_estimate_us(int64_t M, int64_t N, int64_t K, int gs, int bits) {
+  if (const float us = qmm_slice_estimate_us(M, N, K, gs, bits); us > 0.f) return us;
+  if (use_mid_kernel(M, N, K)) return 5.f + qmm_mid_estimate_us(M, N, K, gs);
+  const int64_t cus = compute_units(), tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  const int splits = plan_tail(M, N, K, period_of(gs), (int)cus).splits;
+  if (splits == 1) return 5.f + tiles_estimate_us(tiles, K);
+  const float step_us = 1.68f * (float)(K / BK);
+  return 11.f + step_us * (float)(tiles / cus) + step_us / (float)splits + 0.13f * (float)(tiles % cus * splits);
 }
 
 #ifndef MFQ_ODD_FRAG_ROWS
@@ -1168,9 +1185,9 @@ size_t qmm_min_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits
   if (K % BK) return 0;
   const size_t planes = use_mid_kernel(M, N, K) ? qmm_mid_workspace_bytes(M, N, K, gs)
                                                 : tail_plane_bytes(M, N, plan_tail(M, N, K, period_of(gs), compute_units()));
-  // (not the smaller of the two: a misaligned operand or an epilogue may still send the call to the other kernels)
-  const size_t slice = qmm_slice_workspace_bytes(M, N, K, gs, bits);
-  return planes > slice ? planes : slice;
+  // (the largest: a misaligned operand or an epilogue may still send the call to the other kernels)
+  const size_t slice = qmm_slice_workspace_bytes(M, N, K, gs, bits), wide = qmm_wide_workspace_bytes(M, N, K, gs, bits);
+  return std::max(planes, std::max(slice, wide));
 }
 
 size_t qmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits) {
@@ -1262,6 +1279,10 @@ int launch_qmm_n_ws(const void* x, int dtype, int64_t M, int64_t N, const uint32
 int launch_qmm(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
                void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank, Epilogue epi) {
+  if (const int rc = launch_qmm_wide(x, dtype, M, K, wq, scales, biases, bias, N, gs, bits, y, y_dtype, workspace,
+                                     workspace_bytes, stream, low_rank, epi);
+      rc != MFQ_EUNSUPPORTED)
+    return rc;
   if (const int rc = launch_qmm_slice(x, dtype, M, K, wq, scales, biases, bias, N, gs, bits, y, y_dtype, workspace,
                                       workspace_bytes, stream, low_rank, epi);
       rc != MFQ_EUNSUPPORTED)

@@ -577,6 +577,10 @@ size_t qmm_slice_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bi
   return plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
 }
 
+float qmm_slice_estimate_us(int64_t M, int64_t N, int64_t K, int gs, int bits) {
+  return choose_slice(M, N, K, gs, bits, true).us;
+}
+
 int launch_qmm_slice(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                      const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
                      void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank, Epilogue epi) {

@@ -1,0 +1,90 @@
+"""GPU parity: the GEMM whose wavefronts dequantise into registers (csrc/qmm_wide.hip) at the edges of its 128 x 256 tiles,
+with one quad of steps to a range and several, K whole and cut into ranges, and against the kernels that take the same call
+when scales and biases lie at odd addresses.  The shapes are ones that its rule takes on 256 compute units.
+
+Reference: float64 on the dequantised weights rounded once to the 16-bit type, which is what the kernels multiply.  What
+is left is the rounding of the result (at most 2^-8 of it in bfloat16 and 2^-11 in float16; the bias add rounds once more)
+and the float32 sums (K 2^-24 of the sum of magnitudes, below 2^-12 of a row's largest output on these operands).
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DT = {"bf16": torch.bfloat16, "f16": torch.float16}
+
+
+def _operands(M, K, N, bits, gs, dtype):
+    import mflux_amd
+
+    gen = torch.Generator(device="cuda").manual_seed(83)
+    w = (torch.randn(N, K, generator=gen, device="cuda") * 0.02).to(dtype)
+    x = torch.randn(M, K, generator=gen, device="cuda").to(dtype)
+    bias = (torch.randn(N, generator=gen, device="cuda") * 0.02).to(dtype)
+    packed = mflux_amd.quantize(w, gs, bits)
+    w_hat = mflux_amd.dequantize(*packed, gs, bits, dtype=torch.float32).to(dtype).double()
+    return x, packed, bias, x.double() @ w_hat.t()
+
+
+def _close(y, ref, dtype, roundings):
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    bound = (unit * roundings + 2.0 ** -12) * ref.abs().amax(dim=1)
+    err = (y.double() - ref).abs().amax(dim=1)
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
+def _at_odd_address(t):
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    buf[1:].copy_(t.reshape(-1))
+    return buf[1:].view(t.shape)
+
+
+# rows: part of a tile, a tile, one more, several; columns: ragged (no epilogue), a tile's part, whole tiles
+# K: one quad (256), an even and an uneven cut into ranges, long
+@pytest.mark.parametrize("M,K,N", [(40, 256, 32770), (128, 256, 32770), (257, 256, 20480), (896, 256, 8200), (600, 256, 12288),
+                                   (513, 3072, 4096), (384, 4096, 4100), (1000, 12288, 1032), (129, 6144, 20480)])
+@pytest.mark.parametrize("bits,gs,dtype", [(4, 64, "bf16"), (4, 32, "f16"), (4, 128, "bf16"), (8, 64, "f16"), (8, 64, "bf16"),
+                                           (8, 128, "bf16")])
+def test_tiles_ranges_and_the_other_kernels(M, K, N, bits, gs, dtype):
+    import mflux_amd
+
+    dtype = DT[dtype]
+    x, (wq, s, b), bias, ref = _operands(M, K, N, bits, gs, dtype)
+    y = mflux_amd.quantized_matmul(x, wq, s, b, group_size=gs, bits=bits, bias=bias)
+    _close(y, ref + bias.double(), dtype, 2)
+    other = mflux_amd.quantized_matmul(x, wq, _at_odd_address(s), _at_odd_address(b), group_size=gs, bits=bits, bias=bias)
+    _close(other, ref + bias.double(), dtype, 2)
+    y32 = mflux_amd.quantized_matmul(x.float(), wq, s, b, group_size=gs, bits=bits)  # float32 out: no rounding of the result
+    assert y32.dtype == torch.float32
+    _close(y32, ref, dtype, 0)
+
+
+@pytest.mark.parametrize("M,K,N", [(257, 256, 20480), (640, 12288, 1032)])
+@pytest.mark.parametrize("rank", [16, 48])
+def test_low_rank_update(M, K, N, rank):
+    import mflux_amd
+
+    x, packed, bias, ref = _operands(M, K, N, 4, 64, torch.bfloat16)
+    t, bs = torch.randn(M, rank, device="cuda").bfloat16(), (torch.randn(N, rank, device="cuda") * 0.02).bfloat16()
+    y = mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=4, bias=bias, low_rank=(t, bs))
+    _close(y, ref + bias.double() + t.double() @ bs.double().t(), torch.bfloat16, 2)
+
+
+@pytest.mark.parametrize("M,K,N", [(257, 256, 20480), (385, 6144, 8256), (513, 3072, 4096)])
+def test_epilogues_are_the_separate_operations(M, K, N):
+    """Gate and residual, and SwiGLU, on the linear layer's own values; GELU rounds once where torch's does."""
+    import mflux_amd
+    from mflux_amd import core
+
+    x, packed, bias, _ = _operands(M, K, N, 4, 64, torch.bfloat16)
+    lin = mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=4, bias=bias)
+    gate, res = torch.randn(N, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
+    y = core.quantized_matmul_epilogue(x, *packed, epilogue="gate_residual", group_size=64, bits=4, bias=bias, gate=gate, residual=res)
+    assert torch.equal(y, res + gate * lin)
+    y = core.quantized_matmul_epilogue(x, *packed, epilogue="gelu", group_size=64, bits=4, bias=bias, act_from=N // 2)
+    assert torch.equal(y[:, : N // 2], lin[:, : N // 2])
+    want = torch.nn.functional.gelu(lin[:, N // 2:].double(), approximate="tanh")
+    assert bool(((y[:, N // 2:].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-6).all())
+    y = core.quantized_matmul_epilogue(x, *packed, epilogue="swiglu", group_size=64, bits=4, bias=bias)
+    want = core.swiglu_unstack(lin).double()
+    assert bool(((y.double() - want).abs() <= 2.0 ** -6 * want.abs() + 1e-6).all())  # the sigmoid's last place, twice rounded
