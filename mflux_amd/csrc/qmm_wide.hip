@@ -288,16 +288,20 @@ inline WidePlan plan_wide(int64_t M, int64_t N, int64_t K, int bits, bool may_cu
   return best;
 }
 
-// Taken where its estimate is a tenth below that of the kernel that would run: on the 600 shapes a fifth of the calls, 0.91
-// of their time (geometric mean), the slowest 5 % behind (967 rows x 4096 -> 20480, 169 -> 174 us).  From 1024 rows on the
-// 256 x 256 tiles are ahead (1024 x 3072 -> 12288 83 us against 89).  8 bits in groups of 32 stay with the other kernels: the
-// scales of a quad are sixteen registers more than there are, and 879 rows x 10240 -> 4096 took 163 us against 101.
+// Taken where its estimate is a tenth (257 to 512 rows) or a sixth below that of the kernel that would run.  Of 7400 drawn
+// calls of 55 to 1023 rows those are 714, in 0.88 of their time (geometric mean), the slowest 1 % behind; with a tenth for
+// all rows 1206, but 54 of the added ones 3 to 9 % behind (67 rows x 2560 -> 19456 28.0 -> 30.5 us, 908 x 12288 ->
+// 3072 90 -> 95), where the others' estimates are some 5 % high; with a sixth for all, 257 to 512 rows lose what they gain
+// between the two (320 x 18944 -> 3584, 85 us against 70).  From 1024 rows on the 256 x 256 tiles are ahead (1024 x 3072 ->
+// 12288 83 us against 89).  8 bits in groups of 32 stay with the other kernels: the scales of a quad are sixteen registers
+// more than there are, and 879 rows x 10240 -> 4096 took 163 us against 101.
 inline WidePlan choose_wide(int64_t M, int64_t N, int64_t K, int gs, int bits, bool may_cut) {
   const WidePlan none{0, 0, 0, 0.f};
   if (bits != 4 && (bits != 8 || gs == 32)) return none;
   if (M >= 1024 || K % (4 * TK) || M * K >= (int64_t)1 << 31 || N * K >= (int64_t)1 << 31) return none;
   const WidePlan plan = plan_wide(M, N, K, bits, may_cut);
-  return plan.us < 0.9f * qmm_others_estimate_us(M, N, K, gs, bits) ? plan : none;
+  const float share = M > 256 && M <= 512 ? 0.9f : 0.84f;
+  return plan.us < share * qmm_others_estimate_us(M, N, K, gs, bits) ? plan : none;
 }
 
 template <typename T, int GS, int BITS>

@@ -1,4 +1,4 @@
-// Epilogue shared by the 128-column-tile GEMM kernels (qmm_mid.hip, qmm_n.hip):
+// Epilogue shared by the GEMM kernels of qmm_mid.hip, qmm_n.hip and qmm_wide.hip:
 // a wavefront's 64 x 64 block of float32 sums -> y, rounded, with the bias.
 #pragma once
 

@@ -40,9 +40,9 @@ def _at_odd_address(t):
 
 
 # rows: part of a tile, a tile, one more, several; columns: ragged (no epilogue), a tile's part, whole tiles
-# K: one quad (256), an even and an uneven cut into ranges, long
-@pytest.mark.parametrize("M,K,N", [(40, 256, 32770), (128, 256, 32770), (257, 256, 20480), (896, 256, 8200), (600, 256, 12288),
-                                   (513, 3072, 4096), (384, 4096, 4100), (1000, 12288, 1032), (129, 6144, 20480)])
+# K: one quad (256) and two, an even and an uneven cut into ranges, long
+@pytest.mark.parametrize("M,K,N", [(40, 512, 32770), (128, 512, 32770), (257, 256, 20480), (385, 256, 32770), (600, 256, 24584),
+                                   (384, 4096, 4100), (513, 12288, 1032), (1000, 12288, 1032), (128, 6144, 24584)])
 @pytest.mark.parametrize("bits,gs,dtype", [(4, 64, "bf16"), (4, 32, "f16"), (4, 128, "bf16"), (8, 64, "f16"), (8, 64, "bf16"),
                                            (8, 128, "bf16")])
 def test_tiles_ranges_and_the_other_kernels(M, K, N, bits, gs, dtype):
@@ -70,7 +70,7 @@ def test_low_rank_update(M, K, N, rank):
     _close(y, ref + bias.double() + t.double() @ bs.double().t(), torch.bfloat16, 2)
 
 
-@pytest.mark.parametrize("M,K,N", [(257, 256, 20480), (385, 6144, 8256), (513, 3072, 4096)])
+@pytest.mark.parametrize("M,K,N", [(257, 256, 20480), (385, 6144, 8256), (640, 12288, 1088)])
 def test_epilogues_are_the_separate_operations(M, K, N):
     """Gate and residual, and SwiGLU, on the linear layer's own values; GELU rounds once where torch's does."""
     import mflux_amd
