@@ -515,14 +515,16 @@ inline SlicePlan plan_slice(int64_t M, int64_t N, int64_t K, int bits, bool may_
   return best;
 }
 
-// Taken where its estimate is 7 % below the other kernel's (that estimate and 5 us, as it leaves the launch and the first
-// bytes out).  Over the 700 shapes, of which 460 come here, this leaves 0.80 of the time before (geometric mean), four
-// shapes behind by 4 to 10 % (6 bits 89 rows x 3072 -> 12288, 27.6 us, is the worst) and 1.6 % to a perfect choice.
+// Taken where its estimate is 7 % (8 bits: 16 %) below the other kernel's (that estimate and 5 us, as it leaves the launch
+// and the first bytes out).  Over the 700 shapes, of which 460 come here, this leaves 0.80 of the time before (geometric
+// mean), four shapes behind by 4 to 10 % (6 bits 89 rows x 3072 -> 12288, 27.6 us, is the worst) and 1.6 % to a perfect
+// choice.  Of 2400 drawn calls at 4 bits that come here 8 are 3 to 8 % behind (600 rows x 2560 -> 2560); at 8 bits with 7 %
+// 32 of 1020 were, all from the 169 that 16 % leaves out (138 x 2560 -> 10240 26.8 -> 28.7 us).
 inline SlicePlan choose_slice(int64_t M, int64_t N, int64_t K, int gs, int bits, bool may_cut) {
   const int64_t gran = bits == 3 || bits == 5 ? 128 : 64;
   if (M > 1024 || N % 8 || K % gran || (K / gs) % 2 || M * K >= (int64_t)1 << 31 || N * K >= (int64_t)1 << 31) return SlicePlan();
   const SlicePlan plan = plan_slice(M, N, K, bits, may_cut);
-  return plan.us < 0.93f * (5.f + qmm_mid_estimate_us(M, N, K, gs)) ? plan : SlicePlan();
+  return plan.us < (bits == 8 ? 0.84f : 0.93f) * (5.f + qmm_mid_estimate_us(M, N, K, gs)) ? plan : SlicePlan();
 }
 
 template <typename T, int BITS, int kA, int kB>
