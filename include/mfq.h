@@ -127,12 +127,15 @@ int mfq_dequantize_rows(const uint32_t* wq, const void* scales, const void* bias
  *   biases  [N, K/group_size]      sb_dtype
  *   bias    [N] or NULL            sb_dtype
  *   y       [M, N]                 y_dtype (sb_dtype or MFQ_F32)
- * M <= 16 runs the HBM-bound matvec kernels, larger M one of two MFMA GEMM
+ * M <= 16 runs the HBM-bound matvec kernels, larger M one of the MFMA GEMM
  * kernels: 128-column tiles while 256 x 256 tiles would leave more than half of
  * the compute units idle (unless K is long enough to be cut between those
  * tiles), and below 1024 rows where an estimate of both finds them faster;
- * 256 x 256 tiles otherwise.  3, 5 and 6 bits: one activation row of up to 8192
- * elements has its own kernel, everything else runs on the 128-column-tile GEMM.
+ * 256 x 256 tiles otherwise; up to 1024 rows also 32- and 64-row tiles with K
+ * sliced over a workgroup, and 128 x 256 tiles (4 and 8 bits, K % 256 == 0),
+ * each where its estimate is the lowest.  3, 5 and 6 bits: one activation row of
+ * up to 8192 elements has its own kernel, everything else runs on the sliced or
+ * the 128-column-tile GEMM.
  * Sums are float32, on dequantised weights rounded at most once, to x_dtype -- except in
  * the integer matvec kernels of 4 and 8 bits, where x becomes fixed point (one
  * power of two per row, or per part of a row that a wavefront multiplies, from
