@@ -16,7 +16,8 @@
 // With 240 (4 bits) to 252 registers two wavefronts fit a SIMD.  320 rows x 3584 -> 37888 at 4 bits: 110 us, 0.79 PFLOP/s
 // (143 on 888 tiles of 128 x 128, 129 with those 160 rows high); with x all zeros, which costs less power, 95.  Weight loads
 // in whole cache lines (their share of every line is 32 bytes now) would give some 8 % more, but their way through LDS has no
-// registers left; 96-row tiles took 135 us, 64-row tiles, which dequantise twice as often, 120.
+// registers left (half lines through a private region: 115); 96-row tiles took 135 us, 64-row tiles, which dequantise twice as
+// often, 120.
 #include <type_traits>
 
 #include "common.h"
