@@ -45,6 +45,8 @@ def _compile(src: str) -> str:
 # Kernels whose matrix instructions are inline assembly (result tied to the addend), which the compiler's
 # hazard recognizer cannot see: {source: substring of the kernels' mangled names}.
 ASM_MFMA_KERNELS = {"qmm_frag.hip": "frag_gemm_kernel"}
+# Sources whose loads from memory straight into LDS are inline assembly, with the write of m0 (their LDS base) in front.
+ASM_LDS_LOAD_SOURCES = ("qmm_frag.hip", "qmm_slice.hip")
 
 
 def _parse_blocks(body: str):
@@ -69,6 +71,71 @@ def _wait_states(ins: str) -> int:
     if ins.startswith("s_nop"):
         return int(ins.split()[1], 0) + 1
     return 1
+
+
+def _successors(blocks, index, b):
+    """The blocks control may pass to from block b."""
+    import re
+
+    ins = blocks[b][1]
+    out = []
+    for s in ins:
+        t = re.match(r"s_c?branch\S*\s+(\S+)", s)
+        if t and t.group(1) in index:
+            out.append(index[t.group(1)])
+    last = ins[-1] if ins else ""
+    if not (last.startswith("s_branch") or last.startswith("s_endpgm") or last.startswith("s_setpc")):
+        if b + 1 < len(blocks):
+            out.append(b + 1)
+    return out
+
+
+def check_lds_loads(text: str, where: str = "listing") -> int:
+    """Checks every kernel of the assembly listing `text`: a load from memory into
+    LDS takes its LDS base from m0 and needs one wait state behind a write of it
+    (an s_nop or any other instruction).  The compiler puts that behind its own
+    writes of m0 but not between two instructions of one assembly statement; a load
+    issued too early would land at the base of the load before it.  Follows the
+    control flow as check_listing does.  Returns the number of such loads; raises
+    RuntimeError on a finding or if there is none."""
+    import re
+
+    def is_lds_load(ins):
+        return bool(re.match(r"(global|scratch)_load_lds_|buffer_load\S* .*\blds\b", ins))
+
+    loads = 0
+    for m in re.finditer(r"^(\w+):", text, re.M):
+        end = text.find(".Lfunc_end", m.end())
+        if end < 0:
+            break
+        if "s_endpgm" not in text[m.end():end]:
+            continue  # a symbol of the data sections
+        blocks = _parse_blocks(text[m.end():end])
+        index = {label: i for i, (label, _) in enumerate(blocks) if label}
+
+        def next_instructions(b, i):
+            if i + 1 < len(blocks[b][1]):
+                return [blocks[b][1][i + 1]]
+            found, todo, seen = [], _successors(blocks, index, b), set()
+            while todo:
+                nb = todo.pop()
+                if nb in seen:
+                    continue
+                seen.add(nb)
+                if blocks[nb][1]:
+                    found.append(blocks[nb][1][0])
+                else:
+                    todo += _successors(blocks, index, nb)
+            return found
+
+        for b, (_, ins) in enumerate(blocks):
+            for i, s in enumerate(ins):
+                loads += is_lds_load(s)
+                if re.match(r"s_\w+\s+m0\b", s) and any(map(is_lds_load, next_instructions(b, i))):
+                    raise RuntimeError(f"{where}: {m.group(1)} loads into LDS directly behind a write of m0 ({s})")
+    if not loads:
+        raise RuntimeError(f"{where}: no load into LDS; the check does not see the kernels")
+    return loads
 
 
 def check_listing(text: str, kernel_substring: str, where: str = "listing") -> int:
@@ -111,26 +178,13 @@ def check_listing(text: str, kernel_substring: str, where: str = "listing") -> i
         col_tiles = re.search(r"ELi(\d)ELb[01]EEEv", name)  # the template argument before the last: column tiles per wavefront
         least = 2 * int(col_tiles.group(1)) if col_tiles else 8
 
-        def successors(b):
-            ins = blocks[b][1]
-            out = []
-            for s in ins:
-                t = re.match(r"s_c?branch\S*\s+(\S+)", s)
-                if t and t.group(1) in index:
-                    out.append(index[t.group(1)])
-            last = ins[-1] if ins else ""
-            if not (last.startswith("s_branch") or last.startswith("s_endpgm") or last.startswith("s_setpc")):
-                if b + 1 < len(blocks):
-                    out.append(b + 1)
-            return out
-
         def walk(b, i, budget, visit, seen):
             """Calls visit(instruction) for everything within `budget` wait states behind instruction i of block b."""
             ins = blocks[b][1]
             while budget > 0:
                 i += 1
                 if i >= len(ins):
-                    for nb in successors(b):
+                    for nb in _successors(blocks, index, b):
                         if seen.get(nb, 0) < budget:  # not yet entered with as much distance left
                             seen[nb] = budget
                             walk(nb, -1, budget, visit, seen)
@@ -183,9 +237,10 @@ def check_listing(text: str, kernel_substring: str, where: str = "listing") -> i
 
 
 def check_generated_code(src: str) -> int:
-    """Compiles `src` to assembly (device side) and runs check_listing over the
-    kernels named in ASM_MFMA_KERNELS.  Returns the number of kernels checked;
-    raises on a finding."""
+    """Compiles `src` to assembly (device side) and runs check_lds_loads (for
+    ASM_LDS_LOAD_SOURCES) and check_listing (over the kernels named in
+    ASM_MFMA_KERNELS).  Returns the number of kernels check_listing checked; raises
+    on a finding."""
     import tempfile
 
     with tempfile.TemporaryDirectory() as tmp:
@@ -195,14 +250,17 @@ def check_generated_code(src: str) -> int:
         if res.returncode != 0:
             raise RuntimeError(f"hipcc -S failed on {src}:\n{res.stdout}\n{res.stderr}")
         text = open(asm).read()
-    return check_listing(text, ASM_MFMA_KERNELS[src], src)
+    if src in ASM_LDS_LOAD_SOURCES:
+        check_lds_loads(text, src)
+    return check_listing(text, ASM_MFMA_KERNELS[src], src) if src in ASM_MFMA_KERNELS else 0
 
 
 def build_library(verbose: bool = False) -> str:
     """Always recompiles every translation unit, checks the generated code of the
-    kernels in ASM_MFMA_KERNELS and relinks libmfq.so."""
-    with ThreadPoolExecutor(max_workers=len(SOURCES) + len(ASM_MFMA_KERNELS)) as pool:
-        checks = [pool.submit(check_generated_code, src) for src in ASM_MFMA_KERNELS]
+    sources with assembly in them and relinks libmfq.so."""
+    checked = sorted({*ASM_MFMA_KERNELS, *ASM_LDS_LOAD_SOURCES})
+    with ThreadPoolExecutor(max_workers=len(SOURCES) + len(checked)) as pool:
+        checks = [pool.submit(check_generated_code, src) for src in checked]
         objs = list(pool.map(_compile, SOURCES))
         for c in checks:
             c.result()

@@ -265,6 +265,17 @@ __device__ __forceinline__ void mma16(bf16x8 a, bf16x8 b, f32x4& c) {
 __device__ __forceinline__ void mma16(f16x8 a, f16x8 b, f32x4& c) {
   asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
+// The same with a load from memory into LDS behind it (dma16 below): the matrix instruction is the wait state that the load
+// wants behind the write of m0.
+#define MFQ_MMA16_DMA(type)                                                                                            \
+  "s_mov_b32 m0, %5\n\tv_mfma_f32_16x16x32_" type " %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %3, %4"
+__device__ __forceinline__ void mma16_dma(bf16x8 a, bf16x8 b, f32x4& c, const char* sbase, uint32_t voff, uint32_t lds_addr) {
+  asm volatile(MFQ_MMA16_DMA("bf16") : "+a"(c) : "v"(a), "v"(b), "v"(voff), "s"(sbase), "s"(lds_addr) : "memory", "m0");
+}
+__device__ __forceinline__ void mma16_dma(f16x8 a, f16x8 b, f32x4& c, const char* sbase, uint32_t voff, uint32_t lds_addr) {
+  asm volatile(MFQ_MMA16_DMA("f16") : "+a"(c) : "v"(a), "v"(b), "v"(voff), "s"(sbase), "s"(lds_addr) : "memory", "m0");
+}
+#undef MFQ_MMA16_DMA
 // The first matrix instruction of a tile: the product alone, whatever the registers held.  Stated as an
 // update all the same, so that the tile's sums stay in the registers the previous tile's were in.
 __device__ __forceinline__ void mma16_first(bf16x8 a, bf16x8 b, f32x4& c) {
@@ -356,10 +367,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   // 16 bytes per lane from global memory straight into LDS, 1 KiB per instruction (eight rows of the tile):
   // no registers, no LDS write instructions.  The compiler does not see these loads; it counts only the
   // weight loads, so its own waits can only be stricter than it thinks, and the waits for the tiles
-  // themselves are stated below by count.
+  // themselves are stated below by count.  (s_nop: a load into LDS wants one wait state behind the write of m0,
+  // which the compiler does not see to inside a statement of assembly.)
   const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
   auto dma16 = [&](const char* sbase, uint32_t voff, uint32_t lds_addr) __attribute__((always_inline)) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr)
                  : "memory", "m0");
   };
   int x_cur = 0, x_next = kTileBytes, x_fill = 2 * kTileBytes;  // LDS offsets of the three x tiles
@@ -508,6 +520,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         for (int j = 0; j < kJ; ++j) {
           const int m = kJ * r + j;
           const int g = 16 * half + r;
+          constexpr int kDmaFirst = kJ == 4 ? 6 : 4, kDmaEvery = kJ == 4 ? 7 : 5;  // 8 loads over the pass's 16 kJ slots
+          const bool dma = half == 1 && m >= kDmaFirst && (m - kDmaFirst) % kDmaEvery == 0 && m < kDmaFirst + 8 * kDmaEvery;
           if (kDrain != 0 && half == 0) {
             mma16_first(now[2 * j + half], xf[g & 3], acc[r][j]);
             if constexpr (kDrain == 1) {
@@ -515,6 +529,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
               if (r & 1) drain_read(r >> 1, j);
               if (r >= 2 && !(r & 1)) drain_store((r - 2) >> 1, j);
             }
+          } else if (dma) {
+            const int i = (m - kDmaFirst) / kDmaEvery;
+            mma16_dma(now[2 * j + half], xf[g & 3], acc[r][j], xbytes + (size_t)s_h0 * (BK * 2), xoff[i], fill + 4096u * i);
           } else {
             mma16(now[2 * j + half], xf[g & 3], acc[r][j]);
             if (kDrain == 1 && r == 0) drain_store(7, j);
@@ -527,11 +544,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
             } else {
               now[2 * j1] = *reinterpret_cast<const vec8*>(wfrag + (size_t)s_h0 * kBlockBytes + woff[j1]);
             }
-          }
-          constexpr int kDmaFirst = kJ == 4 ? 6 : 4, kDmaEvery = kJ == 4 ? 7 : 5;  // 8 loads over the pass's 16 kJ slots
-          if (half == 1 && m >= kDmaFirst && (m - kDmaFirst) % kDmaEvery == 0 && m < kDmaFirst + 8 * kDmaEvery) {
-            const int i = (m - kDmaFirst) / kDmaEvery;
-            dma16(xbytes + (size_t)s_h0 * (BK * 2), xoff[i], fill + 4096u * i);
           }
           __builtin_amdgcn_sched_barrier(0);
         }

@@ -121,11 +121,15 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
 
   char* ring = lds + wave * S::kRing;
   const uint32_t ring_addr = (uint32_t)(uintptr_t)ring;
-  auto dma16 = [&](const char* sbase, uint32_t voff, uint32_t lds_addr) __attribute__((always_inline)) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory", "m0");
+  // LDS destination of a lane: lds_addr + offset (a constant) + 16 (4) times its number.  A load into LDS wants one wait
+  // state behind the write of m0, which the compiler does not see to inside a statement of assembly: the s_nop.
+  auto dma16 = [&](const char* sbase, uint32_t voff, uint32_t lds_addr, int offset) __attribute__((always_inline)) {
+    asm volatile("s_add_i32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 ::"v"(voff), "s"(sbase), "s"(lds_addr), "i"(offset) : "memory", "m0", "scc");
   };
-  auto dma4 = [&](const char* sbase, uint32_t voff, uint32_t lds_addr) __attribute__((always_inline)) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory", "m0");
+  auto dma4 = [&](const char* sbase, uint32_t voff, uint32_t lds_addr, int offset) __attribute__((always_inline)) {
+    asm volatile("s_add_i32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                 ::"v"(voff), "s"(sbase), "s"(lds_addr), "i"(offset) : "memory", "m0", "scc");
   };
 
   // ---- what the lane loads
@@ -156,23 +160,23 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
   const char* wbytes = reinterpret_cast<const char*>(wq);
   const uint32_t w_begin = (uint32_t)begin * 8u * BITS, w_end = (uint32_t)(K * BITS / 8 - 16);
   auto load_x = [&](int j, int slot, int i) __attribute__((always_inline)) {
-    dma16(xbytes + (size_t)j * 128, xoff[i], ring_addr + slot * S::kXSlot + 1024 * i);
+    dma16(xbytes + (size_t)j * 128, xoff[i], ring_addr + slot * S::kXSlot, 1024 * i);
   };
   auto load_w = [&](int c) __attribute__((always_inline)) {  // chunk c; pieces past the row's end repeat its last one
 #pragma unroll
     for (int i = 0; i < S::kWLoads; ++i)
       if ((i + 1) * 64 <= S::kWPieces || 64 * i + lane < S::kWPieces)
         dma16(wbytes, wrow[i] + min(wcol[i] + w_begin + (uint32_t)(c * S::kRowPieces * 16), w_end),
-              ring_addr + S::kWBase + (c & 1) * S::kWSlot + 1024 * i);
+              ring_addr + (c & 1) * S::kWSlot, S::kWBase + 1024 * i);
   };
   auto load_s = [&](int win) __attribute__((always_inline)) {
     const uint32_t col = 4u * (uint32_t)min(first_dword + 4 * win + (lane & 3), row_groups / 2 - 1);
-    const uint32_t addr = ring_addr + S::kSBase + (win & 1) * 2 * S::kWinBytes;
+    const uint32_t addr = ring_addr + (win & 1) * 2 * S::kWinBytes;
 #pragma unroll
     for (int i = 0; i < S::kSLoads; ++i)
       if ((i + 1) * 64 <= S::TN * 4 || 64 * i + lane < S::TN * 4) {
-        dma4(reinterpret_cast<const char*>(scales), srow[i] + col, addr + 256 * i);
-        dma4(reinterpret_cast<const char*>(biases), srow[i] + col, addr + S::kWinBytes + 256 * i);
+        dma4(reinterpret_cast<const char*>(scales), srow[i] + col, addr, S::kSBase + 256 * i);
+        dma4(reinterpret_cast<const char*>(biases), srow[i] + col, addr, S::kSBase + S::kWinBytes + 256 * i);
       }
   };
 

@@ -246,6 +246,35 @@ def test_generated_code_of_the_assembly_matrix_kernels():
     assert _build.check_generated_code("qmm_frag.hip") == 18
 
 
+def test_generated_code_of_the_assembly_lds_loads():
+    """The sliced GEMM's loads into LDS: every write of m0 has a wait state in front of
+    the load that takes it (the two-kernel GEMM's are checked with its matrix
+    instructions, above)."""
+    from mflux_amd import _build
+
+    assert _build.check_generated_code("qmm_slice.hip") == 0
+
+
+def test_listing_check_of_lds_loads():
+    """A load into LDS directly behind a write of m0 is refused, over a branch and
+    through an empty block too; an s_nop or another instruction between the two is
+    what the hardware asks for."""
+    from mflux_amd import _build
+
+    load, end = "global_load_lds_dwordx4 v1, s[2:3]", (".LBB0_9", ["s_endpgm"])
+    for write in ("s_mov_b32 m0, s4", "s_add_i32 m0, s4, 0x400"):
+        with pytest.raises(RuntimeError, match="behind a write of m0"):
+            _build.check_lds_loads(_listing([("", [write, load]), end]))
+        for between in ("s_nop 0", "v_add_u32_e32 v9, v9, v9"):
+            assert _build.check_lds_loads(_listing([("", [write, between, load]), end])) == 1
+    hop = [("", ["s_cmp_eq_u32 s0, 0", "s_cbranch_scc1 .LBB0_2"]), (".LBB0_1", ["s_mov_b32 m0, s4"]), (".LBB0_2", []),
+           (".LBB0_3", [load]), end]
+    with pytest.raises(RuntimeError, match="behind a write of m0"):
+        _build.check_lds_loads(_listing(hop))
+    with pytest.raises(RuntimeError, match="no load into LDS"):
+        _build.check_lds_loads(_listing([("", ["s_mov_b32 m0, s4"]), end]))
+
+
 def _listing(blocks, spills=0):
     """A synthetic assembly listing of one kernel, `demo_gemm_kernel`, in the
     form the compiler prints: label lines, one instruction per line, the
