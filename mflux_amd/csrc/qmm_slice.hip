@@ -9,7 +9,7 @@
 // whose partial tiles meet in LDS at the end: no planes, no second launch.
 //   - Each wavefront has a ring of its own in LDS (40 KiB) that it fills with global_load_lds and reads back as matrix
 //     fragments: no barrier in the loop, no registers for what is on its way, and as no load in the loop is the compiler's
-//     every wait is by count and leaves exactly the younger requests in flight.
+//     every wait is by count and leaves the younger requests of x in flight (and of codes, where that pays: see step).
 //   - A request costs the memory path of a compute unit some 1.2 to 2.5 ns per cache line touched, whatever it takes of
 //     the line, so everything comes in whole lines or long runs of one: x in 128 bytes of a row (64 k), codes in chunks
 //     of 128 bytes of a row where the ring has room, scales and biases eight groups at a time.
@@ -42,6 +42,15 @@ struct Shape {
   static constexpr int TM = 16 * kA, TN = 16 * kB;
   static constexpr int kXSlot = TM * 128;                      // 64 k of the tile's rows of x
   static constexpr int kXLoads = TM / 8;                       // load instructions of a slot
+  static constexpr int kInstr = 2 * kA * kB;                   // matrix instructions of a sub-step
+  static constexpr int kReadsAt = kInstr / 3;                  // the next sub-step's fragments are read behind these
+  // load l of a slot is requested behind matrix instruction load_slot(l); those requested when the reads begin
+  static constexpr int load_slot(int l) { return l * kInstr / kXLoads; }
+  static constexpr int loads_before_reads() {
+    int n = 0;
+    for (int l = 0; l < kXLoads; ++l) n += load_slot(l) <= kReadsAt;
+    return n;
+  }
   static constexpr int kWinBytes = TN * 16;                    // a window: scales (or biases) of eight groups
   static constexpr int kSLoads = (TN * 4 + 63) / 64;
   static constexpr int kGran = (BITS == 3 || BITS == 5) ? 2 : 1;  // sub-steps of a wavefront come in multiples of this
@@ -280,20 +289,25 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
   };
 
   u32x4 cur, nxt;
-  constexpr int kInstr = 2 * kA * kB;                    // matrix instructions of a sub-step
-  constexpr int kReadsAt = kInstr / 3;                    // the next sub-step's fragments are read behind these
+  constexpr int kInstr = S::kInstr, kReadsAt = S::kReadsAt;
   auto step = [&](auto more_x_c, auto more_c, Frag& f, Frag& next, int j, int slot) __attribute__((always_inline)) {
     constexpr bool more_x = decltype(more_x_c)::value, more = decltype(more_c)::value;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this sub-step's operands are in registers: their slots are free
     // a chunk's (a window's) last sub-step: its slot takes the one after the next
-    if (j % S::kChunk == S::kChunk - 1 && (j / S::kChunk + 2) * S::kChunk < n) load_w(j / S::kChunk + 2);
+    const bool chunk = j % S::kChunk == S::kChunk - 1 && (j / S::kChunk + 2) * S::kChunk < n;
+    if (chunk) load_w(j / S::kChunk + 2);
     if (more) {
       const int g = (((begin + j) * 64 + 48) >> gs_shift) - g_first, g_next = (((begin + j + 1) * 64) >> gs_shift) - g_first;
       if ((g >> 3) != (g_next >> 3) && ((g >> 3) + 2) * 8 + g_first <= g_last) load_s((g >> 3) + 2);
     }
     const int after = slot + 1 == S::kXSlots ? 0 : slot + 1;
-    // requests of x(j + kXSlots) in front of the wait below
-    constexpr int kIssued = kReadsAt * S::kXLoads / kInstr;
+    // Younger than x(j + 1), which the reads below wait for: the slots behind it, and of x(j + kXSlots) what is requested by
+    // then.  A chunk requested in this sub-step lies between the two: counted where every sub-step requests one (as long as
+    // there is x to request there are codes), and by a branch in rings of two slots of x, which would wait for what they
+    // have just requested (uncounted: 8 bits, 64 x 96, 4 % of the call, 5 bits 2 to 3 %).  In the others that branch costs 1
+    // to 2 %, and a chunk's own sub-step (one in two or four) waits for a part of x(j + 2) instead; a window's (one in
+    // eight groups) does everywhere.
+    constexpr int kYounger = (S::kXSlots - 2) * S::kXLoads + S::loads_before_reads();
 #pragma unroll
     for (int i = 0; i < 2 * kB; ++i) {
 #pragma unroll
@@ -303,12 +317,13 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
         if (more_x) {
 #pragma unroll
           for (int l = 0; l < S::kXLoads; ++l)
-            if (l * kInstr / S::kXLoads == at) load_x(j + S::kXSlots, slot, l);
+            if (S::load_slot(l) == at) load_x(j + S::kXSlots, slot, l);
         }
         if (more) {
           if (at == kReadsAt) {
-            if constexpr (more_x) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S::kXSlots - 2) * S::kXLoads + kIssued) : "memory");
-            else wait_next(j);
+            if constexpr (!more_x) wait_next(j);
+            else if (S::kChunk == 1 || (S::kXSlots == 2 && chunk)) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kYounger + S::kWLoads) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kYounger) : "memory");
           }
 #pragma unroll
           for (int b = 0; b < kB; ++b)
