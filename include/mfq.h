@@ -271,7 +271,9 @@ int mfq_qmm_n_low_rank(const void* x, int x_dtype, int64_t M, int64_t N, const u
  * The copy's values are the ones the fused kernels use (one rounding of
  * fma(code, scale, bias)); the float32 sums run in another order.
  * mfq_qmm_t_workspace_bytes() returns the size this shape would use on the
- * current device (0: no use for one, pass NULL).  A NULL or smaller workspace
+ * current device (0: no use for one, pass NULL): K is cut only where that is
+ * estimated to be the faster, most shapes up to 512 rows run on tiles small
+ * enough without.  A NULL or smaller workspace
  * is not an error: without room for the copy the call runs as mfq_qmm_t does
  * (the fused kernel, K not split), with room for the copy only its tiles run
  * whole.  The workspace must be 16-byte aligned; its contents before and after
@@ -279,6 +281,26 @@ int mfq_qmm_n_low_rank(const void* x, int x_dtype, int64_t M, int64_t N, const u
  * stream.
  */
 size_t mfq_qmm_t_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size, int bits);
+
+/*
+ * Which kernel mfq_qmm_t_ws runs on for a shape, on the current device, with a
+ * 16-bit y, 16-byte aligned operands and the workspace of
+ * mfq_qmm_t_workspace_bytes(): one of MFQ_KERNEL_*, or a negative MFQ_E* for
+ * arguments the call refuses (and MFQ_EUNSUPPORTED for one row of more than
+ * 8192 codes of 3, 5 or 6 bits, which is not answered).  *k_ranges (may be
+ * NULL): into how many ranges K is cut between workgroups, of the last round of
+ * tiles for the 256 x 256 tiles.  For tests and measurements.  Has no
+ * counterpart in the reference.
+ */
+enum mfq_kernel {
+  MFQ_KERNEL_MATVEC = 1,      /* the kernels for up to 16 rows (3, 5, 6 bits: one) */
+  MFQ_KERNEL_SLICED = 2,      /* 32- and 64-row tiles, K sliced over a workgroup */
+  MFQ_KERNEL_WIDE = 3,        /* 128 x 256 tiles */
+  MFQ_KERNEL_TILES_128 = 4,   /* 128-column tiles */
+  MFQ_KERNEL_TILES_256 = 5,   /* 256 x 256 tiles, dequantised in the GEMM */
+  MFQ_KERNEL_TWO_KERNELS = 6  /* 256 x 256 (or 192) tiles on a 16-bit copy of the weight */
+};
+int mfq_qmm_t_kernel(int64_t M, int64_t K, int64_t N, int group_size, int bits, int* k_ranges);
 int mfq_qmm_t_ws(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq,
                  const void* scales, const void* biases, int sb_dtype, const void* bias, int64_t N,
                  int group_size, int bits, void* y, int y_dtype, void* workspace,

@@ -14,6 +14,8 @@ LIB_PATH = os.path.join(_HERE, "csrc", "libmfq.so")
 F32, F16, BF16 = 0, 1, 2
 MFQ_EUNSUPPORTED = -8  # no kernel for this combination of arguments
 EPILOGUE_GELU, EPILOGUE_GATE_RESIDUAL, EPILOGUE_SWIGLU = 1, 2, 3
+# what mfq_qmm_t_kernel answers
+KERNEL_MATVEC, KERNEL_SLICED, KERNEL_WIDE, KERNEL_TILES_128, KERNEL_TILES_256, KERNEL_TWO_KERNELS = range(1, 7)
 MFQ_ESCRATCH = -9  # mfq_qmm_t_static: the K split needs more than the built-in buffer
 
 # every symbol include/mfq.h declares, with its ctypes signature
@@ -34,6 +36,7 @@ SIGNATURES = {
     "mfq_qmm_n_low_rank": (_INT, [_PTR, _INT, _I64, _I64, _PTR, _PTR, _PTR, _INT, _I64, _INT, _INT, _PTR, _PTR, _I64, _PTR,
                                   _INT, _PTR, ctypes.c_size_t, _PTR]),
     "mfq_qmm_t_workspace_bytes": (ctypes.c_size_t, [_I64, _I64, _I64, _INT, _INT]),
+    "mfq_qmm_t_kernel": (_INT, [_I64, _I64, _I64, _INT, _INT, ctypes.POINTER(_INT)]),
     "mfq_qmm_t_ws": (_INT, [_PTR, _INT, _I64, _I64, _PTR, _PTR, _PTR, _INT, _PTR, _I64, _INT, _INT, _PTR, _INT, _PTR,
                             ctypes.c_size_t, _PTR]),
     "mfq_qmm_t_prepared_bytes": (ctypes.c_size_t, [_I64, _I64, _INT]),

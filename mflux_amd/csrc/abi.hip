@@ -91,18 +91,23 @@ int mfq_dequantize_rows(const uint32_t* wq, const void* scales, const void* bias
                                      out, out_dtype, (hipStream_t)stream);
 }
 
+int mfq_qmm_t_kernel(int64_t M, int64_t K, int64_t N, int group_size, int bits, int* k_ranges) {
+  if (int rc = check_common(group_size, bits)) return rc;
+  if (M <= 0 || N <= 0 || K <= 0 || K % group_size || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return MFQ_ESHAPE;
+  const bool odd_bits = bits != 4 && bits != 8;
+  if (odd_bits && M == 1 && K > 8192) return MFQ_EUNSUPPORTED;  // (a GEMM without the workspace that qmm_route() counts on)
+  mfq::QmmRoute route{MFQ_KERNEL_MATVEC, 1, 0, 0};
+  if (M > (odd_bits ? 1 : 16)) route = mfq::qmm_route(M, N, K, group_size, bits);
+  if (k_ranges) *k_ranges = route.ranges;
+  return route.kernel;
+}
+
 size_t mfq_qmm_t_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size, int bits) {
   if (check_common(group_size, bits) != MFQ_OK) return 0;
   if (N <= 0 || K <= 0 || K % group_size || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return 0;
-  if (bits != 4 && bits != 8) {
-    if (M <= 1) return 0;
-    if (mfq::prefer_frag_path(M, N, K, group_size, bits)) return mfq::qmm_workspace_bytes(M, N, K, group_size, bits);
-    const size_t planes = mfq::qmm_mid_workspace_bytes(M, N, K, group_size);
-    const size_t slice = mfq::qmm_slice_workspace_bytes(M, N, K, group_size, bits);
-    return planes > slice ? planes : slice;
-  }
-  if (M <= 16) return 0;
-  return mfq::qmm_workspace_bytes(M, N, K, group_size, bits);
+  if (M <= (bits == 4 || bits == 8 ? 16 : 1)) return 0;
+  const mfq::QmmRoute route = mfq::qmm_route(M, N, K, group_size, bits);
+  return route.copy + route.planes;
 }
 
 int mfq_qmm_t(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
@@ -125,7 +130,7 @@ int mfq_qmm_t_static(const void* x, int x_dtype, int64_t M, int64_t K, const uin
   if (int rc = check_common(group_size, bits)) return rc;
   size_t need = mfq_qmm_t_workspace_bytes(M, K, N, group_size, bits);
   // a scratch copy of the weights that does not fit is done without (the fused kernel); the planes of a K split are not
-  if (need > kScratchBytes && (bits == 4 || bits == 8) && M > 16) need = mfq::qmm_min_workspace_bytes(M, N, K, group_size, bits);
+  if (need > kScratchBytes && (bits == 4 || bits == 8) && M > 16) need = mfq::qmm_route(M, N, K, group_size, bits).planes;
   if (need > kScratchBytes) return MFQ_ESCRATCH;
   void* ws = nullptr;
   if (need) {

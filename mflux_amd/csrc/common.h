@@ -413,10 +413,15 @@ int launch_silu(const void* x, int dtype, int64_t n, void* y, hipStream_t stream
 // t[M, R] = x[M, K] @ A[K, R], A in fragment order ([R/16][K/32][4][16][8]); 16-bit type `dtype`; R % 16 == 0, K % 32 == 0
 int launch_low_rank_down(const void* x, int dtype, int64_t M, int64_t K, const void* at, int64_t R, void* t,
                          hipStream_t stream);
-// what a caller should bring (the K split's planes, or the scratch copy of the two-kernel path where that is
-// preferred) and what the call cannot do without (the planes only)
-size_t qmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits);
-size_t qmm_min_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits);
+// The GEMM that takes a call of more than 16 rows (3, 5 and 6 bits: more than one) with a 16-bit result, 16-byte aligned
+// operands and the workspace given here, by the rules that the launchers follow
+struct QmmRoute {
+  int kernel;     // MFQ_KERNEL_*
+  int ranges;     // of K (of the tail's tiles where those are 256 x 256)
+  size_t copy;    // bytes of the two-kernel path's scratch copy, which a call can do without
+  size_t planes;  // and of a K cut's float32 planes behind it
+};
+QmmRoute qmm_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
 // the two-kernel path (qmm_frag.hip): dequantize once into a 16-bit copy in fragment order, then a GEMM on
 // 16x16x32 matrix instructions; 4 and 8 bits, 16-bit y of x's type, a low-rank update or an epilogue as
 // launch_qmm / launch_qmm_epilogue.
@@ -468,7 +473,8 @@ int launch_qmm_slice(const void* x, int dtype, int64_t M, int64_t K, const uint3
                      const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
                      void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank = LowRank(),
                      Epilogue epi = Epilogue());
-size_t qmm_slice_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits);
+// ranges of K it takes the shape in, each with a float32 plane if there are several; 0: it does not take it
+int qmm_slice_ranges(int64_t M, int64_t N, int64_t K, int gs, int bits);
 // what launch_qmm_slice is estimated to take, 0 where it does not take the shape
 float qmm_slice_estimate_us(int64_t M, int64_t N, int64_t K, int gs, int bits);
 // 128 x 256 tiles that dequantise into registers (qmm_wide.hip): 4 and 8 bits, K % 256 == 0, up to 1024 rows.
@@ -477,10 +483,10 @@ int launch_qmm_wide(const void* x, int dtype, int64_t M, int64_t K, const uint32
                     const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,
                     void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank = LowRank(),
                     Epilogue epi = Epilogue());
-size_t qmm_wide_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits);
+int qmm_wide_ranges(int64_t M, int64_t N, int64_t K, int gs, int bits);
 // what launch_qmm is estimated to take at 4 and 8 bits without launch_qmm_wide (below 1024 rows)
 float qmm_others_estimate_us(int64_t M, int64_t N, int64_t K, int gs, int bits);
-size_t qmm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs);
+int qmm_mid_ranges(int64_t M, int64_t N, int64_t K, int gs);
 // the same kernel for 3, 5 and 6 bits (any M above one row; K % 32 == 0)
 int launch_qmm_mid_stream(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                           const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,

@@ -25,7 +25,6 @@
 //     and costs a third of the kernel's time.
 //   - the k order inside a step is permuted (lane half h covers k 32h..32h+31)
 //     identically for both operands, which the dot product does not notice.
-#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -1181,18 +1180,22 @@ bool prefer_frag_path(int64_t M, int64_t N, int64_t K, int gs, int bits) {
   return M >= least_rows && qmm_frag_shape_ok(M, N, K, bits) && !use_mid_kernel(M, N, K);
 }
 
-size_t qmm_min_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits) {
-  if (K % BK) return 0;
-  const size_t planes = use_mid_kernel(M, N, K) ? qmm_mid_workspace_bytes(M, N, K, gs)
-                                                : tail_plane_bytes(M, N, plan_tail(M, N, K, period_of(gs), compute_units()));
-  // (the largest: a misaligned operand or an epilogue may still send the call to the other kernels)
-  const size_t slice = qmm_slice_workspace_bytes(M, N, K, gs, bits), wide = qmm_wide_workspace_bytes(M, N, K, gs, bits);
-  return std::max(planes, std::max(slice, wide));
-}
-
-size_t qmm_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits) {
-  const size_t planes = qmm_min_workspace_bytes(M, N, K, gs, bits);
-  return prefer_frag_path(M, N, K, gs, bits) ? qmm_frag_copy_bytes(N, K) + planes : planes;
+// In the order of launch_qmm() and launch_qmm_mid_stream().  What sends a call past the wide or the sliced kernel, scales or
+// biases off 4 bytes, also keeps the kernels behind them from cutting K: no planes but those of the kernel named here are
+// ever used.
+QmmRoute qmm_route(int64_t M, int64_t N, int64_t K, int gs, int bits) {
+  const auto whole_planes = [&](int kernel, int ranges) {
+    return QmmRoute{kernel, ranges, 0, ranges > 1 ? (size_t)ranges * M * N * sizeof(float) : 0};
+  };
+  if (K % BK) return whole_planes(MFQ_KERNEL_TILES_128, 1);
+  if (const int ranges = qmm_wide_ranges(M, N, K, gs, bits)) return whole_planes(MFQ_KERNEL_WIDE, ranges);
+  if (const int ranges = qmm_slice_ranges(M, N, K, gs, bits)) return whole_planes(MFQ_KERNEL_SLICED, ranges);
+  const bool two_kernels = prefer_frag_path(M, N, K, gs, bits);
+  if (use_mid_kernel(M, N, K) || (bits != 4 && bits != 8 && !two_kernels))
+    return whole_planes(MFQ_KERNEL_TILES_128, qmm_mid_ranges(M, N, K, gs));
+  const TailPlan plan = plan_tail(M, N, K, period_of(gs), compute_units());
+  return QmmRoute{two_kernels ? MFQ_KERNEL_TWO_KERNELS : MFQ_KERNEL_TILES_256, plan.splits,
+                  two_kernels ? qmm_frag_copy_bytes(N, K) : 0, tail_plane_bytes(M, N, plan)};
 }
 
 int launch_tail_reduce(int dtype, const float* planes, int n_whole, int splits, int tiles_m, int tiles_n,

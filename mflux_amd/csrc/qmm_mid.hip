@@ -492,10 +492,7 @@ int launch_qmm_mid_stream(const void* x, int dtype, int64_t M, int64_t K, const 
                           void* workspace, size_t workspace_bytes, hipStream_t stream, LowRank low_rank,
                           Epilogue epi) {
 #else
-size_t qmm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs) {
-  const MidPlan plan = plan_mid(M, N, K, period_of(gs), compute_units());
-  return plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
-}
+int qmm_mid_ranges(int64_t M, int64_t N, int64_t K, int gs) { return plan_mid(M, N, K, period_of(gs), compute_units()).splits; }
 
 float qmm_mid_estimate_us(int64_t M, int64_t N, int64_t K, int gs) { return plan_mid(M, N, K, period_of(gs), compute_units()).us; }
 

@@ -593,10 +593,7 @@ int launch_bits(SlicePlan plan, const void* x, int64_t M, int64_t K, const uint3
 
 }  // namespace
 
-size_t qmm_slice_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits) {
-  const SlicePlan plan = choose_slice(M, N, K, gs, bits, true);
-  return plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
-}
+int qmm_slice_ranges(int64_t M, int64_t N, int64_t K, int gs, int bits) { return choose_slice(M, N, K, gs, bits, true).splits; }
 
 float qmm_slice_estimate_us(int64_t M, int64_t N, int64_t K, int gs, int bits) {
   return choose_slice(M, N, K, gs, bits, true).us;

@@ -329,10 +329,7 @@ int launch_type(const WidePlan& plan, const void* x, int64_t M, int64_t K, const
 
 }  // namespace
 
-size_t qmm_wide_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits) {
-  const WidePlan plan = choose_wide(M, N, K, gs, bits, true);
-  return plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
-}
+int qmm_wide_ranges(int64_t M, int64_t N, int64_t K, int gs, int bits) { return choose_wide(M, N, K, gs, bits, true).splits; }
 
 int launch_qmm_wide(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                     const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype,

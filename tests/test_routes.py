@@ -1,0 +1,58 @@
+"""Which kernel a quantized product runs on and the workspace it asks for, as the library answers without a GPU (it then
+counts 256 compute units, which is what the shapes below are for)."""
+import ctypes
+
+import pytest
+
+from mflux_amd import _lib
+
+GROUPS = ((4, 64), (4, 32), (4, 128), (8, 64), (8, 128), (3, 64), (5, 32), (6, 64))
+ROWS = (2, 16, 17, 64, 129, 256, 300, 512, 640, 1000, 1024, 1030, 2100, 4608)
+SIZES = ((256, 64), (768, 3072), (1280, 264), (2560, 4096), (3072, 3072), (3072, 12288), (12288, 3072), (3584, 37888), (18944, 520),
+         (2080, 1000))
+
+
+def route(M, K, N, bits, gs):
+    ranges = ctypes.c_int()
+    kernel = _lib.load().mfq_qmm_t_kernel(M, K, N, gs, bits, ctypes.byref(ranges))
+    assert kernel > 0, (kernel, M, K, N, bits, gs)
+    return kernel, ranges.value
+
+
+def workspace(M, K, N, bits, gs):
+    return _lib.load().mfq_qmm_t_workspace_bytes(M, K, N, gs, bits)
+
+
+def test_arguments_are_checked():
+    f = _lib.load().mfq_qmm_t_kernel
+    assert f(4, 128, 8, 48, 4, None) == -2 and f(4, 128, 8, 64, 7, None) == -3
+    for bad in ((0, 128, 8), (4, 100, 8), (4, 128, 0), (1 << 31, 128, 8)):
+        assert f(*bad, 64, 4, None) == -4
+    assert f(1, 8192, 64, 64, 3, None) == _lib.KERNEL_MATVEC and f(1, 8256, 64, 64, 3, None) == _lib.MFQ_EUNSUPPORTED
+    assert f(16, 3072, 64, 64, 4, None) == _lib.KERNEL_MATVEC
+
+
+@pytest.mark.parametrize("bits,gs", GROUPS)
+def test_the_workspace_is_what_the_kernel_uses(bits, gs):
+    """Planes for the ranges of K the kernel named takes and for no other kernel's, the 16-bit copy where that is made."""
+    for M in ROWS:
+        for K, N in SIZES:
+            if K % gs:
+                continue
+            kernel, ranges = route(M, K, N, bits, gs)
+            need = workspace(M, K, N, bits, gs)
+            if kernel == _lib.KERNEL_MATVEC:
+                assert need == 0
+            elif kernel in (_lib.KERNEL_SLICED, _lib.KERNEL_WIDE, _lib.KERNEL_TILES_128):
+                assert need == (ranges * M * N * 4 if ranges > 1 else 0), (M, K, N)
+            else:
+                copy = -(-N // 16) * 16 * K * 2 // 256 * 256 if kernel == _lib.KERNEL_TWO_KERNELS else 0
+                planes = need - copy
+                assert planes % (ranges * 256 * 256 * 4) == 0 and (planes > 0) == (ranges > 1), (M, K, N)
+
+
+@pytest.mark.parametrize("M,K,N", [(256, 3072, 3072), (512, 3072, 3072), (300, 2560, 4096)])
+def test_shapes_that_run_in_one_launch_ask_for_no_planes(M, K, N):
+    for bits, gs in ((4, 64), (4, 128)):
+        assert route(M, K, N, bits, gs) == (_lib.KERNEL_SLICED, 1)
+        assert workspace(M, K, N, bits, gs) == 0
