@@ -495,18 +495,19 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
 
 // ---- which tile, and whether at all.
 //
-// Time of a call by tile, from 700 drawn shapes (17 to 1100 rows, 3 to 8 bits, groups of 32 to 128, cold weights, a stream
-// of launches; the fit is 4 to 9 % rms): 2.5 us and, for each round of workgroups, 2.4 us and the sub-steps of a wavefront
-// times kAlone (one workgroup on the chip) to kAlone + kCrowd (all of it); a cut of K over workgroups costs the launch of
-// the second kernel and its planes, 3.5 us and 5 bytes/ps.
+// Time of a call by tile, from 3000 drawn shapes on each tile (2 to 1023 rows, 3 to 8 bits, groups of 32 to 128, cold weights,
+// a stream of launches; the fit is 7 to 8 % rms): 3.1 us and, for each round of workgroups, `first` (first bytes, partial tiles,
+// store; it grows with the tile) and `step` for every sub-step of a wavefront.  A cut of K over workgroups costs the launch of
+// the second kernel and its planes, 3.4 us and 1.3 bytes/ps.  (With one first cost for all tiles the wide tiles on short K
+// came out up to 40 % too low.)
 struct Tile {
   int rows, columns;
-  float alone[5], crowd;  // us per sub-step at 3, 4, 5, 6, 8 bits
+  float first, step[5];  // us; the step at 3, 4, 5, 6, 8 bits
 };
 constexpr Tile kTiles[] = {
-    {32, 32, {0.42f, 0.385f, 0.49f, 0.465f, 0.40f}, 0.10f}, {64, 32, {0.52f, 0.44f, 0.58f, 0.52f, 0.46f}, 0.13f},
-    {64, 48, {0.67f, 0.55f, 0.71f, 0.68f, 0.59f}, 0.18f},   {64, 64, {0.87f, 0.665f, 0.90f, 0.85f, 0.73f}, 0.20f},
-    {64, 96, {1.17f, 0.91f, 1.36f, 1.25f, 1.08f}, 0.34f},
+    {32, 32, 1.8f, {0.43f, 0.47f, 0.58f, 0.60f, 0.54f}}, {64, 32, 2.7f, {0.58f, 0.55f, 0.64f, 0.65f, 0.59f}},
+    {64, 48, 3.9f, {0.74f, 0.67f, 0.80f, 0.81f, 0.70f}}, {64, 64, 4.8f, {0.91f, 0.74f, 0.97f, 0.96f, 0.83f}},
+    {64, 96, 6.9f, {1.22f, 1.01f, 1.33f, 1.50f, 1.05f}},
 };
 
 struct SlicePlan {
@@ -523,27 +524,34 @@ inline SlicePlan plan_slice(int64_t M, int64_t N, int64_t K, int bits, bool may_
     if (t.rows == 32 && M > 128) continue;  // (every code is then dequantised for five row tiles and more)
     const int64_t tiles = ((M + t.rows - 1) / t.rows) * ((N + t.columns - 1) / t.columns);
     for (int s = 1; s == 1 || (may_cut && s <= 8 && tiles * s <= cus && K / 64 / s >= 8); ++s) {
-      const int64_t items = tiles * s, rounds = (items + cus - 1) / cus;
+      const int64_t rounds = (tiles * s + cus - 1) / cus;
       const int subs = (grains + kWaves * s - 1) / (kWaves * s) * gran;
-      const float load = items < cus ? (float)items / (float)cus : 1.f;
-      float us = 2.5f + (float)rounds * (2.4f + (float)subs * (t.alone[width] + t.crowd * load));
-      if (s > 1) us += 3.5f + (float)(s * M * N) * (4.f / 5e6f);
+      float us = 3.1f + (float)rounds * (t.first + (float)subs * t.step[width]);
+      if (s > 1) us += 3.4f + (float)(s * M * N) * (4.f / 1.3e6f);
       if (best.splits == 0 || us < best.us) best = SlicePlan{t.rows, t.columns, s, us};
     }
   }
   return best;
 }
 
-// Taken where its estimate is 7 % (8 bits: 16 %) below the other kernel's (that estimate and 5 us, as it leaves the launch
-// and the first bytes out).  Over the 700 shapes, of which 460 come here, this leaves 0.80 of the time before (geometric
-// mean), four shapes behind by 4 to 10 % (6 bits 89 rows x 3072 -> 12288, 27.6 us, is the worst) and 1.6 % to a perfect
-// choice.  Of 2400 drawn calls at 4 bits that come here 8 are 3 to 8 % behind (600 rows x 2560 -> 2560); at 8 bits with 7 %
-// 32 of 1020 were, all from the 169 that 16 % leaves out (138 x 2560 -> 10240 26.8 -> 28.7 us).
+// What the 128-column-tile kernel takes on the same shapes: its own estimate leaves out 4.3 us of launch and first bytes,
+// 0.15 us for each plane of a cut, and what a bit stream's codes cost it (3, 5 and 6 bits).
+inline float others_us(int64_t M, int64_t N, int64_t K, int gs, int bits) {
+  const int ranges = qmm_mid_ranges(M, N, K, gs);
+  const float width = bits == 3 ? 1.08f : bits == 4 ? 1.02f : bits == 5 ? 1.16f : bits == 6 ? 1.12f : 1.03f;
+  return 4.3f + width * qmm_mid_estimate_us(M, N, K, gs) + (ranges > 1 ? 0.15f * (float)ranges : 0.f);
+}
+
+// Taken where its estimate is a tenth below that one.  Of 11900 drawn calls (2 to 1023 rows at 3, 5 and 6 bits, 17 to 1023 at 4
+// and 8; model sizes and short K) 6900 are, in 0.71 of the other kernel's time (geometric mean; 2 to 16 rows 0.77), 15 of them
+// 3 % or more behind it and 5 by 6 to 9 % (6 bits 126 rows x 3072 -> 12288 31.0 -> 33.8 us): both estimates are off by some 7 %.
+// Before the tiles' first costs were told apart (2.4 us each) and the other kernel's planes and widths counted, 235 calls were
+// 3 % behind, 123 by more than 6 (6 bits 33 x 768 -> 37888 19.8 -> 27.3 us, 76 x 3072 -> 12288 28.8 -> 33.0).
 inline SlicePlan choose_slice(int64_t M, int64_t N, int64_t K, int gs, int bits, bool may_cut) {
   const int64_t gran = bits == 3 || bits == 5 ? 128 : 64;
   if (M > 1024 || N % 8 || K % gran || (K / gs) % 2 || M * K >= (int64_t)1 << 31 || N * K >= (int64_t)1 << 31) return SlicePlan();
   const SlicePlan plan = plan_slice(M, N, K, bits, may_cut);
-  return plan.us < (bits == 8 ? 0.84f : 0.93f) * (5.f + qmm_mid_estimate_us(M, N, K, gs)) ? plan : SlicePlan();
+  return plan.us < 0.9f * others_us(M, N, K, gs, bits) ? plan : SlicePlan();
 }
 
 template <typename T, int BITS, int kA, int kB>

@@ -56,3 +56,26 @@ def test_shapes_that_run_in_one_launch_ask_for_no_planes(M, K, N):
     for bits, gs in ((4, 64), (4, 128)):
         assert route(M, K, N, bits, gs) == (_lib.KERNEL_SLICED, 1)
         assert workspace(M, K, N, bits, gs) == 0
+
+
+# measured on 256 units, us on the sliced and on the 128-column tiles
+@pytest.mark.parametrize("M,K,N,bits,gs", [
+    (33, 768, 37888, 6, 64),    # 27.3, 19.8
+    (76, 3072, 12288, 6, 64),   # 33.0, 28.8
+    (4, 768, 37888, 6, 128),    # 25.5, 20.9
+    (128, 2560, 9216, 6, 128),  # 30.1, 26.4
+    (442, 768, 3072, 5, 64),    # 15.4, 13.6
+    (358, 1152, 4096, 4, 64),   # 19.7, 17.9
+    (432, 2560, 3840, 4, 64),   # 28.3, 26.6
+])
+def test_the_sliced_kernel_is_left_where_it_is_the_slower(M, K, N, bits, gs):
+    assert route(M, K, N, bits, gs)[0] == _lib.KERNEL_TILES_128
+
+
+@pytest.mark.parametrize("M,K,N,bits,gs", [
+    (840, 3072, 512, 5, 64), (16, 3072, 3072, 6, 64), (2, 2560, 4096, 3, 64), (256, 3072, 3072, 4, 64), (300, 2560, 4096, 6, 64),
+    (208, 6144, 64, 5, 64),     # 11.5, 16.0
+    (159, 3584, 4096, 6, 32),   # 23.5, 27.4
+])
+def test_the_sliced_kernel_is_kept_where_it_is_the_faster(M, K, N, bits, gs):
+    assert route(M, K, N, bits, gs)[0] == _lib.KERNEL_SLICED
