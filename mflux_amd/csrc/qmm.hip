@@ -1304,6 +1304,7 @@ int launch_qmm(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* w
     return launch_qmm_frag(x, dtype, M, K, wq, scales, biases, bias, N, gs, bits, y, workspace, plan.n_whole,
                            plan.splits, stream, low_rank, epi);
   }
+  if (epi.kind != kEpiNone && low_rank.R) return MFQ_EUNSUPPORTED;  // (its 256 x 256 tiles have one or the other)
   if (epi.kind != kEpiNone)
     return launch_qmm_epilogue(x, dtype, M, K, wq, scales, biases, bias, N, gs, bits, y, y_dtype, workspace,
                                workspace_bytes, stream, epi);

@@ -400,7 +400,7 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
     vec8 wf[kB], xf[kA];
 #pragma unroll
     for (int b = 0; b < kB; ++b) {
-      wf[b] = *reinterpret_cast<const vec8*>(lr_bs + (int64_t)min(n0 + 16 * b + r, N - 1) * lr_rank + kk);
+      wf[b] = *reinterpret_cast<const vec8*>(lr_bs + (int64_t)weight_row(16 * b + r) * lr_rank + kk);
       if (!in) wf[b] = zero;
     }
 #pragma unroll

@@ -104,3 +104,34 @@ def test_epilogues_are_the_separate_operations(M, K, N):
     y = core.quantized_matmul_epilogue(x, *packed, epilogue="swiglu", group_size=64, bits=4, bias=bias)
     want = core.swiglu_unstack(lin).double()
     assert bool(((y.double() - want).abs() <= 2.0 ** -6 * want.abs() + 1e-6).all())  # the sigmoid's last place, twice rounded
+
+
+def test_update_and_swiglu_together():
+    """The update's rows are the tile's own weight rows, half of them the gate's and half the up projection's.  The C interface
+    offers no call with both, so the launcher is called itself."""
+    import ctypes
+
+    import mflux_amd
+    from mflux_amd import _lib, core
+
+    class LowRank(ctypes.Structure):
+        _fields_ = [("t", ctypes.c_void_p), ("bs", ctypes.c_void_p), ("R", ctypes.c_int)]
+
+    class Epilogue(ctypes.Structure):
+        _fields_ = [("kind", ctypes.c_int), ("gate", ctypes.c_void_p), ("residual", ctypes.c_void_p), ("act_from", ctypes.c_int)]
+
+    M, K, N, rank = 70, 3072, 1024, 48
+    ptr, i64, i32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
+    launch = getattr(_lib.load(), "_ZN3mfq16launch_qmm_sliceEPKvillPKjS1_S1_S1_liiPviS4_mP12ihipStream_tNS_7LowRankENS_8EpilogueE")
+    launch.restype = i32
+    launch.argtypes = [ptr, i32, i64, i64, ptr, ptr, ptr, ptr, i64, i32, i32, ptr, i32, ptr, ctypes.c_size_t, ptr, LowRank, Epilogue]
+    x, (wq, s, b), bias, _ = _operands(M, K, N, 4, 64, torch.bfloat16)
+    t, bs = torch.randn(M, rank, device="cuda").bfloat16(), (torch.randn(N, rank, device="cuda") * 0.3).bfloat16()
+    y = torch.empty(M, N // 2, device="cuda", dtype=torch.bfloat16)
+    rc = launch(x.data_ptr(), _lib.BF16, M, K, wq.data_ptr(), s.data_ptr(), b.data_ptr(), bias.data_ptr(), N, 64, 4, y.data_ptr(),
+                _lib.BF16, None, 0, torch.cuda.current_stream().cuda_stream, LowRank(t.data_ptr(), bs.data_ptr(), rank),
+                Epilogue(_lib.EPILOGUE_SWIGLU, None, None, 0))
+    assert rc == 0
+    lin = mflux_amd.quantized_matmul(x, wq, s, b, group_size=64, bits=4, bias=bias, low_rank=(t, bs))
+    want = core.swiglu_unstack(lin).double()
+    assert bool(((y.double() - want).abs() <= 2.0 ** -6 * want.abs() + 1e-6).all())
