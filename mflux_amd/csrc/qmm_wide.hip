@@ -289,19 +289,21 @@ inline WidePlan plan_wide(int64_t M, int64_t N, int64_t K, int bits, bool may_cu
   return best;
 }
 
-// Taken where its estimate is a tenth (257 to 512 rows) or a sixth below that of the kernel that would run.  Of 7400 drawn
-// calls of 55 to 1023 rows those are 714, in 0.88 of their time (geometric mean), the slowest 1 % behind; with a tenth for
-// all rows 1206, but 54 of the added ones 3 to 9 % behind (67 rows x 2560 -> 19456 28.0 -> 30.5 us, 908 x 12288 ->
-// 3072 90 -> 95), where the others' estimates are some 5 % high; with a sixth for all, 257 to 512 rows lose what they gain
-// between the two (320 x 18944 -> 3584, 85 us against 70).  From 1024 rows on the 256 x 256 tiles are ahead (1024 x 3072 ->
-// 12288 83 us against 89).  8 bits in groups of 32 stay with the other kernels: the scales of a quad are sixteen registers
-// more than there are, and 879 rows x 10240 -> 4096 took 163 us against 101.
+// Taken where its estimate is a tenth below that of the kernel that would run, up to 128 rows a fifth and from 769 rows on a
+// sixth.  Of 2180 drawn calls of 17 to 1023 rows at 4 and 8 bits with such a K 105 are, in 0.905 of the time (geometric mean),
+// 3 of them 3 to 6 % behind.  Up to 128 rows there is one row of tiles: every code is used once, and weights fetched a quarter
+// line at a time are what the call takes; of 45 calls between a tenth and a fifth 17 were behind (67 rows x 2560 -> 19456 29.1 ->
+// 33.1 us).  From 769 rows on 256-row tiles are well filled, 3 of 10 between a tenth and a sixth were behind (1019 x 12288 -> 3072
+// 89 -> 98 us).  In between the band is worth having (627 x 18944 -> 3072 101 -> 87 us, 135 x 3840 -> 12288 46 -> 42).  Calls of
+// 100 us and more, which the power limit slows, come out up to 15 % low on either side (320 x 3584 -> 37888: 94 for 110).  From
+// 1024 rows on the 256 x 256 tiles are ahead (1024 x 3072 -> 12288 83 us against 89).  8 bits in groups of 32 stay with the other
+// kernels: the scales of a quad are sixteen registers more than there are, and 879 rows x 10240 -> 4096 took 163 us against 101.
 inline WidePlan choose_wide(int64_t M, int64_t N, int64_t K, int gs, int bits, bool may_cut) {
   const WidePlan none{0, 0, 0, 0.f};
   if (bits != 4 && (bits != 8 || gs == 32)) return none;
   if (M >= 1024 || K % (4 * TK) || M * K >= (int64_t)1 << 31 || N * K >= (int64_t)1 << 31) return none;
   const WidePlan plan = plan_wide(M, N, K, bits, may_cut);
-  const float share = M > 256 && M <= 512 ? 0.9f : 0.84f;
+  const float share = M <= 128 ? 0.8f : M <= 768 ? 0.9f : 0.84f;
   return plan.us < share * qmm_others_estimate_us(M, N, K, gs, bits) ? plan : none;
 }
 

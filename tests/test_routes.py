@@ -79,3 +79,17 @@ def test_the_sliced_kernel_is_left_where_it_is_the_slower(M, K, N, bits, gs):
 ])
 def test_the_sliced_kernel_is_kept_where_it_is_the_faster(M, K, N, bits, gs):
     assert route(M, K, N, bits, gs)[0] == _lib.KERNEL_SLICED
+
+
+# measured on 256 units, us on the kernel named and on the other one
+@pytest.mark.parametrize("M,K,N,bits,gs,wide", [
+    (627, 18944, 3072, 4, 64, True),    # 87, 101
+    (135, 3840, 12288, 4, 128, True),   # 42, 46
+    (320, 3584, 37888, 4, 64, True), (320, 3584, 37888, 8, 64, True), (320, 18944, 3584, 4, 64, True), (100, 2304, 38016, 4, 64, True),
+    (67, 2560, 19456, 4, 64, False),    # 29, 33
+    (1019, 12288, 3072, 4, 128, False), # 89, 98
+    (1024, 3072, 12288, 4, 64, False),  # 83, 89
+    (879, 10240, 4096, 8, 32, False),   # 101, 163
+])
+def test_where_the_wide_kernel_is_taken(M, K, N, bits, gs, wide):
+    assert (route(M, K, N, bits, gs)[0] == _lib.KERNEL_WIDE) == wide
