@@ -31,3 +31,18 @@ def raw(t: torch.Tensor) -> np.ndarray:
 
 def to_f64(t: torch.Tensor) -> np.ndarray:
     return t.detach().to(torch.float64).cpu().numpy()
+
+
+def kernel_of(M: int, K: int, N: int, bits: int, group_size: int) -> tuple[int, int]:
+    """The GEMM a product of that shape runs on here (_lib.KERNEL_*) and into how many ranges it cuts K: what a test that is
+    about one kernel asserts, so that a rule that changes cannot leave it testing another.  Shapes are for 256 compute units."""
+    import ctypes
+
+    import pytest
+    from mflux_amd import _lib
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("shapes are chosen for 256 compute units")
+    ranges = ctypes.c_int()
+    kernel = _lib.load().mfq_qmm_t_kernel(M, K, N, group_size, bits, ctypes.byref(ranges))
+    return kernel, ranges.value

@@ -23,12 +23,25 @@ ULP = 2.0 ** -8  # one more rounding to bfloat16, relative to the value
 SHAPES = [
     (2304, 512, 4096, 4, 64),    # 256 x 256 tiles, whole tiles only
     (4400, 1024, 3840, 8, 64),   # 256 x 256 tiles, the short last round cut along K (second kernel)
-    (300, 512, 1024, 4, 64),     # 128-column tiles
-    (512, 3072, 3072, 4, 64),    # 128-column tiles cut along K (second kernel)
-    (200, 1024, 640, 5, 128),    # 5-bit stream
-    (77, 96, 128, 8, 32),        # K % 64 == 32
-    (100, 256, 192, 4, 64),      # 128-row tiles
+    (300, 512, 1024, 4, 64),     # K sliced over a workgroup
+    (512, 3072, 3072, 4, 64),    # the same, several tiles in M
+    (200, 1024, 640, 5, 128),    # the same on a 5-bit stream
+    (77, 96, 128, 8, 32),        # 128-column tiles, K % 64 == 32
+    (100, 256, 192, 4, 64),      # K sliced, wavefronts with one sub-step
+    (1030, 512, 1024, 4, 64),    # 128-column tiles
+    (1030, 1280, 320, 8, 64),    # 128-column tiles cut along K (second kernel)
+    (1030, 1024, 640, 5, 128),   # the same on a 5-bit stream
+    (257, 256, 20480, 4, 64),    # 128 x 256 tiles
 ]
+
+
+def test_the_shapes_run_on_every_kernel():
+    from gpu_util import kernel_of
+    from mflux_amd import _lib
+
+    ran = {(kernel, ranges > 1) for kernel, ranges in (kernel_of(*shape) for shape in SHAPES)}
+    assert ran >= {(_lib.KERNEL_TWO_KERNELS, False), (_lib.KERNEL_TWO_KERNELS, True), (_lib.KERNEL_SLICED, False),
+                   (_lib.KERNEL_TILES_128, False), (_lib.KERNEL_TILES_128, True), (_lib.KERNEL_WIDE, False)}
 
 
 def _operands(o, cfg, M, K, N, bits, gs):

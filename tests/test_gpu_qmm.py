@@ -641,16 +641,20 @@ def test_f16_path(oracle, bits):
 
 @pytest.mark.parametrize("bits,gs", [(4, 64), (8, 64), (4, 32), (8, 32), (4, 128), (8, 128)])
 @pytest.mark.parametrize("M,K,N", [(100, 512, 1000), (128, 3072, 136), (129, 1024, 264), (256, 2048, 520),
-                                   (400, 768, 130), (77, 768, 3072)])
+                                   (400, 768, 130), (77, 768, 3072), (100, 512, 1004), (128, 3072, 140), (129, 1024, 268),
+                                   (256, 2048, 524), (77, 768, 3076)])
 def test_qmm_medium_m(oracle, bits, gs, M, K, N):
-    """The 128-column-tile kernel: 128-row tiles (M <= 128) and 256-row tiles,
-    ragged M and N, K with and without a split, a K that is not a whole number
-    of scale periods (768 with groups of 128), all group sizes; bf16 with bias
-    and float32 output."""
+    """The 128-column-tile kernel (N not a multiple of 8) and the one with K
+    sliced over a workgroup: 128-row tiles (M <= 128) and 256-row tiles, ragged
+    M and N, K with and without a split, a K that is not a whole number of scale
+    periods (768 with groups of 128), all group sizes; bf16 with bias and
+    float32 output."""
     import mflux_amd
-    from gpu_util import to_dev, u32_to_dev
+    from gpu_util import kernel_of, to_dev, u32_to_dev
+    from mflux_amd import _lib
 
     o = oracle
+    assert N % 8 == 0 or kernel_of(M, K, N, bits, gs)[0] == _lib.KERNEL_TILES_128
     args = _case(o, 31, M, K, N, bits, gs=gs)
     ref = _ref(o, *args, bits, gs)
     _assert_close(_run(o, *args, bits, gs), ref)
@@ -671,13 +675,15 @@ def test_qmm_medium_m_odd_n(oracle):
 
 @pytest.mark.parametrize("bits,gs", [(4, 64), (8, 128)])
 def test_qmm_many_rows_long_k_split(oracle, bits, gs):
-    """More than 512 rows, few 256 x 256 tiles and K >= 8192: the large-M
+    """1024 rows or more, few 256 x 256 tiles and K >= 8192: the large-M
     kernel with every tile cut along K across compute units."""
+    from gpu_util import kernel_of
     from mflux_amd import _lib
 
     o = oracle
-    M, K, N = 600, 8192, 256
-    assert _lib.load().mfq_qmm_t_workspace_bytes(M, K, N, gs, bits) >= 2 * M * N * 4
+    M, K, N = 1030, 8192, 256
+    kernel, ranges = kernel_of(M, K, N, bits, gs)
+    assert kernel == _lib.KERNEL_TILES_256 and ranges > 1
     args = _case(o, 33, M, K, N, bits, gs=gs)
     _assert_close(_run(o, *args, bits, gs), _ref(o, *args, bits, gs))
 
@@ -729,7 +735,7 @@ def test_calls_replay_in_a_hip_graph(oracle):
     import mflux_amd
 
     torch.manual_seed(9)
-    shapes = ((1, 3072, 1024, 8), (300, 2048, 520, 4), (2200, 512, 2304, 4))
+    shapes = ((1, 3072, 1024, 8), (300, 2048, 524, 4), (2200, 512, 2304, 4))
     ops = []
     for M, K, N, bits in shapes:
         x = torch.randn(M, K, device="cuda").to(torch.bfloat16)

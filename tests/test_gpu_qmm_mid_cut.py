@@ -28,30 +28,47 @@ def _close(y, ref):
     assert float(err.max()) <= 1e-2
 
 
-# K: 5, 10, 7 and 37 scale periods (groups of 64; half or twice that for 128 and 32) against any number of ranges
+# K: 5, 10, 7 and 37 scale periods (groups of 64; half or twice that for 128 and 32) against any number of ranges.  With
+# columns that are a multiple of 8 the sliced kernel takes these; with 4 more this one does.
 @pytest.mark.parametrize("bits,gs", [(4, 64), (8, 64), (6, 64), (3, 128), (4, 128), (8, 32)])
-@pytest.mark.parametrize("M,K,N", [(17, 1280, 64), (129, 2560, 392), (300, 1792, 1000), (513, 9472, 128), (1000, 1280, 264)])
+@pytest.mark.parametrize("M,K,N", [(17, 1280, 64), (129, 2560, 392), (300, 1792, 1000), (513, 9472, 128), (1000, 1280, 264),
+                                   (17, 1280, 68), (129, 2560, 396), (300, 1792, 1004), (513, 9472, 132), (1000, 1280, 268)])
 def test_unequal_k_ranges(M, K, N, bits, gs):
     import mflux_amd
+    from gpu_util import kernel_of
+    from mflux_amd import _lib
 
     if K % (4 * gs):
         K += 4 * gs - K % (4 * gs)
+    if N % 8:
+        kernel, ranges = kernel_of(M, K, N, bits, gs)
+        assert kernel == _lib.KERNEL_TILES_128 and ranges > 1
     x, packed, bias, ref = _operands(M, K, N, bits, gs, 71)
     _close(mflux_amd.quantized_matmul(x, *packed, group_size=gs, bits=bits, bias=bias), ref + bias.double())
     _close(mflux_amd.quantized_matmul(x.float(), *packed, group_size=gs, bits=bits), ref)
 
 
-@pytest.mark.parametrize("M", [40, 300, 520])
-def test_unequal_k_ranges_with_update_and_epilogue(M):
+# on the sliced kernel, and on this one: 128-row tiles and 256-row ones, few ranges and many
+@pytest.mark.parametrize("M,K,N,bits,here", [
+    (40, 1280, 256, 4, False), (300, 1280, 256, 4, False), (520, 1280, 256, 4, False), (70, 2560, 12296, 4, True),
+    (200, 9728, 3072, 8, True), (256, 12288, 3072, 4, True), (1030, 1280, 264, 4, True), (1100, 2560, 392, 5, True)])
+def test_unequal_k_ranges_with_update_and_epilogue(M, K, N, bits, here):
     """The low-rank update enters once, with the first range; GELU and gate are the reduction's."""
     import mflux_amd
-    from mflux_amd import core
+    from gpu_util import kernel_of
+    from mflux_amd import _lib, core
 
-    x, packed, bias, ref = _operands(M, 1280, 256, 4, 64, 72)
-    t, bs = torch.randn(M, 16, device="cuda").bfloat16(), (torch.randn(256, 16, device="cuda") * 0.02).bfloat16()
-    y = mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=4, bias=bias, low_rank=(t, bs))
+    kernel, ranges = kernel_of(M, K, N, bits, 64)
+    assert (kernel == _lib.KERNEL_TILES_128 and ranges > 1) == here
+    x, packed, bias, ref = _operands(M, K, N, bits, 64, 72)
+    t, bs = torch.randn(M, 16, device="cuda").bfloat16(), (torch.randn(N, 16, device="cuda") * 0.02).bfloat16()
+    y = mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=bits, bias=bias, low_rank=(t, bs))
     _close(y, ref + bias.double() + t.double() @ bs.double().t())
-    y = core.quantized_matmul_epilogue(x, *packed, epilogue="gelu", group_size=64, bits=4, bias=bias)
+    plain = mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=bits, bias=bias)
+    gate, res = torch.randn(N, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
+    y = core.quantized_matmul_epilogue(x, *packed, epilogue="gate_residual", group_size=64, bits=bits, bias=bias, gate=gate, residual=res)
+    assert torch.equal(y, res + gate * plain)
+    y = core.quantized_matmul_epilogue(x, *packed, epilogue="gelu", group_size=64, bits=bits, bias=bias)
     # the linear's 1e-2 of ITS largest output in the row, through a slope of at most 1.13, and one more rounding
     lin = ref + bias.double()
     want = torch.nn.functional.gelu(lin, approximate="tanh")

@@ -1,6 +1,6 @@
 """GPU parity: the GEMM with K sliced over the wavefronts of a workgroup (csrc/qmm_slice.hip), at the edges of its tiles
-(32 and 64 rows; 32, 48, 64 and 96 columns), rings, chunks and windows, and against the 128-column-tile kernel, which
-takes the same call when scales and biases lie at odd addresses.
+(32 and 64 rows; 32, 48, 64 and 96 columns), rings, chunks and windows, and the kernels that take the same call when scales
+and biases lie at odd addresses (the 128-column tiles in their form for those, K whole).
 
 Reference: float64 on the dequantised weights rounded once to the 16-bit type, which is what the kernels multiply.  What
 is left is the rounding of the result (half a unit in the last of 8 or 11 significant bits, at most 2^-8 of it in bfloat16

@@ -1,6 +1,7 @@
 """GPU parity: the GEMM whose wavefronts dequantise into registers (csrc/qmm_wide.hip) at the edges of its 128 x 256 tiles,
 with one quad of steps to a range and several, K whole and cut into ranges, and against the kernels that take the same call
-when scales and biases lie at odd addresses.  The shapes are ones that its rule takes on 256 compute units.
+when scales and biases lie at odd addresses (forms for those, K whole).  The shapes are ones that its rule takes on 256
+compute units, where a test does not say otherwise; the tests ask the library.
 
 Reference: float64 on the dequantised weights rounded once to the 16-bit type, which is what the kernels multiply.  What
 is left is the rounding of the result (at most 2^-8 of it in bfloat16 and 2^-11 in float16; the bias add rounds once more)
@@ -40,14 +41,24 @@ def _at_odd_address(t):
 
 
 # rows: part of a tile, a tile, one more, several; columns: ragged (no epilogue), a tile's part, whole tiles
-# K: one quad (256) and two, an even and an uneven cut into ranges, long
-@pytest.mark.parametrize("M,K,N", [(40, 512, 32770), (128, 512, 32770), (257, 256, 20480), (385, 256, 32770), (600, 256, 24584),
-                                   (384, 4096, 4100), (513, 12288, 1032), (1000, 12288, 1032), (128, 6144, 24584)])
-@pytest.mark.parametrize("bits,gs,dtype", [(4, 64, "bf16"), (4, 32, "f16"), (4, 128, "bf16"), (8, 64, "f16"), (8, 64, "bf16"),
-                                           (8, 128, "bf16")])
+# K: one quad (256) and two, whole over many quads, an even and an uneven cut into ranges, long
+WHOLE = {4: [(100, 2304, 38016), (257, 256, 20480), (385, 256, 32770), (600, 256, 24584), (257, 2816, 16392)],
+         8: [(600, 256, 24584), (257, 2816, 32776)]}
+CUT = {4: [(384, 4096, 4100), (513, 12288, 1032), (1000, 12288, 1032)], 8: [(513, 12288, 1032), (1000, 12288, 1032)]}
+NOT_TAKEN = [(40, 512, 32770), (128, 512, 32770), (128, 6144, 24584)]  # (wide calls of few rows, which are left)
+FORMS = {4: [(64, "bf16"), (32, "f16"), (128, "bf16")], 8: [(64, "f16"), (64, "bf16"), (128, "bf16")]}
+
+
+@pytest.mark.parametrize("M,K,N,bits,gs,dtype", [
+    (*shape, bits, *form) for bits in (4, 8) for shape in WHOLE[bits] + CUT[bits] + NOT_TAKEN for form in FORMS[bits]])
 def test_tiles_ranges_and_the_other_kernels(M, K, N, bits, gs, dtype):
     import mflux_amd
+    from gpu_util import kernel_of
+    from mflux_amd import _lib
 
+    kernel, ranges = kernel_of(M, K, N, bits, gs)
+    assert (kernel == _lib.KERNEL_WIDE) == ((M, K, N) not in NOT_TAKEN)
+    assert kernel != _lib.KERNEL_WIDE or (ranges > 1) == ((M, K, N) in CUT[bits])
     dtype = DT[dtype]
     x, (wq, s, b), bias, ref = _operands(M, K, N, bits, gs, dtype)
     y = mflux_amd.quantized_matmul(x, wq, s, b, group_size=gs, bits=bits, bias=bias)
@@ -59,32 +70,39 @@ def test_tiles_ranges_and_the_other_kernels(M, K, N, bits, gs, dtype):
     _close(y32, ref, dtype, 0)
 
 
-@pytest.mark.parametrize("M,K,N", [(257, 256, 20480), (640, 12288, 1032)])
+@pytest.mark.parametrize("M,K,N,bits", [(257, 256, 20480, 4), (640, 12288, 1032, 4), (257, 2816, 32776, 8)])
 @pytest.mark.parametrize("rank", [16, 48])
-def test_low_rank_update(M, K, N, rank):
+def test_low_rank_update(M, K, N, bits, rank):
     import mflux_amd
+    from gpu_util import kernel_of
+    from mflux_amd import _lib
 
-    x, packed, bias, ref = _operands(M, K, N, 4, 64, torch.bfloat16)
+    assert kernel_of(M, K, N, bits, 64)[0] == _lib.KERNEL_WIDE
+    x, packed, bias, ref = _operands(M, K, N, bits, 64, torch.bfloat16)
     t, bs = torch.randn(M, rank, device="cuda").bfloat16(), (torch.randn(N, rank, device="cuda") * 0.02).bfloat16()
-    y = mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=4, bias=bias, low_rank=(t, bs))
+    y = mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=bits, bias=bias, low_rank=(t, bs))
     _close(y, ref + bias.double() + t.double() @ bs.double().t(), torch.bfloat16, 2)
 
 
-@pytest.mark.parametrize("M,K,N", [(257, 256, 20480), (385, 6144, 8256), (640, 12288, 1088)])
-def test_epilogues_are_the_separate_operations(M, K, N):
+# K whole over one quad of steps and over eleven, and cut
+@pytest.mark.parametrize("M,K,N,bits", [(257, 256, 20480, 4), (257, 2816, 16448, 4), (640, 12288, 1088, 4), (257, 2816, 32832, 8),
+                                        (640, 12288, 1088, 8)])
+def test_epilogues_are_the_separate_operations(M, K, N, bits):
     """Gate and residual, and SwiGLU, on the linear layer's own values; GELU rounds once where torch's does."""
     import mflux_amd
-    from mflux_amd import core
+    from gpu_util import kernel_of
+    from mflux_amd import _lib, core
 
-    x, packed, bias, _ = _operands(M, K, N, 4, 64, torch.bfloat16)
-    lin = mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=4, bias=bias)
+    assert kernel_of(M, K, N, bits, 64)[0] == _lib.KERNEL_WIDE
+    x, packed, bias, _ = _operands(M, K, N, bits, 64, torch.bfloat16)
+    lin = mflux_amd.quantized_matmul(x, *packed, group_size=64, bits=bits, bias=bias)
     gate, res = torch.randn(N, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
-    y = core.quantized_matmul_epilogue(x, *packed, epilogue="gate_residual", group_size=64, bits=4, bias=bias, gate=gate, residual=res)
+    y = core.quantized_matmul_epilogue(x, *packed, epilogue="gate_residual", group_size=64, bits=bits, bias=bias, gate=gate, residual=res)
     assert torch.equal(y, res + gate * lin)
-    y = core.quantized_matmul_epilogue(x, *packed, epilogue="gelu", group_size=64, bits=4, bias=bias, act_from=N // 2)
+    y = core.quantized_matmul_epilogue(x, *packed, epilogue="gelu", group_size=64, bits=bits, bias=bias, act_from=N // 2)
     assert torch.equal(y[:, : N // 2], lin[:, : N // 2])
     want = torch.nn.functional.gelu(lin[:, N // 2:].double(), approximate="tanh")
     assert bool(((y[:, N // 2:].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-6).all())
-    y = core.quantized_matmul_epilogue(x, *packed, epilogue="swiglu", group_size=64, bits=4, bias=bias)
+    y = core.quantized_matmul_epilogue(x, *packed, epilogue="swiglu", group_size=64, bits=bits, bias=bias)
     want = core.swiglu_unstack(lin).double()
     assert bool(((y.double() - want).abs() <= 2.0 ** -6 * want.abs() + 1e-6).all())  # the sigmoid's last place, twice rounded
