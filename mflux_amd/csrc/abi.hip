@@ -194,7 +194,7 @@ int mfq_qmm_t_low_rank(const void* x, int x_dtype, int64_t M, int64_t K, const u
   if (!mfq::aligned16(x) || !mfq::aligned16(wq)) return MFQ_EALIGN;
   if (M > 16 && !mfq::aligned16(y)) return MFQ_EALIGN;  // the GEMM writes y in 16-byte pieces
   if (odd_bits) {
-    // 3, 5, 6 bits: the one-row kernel for the rows it takes, the 128-column-tile GEMM for everything else
+    // 3, 5, 6 bits: the one-row kernel for the rows it takes, the sliced or the 128-column-tile GEMM for everything else
     if (M == 1) {
       const int rc = mfq::launch_qmv_odd(x, x_dtype, M, K, wq, scales, biases, bias, N, group_size, bits, y, y_dtype,
                                          (hipStream_t)stream);

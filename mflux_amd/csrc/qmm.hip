@@ -1138,8 +1138,8 @@ static float tiles_estimate_us(int64_t tiles, int64_t K) {
 // 18944 -> 3584 196 us, 132 on the other kernel).  Below 1024 rows a shape with
 // more tiles goes there too where its rows fill 128-row tiles and rounds of
 // workgroups much better: 320 rows x 3584 -> 37888 150 us on 296 tiles of 256 x 256
-// (one round and 40 tiles cut in two), 129 on 888 of 128 x 128; 600 rows x 3072 ->
-// 12288 70 against 62.
+// (one round and 40 tiles cut in two), 126 on 888 of 128 x 128; 600 rows x 3072 ->
+// 12288 70 against 59.  (At 4 and 8 bits 128 x 256 tiles may take both: launch_qmm().)
 // Both rules take groups of 64 for all.  Groups of 32 can be cut more often (18944 -> 3584, four ranges instead of two),
 // which this kernel gains by and the rule does not see: there 513 .. 768 rows are 8 to 10 % faster on the other kernel,
 // 900 rows 155 us against 144.

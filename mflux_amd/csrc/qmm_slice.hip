@@ -17,8 +17,9 @@
 //     type, every code once per workgroup), requests and LDS reads are dealt out between the matrix instructions by
 //     hand, and the steady state has no branch but one for a chunk's and one for a window's end (with a branch around
 //     every request 16.0 us on the shape below instead of 13.8).
-// Measured, 4 bits in groups of 64, stream of launches, cold weights: 256 rows x 3072 -> 3072 21.9 us on the other kernel
-// (two launches), 13.5 here; 512 rows 24.0 -> 20.0; 64 rows 14.7 -> 10.0.  What bounds it: a sub-step of 64 k on the four
+// Measured, 4 bits in groups of 64, stream of launches, a gigabyte of weights in turn: 256 rows x 3072 -> 3072 22.6 us on the
+// other kernel (two launches), 15.3 here; 512 rows 26.4 -> 22.7; 64 rows 16.2 -> 10.6.  (The figures of attempts, above and
+// below, are of fewer weights in turn, where this kernel took 13.5 to 13.8.)  What bounds it: a sub-step of 64 k on the four
 // wavefronts takes 0.67 us (64 x 48), of which the matrix instructions with the dequantisation between them are 0.34 and
 // 39 KB of direct loads 0.35 to 0.4, which a lone wavefront overlaps in part; 5 us are launch, first bytes and the sum.
 // Tried on this tile and not faster: eight wavefronts with a barrier per step and shared staging (13.9 us; slower from

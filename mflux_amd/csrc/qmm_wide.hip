@@ -13,8 +13,8 @@
 //     sub-step s multiplies its codes 8 s .., and the lane's x fragment is taken from the same k;
 //   - eight codes of each column are dequantised (one float32 fma each, one rounding) while the eight before them are
 //     multiplied; x fragments are read three ahead, over the barrier that ends a step.
-// With 240 (4 bits) to 252 registers two wavefronts fit a SIMD.  320 rows x 3584 -> 37888 at 4 bits: 110 us, 0.79 PFLOP/s
-// (143 on 888 tiles of 128 x 128, 129 with those 160 rows high); with x all zeros, which costs less power, 95.  Weight loads
+// With 240 (4 bits) to 252 registers two wavefronts fit a SIMD.  320 rows x 3584 -> 37888 at 4 bits: 105 to 110 us, 0.79 to 0.83
+// PFLOP/s (126 on 888 tiles of 128 x 128); with x all zeros, which costs less power, 95.  Weight loads
 // in whole cache lines (their share of every line is 32 bytes now) would give some 8 % more, but their way through LDS has no
 // registers left (half lines through a private region: 115); 96-row tiles took 135 us, 64-row tiles, which dequantise twice as
 // often, 120.
