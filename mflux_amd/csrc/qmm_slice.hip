@@ -43,10 +43,12 @@ struct Shape {
   static constexpr int TM = 16 * kA, TN = 16 * kB;
   static constexpr int kXSlot = TM * 128;                      // 64 k of the tile's rows of x
   static constexpr int kXLoads = TM / 8;                       // load instructions of a slot
+  static constexpr int kXGroup = 4;                            // that share a write of m0
   static constexpr int kInstr = 2 * kA * kB;                   // matrix instructions of a sub-step
   static constexpr int kReadsAt = kInstr / 3;                  // the next sub-step's fragments are read behind these
-  // load l of a slot is requested behind matrix instruction load_slot(l); those requested when the reads begin
-  static constexpr int load_slot(int l) { return l * kInstr / kXLoads; }
+  // load l of a slot is requested behind matrix instruction load_slot(l), kXGroup of them together; those requested when the
+  // reads begin
+  static constexpr int load_slot(int l) { return l / kXGroup * kXGroup * kInstr / kXLoads; }
   static constexpr int loads_before_reads() {
     int n = 0;
     for (int l = 0; l < kXLoads; ++l) n += load_slot(l) <= kReadsAt;
@@ -137,17 +139,24 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
     asm volatile("s_add_i32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  ::"v"(voff), "s"(sbase), "s"(lds_addr), "i"(offset) : "memory", "m0", "scc");
   };
+  // Four of them to consecutive KiB of LDS: the instruction's offset counts on both sides, in LDS and in memory.
+  auto dma16x4 = [&](const char* sbase, const uint32_t* voff, uint32_t lds_addr, int offset) __attribute__((always_inline)) {
+    asm volatile("s_add_i32 m0, %5, %6\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %4\n\tglobal_load_lds_dwordx4 %1, %4 offset:1024"
+                 "\n\tglobal_load_lds_dwordx4 %2, %4 offset:2048\n\tglobal_load_lds_dwordx4 %3, %4 offset:3072"
+                 ::"v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(sbase), "s"(lds_addr), "i"(offset) : "memory", "m0", "scc");
+  };
   auto dma4 = [&](const char* sbase, uint32_t voff, uint32_t lds_addr, int offset) __attribute__((always_inline)) {
     asm volatile("s_add_i32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                  ::"v"(voff), "s"(sbase), "s"(lds_addr), "i"(offset) : "memory", "m0", "scc");
   };
 
   // ---- what the lane loads
-  uint32_t xoff[S::kXLoads];  // eight rows, 128 bytes each
+  uint32_t xoff[S::kXLoads];  // eight rows, 128 bytes each; what the instruction's offset adds is taken off here
 #pragma unroll
   for (int i = 0; i < S::kXLoads; ++i) {
     const int row = 8 * i + (lane >> 3);
-    xoff[i] = ((uint32_t)min(m0 + row, M - 1) * (uint32_t)K + 8u * (uint32_t)((lane & 7) ^ swz_mask(row))) * 2u;
+    xoff[i] = ((uint32_t)min(m0 + row, M - 1) * (uint32_t)K + 8u * (uint32_t)((lane & 7) ^ swz_mask(row))) * 2u +
+              1024u * (uint32_t)(S::kXGroup - 1 - i % S::kXGroup);
   }
   // codes: piece p of a chunk is piece p % kRowPieces of row p / kRowPieces
   uint32_t wrow[S::kWLoads], wcol[S::kWLoads];
@@ -166,11 +175,11 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
   const int first_dword = (begin * 64 >> gs_shift) >> 1;  // of the first window; a window begins at an even group
   const int g_first = (begin * 64 >> gs_shift) & ~1, g_last = ((begin + n) * 64 - 1) >> gs_shift;
 
-  const char* xbytes = reinterpret_cast<const char*>(x) + (size_t)begin * 128;
+  const char* xbytes = reinterpret_cast<const char*>(x) + (ptrdiff_t)begin * 128 - 1024 * (S::kXGroup - 1);
   const char* wbytes = reinterpret_cast<const char*>(wq);
   const uint32_t w_begin = (uint32_t)begin * 8u * BITS, w_end = (uint32_t)(K * BITS / 8 - 16);
-  auto load_x = [&](int j, int slot, int i) __attribute__((always_inline)) {
-    dma16(xbytes + (size_t)j * 128, xoff[i], ring_addr + slot * S::kXSlot, 1024 * i);
+  auto load_x = [&](int j, int slot, int i) __attribute__((always_inline)) {  // loads i to i + kXGroup - 1
+    dma16x4(xbytes + (size_t)j * 128, xoff + i, ring_addr + slot * S::kXSlot, 1024 * i);
   };
   auto load_w = [&](int c) __attribute__((always_inline)) {  // chunk c; pieces past the row's end repeat its last one
 #pragma unroll
@@ -317,7 +326,7 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
         acc[a][i % kB] = mfma16(__builtin_bit_cast(vec8, cur), f.x[a][i / kB], acc[a][i % kB]);
         if (more_x) {
 #pragma unroll
-          for (int l = 0; l < S::kXLoads; ++l)
+          for (int l = 0; l < S::kXLoads; l += S::kXGroup)
             if (S::load_slot(l) == at) load_x(j + S::kXSlots, slot, l);
         }
         if (more) {
@@ -349,7 +358,7 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
     for (int j = 0; j < S::kXSlots; ++j)
       if (j < n) {
 #pragma unroll
-        for (int i = 0; i < S::kXLoads; ++i) load_x(j, j, i);
+        for (int i = 0; i < S::kXLoads; i += S::kXGroup) load_x(j, j, i);
         if (j == 0) {
           if (n > S::kChunk) load_w(1);
           if (8 + g_first <= g_last) load_s(1);
@@ -550,7 +559,7 @@ inline float others_us(int64_t M, int64_t N, int64_t K, int gs, int bits) {
 // 3 % behind, 123 by more than 6 (6 bits 33 x 768 -> 37888 19.8 -> 27.3 us, 76 x 3072 -> 12288 28.8 -> 33.0).
 inline SlicePlan choose_slice(int64_t M, int64_t N, int64_t K, int gs, int bits, bool may_cut) {
   const int64_t gran = bits == 3 || bits == 5 ? 128 : 64;
-  if (M > 1024 || N % 8 || K % gran || (K / gs) % 2 || M * K >= (int64_t)1 << 31 || N * K >= (int64_t)1 << 31) return SlicePlan();
+  if (M > 1024 || N % 8 || K % gran || (K / gs) % 2 || M * K >= ((int64_t)1 << 31) - 2048 || N * K >= (int64_t)1 << 31) return SlicePlan();
   const SlicePlan plan = plan_slice(M, N, K, bits, may_cut);
   return plan.us < 0.9f * others_us(M, N, K, gs, bits) ? plan : SlicePlan();
 }
