@@ -13,8 +13,9 @@
 //     sub-step s multiplies its codes 8 s .., and the lane's x fragment is taken from the same k;
 //   - eight codes of each column are dequantised (one float32 fma each, one rounding) while the eight before them are
 //     multiplied; x fragments are read three ahead, over the barrier that ends a step.
-// With 240 (4 bits) to 252 registers two wavefronts fit a SIMD.  320 rows x 3584 -> 37888 at 4 bits: 105 to 110 us, 0.79 to 0.83
-// PFLOP/s (126 on 888 tiles of 128 x 128); with x all zeros, which costs less power, 95.  Weight loads
+// With 240 (4 bits) to 252 registers two wavefronts fit a SIMD.  384 rows x 3584 -> 37888 at 4 bits: 105 to 110 us, 0.95 to
+// 0.99 PFLOP/s, 320 rows, whose last tile leaves half of its matrix work out, 104 (126 on 888 tiles of 128 x 128); before it did,
+// 109, and with x all zeros, which costs less power, 95.  Weight loads
 // in whole cache lines (their share of every line is 32 bytes now) would give some 8 % more, but their way through LDS has no
 // registers left (half lines through a private region: 115); 96-row tiles took 135 us, 64-row tiles, which dequantise twice as
 // often, 120.
@@ -37,7 +38,8 @@ constexpr int kLds = 2 * kBuf > kStage ? 2 * kBuf : kStage;
 __device__ inline int swz(int row, int chunk) { return row * (TK * 2) + ((chunk ^ ((row >> 1) & 7)) << 4); }
 
 // K % 256 == 0: the loop runs over quads of four steps, whose scales of a column are one piece of 512 / GS bytes.
-template <typename T, int GS, int BITS>
+// kShort: the last tile of every column has at most 64 rows, and its workgroups run a loop of their own over those.
+template <typename T, int GS, int BITS, bool kShort>
 __global__ __launch_bounds__(kThreads, 2) void qmm_wide_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
     const uint16_t* __restrict__ biases, const uint16_t* __restrict__ bias, void* __restrict__ y, int y_is_f32, int M,
@@ -45,8 +47,7 @@ __global__ __launch_bounds__(kThreads, 2) void qmm_wide_kernel(
     const uint16_t* __restrict__ lr_bs, int lr_rank, Epilogue epi) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   using vec8 = typename T::vec8;
-  constexpr int kFrags = 4 * kI, kRing = 4, kAhead = kRing - 1;  // x fragments of a step, in flight
-  constexpr int kGate = kFrags - kAhead;                         // in front of this one's instructions the next step's x opens
+  constexpr int kRing = 4, kAhead = kRing - 1;                   // x fragments in flight
   constexpr int kWords = BITS;                                   // of a lane's 32 codes of a step and column
   constexpr int kSWords = 128 / GS;                              // 32-bit words of a column's scales of a quad
   static_assert(BITS == 4 || BITS == 8, "");
@@ -161,26 +162,29 @@ __global__ __launch_bounds__(kThreads, 2) void qmm_wide_kernel(
       return T::pack2(__builtin_fmaf(ubyte_f32(v, 2 * (p & 1)), sv, bv), __builtin_fmaf(ubyte_f32(v, 2 * (p & 1) + 1), sv, bv));
     }
   };
-  auto read_x = [&](int buf, int f) __attribute__((always_inline)) {
-    return *reinterpret_cast<const vec8*>(lds + buf * kBuf + f % kI * 4096 + rd[f / kI]);
+  auto read_x = [&](auto rows_c, int buf, int f) __attribute__((always_inline)) {
+    constexpr int kR = decltype(rows_c)::value;
+    return *reinterpret_cast<const vec8*>(lds + buf * kBuf + f % kR * 4096 + rd[f / kR]);
   };
 
-  // step e of a quad, p of the item
-  auto step = [&](auto e_c, int p) __attribute__((always_inline)) {
-    constexpr int e = decltype(e_c)::value, buf = e & 1;
+  // step e of a quad, p of the item, on the tile's first kR blocks of 32 rows
+  auto step = [&](auto rows_c, auto e_c, int p) __attribute__((always_inline)) {
+    constexpr int kR = decltype(rows_c)::value, e = decltype(e_c)::value, buf = e & 1;
+    constexpr int kFrags = 4 * kR;         // x fragments of a step
+    constexpr int kGate = kFrags - kAhead;  // in front of this one's instructions the next step's x opens
     constexpr std::integral_constant<int, (e + 1) & 3> e_next{};
 #pragma unroll
     for (int f = 0; f < kFrags; ++f) {
-      const int s = f / kI, i = f % kI;
+      const int s = f / kR, i = f % kR;
       if (f == kGate) __syncthreads();  // all of step p's x has been read, step p + 1's is there
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[i][j] = mfma32(__builtin_bit_cast(vec8, wf[s & 1][j]), xf[f % kRing], acc[i][j]);
-      xf[(f + kAhead) % kRing] = f + kAhead < kFrags ? read_x(buf, f + kAhead) : read_x(buf ^ 1, f + kAhead - kFrags);
-      if (f % 2 == 0 && f / 2 < kI) {
+      xf[(f + kAhead) % kRing] = f + kAhead < kFrags ? read_x(rows_c, buf, f + kAhead) : read_x(rows_c, buf ^ 1, f + kAhead - kFrags);
+      if (f % 2 == 0 && f / 2 < kR) {
         *reinterpret_cast<u32x4*>(lds + (buf ^ 1) * kBuf + wr_x + 4096 * (f / 2)) = xr[f / 2];
         load_x(p + 2, f / 2);
       }
-      if (f == 2 * kI) {
+      if (f == 2 * kR) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           if constexpr (e == 3) scale_of(nxt, e_next, j);
@@ -189,12 +193,12 @@ __global__ __launch_bounds__(kThreads, 2) void qmm_wide_kernel(
         if constexpr (e == 3) cur = nxt;
       }
 #pragma unroll
-      for (int q = 8 * i / kI; q < 8 * (i + 1) / kI; ++q) {
+      for (int q = 8 * i / kR; q < 8 * (i + 1) / kR; ++q) {
         const int j = q >> 2;
         wf[(s + 1) & 1][j][q & 3] = s < 3 ? pair(w[buf][j], s + 1, q & 3, sc[buf][j], bi[buf][j])
                                           : pair(w[buf ^ 1][j], 0, q & 3, sc[buf ^ 1][j], bi[buf ^ 1][j]);
       }
-      if (f == 3 * kI) {
+      if (f == 3 * kR) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) load_w(buf, p + 2, j);
         if constexpr (e == 0) {
@@ -206,35 +210,43 @@ __global__ __launch_bounds__(kThreads, 2) void qmm_wide_kernel(
     }
   };
 
+  auto run = [&](auto rows_c) __attribute__((always_inline)) {
+    constexpr int kR = decltype(rows_c)::value;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    load_s(cur, 0, j);
-    load_w(0, 0, j);
-  }
+    for (int j = 0; j < 2; ++j) {
+      load_s(cur, 0, j);
+      load_w(0, 0, j);
+    }
 #pragma unroll
-  for (int i = 0; i < kI; ++i) load_x(0, i);
+    for (int i = 0; i < kR; ++i) load_x(0, i);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) load_w(1, 1, j);
+    for (int j = 0; j < 2; ++j) load_w(1, 1, j);
 #pragma unroll
-  for (int i = 0; i < kI; ++i) {
-    *reinterpret_cast<u32x4*>(lds + wr_x + 4096 * i) = xr[i];
-    load_x(1, i);
-  }
+    for (int i = 0; i < kR; ++i) {
+      *reinterpret_cast<u32x4*>(lds + wr_x + 4096 * i) = xr[i];
+      load_x(1, i);
+    }
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    scale_of(cur, std::integral_constant<int, 0>{}, j);
+    for (int j = 0; j < 2; ++j) {
+      scale_of(cur, std::integral_constant<int, 0>{}, j);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) wf[0][j][q] = pair(w[0][j], 0, q, sc[0][j], bi[0][j]);
-  }
-  __syncthreads();
+      for (int q = 0; q < 4; ++q) wf[0][j][q] = pair(w[0][j], 0, q, sc[0][j], bi[0][j]);
+    }
+    __syncthreads();
 #pragma unroll
-  for (int f = 0; f < kAhead; ++f) xf[f] = read_x(0, f);
-  for (int p = 0; p < steps; p += 4) {
-    step(std::integral_constant<int, 0>{}, p);
-    step(std::integral_constant<int, 1>{}, p + 1);
-    step(std::integral_constant<int, 2>{}, p + 2);
-    step(std::integral_constant<int, 3>{}, p + 3);
-  }
+    for (int f = 0; f < kAhead; ++f) xf[f] = read_x(rows_c, 0, f);
+    for (int p = 0; p < steps; p += 4) {
+      step(rows_c, std::integral_constant<int, 0>{}, p);
+      step(rows_c, std::integral_constant<int, 1>{}, p + 1);
+      step(rows_c, std::integral_constant<int, 2>{}, p + 2);
+      step(rows_c, std::integral_constant<int, 3>{}, p + 3);
+    }
+  };
+  // A tile of at most 64 rows leaves the matrix work of the other half out (its weights are dequantised all the same): 320
+  // rows x 3584 -> 37888 113 -> 107 us, x 18944 -> 3584 67.6 -> 64.8.  A kernel of its own, because both loops in one cost
+  // the whole tiles' up to 1 % (registers; at 8 bits some are spilled in it).
+  if (kShort && M - m0 <= TM / 2) run(std::integral_constant<int, kI / 2>{});
+  else run(std::integral_constant<int, kI>{});
 
   // low-rank update: lr_rank more k, 16-bit and unquantised, straight from memory; of a tile's k ranges the first adds it
   if (split == 0) {
@@ -260,6 +272,9 @@ __global__ __launch_bounds__(kThreads, 2) void qmm_wide_kernel(
     store_block_64x64<T>(half, lds, wave, lane, m0 + 32 * i, n0 + 64 * wave, M, N, bias, y_item, y_is_f32, epi);
   }
 }
+
+// whether the last row of tiles has at most half of its rows
+inline bool short_tiles(int64_t M) { return (M - 1) % TM < TM / 2; }
 
 struct WidePlan {
   int splits;  // 0: not this kernel
@@ -307,16 +322,24 @@ inline WidePlan choose_wide(int64_t M, int64_t N, int64_t K, int gs, int bits, b
   return plan.us < share * qmm_others_estimate_us(M, N, K, gs, bits) ? plan : none;
 }
 
-template <typename T, int GS, int BITS>
-int launch_kernel(const WidePlan& plan, const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
+template <typename T, int GS, int BITS, bool kShort>
+int launch_tiles(const WidePlan& plan, const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                   const void* biases, const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream, LowRank lr,
                   Epilogue epi) {
   const int tiles_m = (int)((M + TM - 1) / TM), tiles_n = (int)((N + TN - 1) / TN);
-  hipLaunchKernelGGL((qmm_wide_kernel<T, GS, BITS>), dim3((unsigned)(tiles_m * tiles_n * plan.splits)), dim3(kThreads), kLds,
+  hipLaunchKernelGGL((qmm_wide_kernel<T, GS, BITS, kShort>), dim3((unsigned)(tiles_m * tiles_n * plan.splits)), dim3(kThreads), kLds,
                      stream, (const uint16_t*)x, wq, (const uint16_t*)scales, (const uint16_t*)biases, (const uint16_t*)bias, y,
                      (int)(y_dtype == MFQ_F32), (int)M, (int)N, (int)K, tiles_m, tiles_n, plan.quads, plan.n_long,
                      (const uint16_t*)lr.t, (const uint16_t*)lr.bs, lr.R, epi);
   return hipGetLastError() == hipSuccess ? MFQ_OK : MFQ_ELAUNCH;
+}
+
+template <typename T, int GS, int BITS>
+int launch_kernel(const WidePlan& plan, const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
+                  const void* biases, const void* bias, int64_t N, void* y, int y_dtype, hipStream_t stream, LowRank lr,
+                  Epilogue epi) {
+  const auto go = [&](auto launch) { return launch(plan, x, M, K, wq, scales, biases, bias, N, y, y_dtype, stream, lr, epi); };
+  return short_tiles(M) ? go(launch_tiles<T, GS, BITS, true>) : go(launch_tiles<T, GS, BITS, false>);
 }
 
 template <typename T>

@@ -106,3 +106,21 @@ def test_epilogues_are_the_separate_operations(M, K, N, bits):
     y = core.quantized_matmul_epilogue(x, *packed, epilogue="swiglu", group_size=64, bits=bits, bias=bias)
     want = core.swiglu_unstack(lin).double()
     assert bool(((y.double() - want).abs() <= 2.0 ** -6 * want.abs() + 1e-6).all())  # the sigmoid's last place, twice rounded
+
+
+# the last tile of a column with 44, 64 (half, the loop of its own) and 65 rows (the whole tile's loop); K whole and cut
+@pytest.mark.parametrize("M", [300, 320, 321])
+@pytest.mark.parametrize("K,N,bits,gs,dtype", [(2816, 16448, 4, 64, "bf16"), (2816, 16448, 4, 32, "f16"), (18944, 3592, 4, 128, "bf16"),
+                                               (2816, 32832, 8, 64, "bf16")])
+def test_a_last_tile_of_half_its_rows(M, K, N, bits, gs, dtype):
+    import mflux_amd
+    from gpu_util import kernel_of
+    from mflux_amd import _lib
+
+    assert kernel_of(M, K, N, bits, gs)[0] == _lib.KERNEL_WIDE
+    x, packed, bias, ref = _operands(M, K, N, bits, gs, DT[dtype])
+    y = mflux_amd.quantized_matmul(x, *packed, group_size=gs, bits=bits, bias=bias)
+    _close(y, ref + bias.double(), DT[dtype], 2)
+    rows = mflux_amd.quantized_matmul(x[:256], *packed, group_size=gs, bits=bits, bias=bias)  # (whole tiles only)
+    if kernel_of(M, K, N, bits, gs) == kernel_of(256, K, N, bits, gs):
+        assert torch.equal(y[:256], rows)
