@@ -460,6 +460,30 @@ int mfq_low_rank_down(const void* x, const void* af, int dtype, int64_t M, int64
 int mfq_low_rank_add(const void* t, const void* bs, int dtype, int64_t M, int64_t N, int64_t rank,
                      void* y, int y_dtype, void* stream);
 
+/*
+ * Training one adapter on a quantized base (src/mflux/models/common/training/lora/target_injector.py:30-33,
+ * linear_lora_layer.py:50-53): what mx.value_and_grad computes beside the two large products.  All arrays
+ * are of the 16-bit type dtype, the sums float32, rounded once; R, the rank the kernels work on, is 16 or
+ * 32 and not below `rank`; K and N are multiples of 32, every pointer but lora_a and lora_b 16-byte aligned.
+ *   mfq_low_rank_pack      lora_a [K, rank], lora_b [rank, N] (any address) ->
+ *                          af [R/16][K/32][4][16][8] as in mfq_low_rank_down, bf [R/16][N/32][4][16][8] the
+ *                          same of lora_b^T, bs [N, R] = scale * lora_b^T and ap [K, R] = lora_a (NULL: not
+ *                          wanted), zeros behind the rank
+ *   mfq_low_rank_forward   t [M, R] = x [M, K] @ lora_a, zeros behind the rank, and tf [R/16][ceil(M/32)][4][16][8]:
+ *                          tf[f][s][q][c][e] = t[32 s + 8 q + e][16 f + c], zeros behind row M
+ *   mfq_low_rank_gradient  gt [M, R] = scale * g [M, N] @ lora_b^T and its gtf (both NULL: not wanted);
+ *                          db [rank, N] = scale * t^T @ g (NULL: not wanted)
+ *   mfq_low_rank_up        out [K, rank] = x [M, K]^T @ t, e.g. the gradient of lora_a with gtf for tf
+ */
+int mfq_low_rank_pack(const void* lora_a, const void* lora_b, int dtype, int64_t K, int64_t N, int64_t rank,
+                      int64_t R, float scale, void* af, void* bf, void* bs, void* ap, void* stream);
+int mfq_low_rank_forward(const void* x, const void* af, int dtype, int64_t M, int64_t K, int64_t rank,
+                         int64_t R, void* t, void* tf, void* stream);
+int mfq_low_rank_gradient(const void* g, const void* bf, const void* tf, int dtype, int64_t M, int64_t N,
+                          int64_t rank, int64_t R, float scale, void* gt, void* gtf, void* db, void* stream);
+int mfq_low_rank_up(const void* x, const void* tf, int dtype, int64_t M, int64_t K, int64_t rank, int64_t R,
+                    void* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

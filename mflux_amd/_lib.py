@@ -50,6 +50,10 @@ SIGNATURES = {
     "mfq_layer_norm_modulate": (_INT, [_PTR, _INT, _I64, _I64, _PTR, _PTR, _I64, ctypes.c_float, _PTR, _PTR]),
     "mfq_silu": (_INT, [_PTR, _INT, _I64, _PTR, _PTR]),
     "mfq_low_rank_down": (_INT, [_PTR, _PTR, _INT, _I64, _I64, _I64, _PTR, _PTR]),
+    "mfq_low_rank_pack": (_INT, [_PTR, _PTR, _INT, _I64, _I64, _I64, _I64, ctypes.c_float, _PTR, _PTR, _PTR, _PTR, _PTR]),
+    "mfq_low_rank_forward": (_INT, [_PTR, _PTR, _INT, _I64, _I64, _I64, _I64, _PTR, _PTR, _PTR]),
+    "mfq_low_rank_gradient": (_INT, [_PTR, _PTR, _PTR, _INT, _I64, _I64, _I64, _I64, ctypes.c_float, _PTR, _PTR, _PTR, _PTR]),
+    "mfq_low_rank_up": (_INT, [_PTR, _PTR, _INT, _I64, _I64, _I64, _I64, _PTR, _PTR]),
     "mfq_low_rank_add": (_INT, [_PTR, _PTR, _INT, _I64, _I64, _I64, _PTR, _INT, _PTR]),
 }
 

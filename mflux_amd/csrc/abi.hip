@@ -361,6 +361,48 @@ int mfq_low_rank_down(const void* x, const void* at, int dtype, int64_t M, int64
   return mfq::launch_low_rank_down(x, dtype, M, K, at, rank, t, (hipStream_t)stream);
 }
 
+static int check_training(int dtype, int64_t rows, int64_t columns, int64_t rank, int64_t R) {
+  if (!is16(dtype)) return MFQ_EDTYPE;
+  if (rank <= 0 || rank > R || (R != 16 && R != 32)) return MFQ_ESHAPE;
+  if (rows <= 0 || columns <= 0 || columns % 32 || rows > INT32_MAX - 64 || columns > (1 << 24)) return MFQ_ESHAPE;
+  return rows * columns < (int64_t)1 << 40 ? MFQ_OK : MFQ_ESHAPE;
+}
+
+int mfq_low_rank_pack(const void* lora_a, const void* lora_b, int dtype, int64_t K, int64_t N, int64_t rank, int64_t R,
+                      float scale, void* af, void* bf, void* bs, void* ap, void* stream) {
+  if (int rc = check_training(dtype, 1, K, rank, R)) return rc;
+  if (int rc = check_training(dtype, 1, N, rank, R)) return rc;
+  if (!lora_a || !lora_b || !af || !bf || !bs) return MFQ_ENULL;
+  if (!mfq::aligned16(af) || !mfq::aligned16(bf) || !mfq::aligned16(bs) || !mfq::aligned16(ap)) return MFQ_EALIGN;
+  return mfq::launch_low_rank_pack(lora_a, lora_b, dtype, K, N, (int)rank, (int)R, scale, af, bf, bs, ap, (hipStream_t)stream);
+}
+
+int mfq_low_rank_forward(const void* x, const void* af, int dtype, int64_t M, int64_t K, int64_t rank, int64_t R, void* t,
+                         void* tf, void* stream) {
+  if (int rc = check_training(dtype, M, K, rank, R)) return rc;
+  if (!x || !af || !t || !tf) return MFQ_ENULL;
+  if (!mfq::aligned16(x) || !mfq::aligned16(af) || !mfq::aligned16(t) || !mfq::aligned16(tf)) return MFQ_EALIGN;
+  return mfq::launch_low_rank_forward(x, dtype, M, K, af, (int)rank, (int)R, t, tf, (hipStream_t)stream);
+}
+
+int mfq_low_rank_gradient(const void* g, const void* bf, const void* tf, int dtype, int64_t M, int64_t N, int64_t rank,
+                          int64_t R, float scale, void* gt, void* gtf, void* db, void* stream) {
+  if (int rc = check_training(dtype, M, N, rank, R)) return rc;
+  if (!g || (gt == nullptr) != (gtf == nullptr) || (gt && !bf) || (db && !tf) || (!gt && !db)) return MFQ_ENULL;
+  if (!mfq::aligned16(g) || !mfq::aligned16(bf) || !mfq::aligned16(tf) || !mfq::aligned16(gt) || !mfq::aligned16(gtf) ||
+      !mfq::aligned16(db))
+    return MFQ_EALIGN;
+  return mfq::launch_low_rank_gradient(g, dtype, M, N, bf, tf, (int)rank, (int)R, scale, gt, gtf, db, (hipStream_t)stream);
+}
+
+int mfq_low_rank_up(const void* x, const void* tf, int dtype, int64_t M, int64_t K, int64_t rank, int64_t R, void* out,
+                    void* stream) {
+  if (int rc = check_training(dtype, M, K, rank, R)) return rc;
+  if (!x || !tf || !out) return MFQ_ENULL;
+  if (!mfq::aligned16(x) || !mfq::aligned16(tf) || !mfq::aligned16(out)) return MFQ_EALIGN;
+  return mfq::launch_low_rank_up(x, dtype, M, K, tf, (int)rank, (int)R, out, (hipStream_t)stream);
+}
+
 int mfq_low_rank_add(const void* t, const void* bs, int dtype, int64_t M, int64_t N, int64_t rank, void* y, int y_dtype,
                      void* stream) {
   if (!is16(dtype)) return MFQ_EDTYPE;

@@ -408,6 +408,15 @@ int launch_qmm_epilogue(const void* x, int dtype, int64_t M, int64_t K, const ui
                         void* workspace, size_t workspace_bytes, hipStream_t stream, Epilogue epi);
 // y[M, N] += t @ bs^T, rounded to y's type (dtype: the type of t, bs and a 16-bit y)
 int launch_low_rank_add(int dtype, LowRank low_rank, int64_t M, int64_t N, void* y, int y_dtype, hipStream_t stream);
+// the products of a trainable adapter with its activations and gradients: see include/mfq.h
+int launch_low_rank_pack(const void* a, const void* b, int dtype, int64_t K, int64_t N, int rank, int R, float scale, void* af,
+                         void* bf, void* bs, void* ap, hipStream_t stream);
+int launch_low_rank_forward(const void* x, int dtype, int64_t M, int64_t K, const void* af, int rank, int R, void* t,
+                            void* tf, hipStream_t stream);
+int launch_low_rank_gradient(const void* g, int dtype, int64_t M, int64_t N, const void* bf, const void* tf, int rank, int R,
+                             float scale, void* gt, void* gtf, void* db, hipStream_t stream);
+int launch_low_rank_up(const void* x, int dtype, int64_t M, int64_t K, const void* tf, int rank, int R, void* out,
+                       hipStream_t stream);
 // y[i] = silu(x[i]), the sigmoid and the product each rounded to the 16-bit type
 int launch_silu(const void* x, int dtype, int64_t n, void* y, hipStream_t stream);
 // t[M, R] = x[M, K] @ A[K, R], A in fragment order ([R/16][K/32][4][16][8]); 16-bit type `dtype`; R % 16 == 0, K % 32 == 0

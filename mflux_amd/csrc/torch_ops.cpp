@@ -285,6 +285,92 @@ Tensor low_rank_down(const Tensor& x, const Tensor& af) {
   return t;
 }
 
+// ---- a trainable adapter's products (include/mfq.h, mfq_low_rank_pack and what follows it)
+int64_t training_rank(int64_t rank) { return rank <= 16 ? 16 : 32; }
+
+void check_factor(const char* fn, const Tensor& t, int64_t rows, int64_t columns, const Tensor& like) {
+  TORCH_CHECK(t.dim() == 2 && t.size(0) == rows && t.size(1) == columns && t.is_contiguous() &&
+                  t.scalar_type() == like.scalar_type() && t.device() == like.device(),
+              fn, ": expected a contiguous [", rows, ", ", columns, "] matrix of ", like.scalar_type(), " on ", like.device());
+}
+
+void check_fragments(const char* fn, const Tensor& t, int64_t steps, const Tensor& like) {
+  TORCH_CHECK(t.dim() == 5 && t.size(1) == steps && t.size(2) == 4 && t.size(3) == 16 && t.size(4) == 8 && t.is_contiguous() &&
+                  t.scalar_type() == like.scalar_type() && t.device() == like.device(),
+              fn, ": expected fragments [R/16, ", steps, ", 4, 16, 8] of ", like.scalar_type(), " on ", like.device());
+}
+
+// lora_A [K, rank], lora_B [rank, N] -> their fragments, scale lora_B^T [N, R] and lora_A [K, R]
+std::tuple<Tensor, Tensor, Tensor, Tensor> low_rank_pack(const Tensor& a, const Tensor& b, double scale) {
+  TORCH_CHECK(a.dim() == 2 && b.dim() == 2, "mfq::low_rank_pack: lora_A [K, rank], lora_B [rank, N]");
+  const int64_t K = a.size(0), rank = a.size(1), N = b.size(1), R = training_rank(rank);
+  check_factor("mfq::low_rank_pack", a, K, rank, a);
+  check_factor("mfq::low_rank_pack", b, rank, N, a);
+  const c10::hip::HIPGuardMasqueradingAsCUDA guard(a.device());
+  Tensor af = at::empty({R / 16, K / 32, 4, 16, 8}, a.options()), bf = at::empty({R / 16, N / 32, 4, 16, 8}, a.options());
+  Tensor bs = at::empty({N, R}, a.options());
+  const bool as_it_is = rank == R && reinterpret_cast<uintptr_t>(a.data_ptr()) % 16 == 0;
+  Tensor ap = as_it_is ? a.detach() : at::empty({K, R}, a.options());
+  check_status("mfq_low_rank_pack",
+               mfq_low_rank_pack(a.data_ptr(), b.data_ptr(), dtype_code(a.scalar_type(), "lora_A"), K, N, rank, R, (float)scale,
+                                 af.data_ptr(), bf.data_ptr(), bs.data_ptr(), as_it_is ? nullptr : ap.data_ptr(), stream_of(a)));
+  return {af, bf, bs, ap};
+}
+
+// t [M, R] = x @ lora_A and its fragments
+std::tuple<Tensor, Tensor> low_rank_forward(const Tensor& x, const Tensor& af, int64_t rank) {
+  TORCH_CHECK(x.dim() == 2, "mfq::low_rank_forward: x [M, K]");
+  const int64_t M = x.size(0), K = x.size(1);
+  check_factor("mfq::low_rank_forward", x, M, K, x);
+  check_fragments("mfq::low_rank_forward", af, K / 32, x);
+  const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  const int64_t R = 16 * af.size(0);
+  Tensor t = at::empty({M, R}, x.options()), tf = at::empty({R / 16, (M + 31) / 32, 4, 16, 8}, x.options());
+  check_status("mfq_low_rank_forward", mfq_low_rank_forward(x.data_ptr(), af.data_ptr(), dtype_code(x.scalar_type(), "x"), M, K,
+                                                            rank, R, t.data_ptr(), tf.data_ptr(), stream_of(x)));
+  return {t, tf};
+}
+
+// (gt [M, R], its fragments, the gradient of lora_B [rank, N]); what is not wanted comes back empty
+std::tuple<Tensor, Tensor, Tensor> low_rank_gradient(const Tensor& g, const Tensor& bf, const Tensor& tf, int64_t rank, double scale,
+                                                     bool want_gt, bool want_db) {
+  TORCH_CHECK(g.dim() == 2, "mfq::low_rank_gradient: g [M, N]");
+  const int64_t M = g.size(0), N = g.size(1);
+  check_factor("mfq::low_rank_gradient", g, M, N, g);
+  check_fragments("mfq::low_rank_gradient", bf, N / 32, g);
+  check_fragments("mfq::low_rank_gradient", tf, (M + 31) / 32, g);
+  TORCH_CHECK(tf.size(0) == bf.size(0), "mfq::low_rank_gradient: fragments of different ranks");
+  const c10::hip::HIPGuardMasqueradingAsCUDA guard(g.device());
+  const int64_t R = 16 * bf.size(0);
+  Tensor gt, gtf, db;
+  if (want_gt) {
+    gt = at::empty({M, R}, g.options());
+    gtf = at::empty({R / 16, (M + 31) / 32, 4, 16, 8}, g.options());
+  } else {
+    gt = gtf = at::empty({0}, g.options());
+  }
+  db = at::empty({want_db ? rank : 0, N}, g.options());
+  if (!want_gt && !want_db) return {gt, gtf, db};
+  check_status("mfq_low_rank_gradient",
+               mfq_low_rank_gradient(g.data_ptr(), bf.data_ptr(), tf.data_ptr(), dtype_code(g.scalar_type(), "g"), M, N, rank, R,
+                                     (float)scale, want_gt ? gt.data_ptr() : nullptr, want_gt ? gtf.data_ptr() : nullptr,
+                                     want_db ? db.data_ptr() : nullptr, stream_of(g)));
+  return {gt, gtf, db};
+}
+
+// x^T @ t [K, rank], t in fragments
+Tensor low_rank_up(const Tensor& x, const Tensor& tf, int64_t rank) {
+  TORCH_CHECK(x.dim() == 2, "mfq::low_rank_up: x [M, K]");
+  const int64_t M = x.size(0), K = x.size(1);
+  check_factor("mfq::low_rank_up", x, M, K, x);
+  check_fragments("mfq::low_rank_up", tf, (M + 31) / 32, x);
+  const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  Tensor out = at::empty({K, rank}, x.options());
+  check_status("mfq_low_rank_up", mfq_low_rank_up(x.data_ptr(), tf.data_ptr(), dtype_code(x.scalar_type(), "x"), M, K, rank,
+                                                  16 * tf.size(0), out.data_ptr(), stream_of(x)));
+  return out;
+}
+
 // y += t @ bs^T in place
 void low_rank_add_(Tensor& y, const Tensor& t, const Tensor& bs) {
   TORCH_CHECK(y.dim() == 2 && t.dim() == 2 && bs.dim() == 2 && y.is_contiguous() && t.is_contiguous() &&
@@ -310,6 +396,10 @@ TORCH_LIBRARY(mfq, m) {
   m.def("layer_norm_modulate(Tensor x, Tensor? scale, Tensor? shift, float eps) -> (Tensor, bool)");
   m.def("low_rank_add_(Tensor(a!) y, Tensor t, Tensor bs) -> ()");
   m.def("low_rank_down(Tensor x, Tensor af) -> Tensor");
+  m.def("low_rank_pack(Tensor lora_a, Tensor lora_b, float scale) -> (Tensor, Tensor, Tensor, Tensor)");
+  m.def("low_rank_forward(Tensor x, Tensor af, int rank) -> (Tensor, Tensor)");
+  m.def("low_rank_gradient(Tensor g, Tensor bf, Tensor tf, int rank, float scale, bool want_gt, bool want_db) -> (Tensor, Tensor, Tensor)");
+  m.def("low_rank_up(Tensor x, Tensor tf, int rank) -> Tensor");
 }
 
 TORCH_LIBRARY_IMPL(mfq, CUDA, m) {  // the HIP backend answers to torch's CUDA dispatch key
@@ -323,4 +413,8 @@ TORCH_LIBRARY_IMPL(mfq, CUDA, m) {  // the HIP backend answers to torch's CUDA d
   m.impl("layer_norm_modulate", layer_norm_modulate);
   m.impl("low_rank_add_", low_rank_add_);
   m.impl("low_rank_down", low_rank_down);
+  m.impl("low_rank_pack", low_rank_pack);
+  m.impl("low_rank_forward", low_rank_forward);
+  m.impl("low_rank_gradient", low_rank_gradient);
+  m.impl("low_rank_up", low_rank_up);
 }

@@ -124,20 +124,30 @@ class _LoRALinearFunction(torch.autograd.Function):
     product three times more (a rank-16 matmul, the scaling, the add: 65 us of a
     step of 410 at 1536 rows, 3072 -> 12288), and backward in bfloat16 scales the
     ``[M, R]`` product of the gradient instead of the gradient.  One rounding where
-    the composition has four."""
+    the composition has four.  The products with the factors are this package's
+    kernels (``own``): the factors packed once per step, then one read of ``x`` and,
+    backward, of ``x`` and of the gradient (304 -> 287 us of that step)."""
 
     @staticmethod
     def forward(ctx, x, lora_a, lora_b, w, scales, biases, bias, scale, group_size, bits):
-        t = torch.matmul(x.reshape(-1, x.shape[-1]), lora_a)
-        ctx.save_for_backward(x, lora_a, lora_b, w, scales, biases, t)
         ctx.meta = (scale, group_size, bits)
-        bs = lora_b if scale == 1.0 else (scale * lora_b.float()).to(lora_b.dtype)
+        ctx.own = lora_a.shape[1] <= _TRAINING_MAX_RANK and lora_b.shape[1] % 32 == 0
+        if ctx.own:
+            ops = _lib.ops()
+            af, bf, bs, ap = ops.low_rank_pack(lora_a.contiguous(), lora_b.contiguous(), scale)
+            t, tf = ops.low_rank_forward(_rows(x), af, lora_a.shape[1])
+            ctx.save_for_backward(x, lora_a, lora_b, w, scales, biases, tf, bf, ap)
+        else:
+            t = torch.matmul(x.reshape(-1, x.shape[-1]), lora_a)
+            ctx.save_for_backward(x, lora_a, lora_b, w, scales, biases, t)
+            bs = _operand((lora_b if scale == 1.0 else (scale * lora_b.float()).to(lora_b.dtype)).t())
+            t = _operand(t)
         return core.quantized_matmul(x, w, scales, biases, True, group_size, bits, bias=bias,
-                                     low_rank=(_operand(t).reshape(*x.shape[:-1], -1), _operand(bs.t())))
+                                     low_rank=(t.reshape(*x.shape[:-1], -1), bs))
 
     @staticmethod
     def backward(ctx, grad_y):
-        x, lora_a, lora_b, w, scales, biases, t = ctx.saved_tensors
+        x, lora_a, lora_b, w, scales, biases, *rest = ctx.saved_tensors
         scale, group_size, bits = ctx.meta
         x2, g = x.reshape(-1, x.shape[-1]), grad_y.reshape(-1, grad_y.shape[-1])
         twice = torch.is_grad_enabled()  # create_graph: everything below in operations that differentiate again
@@ -146,23 +156,45 @@ class _LoRALinearFunction(torch.autograd.Function):
         # young adapter its normal numbers; bfloat16 has float32's range, and the [M, R] products are scaled instead.
         if scale != 1.0 and g.dtype == torch.float16:
             g, scale = scale * g, 1.0
+        need_x, need_a, need_b = ctx.needs_input_grad[:3]
         grad_x = grad_a = grad_b = gt = None
-        if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
+        if ctx.own and not twice:
+            tf, bf, ap = rest
+            ops, rank = _lib.ops(), lora_a.shape[1]
+            rows = _rows(grad_y)
+            gt, gtf, grad_b = ops.low_rank_gradient(rows if scale == ctx.meta[0] else _rows(g), bf, tf, rank, scale,
+                                                    need_x or need_a, need_b)
+            grad_a = ops.low_rank_up(_rows(x), gtf, rank) if need_a else None
+            if need_x:
+                grad_x = core._matmul_untransposed(rows, w, scales, biases, group_size, bits, (gt, ap)).reshape(x.shape)
+            return grad_x, grad_a, grad_b if need_b else None, None, None, None, None, None, None, None
+        if need_x or need_a:
             gt = torch.matmul(g, lora_b.t())
             if scale != 1.0:
                 gt = scale * gt
-        if ctx.needs_input_grad[1]:
+        if need_a:
             grad_a = torch.matmul(x2.t(), gt)
-        if ctx.needs_input_grad[2]:
-            grad_b = torch.matmul((torch.matmul(x2, lora_a) if twice else t).t(), g)
+        if need_b:
+            grad_b = torch.matmul((torch.matmul(x2, lora_a) if twice else rest[0]).t(), g)
             if scale != 1.0:
                 grad_b = scale * grad_b
-        if ctx.needs_input_grad[0]:
+        if need_x:
             update = None if twice else (_operand(gt), _operand(lora_a))
             grad_x = core._matmul_untransposed(grad_y, w, scales, biases, group_size, bits, update)
             if twice:
                 grad_x = grad_x + torch.matmul(gt, lora_a.t()).reshape(grad_x.shape)
         return grad_x, grad_a, grad_b, None, None, None, None, None, None, None
+
+
+# of the kernels in csrc/lora.hip; above, and where N % 32, the products are torch's (rank 64, 1024 rows of 12288: 33 us for
+# the first of them against the BLAS library's 13)
+_TRAINING_MAX_RANK = 32
+
+
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    """``t`` as a contiguous matrix of its last dimension's rows at a 16-byte address."""
+    t = t.reshape(-1, t.shape[-1]).contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def _operand(t: torch.Tensor) -> torch.Tensor:
