@@ -175,7 +175,7 @@ def check_listing(text: str, kernel_substring: str, where: str = "listing") -> i
         body = text[m.end():text.index(".Lfunc_end", m.end())]
         blocks = _parse_blocks(body)
         index = {label: i for i, (label, _) in enumerate(blocks) if label}
-        col_tiles = re.search(r"ELi(\d)ELb[01]EEEv", name)  # the template argument before the last: column tiles per wavefront
+        col_tiles = re.search(r"ELi(\d)(?:ELb[01])+EEEv", name)  # the last number among the template arguments: column tiles per wavefront
         least = 2 * int(col_tiles.group(1)) if col_tiles else 8
 
         def walk(b, i, budget, visit, seen):

@@ -203,7 +203,7 @@ int mfq_qmm_t_low_rank(const void* x, int x_dtype, int64_t M, int64_t K, const u
     }
     if (!mfq::aligned16(y)) return MFQ_EALIGN;
     // many rows and room for the scratch copy: the two-kernel path of the 4- and 8-bit weights
-    if (M > 16 && K % 64 == 0 && y_dtype == x_dtype && workspace && mfq::aligned16(workspace) &&
+    if (M > 16 && K % 64 == 0 && (y_dtype == x_dtype || !rank) && workspace && mfq::aligned16(workspace) &&
         mfq::qmm_frag_shape_ok(M, N, K, bits) && workspace_bytes >= mfq::qmm_frag_copy_bytes(N, K) &&
         mfq::prefer_frag_path(M, N, K, group_size, bits))
       return mfq::launch_qmm(x, x_dtype, M, K, wq, scales, biases, bias, N, group_size, bits, y, y_dtype, workspace,

@@ -440,7 +440,7 @@ bool qmm_frag_shape_ok(int64_t M, int64_t N, int64_t K, int bits);
 bool prefer_frag_path(int64_t M, int64_t N, int64_t K, int gs, int bits);  // where the two-kernel path is the faster
 size_t qmm_frag_copy_bytes(int64_t N, int64_t K);
 int launch_qmm_frag(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
-                    const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, void* workspace,
+                    const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype, void* workspace,
                     int n_whole, int splits, hipStream_t stream, LowRank low_rank, Epilogue epi);
 // the same path for the weight not transposed, y[M, K] = x[M, N] @ dequantize(wq[N, K]): the copy holds W^T
 // (qmm_frag_copy_bytes(K, N) of workspace, the planes of a K cut wherever `planes` points)
@@ -460,7 +460,7 @@ int launch_qmm_n_ws(const void* x, int dtype, int64_t M, int64_t N, const uint32
 int launch_qmm_frag_copy(int dtype, const uint32_t* wq, const void* scales, const void* biases, int64_t N, int64_t K,
                          int gs, int bits, void* copy, hipStream_t stream);
 int launch_qmm_frag_gemm(const void* x, int dtype, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N,
-                         void* y, float* planes, int n_whole, int splits, hipStream_t stream, LowRank low_rank,
+                         void* y, int y_dtype, float* planes, int n_whole, int splits, hipStream_t stream, LowRank low_rank,
                          Epilogue epi);
 // the GEMM on a prepared copy with the K cut planned here: `workspace` takes the planes (without room: whole tiles)
 size_t qmm_prepared_workspace_bytes(int64_t M, int64_t N, int64_t K);

@@ -299,7 +299,10 @@ __device__ __forceinline__ void acc_read(f32x4& c, float (&v)[4]) {
 //     256-column tiles of the same round); without epilogue or K cut
 // kDeferBias: the instantiation for calls with an output bias, whose deferred tile stores (do_step) add it
 //     (apart, because the add in the slots of the other costs the calls without a bias a fifth of that pass)
-template <typename T, bool kEpi, bool kCut, bool kLowRank, int kJ = 4, bool kDeferBias = false>
+// kF32: y is float32 (activations that arrive in float32): the sums, and the bias, unrounded; without update, epilogue or
+//     deferred stores.  On the one-kernel path, where such calls were, 4096 x 3072 -> 3072 at 4 bits took 95 us with the
+//     rounding of x, 81 here; 6 bits 1536 x 3072 -> 12288 164 and 130; 2048 x 3072 -> 3072, where the two are level, 56
+template <typename T, bool kEpi, bool kCut, bool kLowRank, int kJ = 4, bool kDeferBias = false, bool kF32 = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void frag_gemm_kernel(
     const uint16_t* __restrict__ x, const char* __restrict__ wfrag, const uint16_t* __restrict__ bias,
     void* __restrict__ y, int M, int N, int K, int tiles_m, int tiles_n, int n_whole, int tail_splits,
@@ -309,6 +312,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   using vec8 = typename T::vec8;
   static_assert(kJ == 4 || (kJ == 3 && !kEpi && !kCut), "192-column tiles: plain whole tiles only");
   static_assert(!kDeferBias || (!kEpi && kJ == 4), "deferred stores with a bias: plain 256-column tiles");
+  static_assert(!kF32 || (!kEpi && !kLowRank && !kDeferBias), "float32 y: the linear alone");
   constexpr int kBN = 64 * kJ;  // columns of a tile
   const int n_tiles = tiles_m * tiles_n;
   const int n_items = n_whole + (n_tiles - n_whole) * tail_splits;
@@ -338,6 +342,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     }
     tile_origin(tile, tiles_m, tiles_n, it.m0, it.n0);
     it.n0 = it.n0 / BN * kBN;
+    if constexpr (kF32) {  // (the compiler keeps them in vector registers otherwise, where the loads' addresses cannot be)
+      it.first_step = __builtin_amdgcn_readfirstlane(it.first_step);
+      it.n_steps = __builtin_amdgcn_readfirstlane(it.n_steps);
+    }
     return it;
   };
   const int t = threadIdx.x;
@@ -806,6 +814,48 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     }
   };
 
+  // A whole tile as float32: the planes' transpose, 64 kJ / 4 pieces of 16 bytes to a row of the tile, the bias added to the
+  // sums on the way out.
+  auto store_tile_f32 = [&](auto with_bias, int m0, int n0) {
+    constexpr bool kBias = decltype(with_bias)::value;
+    constexpr int kPieces = 4 * kJ, kStride = 16 * kPieces + 16;
+    static_assert(32 * kStride <= kStageBytes, "the float32 staging fits the wavefront's region");
+    int lane_e = lane;
+    asm volatile("" : "+v"(lane_e));
+    const int c16 = lane_e & 15;
+    const int q = lane_e >> 4;
+    const int lane = lane_e;
+    char* stage = lds + kXBuffers * kTileBytes + wave * kStageBytes;
+    float* bias_f = reinterpret_cast<float*>(lds + kXBuffers * kTileBytes + 4 * kStageBytes + wave * kBiasBytes);
+    float* yout = reinterpret_cast<float*>(out_base);
+    if constexpr (kBias) bias_f[lane] = T::to_f32(out_bias[min(n0 + wn + lane, N - 1)]);
+#pragma unroll
+    for (int pass = 0; pass < 8; ++pass) {
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) {
+#pragma unroll
+        for (int r2 = 0; r2 < 2; ++r2) {
+          const int r = 2 * pass + r2;
+          *reinterpret_cast<float4*>(stage + (16 * r2 + c16) * kStride + (16 * j + 4 * q) * 4) =
+              make_float4(acc[r][j][0], acc[r][j][1], acc[r][j][2], acc[r][j][3]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int k = 0; k < kPieces / 2; ++k) {
+        const int idx = 64 * k + lane, rl = idx / kPieces, piece = idx - rl * kPieces;
+        float4 v = *reinterpret_cast<const float4*>(stage + rl * kStride + 16 * piece);
+        if constexpr (kBias) {
+          const float4 b = *reinterpret_cast<const float4*>(bias_f + 4 * piece);
+          v.x += b.x, v.y += b.y, v.z += b.z, v.w += b.w;
+        }
+        const int row = m0 + 32 * pass + rl, col = wn + 4 * piece;
+        if (row < M && n0 + col < N) *reinterpret_cast<float4*>(yout + (int64_t)(row - m0) * out_stride + col) = v;
+        if (k & 1) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
   // The items of this workgroup in sequence: first its whole tiles, then (kCut) its k ranges of tail tiles.
   // The two kinds run through two instantiations of the same loop, each with one kind of store behind it: with
   // both stores behind one loop the compiler reads the accumulators ahead of the branch and spills them.
@@ -817,7 +867,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
       const int m0 = item.m0, n0 = item.n0;
       const int steps = item.n_steps, s0 = item.first_step;
       if constexpr (!kPlanes) {
-        out_base = static_cast<char*>(y) + ((size_t)m0 * N + n0) * 2;
+        out_base = static_cast<char*>(y) + ((size_t)m0 * N + n0) * (kF32 ? 4 : 2);
         out_stride = N;
         if constexpr (kEpi) {
           if (epi.kind == kEpiSwiglu) {
@@ -844,7 +894,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
       {
         const bool last = steps == 2;
         const int s_even = last ? s_next : s0 + 2;
-        do_step(std::integral_constant<int, (kPlanes || kEpi) ? 3 : 1>{}, last, wa, wb, s0 + 1, s_even);
+        do_step(std::integral_constant<int, (kPlanes || kEpi || kF32) ? 3 : 1>{}, last, wa, wb, s0 + 1, s_even);
         do_step(std::integral_constant<int, 0>{}, false, wb, wa, s_even, last ? s_next + 1 : s0 + 3);
       }
       for (int p = 2; p < steps; p += 2) {
@@ -857,7 +907,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         if (s0 == 0) low_rank_steps(m0, n0);  // once per tile: by the item that has its first k range
       }
       primed = has_next;
-      if constexpr (!kPlanes && !kEpi) {
+      if constexpr (!kPlanes && !kEpi && !kF32) {
         // A tile with all of its rows and columns inside y, followed by another whole tile, leaves its sums in
         // the accumulators: the next tile's first step stores them (a bias: in the kDeferBias instantiation).
         if (seq + (int)gridDim.x < end && m0 + BM <= M && n0 + kBN <= N && (kDeferBias || !out_bias)) {
@@ -873,6 +923,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
       settle();
       if constexpr (kPlanes) {
         store_plane(planes + (size_t)item.plane * (BM * BN));
+      } else if constexpr (kF32) {
+        if (out_bias) store_tile_f32(std::true_type{}, m0, n0);
+        else store_tile_f32(std::false_type{}, m0, n0);
       } else if (out_bias) {
         store_tile_staged(std::true_type{}, m0, n0);
       } else {
@@ -925,10 +978,10 @@ int launch_dequant(const uint32_t* wq, const void* scales, const void* biases, i
   return launch_dequant_bits<T, 128>(wq, scales, biases, bits, out, N, K, stream);
 }
 
-template <typename T, bool kEpi, bool kCut, bool kLowRank, int kJ = 4, bool kDeferBias = false>
+template <typename T, bool kEpi, bool kCut, bool kLowRank, int kJ = 4, bool kDeferBias = false, bool kF32 = false>
 int launch_gemm(const void* x, int64_t M, int64_t K, const void* wfrag, const void* bias, int64_t N, void* y,
                 int n_whole, int splits, float* planes, hipStream_t stream, LowRank lr, Epilogue epi) {
-  auto kernel = frag_gemm_kernel<T, kEpi, kCut, kLowRank, kJ, kDeferBias>;
+  auto kernel = frag_gemm_kernel<T, kEpi, kCut, kLowRank, kJ, kDeferBias, kF32>;
   static PerDeviceInt configured;
   if (!raise_lds_limit(configured, reinterpret_cast<const void*>(kernel), kLdsBytes)) return MFQ_ELAUNCH;
   const int tiles_m = (int)((M + BM - 1) / BM);
@@ -941,12 +994,13 @@ int launch_gemm(const void* x, int64_t M, int64_t K, const void* wfrag, const vo
                      splits, planes, (const uint16_t*)lr.t, (const uint16_t*)lr.bs, lr.R, epi);
   if (hipGetLastError() != hipSuccess) return MFQ_ELAUNCH;
   if (splits > 1)
-    return launch_tail_reduce(T::code, planes, n_whole, splits, tiles_m, tiles_n, bias, M, N, y, T::code, stream, epi);
+    return launch_tail_reduce(T::code, planes, n_whole, splits, tiles_m, tiles_n, bias, M, N, y, kF32 ? MFQ_F32 : T::code, stream,
+                              epi);
   return MFQ_OK;
 }
 
 template <typename T>
-int launch_gemm_typed(const void* x, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N, void* y,
+int launch_gemm_typed(const void* x, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N, void* y, int y_dtype,
                       float* planes, int n_whole, int splits, hipStream_t stream, LowRank lr, Epilogue epi) {
   auto go = [&](auto e, auto c, auto l) {
     return launch_gemm<T, decltype(e)::value, decltype(c)::value, decltype(l)::value>(
@@ -957,6 +1011,12 @@ int launch_gemm_typed(const void* x, int64_t M, int64_t K, const void* copy, con
   // 192-column tiles where they fit one round of workgroups (the 256-column tiles of the same shape then do
   // too, with a third more work on each of fewer workgroups), unless the plan cuts that round along K
   const int64_t tiles_192 = ((M + BM - 1) / BM) * ((N + 191) / 192);
+  if (y_dtype == MFQ_F32) {
+    if (splits == 1 && tiles_192 <= compute_units())
+      return launch_gemm<T, false, false, false, 3, false, true>(x, M, K, copy, bias, N, y, (int)tiles_192, 1, planes, stream, lr, epi);
+    return splits > 1 ? launch_gemm<T, false, true, false, 4, false, true>(x, M, K, copy, bias, N, y, n_whole, splits, planes, stream, lr, epi)
+                      : launch_gemm<T, false, false, false, 4, false, true>(x, M, K, copy, bias, N, y, n_whole, 1, planes, stream, lr, epi);
+  }
   if (epi.kind == kEpiNone && splits == 1 && tiles_192 <= compute_units()) {
     if (lr.R)
       return launch_gemm<T, false, false, true, 3>(x, M, K, copy, bias, N, y, (int)tiles_192, 1, planes, stream, lr, epi);
@@ -995,17 +1055,18 @@ int launch_qmm_frag_copy(int dtype, const uint32_t* wq, const void* scales, cons
 }
 
 int launch_qmm_frag_gemm(const void* x, int dtype, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N,
-                         void* y, float* planes, int n_whole, int splits, hipStream_t stream, LowRank lr,
+                         void* y, int y_dtype, float* planes, int n_whole, int splits, hipStream_t stream, LowRank lr,
                          Epilogue epi) {
   if (!qmm_frag_shape_ok(M, N, K, 4)) return MFQ_EUNSUPPORTED;
+  if (y_dtype != dtype && (y_dtype != MFQ_F32 || lr.R || epi.kind != kEpiNone)) return MFQ_EUNSUPPORTED;
   if (lr.R && (epi.kind != kEpiNone || lr.R % 16)) return MFQ_EUNSUPPORTED;
   // 32-bit byte offsets into the update's operands
   if ((M + BM) * lr.R >= (int64_t)1 << 31 || (N + BN) * lr.R >= (int64_t)1 << 31) return MFQ_EUNSUPPORTED;
   if (splits > 1 && ((K / BK) % splits || (K / BK / splits) % 2)) return MFQ_EUNSUPPORTED;  // ranges of whole pairs of steps
   if (dtype == MFQ_BF16)
-    return launch_gemm_typed<BF16>(x, M, K, copy, bias, N, y, planes, n_whole, splits, stream, lr, epi);
+    return launch_gemm_typed<BF16>(x, M, K, copy, bias, N, y, y_dtype, planes, n_whole, splits, stream, lr, epi);
   if (dtype == MFQ_F16)
-    return launch_gemm_typed<F16>(x, M, K, copy, bias, N, y, planes, n_whole, splits, stream, lr, epi);
+    return launch_gemm_typed<F16>(x, M, K, copy, bias, N, y, y_dtype, planes, n_whole, splits, stream, lr, epi);
   return MFQ_EDTYPE;
 }
 
@@ -1045,18 +1106,18 @@ int launch_qmm_frag_n(const void* x, int dtype, int64_t M, int64_t N, const uint
   if (dtype == MFQ_BF16) rc = launch_dequant_t<BF16>(wq, scales, biases, gs, bits, workspace, N, K, stream);
   if (dtype == MFQ_F16) rc = launch_dequant_t<F16>(wq, scales, biases, gs, bits, workspace, N, K, stream);
   if (rc) return rc;
-  return launch_qmm_frag_gemm(x, dtype, M, N, workspace, nullptr, K, y, planes, n_whole, splits, stream, low_rank,
+  return launch_qmm_frag_gemm(x, dtype, M, N, workspace, nullptr, K, y, dtype, planes, n_whole, splits, stream, low_rank,
                               Epilogue());
 }
 
 int launch_qmm_frag(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
-                    const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, void* workspace,
+                    const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype, void* workspace,
                     int n_whole, int splits, hipStream_t stream, LowRank lr, Epilogue epi) {
   if (!qmm_frag_shape_ok(M, N, K, bits)) return MFQ_EUNSUPPORTED;
   if (int rc = launch_qmm_frag_copy(dtype, wq, scales, biases, N, K, gs, bits, workspace, stream)) return rc;
   // the planes of a K cut lie behind the copy
   float* planes = reinterpret_cast<float*>(static_cast<char*>(workspace) + qmm_frag_copy_bytes(N, K));
-  return launch_qmm_frag_gemm(x, dtype, M, K, workspace, bias, N, y, planes, n_whole, splits, stream, lr, epi);
+  return launch_qmm_frag_gemm(x, dtype, M, K, workspace, bias, N, y, y_dtype, planes, n_whole, splits, stream, lr, epi);
 }
 
 }  // namespace mfq

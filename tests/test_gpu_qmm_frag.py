@@ -438,3 +438,30 @@ def test_quantized_linear_prepare():
                                 mflux_amd.nn.QuantizedLinear(1024, 512, bits=8, device="cuda"), odd, narrow)
     assert mflux_amd.nn.prepare(model) == 2 * (1024 * 512 + 512 * 1024 + 3072 * 512)
     assert mflux_amd.nn.prepare(model, min_output_dims=1024) == 2 * (1024 * 512 + 3072 * 512)
+
+
+# 192-column tiles (one round of them), 256-column tiles whole and with a K cut, ragged rows and columns; 4, 8 and odd bits
+@pytest.mark.parametrize("M,K,N", [(4096, 256, 3072), (4001, 512, 3064), (2310, 256, 12296), (4360, 512, 5128), (6889, 3072, 3072),
+                                   (2817, 1024, 6152)])
+@pytest.mark.parametrize("bits,gs,dtype", [(4, 64, torch.bfloat16), (8, 32, torch.float16), (6, 128, torch.bfloat16)])
+@pytest.mark.parametrize("has_bias", [False, True])
+def test_float32_results(M, K, N, bits, gs, dtype, has_bias):
+    """Float32 activations are rounded to the weights' type on entry; what is left are the float32 sums (K 2^-24 of the sum of
+    magnitudes, below 2^-12 of a row's largest output on these operands) and the bias, added to them unrounded."""
+    import mflux_amd
+    from gpu_util import kernel_of
+    from mflux_amd import _lib, core
+
+    assert kernel_of(M, K, N, bits, gs) == (_lib.KERNEL_TWO_KERNELS, 3 if K == 3072 else 1)
+    gen = torch.Generator(device="cuda").manual_seed(97)
+    packed = mflux_amd.quantize((torch.randn(N, K, generator=gen, device="cuda") * 0.02).to(dtype), gs, bits)
+    x = torch.randn(M, K, generator=gen, device="cuda")
+    bias = torch.randn(N, generator=gen, device="cuda").to(dtype) if has_bias else None
+    y = core.quantized_matmul(x, *packed, True, gs, bits, bias=bias)
+    assert y.dtype == torch.float32
+    w_hat = mflux_amd.dequantize(*packed, gs, bits, dtype=torch.float32).to(dtype).double()
+    ref = x.to(dtype).double() @ w_hat.t()
+    bound = 2.0 ** -12 * ref.abs().amax(dim=1)
+    if has_bias:
+        ref, bound = ref + bias.double(), bound + 2.0 ** -23 * float(bias.abs().max())
+    assert bool(((y.double() - ref).abs().amax(dim=1) <= bound).all())
