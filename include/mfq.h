@@ -289,7 +289,8 @@ size_t mfq_qmm_t_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size
  * arguments the call refuses (and MFQ_EUNSUPPORTED for one row of more than
  * 8192 codes of 3, 5 or 6 bits, which is not answered).  *k_ranges (may be
  * NULL): into how many ranges K is cut between workgroups, of the last round of
- * tiles for the 256 x 256 tiles.  For tests and measurements.  Has no
+ * tiles for the 256 x 256 tiles (calls without an epilogue may run whole tiles
+ * of 192 columns instead of that cut).  For tests and measurements.  Has no
  * counterpart in the reference.
  */
 enum mfq_kernel {

@@ -295,8 +295,7 @@ __device__ __forceinline__ void acc_read(f32x4& c, float (&v)[4]) {
 // shapes that run whole tiles only is what it is without it: the plane store costs the epilogue registers)
 // kLowRank: lr_rank more k behind the item's own (a LoRA update, see qmm.hip), read straight from memory
 // kJ: column tiles of 16 per wavefront, i.e. tiles of 256 rows x 64 kJ columns: 4, or 3 (192 columns) for
-//     shapes whose 192-column tiles fit one round of workgroups (a quarter less work per workgroup than the
-//     256-column tiles of the same round); without epilogue or K cut
+//     shapes whose rounds of workgroups they fill better (prefer_192); without epilogue or K cut
 // kDeferBias: the instantiation for calls with an output bias, whose deferred tile stores (do_step) add it
 //     (apart, because the add in the slots of the other costs the calls without a bias a fifth of that pass)
 // kF32: y is float32 (activations that arrive in float32): the sums, and the bias, unrounded; without update, epilogue or
@@ -999,6 +998,23 @@ int launch_gemm(const void* x, int64_t M, int64_t K, const void* wfrag, const vo
   return MFQ_OK;
 }
 
+// 192-column tiles instead of 256 (`splits`: the cut that those have).  Where they fit one round of workgroups the 256-column
+// tiles do too, with a third more work on each of fewer.  Where 256-column tiles leave a short last round, two or three whole
+// rounds of three quarters of the work are less than one or two and what is left, cut along K (planes written, read and added)
+// or not: of 130 drawn calls between 2048 and 8192 rows with such a round those that the cut does not serve took 0.84 to 0.91 of
+// the time (5890 x 3072 -> 3840 134.6 us -> 116.7), those it does 0.90 to 0.99 with at least 0.22 of a round behind the first
+// (7110 x 3072 -> 3072 123 -> 112, 6889 rows 126 -> 122), from 0.27 on where K is long (5711 x 6144 -> 3840 213 -> 206); with
+// less 0.98 to 1.11, with 12288 k 1.04 and more.  Behind two rounds 0.92 to 0.996 from 0.05 of a round on.
+inline bool prefer_192(int64_t M, int64_t N, int64_t K, int splits) {
+  const int64_t cus = compute_units(), rows = (M + BM - 1) / BM;
+  const int64_t tiles_256 = rows * ((N + BN - 1) / BN), tiles_192 = rows * ((N + 191) / 192);
+  const int64_t rounds = (tiles_192 + cus - 1) / cus, rest = tiles_256 - (rounds - 1) * cus;
+  if (rounds == 1) return splits == 1;
+  if (rounds > 3 || rest <= 0) return false;
+  if (splits == 1) return true;
+  return rounds == 2 ? K <= 8192 && rest * 100 >= cus * (K <= 4096 ? 22 : 27) : K <= 6144 && rest * 100 >= cus * 5;
+}
+
 template <typename T>
 int launch_gemm_typed(const void* x, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N, void* y, int y_dtype,
                       float* planes, int n_whole, int splits, hipStream_t stream, LowRank lr, Epilogue epi) {
@@ -1008,16 +1024,15 @@ int launch_gemm_typed(const void* x, int64_t M, int64_t K, const void* copy, con
   };
   const std::true_type yes{};
   const std::false_type no{};
-  // 192-column tiles where they fit one round of workgroups (the 256-column tiles of the same shape then do
-  // too, with a third more work on each of fewer workgroups), unless the plan cuts that round along K
   const int64_t tiles_192 = ((M + BM - 1) / BM) * ((N + 191) / 192);
+  const bool narrow = epi.kind == kEpiNone && prefer_192(M, N, K, splits);
   if (y_dtype == MFQ_F32) {
-    if (splits == 1 && tiles_192 <= compute_units())
+    if (narrow)
       return launch_gemm<T, false, false, false, 3, false, true>(x, M, K, copy, bias, N, y, (int)tiles_192, 1, planes, stream, lr, epi);
     return splits > 1 ? launch_gemm<T, false, true, false, 4, false, true>(x, M, K, copy, bias, N, y, n_whole, splits, planes, stream, lr, epi)
                       : launch_gemm<T, false, false, false, 4, false, true>(x, M, K, copy, bias, N, y, n_whole, 1, planes, stream, lr, epi);
   }
-  if (epi.kind == kEpiNone && splits == 1 && tiles_192 <= compute_units()) {
+  if (narrow) {
     if (lr.R)
       return launch_gemm<T, false, false, true, 3>(x, M, K, copy, bias, N, y, (int)tiles_192, 1, planes, stream, lr, epi);
     return launch_gemm<T, false, false, false, 3>(x, M, K, copy, bias, N, y, (int)tiles_192, 1, planes, stream, lr, epi);

@@ -440,9 +440,9 @@ def test_quantized_linear_prepare():
     assert mflux_amd.nn.prepare(model, min_output_dims=1024) == 2 * (1024 * 512 + 3072 * 512)
 
 
-# 192-column tiles (one round of them), 256-column tiles whole and with a K cut, ragged rows and columns; 4, 8 and odd bits
-@pytest.mark.parametrize("M,K,N", [(4096, 256, 3072), (4001, 512, 3064), (2310, 256, 12296), (4360, 512, 5128), (6889, 3072, 3072),
-                                   (2817, 1024, 6152)])
+# 192-column tiles (one round of them, two), 256-column tiles whole and with a K cut (264 tiles), ragged rows and columns; 4, 8 and odd bits
+@pytest.mark.parametrize("M,K,N", [(4096, 256, 3072), (4001, 512, 3064), (2310, 256, 12296), (4360, 512, 5128), (6889, 512, 3072),
+                                   (5632, 3072, 3072), (2817, 1024, 6152)])
 @pytest.mark.parametrize("bits,gs,dtype", [(4, 64, torch.bfloat16), (8, 32, torch.float16), (6, 128, torch.bfloat16)])
 @pytest.mark.parametrize("has_bias", [False, True])
 def test_float32_results(M, K, N, bits, gs, dtype, has_bias):
@@ -452,7 +452,7 @@ def test_float32_results(M, K, N, bits, gs, dtype, has_bias):
     from gpu_util import kernel_of
     from mflux_amd import _lib, core
 
-    assert kernel_of(M, K, N, bits, gs) == (_lib.KERNEL_TWO_KERNELS, 3 if K == 3072 else 1)
+    assert kernel_of(M, K, N, bits, gs) == (_lib.KERNEL_TWO_KERNELS, (6 if gs == 128 else 12) if K == 3072 else 1)
     gen = torch.Generator(device="cuda").manual_seed(97)
     packed = mflux_amd.quantize((torch.randn(N, K, generator=gen, device="cuda") * 0.02).to(dtype), gs, bits)
     x = torch.randn(M, K, generator=gen, device="cuda")
@@ -465,3 +465,34 @@ def test_float32_results(M, K, N, bits, gs, dtype, has_bias):
     if has_bias:
         ref, bound = ref + bias.double(), bound + 2.0 ** -23 * float(bias.abs().max())
     assert bool(((y.double() - ref).abs().amax(dim=1) <= bound).all())
+
+
+# one round of 192-column tiles and a part of one, whole rounds, three of them; ragged rows and columns; a cut of the 256-column
+# tiles' tail that is left for them (6889 rows: 324 tiles) and none
+@pytest.mark.parametrize("M,K,N", [(6889, 3072, 3072), (6000, 256, 3840), (5890, 1152, 3848), (2683, 1152, 12296), (8192, 256, 3072)])
+@pytest.mark.parametrize("bits,gs,dtype", [(4, 64, torch.bfloat16), (8, 32, torch.float16), (5, 128, torch.bfloat16)])
+def test_rounds_of_192_column_tiles(M, K, N, bits, gs, dtype):
+    """Against float64 on the weights rounded once: a rounding of the result (at most 2^-8 of it, 2^-11 in float16), the bias add
+    once more, the float32 sums (below 2^-12 of a row's largest output here)."""
+    import mflux_amd
+    from gpu_util import kernel_of
+    from mflux_amd import _lib, core
+
+    assert kernel_of(M, K, N, bits, gs)[0] == _lib.KERNEL_TWO_KERNELS
+    gen = torch.Generator(device="cuda").manual_seed(98)
+    packed = mflux_amd.quantize((torch.randn(N, K, generator=gen, device="cuda") * 0.02).to(dtype), gs, bits)
+    x = torch.randn(M, K, generator=gen, device="cuda").to(dtype)
+    bias = torch.randn(N, generator=gen, device="cuda").to(dtype)
+    t, bs = torch.randn(M, 48, generator=gen, device="cuda").to(dtype), (torch.randn(N, 48, generator=gen, device="cuda") * 0.1).to(dtype)
+    ref = x.double() @ mflux_amd.dequantize(*packed, gs, bits, dtype=torch.float32).to(dtype).double().t()
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+
+    def close(y, want, roundings):
+        largest = want.abs().amax(dim=1) + (float(bias.abs().max()) if roundings == 2 else 0.0)
+        assert bool(((y.double() - want).abs().amax(dim=1) <= (roundings * unit + 2.0 ** -12) * largest).all())
+
+    close(core.quantized_matmul(x, *packed, True, gs, bits), ref, 1)
+    close(core.quantized_matmul(x, *packed, True, gs, bits, bias=bias), ref + bias.double(), 2)
+    close(core.quantized_matmul(x, *packed, True, gs, bits, bias=bias, low_rank=(t, bs)),
+          ref + t.double() @ bs.double().t() + bias.double(), 2)
+    close(core.quantized_matmul(x.float(), *packed, True, gs, bits), ref, 0)
