@@ -391,6 +391,13 @@ int mfq_qmv_silu(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_
 int mfq_silu(const void* x, int dtype, int64_t n, void* y, void* stream);
 
 /*
+ * y[i] = x[i] rounded to the 16-bit type dtype (nearest even), i < n: float32
+ * activations on their way into the products above, which take them in the
+ * scales' type.  y 16-byte aligned.
+ */
+int mfq_round(const float* x, int64_t n, int dtype, void* y, void* stream);
+
+/*
  * A quantized linear layer with LoRA adapters on it in one call:
  *   y = x @ dequantize(wq, scales, biases)^T + t @ bs^T (+ bias).
  * Replaces the body of LoRALinear.__call__

@@ -49,6 +49,7 @@ SIGNATURES = {
     "mfq_qmv_silu": (_INT, [_PTR, _INT, _I64, _I64, _PTR, _PTR, _PTR, _INT, _PTR, _I64, _INT, _INT, _PTR, _INT, _PTR]),
     "mfq_layer_norm_modulate": (_INT, [_PTR, _INT, _I64, _I64, _PTR, _PTR, _I64, ctypes.c_float, _PTR, _PTR]),
     "mfq_silu": (_INT, [_PTR, _INT, _I64, _PTR, _PTR]),
+    "mfq_round": (_INT, [_PTR, _I64, _INT, _PTR, _PTR]),
     "mfq_low_rank_down": (_INT, [_PTR, _PTR, _INT, _I64, _I64, _I64, _PTR, _PTR]),
     "mfq_low_rank_pack": (_INT, [_PTR, _PTR, _INT, _I64, _I64, _I64, _I64, ctypes.c_float, _PTR, _PTR, _PTR, _PTR, _PTR]),
     "mfq_low_rank_forward": (_INT, [_PTR, _PTR, _INT, _I64, _I64, _I64, _I64, _PTR, _PTR, _PTR]),

@@ -224,7 +224,10 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     ``_quantized_matmul_forward``.  Differentiable with respect to ``x`` and
     ``bias``; ``low_rank`` (inference only) is described there."""
     if transpose and low_rank is None and mode == "affine":
-        y = _lib.native().linear(x, w, scales, biases, bias, group_size, bits)
+        native = _lib.native()
+        y = native.linear(x, w, scales, biases, bias, group_size, bits)
+        if y is None:
+            y = native.linear_float32(x, w, scales, biases, bias, group_size, bits)
         if y is not None:
             return y
     _check_mode("quantized_matmul", mode)

@@ -338,6 +338,14 @@ int mfq_silu(const void* x, int dtype, int64_t n, void* y, void* stream) {
   return mfq::launch_silu(x, dtype, n, y, (hipStream_t)stream);
 }
 
+int mfq_round(const float* x, int64_t n, int dtype, void* y, void* stream) {
+  if (!is16(dtype)) return MFQ_EDTYPE;
+  if (n <= 0 || n > (int64_t)1 << 40) return MFQ_ESHAPE;
+  if (!x || !y) return MFQ_ENULL;
+  if (!mfq::aligned16(y)) return MFQ_EALIGN;
+  return mfq::launch_round(x, n, dtype, y, (hipStream_t)stream);
+}
+
 int mfq_layer_norm_modulate(const void* x, int dtype, int64_t M, int64_t K, const void* scale, const void* shift,
                             int64_t rows_per_vector, float eps, void* y, void* stream) {
   if (!is16(dtype)) return MFQ_EDTYPE;

@@ -419,6 +419,8 @@ int launch_low_rank_up(const void* x, int dtype, int64_t M, int64_t K, const voi
                        hipStream_t stream);
 // y[i] = silu(x[i]), the sigmoid and the product each rounded to the 16-bit type
 int launch_silu(const void* x, int dtype, int64_t n, void* y, hipStream_t stream);
+// y[i] = x[i] rounded to the 16-bit type
+int launch_round(const float* x, int64_t n, int dtype, void* y, hipStream_t stream);
 // t[M, R] = x[M, K] @ A[K, R], A in fragment order ([R/16][K/32][4][16][8]); 16-bit type `dtype`; R % 16 == 0, K % 32 == 0
 int launch_low_rank_down(const void* x, int dtype, int64_t M, int64_t K, const void* at, int64_t R, void* t,
                          hipStream_t stream);

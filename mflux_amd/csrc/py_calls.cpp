@@ -65,6 +65,7 @@ struct Linear {
   Tensor x, wq, scales, biases, bias;
   int64_t gs = 0, bits = 0, M = 0, K = 0, N = 0;
   int dtype = 0;
+  bool float32 = false;  // x is float32, and so is y
 
   bool parse(PyObject* const* args) {
     return tensor_arg(args[0], &x) && tensor_arg(args[1], &wq) && tensor_arg(args[2], &scales) &&
@@ -81,7 +82,8 @@ struct Linear {
     if (t == at::kBFloat16) dtype = MFQ_BF16;
     else if (t == at::kHalf) dtype = MFQ_F16;
     else return false;
-    if (wq.scalar_type() != at::kUInt32 || biases.scalar_type() != t || x.scalar_type() != t) return false;
+    if (wq.scalar_type() != at::kUInt32 || biases.scalar_type() != t || x.scalar_type() != (float32 ? at::kFloat : t))
+      return false;
     if (wq.dim() != 2 || scales.dim() != 2 || biases.sizes() != scales.sizes() || x.dim() < 1) return false;
     if ((gs != 32 && gs != 64 && gs != 128) || (bits != 3 && bits != 4 && bits != 5 && bits != 6 && bits != 8)) return false;
     N = wq.size(0);
@@ -143,6 +145,31 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
                     y_p, p.dtype, ws_p, ws_bytes, in.stream);
   Py_END_ALLOW_THREADS
   return result("mfq_qmm_t_ws", rc, y);
+  END_HANDLE_TH_ERRORS
+}
+
+// linear_float32(x, weight, scales, biases, bias or None, group_size, bits) -> y or None: float32 x, rounded to the scales' type
+// for the product, whose sums and bias are the float32 result
+PyObject* linear_float32(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  Linear p;
+  p.float32 = true;
+  if (n != 7 || !p.parse(args)) Py_RETURN_NONE;
+  RECORD_FUNCTION("mfq::qmm_t", p.inputs());
+  const c10::hip::HIPGuardMasqueradingAsCUDA on_device(p.x.device());
+  Tensor y = p.out(p.N), rounded = at::empty({p.M, p.K}, p.scales.options().requires_grad(false)), ws;
+  const size_t ws_bytes = mfq_qmm_t_workspace_bytes(p.M, p.K, p.N, (int)p.gs, (int)p.bits);
+  if (ws_bytes) ws = p.workspace(ws_bytes);
+  const Linear::Pointers in = p.pointers();
+  void *y_p = y.data_ptr(), *r_p = rounded.data_ptr(), *ws_p = ws_bytes ? ws.data_ptr() : nullptr;
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = mfq_round(static_cast<const float*>(in.x), p.M * p.K, p.dtype, r_p, in.stream);
+  if (rc == MFQ_OK)
+    rc = mfq_qmm_t_ws(r_p, p.dtype, p.M, p.K, in.wq, in.scales, in.biases, p.dtype, in.bias, p.N, (int)p.gs, (int)p.bits, y_p,
+                      MFQ_F32, ws_p, ws_bytes, in.stream);
+  Py_END_ALLOW_THREADS
+  return result("mfq_round, mfq_qmm_t_ws", rc, y);
   END_HANDLE_TH_ERRORS
 }
 
@@ -221,6 +248,7 @@ PyObject* epilogue_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 PyMethodDef kMethods[] = {
     {"linear", (PyCFunction)(void*)linear, METH_FASTCALL, "x @ dequantize(w).T (+ bias), or None"},
+    {"linear_float32", (PyCFunction)(void*)linear_float32, METH_FASTCALL, "the same of a float32 x, or None"},
     {"silu_linear", (PyCFunction)(void*)silu_linear, METH_FASTCALL, "silu(x) @ dequantize(w).T (+ bias), or None"},
     {"epilogue_linear", (PyCFunction)(void*)epilogue_linear, METH_FASTCALL, "a linear with its epilogue, or None"},
     {nullptr, nullptr, 0, nullptr}};

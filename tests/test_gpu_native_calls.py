@@ -131,3 +131,23 @@ def test_epilogues_same_bits_as_the_operator(epilogue, act_from, bits):
     got = _lib.native().epilogue_linear(x, *w, 64, bits, core.EPILOGUES[epilogue], None, None, act_from)
     ref, ok = _lib.ops().qmm_t_epilogue(x.reshape(-1, 256), *w, 64, bits, core.EPILOGUES[epilogue], None, None, act_from)
     assert ok and got.shape == (2, 20, ref.shape[-1]) and torch.equal(got, ref.reshape(got.shape))
+
+
+@pytest.mark.parametrize("bits,dtype,shape", [(8, torch.bfloat16, (1, 256)), (4, torch.float16, (2, 3, 256)), (6, torch.bfloat16, (40, 256)),
+                                              (4, torch.bfloat16, (1, 300, 256)), (4, torch.bfloat16, (256,)), (5, torch.float16, (7, 256)),
+                                              (4, torch.bfloat16, (2304, 256))])
+def test_float32_activations_are_the_operator_on_rounded_ones(bits, dtype, shape):
+    from mflux_amd import _lib
+
+    layer = _layer(256, 192, bits, bias=bits != 4, dtype=dtype)
+    x = torch.randn(shape, device="cuda") * 3
+    x.view(-1)[:4] = torch.tensor([1 + 2 ** -8, 1 + 3 * 2 ** -8, -1e-40, 3e38 if dtype == torch.bfloat16 else 65519.0])  # ties, tiny, large
+    w = layer._operands()
+    y = _lib.native().linear_float32(x, *w, 64, bits)
+    ref, ok = _lib.ops().qmm_t(x.reshape(-1, 256).to(dtype), *w, 64, bits, torch.float32, None, None)
+    assert ok and y.dtype == torch.float32 and y.shape == (*shape[:-1], 192) and torch.equal(y, ref.reshape(y.shape))
+    assert torch.equal(y, layer(x))
+    shifted = torch.empty(x.numel() + 1, device="cuda")[1:].view(shape).copy_(x)  # at an address of its own
+    assert torch.equal(_lib.native().linear_float32(shifted, *w, 64, bits), y)
+    for other in (x.to(dtype), x.double(), x.clone().requires_grad_(True), x.cpu()):
+        assert _lib.native().linear_float32(other, *w, 64, bits) is None
