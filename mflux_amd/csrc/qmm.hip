@@ -859,6 +859,34 @@ inline TailPlan plan_tail(int64_t M, int64_t N, int64_t K, int period, int cus) 
 
 inline int period_of(int gs) { return 4 * gs / BK; }
 
+// The sum of `splits` planes at one place, first to last.  All of a sum's loads are on their way before the first is waited
+// for: as a loop over a count known at run time they went one after another, each with the memory's whole latency.
+template <int S>
+__device__ inline float4 sum_of_planes(const float* p, size_t stride) {
+  float4 v[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) v[s] = *reinterpret_cast<const float4*>(p + s * stride);
+#pragma unroll
+  for (int s = 1; s < S; ++s) v[0].x += v[s].x, v[0].y += v[s].y, v[0].z += v[s].z, v[0].w += v[s].w;
+  return v[0];
+}
+__device__ inline float4 sum_of_planes(const float* p, size_t stride, int splits) {
+  switch (splits) {
+    case 2: return sum_of_planes<2>(p, stride);
+    case 3: return sum_of_planes<3>(p, stride);
+    case 4: return sum_of_planes<4>(p, stride);
+    case 5: return sum_of_planes<5>(p, stride);
+    case 6: return sum_of_planes<6>(p, stride);
+    default: break;
+  }
+  float4 sum = sum_of_planes<7>(p, stride);
+  for (int s = 7; s < splits; ++s) {
+    const float4 v = *reinterpret_cast<const float4*>(p + s * stride);
+    sum.x += v.x, sum.y += v.y, sum.z += v.z, sum.w += v.w;
+  }
+  return sum;
+}
+
 // y = sum of `splits` dense float32 planes of M x N (+ bias), through the epilogue: the second kernel of
 // the 128-column-tile GEMM's K split.
 template <typename T>
@@ -866,33 +894,38 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
                                                             int64_t plane_elems, const uint16_t* __restrict__ bias,
                                                             int N, void* __restrict__ y, int y_is_f32, Epilogue epi) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  // the value of the linear layer in column c: rounded, then the bias added and rounded again, as the fused
+  // the value of the linear layer, bv its column's bias: rounded, then the bias added and rounded again, as the fused
   // epilogue does (float32 y: one float32 sum)
-  auto linear = [&](float v, int c) {
-    const float bv = bias ? T::to_f32(bias[c]) : 0.f;
+  auto linear = [&](float v, float bv) {
     if (y_is_f32) return v + bv;
     const float h = round_to<T>(v);
     return bias ? round_to<T>(h + bv) : h;
   };
-  auto sum4 = [&](int64_t q) {
-    float4 sum = reinterpret_cast<const float4*>(planes)[q];
-    for (int sp = 1; sp < splits; ++sp) {
-      const float4 v = reinterpret_cast<const float4*>(planes + sp * plane_elems)[q];
-      sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
-    }
-    return sum;
+  auto bias4 = [&](int c, float (&b)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = bias ? T::to_f32(bias[c + e]) : 0.f;
   };
+  auto sum4 = [&](int64_t q) { return sum_of_planes(planes + 4 * q, plane_elems, splits); };
   // four consecutive outputs per thread when rows are a multiple of four long
   // (a quad then never straddles two rows), one otherwise
   if ((N & 3) == 0) {
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < plane_elems / 4; q += stride) {
       const int col = (int)((q * 4) % N);
       if (epi.kind == kEpiSwiglu && (col & 32)) continue;  // the up projection's columns are read by the gate's threads
+      float b[4];
+      bias4(col, b);
+      uint2 g = {0, 0}, r = {0, 0};  // requested ahead of the sum
+      if (epi.kind == kEpiGateResidual) {
+        g = *reinterpret_cast<const uint2*>(epi.gate + col);
+        r = reinterpret_cast<const uint2*>(epi.residual)[q];
+      }
       const float4 sum = sum4(q);
-      float v[4] = {linear(sum.x, col), linear(sum.y, col + 1), linear(sum.z, col + 2), linear(sum.w, col + 3)};
+      float v[4] = {linear(sum.x, b[0]), linear(sum.y, b[1]), linear(sum.z, b[2]), linear(sum.w, b[3])};
       if (epi.kind == kEpiSwiglu) {  // N % 64 == 0; y is [M, N/2]
         const float4 ups = sum4(q + 8);
-        const float u[4] = {linear(ups.x, col + 32), linear(ups.y, col + 33), linear(ups.z, col + 34), linear(ups.w, col + 35)};
+        float bu[4];
+        bias4(col + 32, bu);
+        const float u[4] = {linear(ups.x, bu[0]), linear(ups.y, bu[1]), linear(ups.z, bu[2]), linear(ups.w, bu[3])};
         const int64_t row = (q * 4) / N;
         uint2 pk;
         pk.x = T::pack2(epi_swiglu<T>(v[0], u[0]), epi_swiglu<T>(v[1], u[1]));
@@ -905,8 +938,6 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
         for (int c = 0; c < 4; ++c) v[c] = epi_gelu<T>(v[c]);
       }
       if (epi.kind == kEpiGateResidual) {
-        const uint2 g = *reinterpret_cast<const uint2*>(epi.gate + col);
-        const uint2 r = reinterpret_cast<const uint2*>(epi.residual)[q];
         v[0] = epi_gate_residual<T>(v[0], lo_f32<T>(g.x), lo_f32<T>(r.x));
         v[1] = epi_gate_residual<T>(v[1], hi_f32<T>(g.x), hi_f32<T>(r.x));
         v[2] = epi_gate_residual<T>(v[2], lo_f32<T>(g.y), lo_f32<T>(r.y));
@@ -922,7 +953,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < plane_elems; i += stride) {
       float sum = planes[i];
       for (int sp = 1; sp < splits; ++sp) sum += planes[sp * plane_elems + i];
-      const float v = linear(sum, (int)(i % N));
+      const float v = linear(sum, bias ? T::to_f32(bias[i % N]) : 0.f);
       if (y_is_f32) {
         reinterpret_cast<float*>(y)[i] = v;
       } else {
@@ -948,14 +979,7 @@ __global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restric
   if (row >= M || col >= N) return;
   if (epi.kind == kEpiSwiglu && (c & 32)) return;  // the up projection's columns are read by the gate's threads
   const float* src = planes + (size_t)tail_tile * splits * (BM * BN) + r * BN + c;
-  auto sum_at = [&](const float* p) {
-    float4 sum = *reinterpret_cast<const float4*>(p);
-    for (int sp = 1; sp < splits; ++sp) {
-      const float4 v = *reinterpret_cast<const float4*>(p + (size_t)sp * (BM * BN));
-      sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
-    }
-    return sum;
-  };
+  auto sum_at = [&](const float* p) { return sum_of_planes(p, BM * BN, splits); };
   // the value of the linear layer in column cc: rounded, then the bias added and rounded again, as the fused
   // epilogue does (float32 y: one float32 sum)
   auto linear = [&](float v, int cc) {
@@ -1218,7 +1242,7 @@ int launch_splitk_reduce(int dtype, const void* planes, int splits, int64_t M, i
   const int64_t plane = M * N;
   const int64_t threads = (N & 3) == 0 ? plane / 4 : plane;
   const int64_t blocks = (threads + 255) / 256;
-  const int cap = compute_units() * 8;
+  const int cap = compute_units() * 64;
   const dim3 grid((unsigned)(blocks < cap ? blocks : cap));
   if (dtype == MFQ_BF16) {
     hipLaunchKernelGGL((splitk_reduce_kernel<BF16>), grid, dim3(256), 0, stream, (const float*)planes, splits, plane,
