@@ -260,8 +260,8 @@ int mfq_qmm_n_low_rank(const void* x, int x_dtype, int64_t M, int64_t N, const u
  * cut into ranges that run on different compute units, each range accumulates
  * into its own float32 plane of the workspace, and a second kernel adds the
  * planes, rounds and applies the bias (same two roundings as the fused
- * epilogue).  Large calls -- 16-bit y, K a multiple of 128, at least 2048
- * activation rows at 4 or 8 bits and 1024 at 3, 5 or 6 (where it starts to
+ * epilogue).  Large calls -- K a multiple of 128, from 1281 to 2048
+ * activation rows on at 4 or 8 bits and 1024 at 3, 5 or 6 (where it starts to
  * pay), e.g. the single-stream
  * linears of FLUX.1 at M = 4608 -- use the workspace first for a 16-bit copy of
  * the dequantised weights (round_up(N, 16) * K * 2 bytes rounded up to 256,

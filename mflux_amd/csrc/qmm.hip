@@ -1196,12 +1196,27 @@ constexpr int64_t kOddBitsFragRows = MFQ_ODD_FRAG_ROWS;
 
 // The two-kernel path (qmm_frag.hip: a 16-bit scratch copy of the weights in fragment order, then a lean
 // GEMM) takes the shapes it wins on: at least eight rows of tiles to spread the copy over.  It cuts K for
-// the tail of the tile sequence by the same plan as the fused kernel.
+// the tail of the tile sequence by the same plan as the fused kernel, or takes narrower tiles there.
+// 4 and 8 bits, 35 drawn shapes of 1793 to 2047 rows (all group sizes, float32 results, low-rank updates): 0.60 to 1.01 of the
+// fused kernel's time (1985 x 2560 -> 9216 107 us -> 102, 1951 x 15360 -> 4304 303 -> 248).  With seven rows of tiles and six the
+// two are level by themselves, and between other kernels the copy's traffic costs more (a training step at 1536 x 3072 -> 12288
+// 283 us, 293 with the copy), except (1281 rows and more) where the narrower tiles take two or three rounds in the place of a
+// short last one (1661 x 2560 -> 12288 137 us -> 112, 1616 x 3072 -> 12288 131 -> 119), and where K is not whole scale periods and
+// the fused kernel reads its scales step by step (1493 x 3840 -> 12288 in groups of 128 236 us -> 148, 1401 x 1152 -> 12288 74 ->
+// 59; 1055 rows 42 -> 47).
+// Below 2048 rows a last round of up to eight tiles, cut, stays with the fused kernel, though it takes 2 to 9 % more there (2040 x
+// 3072 -> 8448 115 us, 106 here): mfq_qmm_t_static holds the planes of such a cut and no copy, and gives mfq_qmm_t_ws's bits.
 bool prefer_frag_path(int64_t M, int64_t N, int64_t K, int gs, int bits) {
+  if (!qmm_frag_shape_ok(M, N, K, bits) || use_mid_kernel(M, N, K)) return false;
   // (3, 5 and 6 bits: the alternative is the 128-column-tile kernel with its codes cut out of a bit stream,
   // which the copy overtakes much earlier)
-  const int64_t least_rows = (bits == 4 || bits == 8) ? 2048 : kOddBitsFragRows;
-  return M >= least_rows && qmm_frag_shape_ok(M, N, K, bits) && !use_mid_kernel(M, N, K);
+  if (bits != 4 && bits != 8) return M >= kOddBitsFragRows;
+  if (M >= 8 * BM) return true;
+  if (M <= 5 * BM) return false;
+  const int64_t cus = compute_units(), rest = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) % cus;
+  const int splits = plan_tail(M, N, K, period_of(gs), (int)cus).splits;
+  if (splits > 1 && rest <= 8) return false;
+  return M > 7 * BM || K / BK % period_of(gs) || qmm_frag_narrow_rounds(M, N, K, splits);
 }
 
 // In the order of launch_qmm() and launch_qmm_mid_stream().  What sends a call past the wide or the sliced kernel, scales or

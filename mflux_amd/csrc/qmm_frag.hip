@@ -1,4 +1,4 @@
-// Large-M quantized GEMM in two kernels (from 2048 activation rows on, where the copy starts to pay):
+// Large-M quantized GEMM in two kernels (from six to eight rows of its tiles on, where the copy starts to pay):
 //   1. dequant_frag_kernel expands the packed weights ONCE per call into 16-bit values
 //      (w_hat = round(fma(code, scale, bias)), the same single rounding as the fused
 //      kernels) and writes them in the order the matrix instructions consume them:
@@ -1049,6 +1049,10 @@ int launch_gemm_typed(const void* x, int64_t M, int64_t K, const void* copy, con
 }
 
 }  // namespace
+
+bool qmm_frag_narrow_rounds(int64_t M, int64_t N, int64_t K, int splits) {
+  return ((M + BM - 1) / BM) * ((N + 191) / 192) > compute_units() && prefer_192(M, N, K, splits);
+}
 
 bool qmm_frag_shape_ok(int64_t M, int64_t N, int64_t K, int bits) {
   // whole pairs of k steps and at least two of them; whole 16-byte pieces of y; 32-bit byte offsets into x
