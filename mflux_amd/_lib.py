@@ -113,14 +113,14 @@ class _NotBuilt:
     """Stands in for the C functions where the libraries are not built: every call takes the
     general route, which words argument errors first and then says what is missing."""
 
-    linear = silu_linear = epilogue_linear = staticmethod(lambda *args: None)
+    linear = linear_float32 = silu_linear = epilogue_linear = staticmethod(lambda *args: None)
 
 
 def native():
     """The Python C functions of csrc/py_calls.cpp, which live in the same library
-    as the ops: ``linear``, ``silu_linear`` and ``epilogue_linear`` take the
-    ordinary call of a quantized linear straight to the C ABI and return None
-    for anything else."""
+    as the ops: ``linear``, ``linear_float32``, ``silu_linear`` and
+    ``epilogue_linear`` take the ordinary call of a quantized linear straight to
+    the C ABI and return None for anything else."""
     global _native
     if _native is None:
         import importlib.machinery
