@@ -13,7 +13,7 @@ from concurrent.futures import ThreadPoolExecutor
 
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.path.join(CSRC, "libmfq.so")
-SOURCES = ("abi.hip", "quantize.hip", "qmv.hip", "qmv_dot.hip", "qmv_quad.hip", "qmv_odd.hip", "qmv_oct.hip", "qmv_oct4.hip", "qmm.hip", "qmm_epi.hip", "qmm_mid.hip", "qmm_mid_stream.hip", "qmm_slice.hip", "qmm_wide.hip", "qmm_n.hip", "qmm_frag.hip", "lora.hip", "norm.hip")
+SOURCES = ("abi.hip", "quantize.hip", "qmv.hip", "qmv_dot.hip", "qmv_quad.hip", "qmv_odd.hip", "qmv_oct.hip", "qmv_oct4.hip", "qmm.hip", "qmm_epi.hip", "qmm_mid.hip", "qmm_mid_stream.hip", "qmm_slice.hip", "qmm_wide.hip", "qmm_n.hip", "qmm_frag.hip", "qmm_frag_f32.hip", "lora.hip", "norm.hip")
 
 # -ffp-contract=off, correctly rounded division and preserved denormals make
 # the quantize kernel's float32 arithmetic the same IEEE operations as the
@@ -44,9 +44,9 @@ def _compile(src: str) -> str:
 
 # Kernels whose matrix instructions are inline assembly (result tied to the addend), which the compiler's
 # hazard recognizer cannot see: {source: substring of the kernels' mangled names}.
-ASM_MFMA_KERNELS = {"qmm_frag.hip": "frag_gemm_kernel"}
+ASM_MFMA_KERNELS = {"qmm_frag.hip": "frag_gemm_kernel", "qmm_frag_f32.hip": "frag_gemm_kernel"}
 # Sources whose loads from memory straight into LDS are inline assembly, with the write of m0 (their LDS base) in front.
-ASM_LDS_LOAD_SOURCES = ("qmm_frag.hip", "qmm_slice.hip")
+ASM_LDS_LOAD_SOURCES = ("qmm_frag.hip", "qmm_frag_f32.hip", "qmm_slice.hip")
 
 
 def _parse_blocks(body: str):

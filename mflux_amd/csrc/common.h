@@ -465,6 +465,9 @@ int launch_qmm_frag_copy(int dtype, const uint32_t* wq, const void* scales, cons
 int launch_qmm_frag_gemm(const void* x, int dtype, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N,
                          void* y, int y_dtype, float* planes, int n_whole, int splits, hipStream_t stream, LowRank low_rank,
                          Epilogue epi);
+// the same with float32 y, no update and no epilogue (launch_qmm_frag_gemm has checked the arguments)
+int launch_qmm_frag_gemm_f32(const void* x, int dtype, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N,
+                             void* y, float* planes, int n_whole, int splits, hipStream_t stream);
 // the GEMM on a prepared copy with the K cut planned here: `workspace` takes the planes (without room: whole tiles)
 size_t qmm_prepared_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int launch_qmm_prepared(const void* x, int dtype, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N,

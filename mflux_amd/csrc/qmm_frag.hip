@@ -301,6 +301,7 @@ __device__ __forceinline__ void acc_read(f32x4& c, float (&v)[4]) {
 // kF32: y is float32 (activations that arrive in float32): the sums, and the bias, unrounded; without update, epilogue or
 //     deferred stores.  On the one-kernel path, where such calls were, 4096 x 3072 -> 3072 at 4 bits took 95 us with the
 //     rounding of x, 81 here; 6 bits 1536 x 3072 -> 12288 164 and 130; 2048 x 3072 -> 3072, where the two are level, 56
+//     (compiled in qmm_frag_f32.hip)
 template <typename T, bool kEpi, bool kCut, bool kLowRank, int kJ = 4, bool kDeferBias = false, bool kF32 = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void frag_gemm_kernel(
     const uint16_t* __restrict__ x, const char* __restrict__ wfrag, const uint16_t* __restrict__ bias,
@@ -1015,8 +1016,30 @@ inline bool prefer_192(int64_t M, int64_t N, int64_t K, int splits) {
   return rounds == 2 ? K <= 8192 && rest * 100 >= cus * (K <= 4096 ? 22 : 27) : K <= 6144 && rest * 100 >= cus * 5;
 }
 
+#ifdef MFQ_FRAG_F32
 template <typename T>
-int launch_gemm_typed(const void* x, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N, void* y, int y_dtype,
+int launch_gemm_f32(const void* x, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N, void* y,
+                    float* planes, int n_whole, int splits, hipStream_t stream) {
+  const Epilogue none;
+  if (prefer_192(M, N, K, splits))
+    return launch_gemm<T, false, false, false, 3, false, true>(
+        x, M, K, copy, bias, N, y, (int)(((M + BM - 1) / BM) * ((N + 191) / 192)), 1, planes, stream, LowRank(), none);
+  return splits > 1 ? launch_gemm<T, false, true, false, 4, false, true>(x, M, K, copy, bias, N, y, n_whole, splits, planes,
+                                                                         stream, LowRank(), none)
+                    : launch_gemm<T, false, false, false, 4, false, true>(x, M, K, copy, bias, N, y, n_whole, 1, planes,
+                                                                          stream, LowRank(), none);
+}
+
+}  // namespace
+
+int launch_qmm_frag_gemm_f32(const void* x, int dtype, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N,
+                             void* y, float* planes, int n_whole, int splits, hipStream_t stream) {
+  return dtype == MFQ_BF16 ? launch_gemm_f32<BF16>(x, M, K, copy, bias, N, y, planes, n_whole, splits, stream)
+                           : launch_gemm_f32<F16>(x, M, K, copy, bias, N, y, planes, n_whole, splits, stream);
+}
+#else
+template <typename T>
+int launch_gemm_typed(const void* x, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N, void* y,
                       float* planes, int n_whole, int splits, hipStream_t stream, LowRank lr, Epilogue epi) {
   auto go = [&](auto e, auto c, auto l) {
     return launch_gemm<T, decltype(e)::value, decltype(c)::value, decltype(l)::value>(
@@ -1026,12 +1049,6 @@ int launch_gemm_typed(const void* x, int64_t M, int64_t K, const void* copy, con
   const std::false_type no{};
   const int64_t tiles_192 = ((M + BM - 1) / BM) * ((N + 191) / 192);
   const bool narrow = epi.kind == kEpiNone && prefer_192(M, N, K, splits);
-  if (y_dtype == MFQ_F32) {
-    if (narrow)
-      return launch_gemm<T, false, false, false, 3, false, true>(x, M, K, copy, bias, N, y, (int)tiles_192, 1, planes, stream, lr, epi);
-    return splits > 1 ? launch_gemm<T, false, true, false, 4, false, true>(x, M, K, copy, bias, N, y, n_whole, splits, planes, stream, lr, epi)
-                      : launch_gemm<T, false, false, false, 4, false, true>(x, M, K, copy, bias, N, y, n_whole, 1, planes, stream, lr, epi);
-  }
   if (narrow) {
     if (lr.R)
       return launch_gemm<T, false, false, true, 3>(x, M, K, copy, bias, N, y, (int)tiles_192, 1, planes, stream, lr, epi);
@@ -1082,11 +1099,12 @@ int launch_qmm_frag_gemm(const void* x, int dtype, int64_t M, int64_t K, const v
   // 32-bit byte offsets into the update's operands
   if ((M + BM) * lr.R >= (int64_t)1 << 31 || (N + BN) * lr.R >= (int64_t)1 << 31) return MFQ_EUNSUPPORTED;
   if (splits > 1 && ((K / BK) % splits || (K / BK / splits) % 2)) return MFQ_EUNSUPPORTED;  // ranges of whole pairs of steps
+  if (dtype != MFQ_BF16 && dtype != MFQ_F16) return MFQ_EDTYPE;
+  if (y_dtype == MFQ_F32)
+    return launch_qmm_frag_gemm_f32(x, dtype, M, K, copy, bias, N, y, planes, n_whole, splits, stream);
   if (dtype == MFQ_BF16)
-    return launch_gemm_typed<BF16>(x, M, K, copy, bias, N, y, y_dtype, planes, n_whole, splits, stream, lr, epi);
-  if (dtype == MFQ_F16)
-    return launch_gemm_typed<F16>(x, M, K, copy, bias, N, y, y_dtype, planes, n_whole, splits, stream, lr, epi);
-  return MFQ_EDTYPE;
+    return launch_gemm_typed<BF16>(x, M, K, copy, bias, N, y, planes, n_whole, splits, stream, lr, epi);
+  return launch_gemm_typed<F16>(x, M, K, copy, bias, N, y, planes, n_whole, splits, stream, lr, epi);
 }
 
 namespace {
@@ -1138,5 +1156,6 @@ int launch_qmm_frag(const void* x, int dtype, int64_t M, int64_t K, const uint32
   float* planes = reinterpret_cast<float*>(static_cast<char*>(workspace) + qmm_frag_copy_bytes(N, K));
   return launch_qmm_frag_gemm(x, dtype, M, K, workspace, bias, N, y, y_dtype, planes, n_whole, splits, stream, lr, epi);
 }
+#endif  // MFQ_FRAG_F32
 
 }  // namespace mfq

@@ -246,6 +246,14 @@ def test_generated_code_of_the_assembly_matrix_kernels():
     assert _build.check_generated_code("qmm_frag.hip") == 18
 
 
+def test_generated_code_of_the_float32_matrix_kernels():
+    """The same check of the kernels that leave float32 results: two types x plain / cut
+    along K / 192-column tiles."""
+    from mflux_amd import _build
+
+    assert _build.check_generated_code("qmm_frag_f32.hip") == 6
+
+
 def test_generated_code_of_the_assembly_lds_loads():
     """The sliced GEMM's loads into LDS: every write of m0 has a wait state in front of
     the load that takes it (the two-kernel GEMM's are checked with its matrix
