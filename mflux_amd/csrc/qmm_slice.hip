@@ -5,7 +5,7 @@
 //
 // The 128-column-tile kernel (qmm_mid.hip) fills the chip on such shapes by cutting K into ranges, each with a float32
 // plane of the output that a second launch reads back.  Here a tile is small enough that there is one for every compute
-// unit with K whole -- 64 rows x 32, 48, 64 or 96 columns, 32 x 32 -- and K is cut over the four wavefronts of its workgroup,
+// unit with K whole -- 64 rows x 32, 48, 64, 80 or 96 columns, 32 x 32 -- and K is cut over the four wavefronts of its workgroup,
 // whose partial tiles meet in LDS at the end: no planes, no second launch.
 //   - Each wavefront has a ring of its own in LDS (40 KiB) that it fills with global_load_lds and reads back as matrix
 //     fragments: no barrier in the loop, no registers for what is on its way, and as no load in the loop is the compiler's
@@ -510,6 +510,13 @@ __global__ __launch_bounds__(kThreads, 1) void qmm_slice_kernel(
 // store; it grows with the tile) and `step` for every sub-step of a wavefront.  A cut of K over workgroups costs the launch of
 // the second kernel and its planes, 3.4 us and 1.3 bytes/ps.  (With one first cost for all tiles the wide tiles on short K
 // came out up to 40 % too low.)
+// 80 columns: the widest tile whose ring still holds three slots of x with two sub-steps of 4-bit codes (96 columns: one), or
+// with 8-bit codes (96: two slots of x).  Where 64 columns take a round more, or the 128-column kernel a cut: 170 drawn calls
+// of 17 to 512 rows, K whole, 0.70 to 1.02 of the time without it, 0.88 in the mean (48 rows x 3584 -> 37888 at 4 bits 44.0 us ->
+// 38.8, at 6 bits 21 rows 55.4 -> 42.0; 35 x 4096 -> 20480 at 8 bits 25.8 -> 24.3; 512 x 3072 -> 2560 at 4 bits 18.9 -> 17.0).
+// With K cut over workgroups 0.97 to 1.06 (6 bits 44 x 18944 -> 3584 in groups of 32 31.6 -> 33.1): such cuts keep the other
+// tiles.  At 3 bits 96 columns take no longer where they are no more rounds (17 x 4096 -> 20480 24.1, 25.0): its step is set
+// above theirs.
 struct Tile {
   int rows, columns;
   float first, step[5];  // us; the step at 3, 4, 5, 6, 8 bits
@@ -517,7 +524,7 @@ struct Tile {
 constexpr Tile kTiles[] = {
     {32, 32, 1.8f, {0.43f, 0.47f, 0.58f, 0.60f, 0.54f}}, {64, 32, 2.7f, {0.58f, 0.55f, 0.64f, 0.65f, 0.59f}},
     {64, 48, 3.9f, {0.74f, 0.67f, 0.80f, 0.81f, 0.70f}}, {64, 64, 4.8f, {0.91f, 0.74f, 0.97f, 0.96f, 0.83f}},
-    {64, 96, 6.9f, {1.22f, 1.01f, 1.33f, 1.50f, 1.05f}},
+    {64, 80, 5.9f, {1.33f, 0.87f, 1.15f, 1.10f, 0.94f}}, {64, 96, 6.9f, {1.22f, 1.01f, 1.33f, 1.50f, 1.05f}},
 };
 
 struct SlicePlan {
@@ -525,15 +532,16 @@ struct SlicePlan {
   float us = 0.f;
 };
 
-inline SlicePlan plan_slice(int64_t M, int64_t N, int64_t K, int bits, bool may_cut) {
+inline SlicePlan plan_slice(int64_t M, int64_t N, int64_t K, int bits, bool may_cut, bool with_80 = true) {
   const int64_t cus = compute_units();
   const int gran = bits == 3 || bits == 5 ? 2 : 1, grains = (int)(K / (64 * gran));
   const int width = bits == 3 ? 0 : bits == 4 ? 1 : bits == 5 ? 2 : bits == 6 ? 3 : 4;
   SlicePlan best;
   for (const Tile& t : kTiles) {
+    if (t.columns == 80 && !with_80) continue;
     if (t.rows == 32 && M > 128) continue;  // (every code is then dequantised for five row tiles and more)
     const int64_t tiles = ((M + t.rows - 1) / t.rows) * ((N + t.columns - 1) / t.columns);
-    for (int s = 1; s == 1 || (may_cut && s <= 8 && tiles * s <= cus && K / 64 / s >= 8); ++s) {
+    for (int s = 1; s == 1 || (may_cut && t.columns != 80 && s <= 8 && tiles * s <= cus && K / 64 / s >= 8); ++s) {
       const int64_t rounds = (tiles * s + cus - 1) / cus;
       const int subs = (grains + kWaves * s - 1) / (kWaves * s) * gran;
       float us = 3.1f + (float)rounds * (t.first + (float)subs * t.step[width]);
@@ -561,7 +569,9 @@ inline SlicePlan choose_slice(int64_t M, int64_t N, int64_t K, int gs, int bits,
   const int64_t gran = bits == 3 || bits == 5 ? 128 : 64;
   if (M > 1024 || N % 8 || K % gran || (K / gs) % 2 || M * K >= ((int64_t)1 << 31) - 2048 || N * K >= (int64_t)1 << 31) return SlicePlan();
   const SlicePlan plan = plan_slice(M, N, K, bits, may_cut);
-  return plan.us < 0.9f * others_us(M, N, K, gs, bits) ? plan : SlicePlan();
+  // (the 80 columns were measured against the other kernel in groups of 32 and 64: in groups of 128 they take no calls from it)
+  const float us = gs == 128 ? plan_slice(M, N, K, bits, may_cut, false).us : plan.us;
+  return us < 0.9f * others_us(M, N, K, gs, bits) ? plan : SlicePlan();
 }
 
 template <typename T, int BITS, int kA, int kB>
@@ -592,6 +602,7 @@ int launch_tile(SlicePlan plan, const void* x, int64_t M, int64_t K, const uint3
     case 32: return go(launch_kernel<T, BITS, 4, 2>);
     case 48: return go(launch_kernel<T, BITS, 4, 3>);
     case 64: return go(launch_kernel<T, BITS, 4, 4>);
+    case 80: return go(launch_kernel<T, BITS, 4, 5>);
     default: return go(launch_kernel<T, BITS, 4, 6>);
   }
 }

@@ -135,3 +135,25 @@ def test_update_and_swiglu_together():
     lin = mflux_amd.quantized_matmul(x, wq, s, b, group_size=64, bits=4, bias=bias, low_rank=(t, bs))
     want = core.swiglu_unstack(lin).double()
     assert bool(((y.double() - want).abs() <= 2.0 ** -6 * want.abs() + 1e-6).all())
+
+
+# whole and ragged last tiles of columns and rows; K: a wavefront's sub-steps fewer than the ring holds, and more
+@pytest.mark.parametrize("M,K,N,bits,gs,dtype", [
+    (449, 1280, 2552, 4, 64, "bf16"), (449, 1280, 2552, 8, 64, "f16"), (449, 1280, 2552, 6, 32, "bf16"), (449, 1280, 2560, 5, 64, "f16"),
+    (300, 1024, 4072, 3, 64, "bf16"), (33, 2560, 19448, 4, 32, "f16"), (64, 2560, 19456, 8, 64, "bf16")])
+def test_tiles_of_80_columns(M, K, N, bits, gs, dtype):
+    import mflux_amd
+    from mflux_amd import core
+
+    dtype = DT[dtype]
+    x, packed, bias, ref = _operands(M, K, N, bits, gs, dtype)
+    y = mflux_amd.quantized_matmul(x, *packed, group_size=gs, bits=bits, bias=bias)
+    _close(y, ref + bias.double(), dtype, 2)
+    _close(mflux_amd.quantized_matmul(x.float(), *packed, group_size=gs, bits=bits), ref, dtype, 0)
+    t, bs = torch.randn(M, 48, device="cuda").to(dtype), (torch.randn(N, 48, device="cuda") * 0.02).to(dtype)
+    y_lr = mflux_amd.quantized_matmul(x, *packed, group_size=gs, bits=bits, bias=bias, low_rank=(t, bs))
+    _close(y_lr, ref + bias.double() + t.double() @ bs.double().t(), dtype, 2)
+    if N % 64 == 0:  # half of a tile's columns the gate's, half the up projection's
+        z = core.quantized_matmul_epilogue(x, *packed, epilogue="swiglu", group_size=gs, bits=bits, bias=bias)
+        want = core.swiglu_unstack(y).double()
+        assert bool(((z.double() - want).abs() <= 2.0 ** -6 * want.abs() + 1e-6).all())
