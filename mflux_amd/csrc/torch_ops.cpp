@@ -300,7 +300,8 @@ void check_fragments(const char* fn, const Tensor& t, int64_t steps, const Tenso
               fn, ": expected fragments [R/16, ", steps, ", 4, 16, 8] of ", like.scalar_type(), " on ", like.device());
 }
 
-// lora_A [K, rank], lora_B [rank, N] -> their fragments, scale lora_B^T [N, R] and lora_A [K, R]
+// lora_A [K, rank], lora_B [rank, N] -> their fragments, scale lora_B^T [N, R] and lora_A [K, R]: new tensors all, also at the
+// ranks where lora_A needs no padding, so that backward sees the factors that forward saw, whatever is written to them between
 std::tuple<Tensor, Tensor, Tensor, Tensor> low_rank_pack(const Tensor& a, const Tensor& b, double scale) {
   TORCH_CHECK(a.dim() == 2 && b.dim() == 2, "mfq::low_rank_pack: lora_A [K, rank], lora_B [rank, N]");
   const int64_t K = a.size(0), rank = a.size(1), N = b.size(1), R = training_rank(rank);
@@ -308,12 +309,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> low_rank_pack(const Tensor& a, const 
   check_factor("mfq::low_rank_pack", b, rank, N, a);
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(a.device());
   Tensor af = at::empty({R / 16, K / 32, 4, 16, 8}, a.options()), bf = at::empty({R / 16, N / 32, 4, 16, 8}, a.options());
-  Tensor bs = at::empty({N, R}, a.options());
-  const bool as_it_is = rank == R && reinterpret_cast<uintptr_t>(a.data_ptr()) % 16 == 0;
-  Tensor ap = as_it_is ? a.detach() : at::empty({K, R}, a.options());
+  Tensor bs = at::empty({N, R}, a.options()), ap = at::empty({K, R}, a.options());
   check_status("mfq_low_rank_pack",
                mfq_low_rank_pack(a.data_ptr(), b.data_ptr(), dtype_code(a.scalar_type(), "lora_A"), K, N, rank, R, (float)scale,
-                                 af.data_ptr(), bf.data_ptr(), bs.data_ptr(), as_it_is ? nullptr : ap.data_ptr(), stream_of(a)));
+                                 af.data_ptr(), bf.data_ptr(), bs.data_ptr(), ap.data_ptr(), stream_of(a)));
   return {af, bf, bs, ap};
 }
 

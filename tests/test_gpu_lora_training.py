@@ -94,3 +94,25 @@ def test_gradients_that_are_not_wanted_or_not_contiguous():
     y = layer(frozen)
     for a, b in zip(torch.autograd.grad(y, inputs[1:], row.expand(2, 24, 320)), want[1:]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("rank", [6, 16, 32])
+def test_packed_factors_are_copies(rank):
+    """No output of the packing is a view of a factor, padded or not, so backward's input gradient is that of the factors
+    that forward saw, also when one is written to behind autograd's back before it."""
+    from mflux_amd import _lib, lora, nn
+
+    torch.manual_seed(98)
+    a, b = torch.randn(64, rank, device="cuda").bfloat16(), torch.randn(rank, 96, device="cuda").bfloat16()
+    storages = {t.untyped_storage().data_ptr() for t in (a, b)}
+    for t in _lib.ops().low_rank_pack(a, b, 1.0):
+        assert t.untyped_storage().data_ptr() not in storages
+    lin = torch.nn.Linear(256, 320, device="cuda", dtype=torch.bfloat16)
+    layer = lora.LoRALinear.from_linear(nn.QuantizedLinear.from_linear(lin, 64, 4), r=rank, scale=1.0)
+    layer.lora_B.data.normal_(std=0.5)
+    x, g = torch.randn(40, 256, device="cuda").bfloat16().requires_grad_(True), torch.randn(40, 320, device="cuda").bfloat16()
+    want, = torch.autograd.grad(layer(x), x, g)
+    y = layer(x)
+    layer.lora_A.data.zero_()
+    layer.lora_B.data.zero_()
+    assert torch.equal(torch.autograd.grad(y, x, g)[0], want)
