@@ -463,7 +463,8 @@ __global__ __launch_bounds__(256) void low_rank_pack_kernel(const uint16_t* __re
   for (int e = 0; e < 8; ++e) v[e] = at[e] < 0 ? (uint16_t)0 : src[at[e]];
   if (factor != 1.f) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = T::from_f32(T::to_f32(v[e]) * factor);
+    for (int e = 0; e < 8; ++e)
+      if (at[e] >= 0) v[e] = T::from_f32(T::to_f32(v[e]) * factor);  // (zero times an infinite scale is no zero)
   }
   u32x4 o;
 #pragma unroll

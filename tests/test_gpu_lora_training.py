@@ -116,3 +116,24 @@ def test_packed_factors_are_copies(rank):
     layer.lora_A.data.zero_()
     layer.lora_B.data.zero_()
     assert torch.equal(torch.autograd.grad(y, x, g)[0], want)
+
+
+@pytest.mark.parametrize("scale", [float("inf"), float("nan"), -3.0])
+def test_a_scale_reaches_the_factor_alone(scale):
+    """The columns a rank is padded by stay zero under any scale; with an infinite one they would make NaN of every output,
+    where the composition has infinities."""
+    from mflux_amd import _lib, lora, nn
+
+    torch.manual_seed(99)
+    a, b = torch.randn(64, 6, device="cuda").bfloat16(), torch.randn(6, 96, device="cuda").bfloat16()
+    bs = _lib.ops().low_rank_pack(a, b, scale)[2]
+    want = torch.nn.functional.pad((scale * b.float()).bfloat16().t(), (0, 10))
+    assert torch.equal(bs.view(torch.int16)[:, 6:], torch.zeros_like(bs.view(torch.int16)[:, 6:]))
+    assert torch.equal(torch.nan_to_num(bs), torch.nan_to_num(want))
+    lin = torch.nn.Linear(256, 320, device="cuda", dtype=torch.bfloat16)
+    layer = lora.LoRALinear.from_linear(nn.QuantizedLinear.from_linear(lin, 64, 4), r=6, scale=scale)
+    layer.lora_A.data.abs_()
+    layer.lora_B.data.normal_(std=0.02).abs_()
+    x = torch.randn(50, 256, device="cuda").abs().bfloat16().requires_grad_(True)
+    got, want = layer(x), lora._composed(layer.linear, [layer], x)
+    assert torch.equal(torch.isfinite(got), torch.isfinite(want)) and torch.equal(torch.isnan(got), torch.isnan(want))
