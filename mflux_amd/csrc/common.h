@@ -472,7 +472,7 @@ int launch_qmm_frag_gemm_f32(const void* x, int dtype, int64_t M, int64_t K, con
 size_t qmm_prepared_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int launch_qmm_prepared(const void* x, int dtype, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N,
                         void* y, void* workspace, size_t workspace_bytes, hipStream_t stream);
-// y tiles = sums of the planes of a K cut (+ bias, epilogue): the second kernel of qmm.hip's and qmm_frag.hip's cut
+// y tiles = sums of the planes of a K cut, at least two (+ bias, epilogue): the second kernel of qmm.hip's and qmm_frag.hip's cut
 int launch_tail_reduce(int dtype, const float* planes, int n_whole, int splits, int tiles_m, int tiles_n,
                        const void* bias, int64_t M, int64_t N, void* y, int y_dtype, hipStream_t stream, Epilogue epi);
 // the 128-column-tile kernel for a few hundred activation rows, and for any M when K % 64 == 32
@@ -514,7 +514,7 @@ int launch_qmm_n(const void* x, int dtype, int64_t M, int64_t N, const uint32_t*
 // [M / rows_per_vector, K] or both nullptr
 int launch_layer_norm_modulate(const void* x, int dtype, int64_t M, int64_t K, const void* scale, const void* shift,
                                int64_t rows_per_vector, float eps, void* y, hipStream_t stream);
-// y = sum of `splits` float32 planes of M x N (+ bias), rounded to y's type; dtype is the type of bias and 16-bit y
+// y = sum of `splits` (at least two) float32 planes of M x N (+ bias), rounded to y's type; dtype is the type of bias and 16-bit y
 int launch_splitk_reduce(int dtype, const void* planes, int splits, int64_t M, int64_t N, const void* bias, void* y,
                          int y_dtype, hipStream_t stream, Epilogue epi = Epilogue());
 

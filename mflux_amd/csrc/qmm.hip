@@ -859,8 +859,9 @@ inline TailPlan plan_tail(int64_t M, int64_t N, int64_t K, int period, int cus) 
 
 inline int period_of(int gs) { return 4 * gs / BK; }
 
-// The sum of `splits` planes at one place, first to last.  All of a sum's loads are on their way before the first is waited
-// for: as a loop over a count known at run time they went one after another, each with the memory's whole latency.
+// The sum of `splits` planes at one place, first to last, splits >= 2.  The loads of up to seven planes are on their way
+// together: as a loop over a count known at run time they went one after another, each with the memory's whole latency, as those
+// of the eighth plane and the ones behind it still do.
 template <int S>
 __device__ inline float4 sum_of_planes(const float* p, size_t stride) {
   float4 v[S];
@@ -1239,6 +1240,7 @@ QmmRoute qmm_route(int64_t M, int64_t N, int64_t K, int gs, int bits) {
 
 int launch_tail_reduce(int dtype, const float* planes, int n_whole, int splits, int tiles_m, int tiles_n,
                        const void* bias, int64_t M, int64_t N, void* y, int y_dtype, hipStream_t stream, Epilogue epi) {
+  if (splits < 2) return MFQ_ESHAPE;  // (sum_of_planes)
   const unsigned blocks = (unsigned)(tiles_m * tiles_n - n_whole) * (BM * BN / 4 / 256);
   if (dtype == MFQ_BF16) {
     hipLaunchKernelGGL((tail_reduce_kernel<BF16>), dim3(blocks), dim3(256), 0, stream, planes, n_whole, splits, tiles_m,
@@ -1254,6 +1256,7 @@ int launch_tail_reduce(int dtype, const float* planes, int n_whole, int splits, 
 
 int launch_splitk_reduce(int dtype, const void* planes, int splits, int64_t M, int64_t N, const void* bias, void* y,
                          int y_dtype, hipStream_t stream, Epilogue epi) {
+  if (splits < 2) return MFQ_ESHAPE;  // (sum_of_planes)
   const int64_t plane = M * N;
   const int64_t threads = (N & 3) == 0 ? plane / 4 : plane;
   const int64_t blocks = (threads + 255) / 256;

@@ -231,6 +231,24 @@ def test_abi_validation_clean_under_host_sanitizers():
     assert "every refusal clean" in _build.sanitize_abi()
 
 
+def test_sums_of_planes_refuse_fewer_than_two():
+    """The two kernels that add up the planes of a K cut read at least two of them: a call with one is refused before it is
+    launched.  (No C function reaches them with one; the launchers are called themselves.)"""
+    from mflux_amd import _lib
+
+    class Epilogue(ctypes.Structure):
+        _fields_ = [("kind", ctypes.c_int), ("gate", ctypes.c_void_p), ("residual", ctypes.c_void_p), ("act_from", ctypes.c_int)]
+
+    ptr, i64, i32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
+    dense = getattr(_lib.load(), "_ZN3mfq20launch_splitk_reduceEiPKvillS1_PviP12ihipStream_tNS_8EpilogueE")
+    dense.restype, dense.argtypes = i32, [i32, ptr, i32, i64, i64, ptr, ptr, i32, ptr, Epilogue]
+    tiles = getattr(_lib.load(), "_ZN3mfq18launch_tail_reduceEiPKfiiiiPKvllPviP12ihipStream_tNS_8EpilogueE")
+    tiles.restype, tiles.argtypes = i32, [i32, ptr, i32, i32, i32, i32, ptr, i64, i64, ptr, i32, ptr, Epilogue]
+    for splits in (1, 0, -1):
+        assert dense(_lib.BF16, 256, splits, 64, 64, None, 256, _lib.BF16, None, Epilogue()) == -4
+        assert tiles(_lib.BF16, 256, 0, splits, 1, 1, None, 64, 64, 256, _lib.BF16, None, Epilogue()) == -4
+
+
 def test_generated_code_of_the_assembly_matrix_kernels():
     """The two-kernel GEMM states its matrix instruction as assembly (result tied
     to the addend), which hides it from the compiler's hazard recognizer; the
