@@ -226,7 +226,7 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     if transpose and low_rank is None and mode == "affine":
         native = _lib.native()
         y = native.linear(x, w, scales, biases, bias, group_size, bits)
-        if y is None:
+        if y is None and getattr(x, "dtype", None) is torch.float32:
             y = native.linear_float32(x, w, scales, biases, bias, group_size, bits)
         if y is not None:
             return y

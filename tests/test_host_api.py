@@ -66,6 +66,26 @@ def test_argument_errors_without_the_built_libraries(monkeypatch):
         mflux_amd.quantized_matmul(x, wq, s, s)
 
 
+def test_the_native_call_of_float32_activations_is_tried_on_those_alone(monkeypatch):
+    """Operands of another type that the native call leaves are looked over once, not twice, on their way to the general route."""
+    from mflux_amd import _lib
+
+    tried = []
+
+    class Native:
+        linear = staticmethod(lambda *args: tried.append("16 bit"))
+        linear_float32 = staticmethod(lambda *args: tried.append("float32"))
+
+    monkeypatch.setattr(_lib, "native", lambda: Native)
+    wq = torch.zeros(8, 16, dtype=torch.uint32)
+    s = torch.zeros(8, 2, dtype=torch.bfloat16)
+    for dtype, want in ((torch.bfloat16, ["16 bit"]), (torch.float64, ["16 bit"]), (torch.float32, ["16 bit", "float32"])):
+        tried.clear()
+        with pytest.raises(RuntimeError, match="no CPU fallback"):
+            mflux_amd.quantized_matmul(torch.zeros(2, 128, dtype=dtype), wq, s, s)
+        assert tried == want
+
+
 def test_quantized_matmul_shape_errors():
     wq = torch.zeros(8, 16, dtype=torch.uint32)
     s = torch.zeros(8, 2, dtype=torch.bfloat16)
