@@ -79,7 +79,7 @@ def test_the_native_call_of_float32_activations_is_tried_on_those_alone(monkeypa
     monkeypatch.setattr(_lib, "native", lambda: Native)
     wq = torch.zeros(8, 16, dtype=torch.uint32)
     s = torch.zeros(8, 2, dtype=torch.bfloat16)
-    for dtype, want in ((torch.bfloat16, ["16 bit"]), (torch.float64, ["16 bit"]), (torch.float32, ["16 bit", "float32"])):
+    for dtype, want in ((torch.bfloat16, ["16 bit"]), (torch.float16, ["16 bit"]), (torch.float32, ["16 bit", "float32"])):
         tried.clear()
         with pytest.raises(RuntimeError, match="no CPU fallback"):
             mflux_amd.quantized_matmul(torch.zeros(2, 128, dtype=dtype), wq, s, s)
