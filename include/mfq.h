@@ -271,7 +271,7 @@ int mfq_qmm_n_low_rank(const void* x, int x_dtype, int64_t M, int64_t N, const u
  * The copy's values are the ones the fused kernels use (one rounding of
  * fma(code, scale, bias)); the float32 sums run in another order.
  * mfq_qmm_t_workspace_bytes() returns the size this shape would use on the
- * current device (0: no use for one, pass NULL): K is cut only where that is
+ * current device, whatever the kind of call (0: no use for one, pass NULL): K is cut only where that is
  * estimated to be the faster, most shapes up to 512 rows run on tiles small
  * enough without.  A NULL or smaller workspace
  * is not an error: without room for the copy the call runs as mfq_qmm_t does
@@ -292,6 +292,12 @@ size_t mfq_qmm_t_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size
  * tiles for the 256 x 256 tiles (calls without an epilogue may run whole tiles
  * of 192 columns instead of that cut).  For tests and measurements.  Has no
  * counterpart in the reference.
+ *
+ * mfq_qmm_t_plan answers the same for one kind of call -- `epilogue` 0:
+ * mfq_qmm_t_ws and mfq_qmm_t_low_rank, MFQ_EPILOGUE_*: mfq_qmm_t_epilogue, which
+ * has rules of its own about the copy of the weights -- with the workspace that
+ * kind uses, *workspace_bytes (may be NULL), where mfq_qmm_t_workspace_bytes()
+ * is enough for every kind.
  */
 enum mfq_kernel {
   MFQ_KERNEL_MATVEC = 1,      /* the kernels for up to 16 rows (3, 5, 6 bits: one) */
@@ -302,6 +308,8 @@ enum mfq_kernel {
   MFQ_KERNEL_TWO_KERNELS = 6  /* 256 x 256 (or 192) tiles on a 16-bit copy of the weight */
 };
 int mfq_qmm_t_kernel(int64_t M, int64_t K, int64_t N, int group_size, int bits, int* k_ranges);
+int mfq_qmm_t_plan(int64_t M, int64_t K, int64_t N, int group_size, int bits, int epilogue, int* k_ranges,
+                   size_t* workspace_bytes);
 int mfq_qmm_t_ws(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq,
                  const void* scales, const void* biases, int sb_dtype, const void* bias, int64_t N,
                  int group_size, int bits, void* y, int y_dtype, void* workspace,

@@ -110,6 +110,23 @@ size_t mfq_qmm_t_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size
   return route.copy + route.planes;
 }
 
+int mfq_qmm_t_plan(int64_t M, int64_t K, int64_t N, int group_size, int bits, int epilogue, int* k_ranges,
+                   size_t* workspace_bytes) {
+  if (workspace_bytes) *workspace_bytes = 0;
+  if (epilogue < 0 || epilogue > MFQ_EPILOGUE_SWIGLU) return MFQ_ESHAPE;
+  int ranges = 1;
+  const int kernel = mfq_qmm_t_kernel(M, K, N, group_size, bits, &ranges);
+  if (kernel < 0) return kernel;
+  if (epilogue && (M <= 16 || N % 8)) return MFQ_EUNSUPPORTED;
+  if (epilogue == MFQ_EPILOGUE_SWIGLU && N % 64) return MFQ_ESHAPE;
+  mfq::QmmRoute route{kernel, ranges, 0, 0};
+  if (kernel != MFQ_KERNEL_MATVEC)
+    route = epilogue ? mfq::qmm_epilogue_route(M, N, K, group_size, bits) : mfq::qmm_route(M, N, K, group_size, bits);
+  if (k_ranges) *k_ranges = route.ranges;
+  if (workspace_bytes) *workspace_bytes = route.copy + route.planes;
+  return route.kernel;
+}
+
 int mfq_qmm_t(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
               const void* biases, int sb_dtype, const void* bias, int64_t N, int group_size, int bits, void* y,
               int y_dtype, void* stream) {

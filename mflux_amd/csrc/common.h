@@ -433,6 +433,8 @@ struct QmmRoute {
   size_t planes;  // and of a K cut's float32 planes behind it
 };
 QmmRoute qmm_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
+// the same of a call with an epilogue
+QmmRoute qmm_epilogue_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
 // the two-kernel path (qmm_frag.hip): dequantize once into a 16-bit copy in fragment order, then a GEMM on
 // 16x16x32 matrix instructions; 4 and 8 bits, 16-bit y of x's type, a low-rank update or an epilogue as
 // launch_qmm / launch_qmm_epilogue.
@@ -440,7 +442,8 @@ QmmRoute qmm_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
 // K cut (n_whole whole tiles, the others in `splits` ranges of whole pairs of k steps; splits == 1: no cut)
 bool qmm_frag_shape_ok(int64_t M, int64_t N, int64_t K, int bits);
 bool qmm_frag_narrow_rounds(int64_t M, int64_t N, int64_t K, int splits);  // 192-column tiles in several rounds
-bool prefer_frag_path(int64_t M, int64_t N, int64_t K, int gs, int bits);  // where the two-kernel path is the faster
+// where the two-kernel path is the faster
+bool prefer_frag_path(int64_t M, int64_t N, int64_t K, int gs, int bits, bool epilogue = false);
 size_t qmm_frag_copy_bytes(int64_t N, int64_t K);
 int launch_qmm_frag(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,
                     const void* biases, const void* bias, int64_t N, int gs, int bits, void* y, int y_dtype, void* workspace,

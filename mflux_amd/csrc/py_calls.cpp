@@ -232,7 +232,8 @@ PyObject* epilogue_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   RECORD_FUNCTION("mfq::qmm_t_epilogue", p.inputs());
   const c10::hip::HIPGuardMasqueradingAsCUDA on_device(p.x.device());
   Tensor y = p.out(epilogue == MFQ_EPILOGUE_SWIGLU ? p.N / 2 : p.N), ws;
-  const size_t ws_bytes = mfq_qmm_t_workspace_bytes(p.M, p.K, p.N, (int)p.gs, (int)p.bits);
+  size_t ws_bytes = 0;
+  mfq_qmm_t_plan(p.M, p.K, p.N, (int)p.gs, (int)p.bits, (int)epilogue, nullptr, &ws_bytes);
   if (ws_bytes) ws = p.workspace(ws_bytes);
   const Linear::Pointers in = p.pointers();
   void *y_p = y.data_ptr(), *ws_p = ws_bytes ? ws.data_ptr() : nullptr;

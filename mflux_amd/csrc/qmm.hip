@@ -1196,28 +1196,36 @@ float qmm_others_estimate_us(int64_t M, int64_t N, int64_t K, int gs, int bits) 
 constexpr int64_t kOddBitsFragRows = MFQ_ODD_FRAG_ROWS;
 
 // The two-kernel path (qmm_frag.hip: a 16-bit scratch copy of the weights in fragment order, then a lean
-// GEMM) takes the shapes it wins on: at least eight rows of tiles to spread the copy over.  It cuts K for
+// GEMM) takes the shapes it wins on: enough rows of tiles to spread the copy over.  It cuts K for
 // the tail of the tile sequence by the same plan as the fused kernel, or takes narrower tiles there.
-// 4 and 8 bits, 35 drawn shapes of 1793 to 2047 rows (all group sizes, float32 results, low-rank updates): 0.60 to 1.01 of the
-// fused kernel's time (1985 x 2560 -> 9216 107 us -> 102, 1951 x 15360 -> 4304 303 -> 248).  With seven rows of tiles and six the
-// two are level by themselves, and between other kernels the copy's traffic costs more (a training step at 1536 x 3072 -> 12288
-// 283 us, 293 with the copy), except (1281 rows and more) where the narrower tiles take two or three rounds in the place of a
-// short last one (1661 x 2560 -> 12288 137 us -> 112, 1616 x 3072 -> 12288 131 -> 119), and where K is not whole scale periods and
-// the fused kernel reads its scales step by step (1493 x 3840 -> 12288 in groups of 128 236 us -> 148, 1401 x 1152 -> 12288 74 ->
-// 59; 1055 rows 42 -> 47).
-// Below 2048 rows a last round of up to eight tiles, cut, stays with the fused kernel, though it takes 2 to 9 % more there (2040 x
-// 3072 -> 8448 115 us, 106 here): mfq_qmm_t_static holds the planes of such a cut and no copy, and gives mfq_qmm_t_ws's bits.
-bool prefer_frag_path(int64_t M, int64_t N, int64_t K, int gs, int bits) {
+// 4 and 8 bits, eight rows of tiles (1793 to 2047 rows): of 35 drawn shapes (all group sizes, float32 results, low-rank updates)
+// 0.60 to 1.01 of the fused kernel's time (1985 x 2560 -> 9216 107 us -> 102, 1951 x 15360 -> 4304 303 -> 248), with an epilogue
+// 0.91 to 0.98 by itself and 0.94 to 0.97 between other kernels (Z-Image's feed-forward, 1850 rows at 8 bits 486 us -> 456; a
+// single-stream block of 2000 rows at 4 489 -> 463).  With seven rows of tiles and six the two are level by themselves, and
+// between other kernels the copy's traffic costs more (a training step at 1536 x 3072 -> 12288 283 us, 293 with the copy), except
+// from 1281 rows on
+//   - where the narrower tiles take two or three rounds in the place of a short last one (1661 x 2560 -> 12288 137 us -> 112,
+//     1616 x 3072 -> 12288 131 -> 119).  Calls with an epilogue do not run those: 3840 -> 20480 with SwiGLU, whose 560 tiles leave
+//     such a round, is 0.94 to 0.98 of the fused kernel's time by itself and makes the feed-forward it stands in 1.02 to 1.034
+//     times as long (1664 rows 407 us -> 421);
+//   - where K is not whole scale periods and the fused kernel reads its scales step by step (1493 x 3840 -> 12288 in groups of
+//     128 236 us -> 148, 1401 x 1152 -> 12288 74 -> 59; 1055 rows 42 -> 47; GELU on 1281 to 1792 x 3840 -> 15360 0.68 to 0.73).
+// Below 2048 rows a last round of up to eight tiles, cut, stays with the fused kernel.  Where those are all there are (up to 256
+// columns) it is level or ahead: 1920 rows x 9728 -> 64 in groups of 64 31 us on either at 4 bits, 31 against 32 at 8, in groups
+// of 128 29 against 32, 15360 -> 64 36 against 41.  Behind whole rounds it takes 0 to 9 % more (2040 x 3072 -> 8448 115 us against
+// 106, 6144 -> 8448 194 against 190, 768 -> 8448 49 on either); what stays the same there is that mfq_qmm_t_static, whose buffer
+// holds the planes of up to sixteen ranges of them and seldom the copy, gives mfq_qmm_t_ws's bits.
+bool prefer_frag_path(int64_t M, int64_t N, int64_t K, int gs, int bits, bool epilogue) {
   if (!qmm_frag_shape_ok(M, N, K, bits) || use_mid_kernel(M, N, K)) return false;
   // (3, 5 and 6 bits: the alternative is the 128-column-tile kernel with its codes cut out of a bit stream,
-  // which the copy overtakes much earlier)
-  if (bits != 4 && bits != 8) return M >= kOddBitsFragRows;
+  // which the copy overtakes much earlier; that kernel has the epilogues)
+  if (bits != 4 && bits != 8) return M >= kOddBitsFragRows && !epilogue;
   if (M >= 8 * BM) return true;
   if (M <= 5 * BM) return false;
   const int64_t cus = compute_units(), rest = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) % cus;
   const int splits = plan_tail(M, N, K, period_of(gs), (int)cus).splits;
   if (splits > 1 && rest <= 8) return false;
-  return M > 7 * BM || K / BK % period_of(gs) || qmm_frag_narrow_rounds(M, N, K, splits);
+  return M > 7 * BM || K / BK % period_of(gs) || (!epilogue && qmm_frag_narrow_rounds(M, N, K, splits));
 }
 
 // In the order of launch_qmm() and launch_qmm_mid_stream().  What sends a call past the wide or the sliced kernel, scales or
@@ -1236,6 +1244,21 @@ QmmRoute qmm_route(int64_t M, int64_t N, int64_t K, int gs, int bits) {
   const TailPlan plan = plan_tail(M, N, K, period_of(gs), compute_units());
   return QmmRoute{two_kernels ? MFQ_KERNEL_TWO_KERNELS : MFQ_KERNEL_TILES_256, plan.splits,
                   two_kernels ? qmm_frag_copy_bytes(N, K) : 0, tail_plane_bytes(M, N, plan)};
+}
+
+QmmRoute qmm_epilogue_route(int64_t M, int64_t N, int64_t K, int gs, int bits) {
+  QmmRoute route = qmm_route(M, N, K, gs, bits);
+  if (route.kernel != MFQ_KERNEL_TWO_KERNELS || prefer_frag_path(M, N, K, gs, bits, true)) return route;
+  if (bits == 4 || bits == 8) {  // the same cut on the fused kernel
+    route.kernel = MFQ_KERNEL_TILES_256;
+    route.copy = 0;
+    return route;
+  }
+  // 3, 5 and 6 bits: a cut as far as the workspace of a call without an epilogue has room for its planes
+  const int ranges = qmm_mid_ranges(M, N, K, gs);
+  const size_t planes = (size_t)ranges * M * N * sizeof(float);
+  const bool cut = ranges > 1 && planes <= route.copy + route.planes;
+  return QmmRoute{MFQ_KERNEL_TILES_128, cut ? ranges : 1, 0, cut ? planes : 0};
 }
 
 int launch_tail_reduce(int dtype, const float* planes, int n_whole, int splits, int tiles_m, int tiles_n,
@@ -1338,7 +1361,8 @@ int launch_qmm(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* w
   // the two-kernel path where it wins and the caller has brought room for the scratch copy (and, behind it, for
   // the planes of the K cut: without those the tiles run whole)
   if ((y_dtype == dtype || (!low_rank.R && epi.kind == kEpiNone)) && workspace && aligned16(workspace) &&
-      !(low_rank.R && epi.kind != kEpiNone) && workspace_bytes >= qmm_frag_copy_bytes(N, K) && prefer_frag_path(M, N, K, gs, bits)) {
+      !(low_rank.R && epi.kind != kEpiNone) && workspace_bytes >= qmm_frag_copy_bytes(N, K) &&
+      prefer_frag_path(M, N, K, gs, bits, epi.kind != kEpiNone)) {
     const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     TailPlan plan = plan_tail(M, N, K, period_of(gs), compute_units());
     if (plan.splits > 1 && workspace_bytes < qmm_frag_copy_bytes(N, K) + tail_plane_bytes(M, N, plan))

@@ -176,7 +176,8 @@ std::tuple<Tensor, bool> qmm_t_epilogue(const Tensor& x, const Tensor& wq, const
   const int64_t n_out = epilogue == MFQ_EPILOGUE_SWIGLU ? m.N / 2 : m.N;
   Tensor y = at::empty({m.M, n_out}, x.options());
   if (m.M == 0) return {y, true};
-  const size_t ws_bytes = mfq_qmm_t_workspace_bytes(m.M, m.K, m.N, (int)group_size, (int)bits);
+  size_t ws_bytes = 0;
+  mfq_qmm_t_plan(m.M, m.K, m.N, (int)group_size, (int)bits, (int)epilogue, nullptr, &ws_bytes);
   Tensor ws;
   if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
   const int rc = mfq_qmm_t_epilogue(x.data_ptr(), m.sb, m.M, m.K, static_cast<const uint32_t*>(wq.data_ptr()),

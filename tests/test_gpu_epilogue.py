@@ -197,3 +197,53 @@ def test_epilogue_module_helpers_and_composed_paths(oracle):
         mflux_amd.quantized_matmul_epilogue(x32, q1.weight, q1.scales, q1.biases, epilogue="relu", bits=8)
     with pytest.raises(ValueError, match="needs gate and residual"):
         mflux_amd.quantized_matmul_epilogue(x32, q1.weight, q1.scales, q1.biases, epilogue="gate_residual", bits=8)
+
+
+# seven rows of tiles whose plain calls take 192-column tiles (with an epilogue the fused kernel, whole and cut), eight rows, K not
+# whole scale periods
+@pytest.mark.parametrize("M,K,N,bits,gs,copies", [(1600, 1024, 10304, 4, 64, False), (1792, 768, 13312, 8, 64, False),
+                                                  (1540, 3840, 20480, 4, 64, False), (1900, 1024, 5120, 4, 64, True),
+                                                  (1300, 768, 13312, 4, 128, True)])
+def test_below_2048_rows_the_copy_is_made_where_it_pays_with_the_epilogue(M, K, N, bits, gs, copies):
+    """The call runs the kernel that mfq_qmm_t_plan names (the same bits as with that kernel's workspace and no more), and the
+    values are the separate operations', on float64 sums: three roundings to bfloat16 (SwiGLU four) and float32 sums."""
+    import ctypes
+
+    import mflux_amd
+    from gpu_util import kernel_of
+    from mflux_amd import _lib, core
+
+    lib = _lib.load()
+    assert kernel_of(M, K, N, bits, gs)[0] == _lib.KERNEL_TWO_KERNELS
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    packed = mflux_amd.quantize((torch.randn(N, K, generator=gen, device="cuda") * 0.05).bfloat16(), gs, bits)
+    bias, gate = (torch.randn(N, generator=gen, device="cuda").bfloat16() for _ in range(2))
+    residual = torch.randn(M, N, generator=gen, device="cuda").bfloat16()
+    lin = x.double() @ mflux_amd.dequantize(*packed, gs, bits, dtype=torch.float32).bfloat16().double().t() + bias.double()
+    g, u = lin.reshape(M, -1, 2, 32).unbind(2)
+    want = {"gelu": torch.nn.functional.gelu(lin, approximate="tanh"), "gate_residual": residual.double() + gate.double() * lin,
+            "swiglu": (torch.nn.functional.silu(g) * u).reshape(M, -1)}
+    for name, ref in want.items():
+        epilogue = core.EPILOGUES[name]
+        y = core.quantized_matmul_epilogue(x, *packed, epilogue=name, group_size=gs, bits=bits, bias=bias,
+                                           gate=gate if name == "gate_residual" else None,
+                                           residual=residual if name == "gate_residual" else None)
+        largest = ref.abs().amax(dim=1, keepdim=True)
+        assert bool(((y.double() - ref).abs() <= (4 * ULP + 2.0 ** -12) * largest).all())
+        need = ctypes.c_size_t()
+        kernel = lib.mfq_qmm_t_plan(M, K, N, gs, bits, epilogue, None, ctypes.byref(need))
+        assert kernel == (_lib.KERNEL_TWO_KERNELS if copies else _lib.KERNEL_TILES_256)
+        ws = torch.empty(max(need.value, 16), dtype=torch.uint8, device="cuda")
+        y_c = torch.full_like(y, float("nan"))
+        assert lib.mfq_qmm_t_epilogue(x.data_ptr(), _lib.BF16, M, K, *(t.data_ptr() for t in packed), _lib.BF16, bias.data_ptr(), N, gs,
+                                      bits, epilogue, gate.data_ptr(), residual.data_ptr(), 0, y_c.data_ptr(), _lib.BF16,
+                                      ws.data_ptr(), need.value, torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(y, y_c)
+        # room for a copy that the rule does not make changes nothing
+        more = torch.empty(lib.mfq_qmm_t_workspace_bytes(M, K, N, gs, bits), dtype=torch.uint8, device="cuda")
+        y_m = torch.full_like(y, float("nan"))
+        assert lib.mfq_qmm_t_epilogue(x.data_ptr(), _lib.BF16, M, K, *(t.data_ptr() for t in packed), _lib.BF16, bias.data_ptr(), N, gs,
+                                      bits, epilogue, gate.data_ptr(), residual.data_ptr(), 0, y_m.data_ptr(), _lib.BF16,
+                                      more.data_ptr(), more.numel(), torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(y, y_m)

@@ -93,3 +93,57 @@ def test_the_sliced_kernel_is_kept_where_it_is_the_faster(M, K, N, bits, gs):
 ])
 def test_where_the_wide_kernel_is_taken(M, K, N, bits, gs, wide):
     assert (route(M, K, N, bits, gs)[0] == _lib.KERNEL_WIDE) == wide
+
+
+def plan(M, K, N, bits, gs, epilogue):
+    ranges, need = ctypes.c_int(), ctypes.c_size_t()
+    kernel = _lib.load().mfq_qmm_t_plan(M, K, N, gs, bits, epilogue, ctypes.byref(ranges), ctypes.byref(need))
+    return kernel, ranges.value, need.value
+
+
+# measured on 256 units between a block's other kernels, us with the copy of the weights and without
+@pytest.mark.parametrize("M,K,N,bits,gs,kernel", [
+    (1600, 3840, 20480, 4, 64, _lib.KERNEL_TILES_256),     # 419, 407
+    (1792, 3840, 20480, 8, 64, _lib.KERNEL_TILES_256),     # 444, 434
+    (1600, 3072, 12288, 4, 64, _lib.KERNEL_TILES_256),
+    (1793, 3840, 20480, 4, 64, _lib.KERNEL_TWO_KERNELS),   # 443, 458 (1850 rows)
+    (2000, 3072, 21504, 8, 64, _lib.KERNEL_TWO_KERNELS),   # 479, 506
+    (1281, 3840, 15360, 4, 128, _lib.KERNEL_TWO_KERNELS),  # K not whole scale periods: 208, 288 by itself
+    (1600, 3072, 12288, 6, 64, _lib.KERNEL_TILES_128),
+])
+def test_where_calls_with_an_epilogue_copy_the_weights(M, K, N, bits, gs, kernel):
+    """From 1281 to 1792 rows the two-kernel path is taken for its rounds of 192-column tiles, which have no epilogue: calls with
+    one stay with the fused kernel, and ask for its planes only."""
+    assert route(M, K, N, bits, gs)[0] == _lib.KERNEL_TWO_KERNELS
+    for epilogue in (_lib.EPILOGUE_GELU, _lib.EPILOGUE_GATE_RESIDUAL, _lib.EPILOGUE_SWIGLU):
+        got, ranges, need = plan(M, K, N, bits, gs, epilogue)
+        assert got == kernel
+        copy = N * K * 2 if kernel == _lib.KERNEL_TWO_KERNELS else 0
+        tail = -(-M // 256) * -(-N // 256) % 256 * ranges * 256 * 256 * 4 if ranges > 1 else 0
+        assert need == copy + (ranges * M * N * 4 if kernel == _lib.KERNEL_TILES_128 and ranges > 1 else tail)
+
+
+@pytest.mark.parametrize("bits,gs", GROUPS)
+def test_plans_agree_with_the_general_answers(bits, gs):
+    for M in (*ROWS, 1281, 1600, 1900, 6889):
+        for K, N in SIZES:
+            if K % gs:
+                continue
+            kernel, ranges = route(M, K, N, bits, gs)
+            most = workspace(M, K, N, bits, gs)
+            for epilogue in range(4):
+                got, r, need = plan(M, K, N, bits, gs, epilogue)
+                if epilogue and (M <= 16 or (epilogue == _lib.EPILOGUE_SWIGLU and N % 64)):
+                    assert got < 0 and need == 0
+                    continue
+                assert got > 0 and need <= most
+                if not epilogue:
+                    assert (got, r, need) == (kernel, ranges, most)
+                elif kernel != _lib.KERNEL_TWO_KERNELS:
+                    assert (got, r, need) == (kernel, ranges, most)
+
+
+def test_plan_checks_its_arguments():
+    assert plan(4, 128, 8, 4, 48, 0) == (-2, 0, 0) and plan(40, 128, 64, 4, 64, 4)[0] == -4 and plan(40, 128, 64, 4, 64, -1)[0] == -4
+    assert plan(40, 128, 12, 4, 64, _lib.EPILOGUE_GELU)[0] == _lib.MFQ_EUNSUPPORTED
+    assert plan(16, 3072, 64, 4, 64, 0) == (_lib.KERNEL_MATVEC, 1, 0)
