@@ -294,10 +294,11 @@ size_t mfq_qmm_t_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size
  * counterpart in the reference.
  *
  * mfq_qmm_t_plan answers the same for one kind of call -- `epilogue` 0:
- * mfq_qmm_t_ws and mfq_qmm_t_low_rank, MFQ_EPILOGUE_*: mfq_qmm_t_epilogue, which
- * has rules of its own about the copy of the weights -- with the workspace that
- * kind uses, *workspace_bytes (may be NULL), where mfq_qmm_t_workspace_bytes()
- * is enough for every kind.
+ * mfq_qmm_t_ws, and mfq_qmm_t_low_rank with a 16-bit y; MFQ_EPILOGUE_*:
+ * mfq_qmm_t_epilogue, which has rules of its own about the copy of the weights --
+ * with the workspace that kind uses, *workspace_bytes (may be NULL), where
+ * mfq_qmm_t_workspace_bytes() is enough for every kind.  Whole 192-column tiles
+ * have one range and no planes there.
  */
 enum mfq_kernel {
   MFQ_KERNEL_MATVEC = 1,      /* the kernels for up to 16 rows (3, 5, 6 bits: one) */
@@ -354,8 +355,9 @@ int mfq_qmm_t_prepared(const void* x, int dtype, int64_t M, int64_t K, const voi
  * same tolerance, other bits).  A shape whose split needs more than the
  * buffer holds is refused with MFQ_ESCRATCH and nothing is launched (on a
  * 256-CU device: the last, short round of 256 x 256 tiles cut into more than
- * 128 planes, e.g. M = 6889 against 3072 -> 3072; use mfq_qmm_t_ws or
- * mfq_qmm_t there).  All calls on one GPU share that GPU's buffer: calls that
+ * 128 planes, e.g. M = 6889 against 3072 -> 3072, also where mfq_qmm_t_ws
+ * would run narrower tiles instead of the cut; use mfq_qmm_t_ws or mfq_qmm_t
+ * there).  All calls on one GPU share that GPU's buffer: calls that
  * overlap on one GPU (two streams, two threads) race; order them on one
  * stream.  The buffer's contents between calls are undefined; nothing in it
  * has to be zero.  The first call on a device looks the buffer's address up

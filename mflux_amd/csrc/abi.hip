@@ -121,7 +121,7 @@ int mfq_qmm_t_plan(int64_t M, int64_t K, int64_t N, int group_size, int bits, in
   if (epilogue == MFQ_EPILOGUE_SWIGLU && N % 64) return MFQ_ESHAPE;
   mfq::QmmRoute route{kernel, ranges, 0, 0};
   if (kernel != MFQ_KERNEL_MATVEC)
-    route = epilogue ? mfq::qmm_epilogue_route(M, N, K, group_size, bits) : mfq::qmm_route(M, N, K, group_size, bits);
+    route = epilogue ? mfq::qmm_epilogue_route(M, N, K, group_size, bits) : mfq::qmm_linear_route(M, N, K, group_size, bits);
   if (k_ranges) *k_ranges = route.ranges;
   if (workspace_bytes) *workspace_bytes = route.copy + route.planes;
   return route.kernel;

@@ -433,7 +433,8 @@ struct QmmRoute {
   size_t planes;  // and of a K cut's float32 planes behind it
 };
 QmmRoute qmm_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
-// the same of a call with an epilogue
+// the same of a call without an epilogue alone (whole 192-column tiles have no planes), and of one with an epilogue
+QmmRoute qmm_linear_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
 QmmRoute qmm_epilogue_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
 // the two-kernel path (qmm_frag.hip): dequantize once into a 16-bit copy in fragment order, then a GEMM on
 // 16x16x32 matrix instructions; 4 and 8 bits, 16-bit y of x's type, a low-rank update or an epilogue as
@@ -441,6 +442,8 @@ QmmRoute qmm_epilogue_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
 // workspace (16-byte aligned): qmm_frag_copy_bytes(N, K) for the copy and, behind it, the float32 planes of a
 // K cut (n_whole whole tiles, the others in `splits` ranges of whole pairs of k steps; splits == 1: no cut)
 bool qmm_frag_shape_ok(int64_t M, int64_t N, int64_t K, int bits);
+// 192-column tiles, whole, where 256-column ones would be cut into `splits` (calls without an epilogue)
+bool qmm_frag_narrow(int64_t M, int64_t N, int64_t K, int splits);
 bool qmm_frag_narrow_rounds(int64_t M, int64_t N, int64_t K, int splits);  // 192-column tiles in several rounds
 // where the two-kernel path is the faster
 bool prefer_frag_path(int64_t M, int64_t N, int64_t K, int gs, int bits, bool epilogue = false);

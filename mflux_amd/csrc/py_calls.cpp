@@ -104,6 +104,11 @@ struct Linear {
     shape.back() = n;
     return at::empty(shape, x.options().requires_grad(false));
   }
+  size_t workspace_bytes(int epilogue) const {
+    size_t bytes = 0;
+    mfq_qmm_t_plan(M, K, N, (int)gs, (int)bits, epilogue, nullptr, &bytes);
+    return bytes;
+  }
   Tensor workspace(size_t bytes) const { return at::empty({(int64_t)bytes}, x.options().dtype(at::kByte).requires_grad(false)); }
   std::vector<c10::IValue> inputs() const { return {x, wq, scales, biases, bias, gs, bits}; }  // for a profiler
 
@@ -135,7 +140,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   RECORD_FUNCTION("mfq::qmm_t", p.inputs());
   const c10::hip::HIPGuardMasqueradingAsCUDA on_device(p.x.device());
   Tensor y = p.out(p.N), ws;
-  const size_t ws_bytes = mfq_qmm_t_workspace_bytes(p.M, p.K, p.N, (int)p.gs, (int)p.bits);
+  const size_t ws_bytes = p.workspace_bytes(0);
   if (ws_bytes) ws = p.workspace(ws_bytes);
   const Linear::Pointers in = p.pointers();
   void *y_p = y.data_ptr(), *ws_p = ws_bytes ? ws.data_ptr() : nullptr;
@@ -158,7 +163,7 @@ PyObject* linear_float32(PyObject*, PyObject* const* args, Py_ssize_t n) {
   RECORD_FUNCTION("mfq::qmm_t", p.inputs());
   const c10::hip::HIPGuardMasqueradingAsCUDA on_device(p.x.device());
   Tensor y = p.out(p.N), rounded = at::empty({p.M, p.K}, p.scales.options().requires_grad(false)), ws;
-  const size_t ws_bytes = mfq_qmm_t_workspace_bytes(p.M, p.K, p.N, (int)p.gs, (int)p.bits);
+  const size_t ws_bytes = p.workspace_bytes(0);
   if (ws_bytes) ws = p.workspace(ws_bytes);
   const Linear::Pointers in = p.pointers();
   void *y_p = y.data_ptr(), *r_p = rounded.data_ptr(), *ws_p = ws_bytes ? ws.data_ptr() : nullptr;
@@ -232,8 +237,7 @@ PyObject* epilogue_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   RECORD_FUNCTION("mfq::qmm_t_epilogue", p.inputs());
   const c10::hip::HIPGuardMasqueradingAsCUDA on_device(p.x.device());
   Tensor y = p.out(epilogue == MFQ_EPILOGUE_SWIGLU ? p.N / 2 : p.N), ws;
-  size_t ws_bytes = 0;
-  mfq_qmm_t_plan(p.M, p.K, p.N, (int)p.gs, (int)p.bits, (int)epilogue, nullptr, &ws_bytes);
+  const size_t ws_bytes = p.workspace_bytes((int)epilogue);
   if (ws_bytes) ws = p.workspace(ws_bytes);
   const Linear::Pointers in = p.pointers();
   void *y_p = y.data_ptr(), *ws_p = ws_bytes ? ws.data_ptr() : nullptr;

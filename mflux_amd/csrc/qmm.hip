@@ -1246,6 +1246,12 @@ QmmRoute qmm_route(int64_t M, int64_t N, int64_t K, int gs, int bits) {
                   two_kernels ? qmm_frag_copy_bytes(N, K) : 0, tail_plane_bytes(M, N, plan)};
 }
 
+QmmRoute qmm_linear_route(int64_t M, int64_t N, int64_t K, int gs, int bits) {
+  QmmRoute route = qmm_route(M, N, K, gs, bits);
+  if (route.kernel == MFQ_KERNEL_TWO_KERNELS && qmm_frag_narrow(M, N, K, route.ranges)) route.ranges = 1, route.planes = 0;
+  return route;
+}
+
 QmmRoute qmm_epilogue_route(int64_t M, int64_t N, int64_t K, int gs, int bits) {
   QmmRoute route = qmm_route(M, N, K, gs, bits);
   if (route.kernel != MFQ_KERNEL_TWO_KERNELS || prefer_frag_path(M, N, K, gs, bits, true)) return route;
@@ -1300,7 +1306,8 @@ int launch_splitk_reduce(int dtype, const void* planes, int splits, int64_t M, i
 // The K cut of the two-kernel path's GEMM when the copy is already there: ranges of whole pairs of k steps.
 size_t qmm_prepared_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (K % (2 * BK)) return 0;
-  return tail_plane_bytes(M, N, plan_tail(M, N, K, 2, compute_units()));
+  const TailPlan plan = plan_tail(M, N, K, 2, compute_units());
+  return qmm_frag_narrow(M, N, K, plan.splits) ? 0 : tail_plane_bytes(M, N, plan);
 }
 
 int launch_qmm_prepared(const void* x, int dtype, int64_t M, int64_t K, const void* copy, const void* bias, int64_t N,
@@ -1322,7 +1329,8 @@ static bool prefer_frag_n(int64_t M, int64_t N, int64_t K, int bits) {
 
 size_t qmm_n_workspace_bytes(int64_t M, int64_t N, int64_t K, int gs, int bits) {
   if (!prefer_frag_n(M, N, K, bits)) return 0;
-  return qmm_frag_copy_bytes(K, N) + tail_plane_bytes(M, K, plan_tail(M, K, N, 2, compute_units()));
+  const TailPlan plan = plan_tail(M, K, N, 2, compute_units());
+  return qmm_frag_copy_bytes(K, N) + (qmm_frag_narrow(M, K, N, plan.splits) ? 0 : tail_plane_bytes(M, K, plan));
 }
 
 int launch_qmm_n_ws(const void* x, int dtype, int64_t M, int64_t N, const uint32_t* wq, const void* scales,

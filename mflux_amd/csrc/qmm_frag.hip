@@ -1067,6 +1067,8 @@ int launch_gemm_typed(const void* x, int64_t M, int64_t K, const void* copy, con
 
 }  // namespace
 
+bool qmm_frag_narrow(int64_t M, int64_t N, int64_t K, int splits) { return prefer_192(M, N, K, splits); }
+
 bool qmm_frag_narrow_rounds(int64_t M, int64_t N, int64_t K, int splits) {
   return ((M + BM - 1) / BM) * ((N + 191) / 192) > compute_units() && prefer_192(M, N, K, splits);
 }

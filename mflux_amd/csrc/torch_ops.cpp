@@ -139,7 +139,11 @@ std::tuple<Tensor, bool> qmm_t(const Tensor& x, const Tensor& wq, const Tensor& 
     t = lr_t->data_ptr();
     bs = lr_bs->data_ptr();
   }
-  const size_t ws_bytes = mfq_qmm_t_workspace_bytes(m.M, m.K, m.N, (int)group_size, (int)bits);
+  size_t ws_bytes = 0;
+  if (rank && out_dtype == at::kFloat)  // (an update with a float32 result: the kernels that dequantise in the GEMM)
+    ws_bytes = mfq_qmm_t_workspace_bytes(m.M, m.K, m.N, (int)group_size, (int)bits);
+  else
+    mfq_qmm_t_plan(m.M, m.K, m.N, (int)group_size, (int)bits, 0, nullptr, &ws_bytes);
   Tensor ws;
   if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
   const int rc = mfq_qmm_t_low_rank(x.data_ptr(), m.sb, m.M, m.K, static_cast<const uint32_t*>(wq.data_ptr()),

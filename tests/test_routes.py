@@ -137,10 +137,26 @@ def test_plans_agree_with_the_general_answers(bits, gs):
                     assert got < 0 and need == 0
                     continue
                 assert got > 0 and need <= most
-                if not epilogue:
+                if not epilogue and need != most:  # whole 192-column tiles in the place of the cut
+                    assert got == kernel == _lib.KERNEL_TWO_KERNELS and r == 1 < ranges and need == -(-N // 16) * 16 * K * 2
+                elif not epilogue:
                     assert (got, r, need) == (kernel, ranges, most)
                 elif kernel != _lib.KERNEL_TWO_KERNELS:
                     assert (got, r, need) == (kernel, ranges, most)
+
+
+def test_whole_192_column_tiles_ask_for_no_planes():
+    """Calls without an epilogue, the input gradient and prepared copies: of the copy, or of nothing, where the tail's cut is not run."""
+    lib = _lib.load()
+    copy = 3072 * 3072 * 2
+    assert plan(6889, 3072, 3072, 4, 64, 0) == (_lib.KERNEL_TWO_KERNELS, 1, copy)
+    assert plan(6889, 3072, 3072, 4, 64, _lib.EPILOGUE_GELU) == (_lib.KERNEL_TWO_KERNELS, 3, copy + 68 * 3 * 256 * 256 * 4)
+    assert lib.mfq_qmm_n_workspace_bytes(6889, 3072, 3072, 64, 4) == copy
+    assert lib.mfq_qmm_t_prepared_workspace_bytes(6889, 3072, 3072) == 0
+    # a cut that is run: its planes
+    assert plan(2100, 2048, 7440, 4, 64, 0) == (_lib.KERNEL_TWO_KERNELS, 8, 7440 * 2048 * 2 + 14 * 8 * 256 * 256 * 4)
+    assert lib.mfq_qmm_n_workspace_bytes(4700, 1024, 3520, 64, 4) > 3520 * 1024 * 2
+    assert lib.mfq_qmm_t_prepared_workspace_bytes(2100, 2048, 7440) > 0
 
 
 def test_plan_checks_its_arguments():
