@@ -298,7 +298,9 @@ size_t mfq_qmm_t_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size
  * mfq_qmm_t_epilogue, which has rules of its own about the copy of the weights --
  * with the workspace that kind uses, *workspace_bytes (may be NULL), where
  * mfq_qmm_t_workspace_bytes() is enough for every kind.  Whole 192-column tiles
- * have one range and no planes there.
+ * have one range and no planes there.  *tile_rows and *tile_columns (NULL, or
+ * both): the tile of the output that a workgroup of the kernel computes, 0 for
+ * the matvecs.
  */
 enum mfq_kernel {
   MFQ_KERNEL_MATVEC = 1,      /* the kernels for up to 16 rows (3, 5, 6 bits: one) */
@@ -310,7 +312,7 @@ enum mfq_kernel {
 };
 int mfq_qmm_t_kernel(int64_t M, int64_t K, int64_t N, int group_size, int bits, int* k_ranges);
 int mfq_qmm_t_plan(int64_t M, int64_t K, int64_t N, int group_size, int bits, int epilogue, int* k_ranges,
-                   size_t* workspace_bytes);
+                   int* tile_rows, int* tile_columns, size_t* workspace_bytes);
 int mfq_qmm_t_ws(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq,
                  const void* scales, const void* biases, int sb_dtype, const void* bias, int64_t N,
                  int group_size, int bits, void* y, int y_dtype, void* workspace,

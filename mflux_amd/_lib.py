@@ -36,7 +36,8 @@ SIGNATURES = {
     "mfq_qmm_n_low_rank": (_INT, [_PTR, _INT, _I64, _I64, _PTR, _PTR, _PTR, _INT, _I64, _INT, _INT, _PTR, _PTR, _I64, _PTR,
                                   _INT, _PTR, ctypes.c_size_t, _PTR]),
     "mfq_qmm_t_workspace_bytes": (ctypes.c_size_t, [_I64, _I64, _I64, _INT, _INT]),
-    "mfq_qmm_t_plan": (_INT, [_I64, _I64, _I64, _INT, _INT, _INT, ctypes.POINTER(_INT), ctypes.POINTER(ctypes.c_size_t)]),
+    "mfq_qmm_t_plan": (_INT, [_I64, _I64, _I64, _INT, _INT, _INT, ctypes.POINTER(_INT), ctypes.POINTER(_INT), ctypes.POINTER(_INT),
+                              ctypes.POINTER(ctypes.c_size_t)]),
     "mfq_qmm_t_kernel": (_INT, [_I64, _I64, _I64, _INT, _INT, ctypes.POINTER(_INT)]),
     "mfq_qmm_t_ws": (_INT, [_PTR, _INT, _I64, _I64, _PTR, _PTR, _PTR, _INT, _PTR, _I64, _INT, _INT, _PTR, _INT, _PTR,
                             ctypes.c_size_t, _PTR]),

@@ -110,8 +110,8 @@ size_t mfq_qmm_t_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size
   return route.copy + route.planes;
 }
 
-int mfq_qmm_t_plan(int64_t M, int64_t K, int64_t N, int group_size, int bits, int epilogue, int* k_ranges,
-                   size_t* workspace_bytes) {
+int mfq_qmm_t_plan(int64_t M, int64_t K, int64_t N, int group_size, int bits, int epilogue, int* k_ranges, int* tile_rows,
+                   int* tile_columns, size_t* workspace_bytes) {
   if (workspace_bytes) *workspace_bytes = 0;
   if (epilogue < 0 || epilogue > MFQ_EPILOGUE_SWIGLU) return MFQ_ESHAPE;
   int ranges = 1;
@@ -124,6 +124,7 @@ int mfq_qmm_t_plan(int64_t M, int64_t K, int64_t N, int group_size, int bits, in
     route = epilogue ? mfq::qmm_epilogue_route(M, N, K, group_size, bits) : mfq::qmm_linear_route(M, N, K, group_size, bits);
   if (k_ranges) *k_ranges = route.ranges;
   if (workspace_bytes) *workspace_bytes = route.copy + route.planes;
+  if (tile_rows && tile_columns) mfq::qmm_route_tile(route, M, N, K, group_size, bits, !epilogue, tile_rows, tile_columns);
   return route.kernel;
 }
 

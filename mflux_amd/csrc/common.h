@@ -436,6 +436,10 @@ QmmRoute qmm_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
 // the same of a call without an epilogue alone (whole 192-column tiles have no planes), and of one with an epilogue
 QmmRoute qmm_linear_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
 QmmRoute qmm_epilogue_route(int64_t M, int64_t N, int64_t K, int gs, int bits);
+// the tile of the kernel that a route names (linear: qmm_linear_route's); a matvec has none
+void qmm_route_tile(const QmmRoute& route, int64_t M, int64_t N, int64_t K, int gs, int bits, bool linear, int* rows, int* columns);
+void qmm_slice_tile(int64_t M, int64_t N, int64_t K, int gs, int bits, int* rows, int* columns);
+int qmm_mid_rows(int64_t M, int64_t N, int64_t K, int gs, bool cut);
 // the two-kernel path (qmm_frag.hip): dequantize once into a 16-bit copy in fragment order, then a GEMM on
 // 16x16x32 matrix instructions; 4 and 8 bits, 16-bit y of x's type, a low-rank update or an epilogue as
 // launch_qmm / launch_qmm_epilogue.

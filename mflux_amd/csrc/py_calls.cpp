@@ -106,7 +106,7 @@ struct Linear {
   }
   size_t workspace_bytes(int epilogue) const {
     size_t bytes = 0;
-    mfq_qmm_t_plan(M, K, N, (int)gs, (int)bits, epilogue, nullptr, &bytes);
+    mfq_qmm_t_plan(M, K, N, (int)gs, (int)bits, epilogue, nullptr, nullptr, nullptr, &bytes);
     return bytes;
   }
   Tensor workspace(size_t bytes) const { return at::empty({(int64_t)bytes}, x.options().dtype(at::kByte).requires_grad(false)); }

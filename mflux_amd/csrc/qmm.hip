@@ -1267,6 +1267,18 @@ QmmRoute qmm_epilogue_route(int64_t M, int64_t N, int64_t K, int gs, int bits) {
   return QmmRoute{MFQ_KERNEL_TILES_128, cut ? ranges : 1, 0, cut ? planes : 0};
 }
 
+void qmm_route_tile(const QmmRoute& route, int64_t M, int64_t N, int64_t K, int gs, int bits, bool linear, int* rows, int* columns) {
+  *rows = *columns = 0;
+  switch (route.kernel) {
+    case MFQ_KERNEL_SLICED: qmm_slice_tile(M, N, K, gs, bits, rows, columns); break;
+    case MFQ_KERNEL_WIDE: *rows = 128, *columns = 256; break;
+    case MFQ_KERNEL_TILES_128: *rows = qmm_mid_rows(M, N, K, gs, route.ranges > 1), *columns = 128; break;
+    case MFQ_KERNEL_TILES_256: *rows = BM, *columns = BN; break;
+    case MFQ_KERNEL_TWO_KERNELS: *rows = BM, *columns = linear && qmm_frag_narrow(M, N, K, route.ranges) ? 192 : BN; break;
+    default: break;
+  }
+}
+
 int launch_tail_reduce(int dtype, const float* planes, int n_whole, int splits, int tiles_m, int tiles_n,
                        const void* bias, int64_t M, int64_t N, void* y, int y_dtype, hipStream_t stream, Epilogue epi) {
   if (splits < 2) return MFQ_ESHAPE;  // (sum_of_planes)

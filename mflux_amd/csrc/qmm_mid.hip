@@ -494,6 +494,10 @@ int launch_qmm_mid_stream(const void* x, int dtype, int64_t M, int64_t K, const 
 #else
 int qmm_mid_ranges(int64_t M, int64_t N, int64_t K, int gs) { return plan_mid(M, N, K, period_of(gs), compute_units()).splits; }
 
+int qmm_mid_rows(int64_t M, int64_t N, int64_t K, int gs, bool cut) {
+  return tile_m(plan_mid(M, N, K, period_of(gs), compute_units(), cut).waves_m);
+}
+
 float qmm_mid_estimate_us(int64_t M, int64_t N, int64_t K, int gs) { return plan_mid(M, N, K, period_of(gs), compute_units()).us; }
 
 int launch_qmm_mid(const void* x, int dtype, int64_t M, int64_t K, const uint32_t* wq, const void* scales,

@@ -624,6 +624,12 @@ int launch_bits(SlicePlan plan, const void* x, int64_t M, int64_t K, const uint3
 
 int qmm_slice_ranges(int64_t M, int64_t N, int64_t K, int gs, int bits) { return choose_slice(M, N, K, gs, bits, true).splits; }
 
+void qmm_slice_tile(int64_t M, int64_t N, int64_t K, int gs, int bits, int* rows, int* columns) {
+  const SlicePlan plan = choose_slice(M, N, K, gs, bits, true);
+  *rows = plan.rows;
+  *columns = plan.columns;
+}
+
 float qmm_slice_estimate_us(int64_t M, int64_t N, int64_t K, int gs, int bits) {
   return choose_slice(M, N, K, gs, bits, true).us;
 }

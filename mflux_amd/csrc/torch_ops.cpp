@@ -143,7 +143,7 @@ std::tuple<Tensor, bool> qmm_t(const Tensor& x, const Tensor& wq, const Tensor& 
   if (rank && out_dtype == at::kFloat)  // (an update with a float32 result: the kernels that dequantise in the GEMM)
     ws_bytes = mfq_qmm_t_workspace_bytes(m.M, m.K, m.N, (int)group_size, (int)bits);
   else
-    mfq_qmm_t_plan(m.M, m.K, m.N, (int)group_size, (int)bits, 0, nullptr, &ws_bytes);
+    mfq_qmm_t_plan(m.M, m.K, m.N, (int)group_size, (int)bits, 0, nullptr, nullptr, nullptr, &ws_bytes);
   Tensor ws;
   if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
   const int rc = mfq_qmm_t_low_rank(x.data_ptr(), m.sb, m.M, m.K, static_cast<const uint32_t*>(wq.data_ptr()),
@@ -181,7 +181,7 @@ std::tuple<Tensor, bool> qmm_t_epilogue(const Tensor& x, const Tensor& wq, const
   Tensor y = at::empty({m.M, n_out}, x.options());
   if (m.M == 0) return {y, true};
   size_t ws_bytes = 0;
-  mfq_qmm_t_plan(m.M, m.K, m.N, (int)group_size, (int)bits, (int)epilogue, nullptr, &ws_bytes);
+  mfq_qmm_t_plan(m.M, m.K, m.N, (int)group_size, (int)bits, (int)epilogue, nullptr, nullptr, nullptr, &ws_bytes);
   Tensor ws;
   if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, x.options().dtype(at::kByte));
   const int rc = mfq_qmm_t_epilogue(x.data_ptr(), m.sb, m.M, m.K, static_cast<const uint32_t*>(wq.data_ptr()),

@@ -46,3 +46,18 @@ def kernel_of(M: int, K: int, N: int, bits: int, group_size: int) -> tuple[int, 
     ranges = ctypes.c_int()
     kernel = _lib.load().mfq_qmm_t_kernel(M, K, N, group_size, bits, ctypes.byref(ranges))
     return kernel, ranges.value
+
+
+def tile_of(M: int, K: int, N: int, bits: int, group_size: int, epilogue: int = 0) -> tuple[int, int, int]:
+    """The same with the tile: the GEMM of a call without an epilogue (or with the one named) and the rows and columns of the
+    output that a workgroup of it computes."""
+    import ctypes
+
+    import pytest
+    from mflux_amd import _lib
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("shapes are chosen for 256 compute units")
+    rows, columns = ctypes.c_int(), ctypes.c_int()
+    kernel = _lib.load().mfq_qmm_t_plan(M, K, N, group_size, bits, epilogue, None, ctypes.byref(rows), ctypes.byref(columns), None)
+    return kernel, rows.value, columns.value

@@ -232,7 +232,7 @@ def test_below_2048_rows_the_copy_is_made_where_it_pays_with_the_epilogue(M, K, 
         largest = ref.abs().amax(dim=1, keepdim=True)
         assert bool(((y.double() - ref).abs() <= (4 * ULP + 2.0 ** -12) * largest).all())
         need = ctypes.c_size_t()
-        kernel = lib.mfq_qmm_t_plan(M, K, N, gs, bits, epilogue, None, ctypes.byref(need))
+        kernel = lib.mfq_qmm_t_plan(M, K, N, gs, bits, epilogue, None, None, None, ctypes.byref(need))
         assert kernel == (_lib.KERNEL_TWO_KERNELS if copies else _lib.KERNEL_TILES_256)
         ws = torch.empty(max(need.value, 16), dtype=torch.uint8, device="cuda")
         y_c = torch.full_like(y, float("nan"))

@@ -449,9 +449,10 @@ def test_float32_results(M, K, N, bits, gs, dtype, has_bias):
     """Float32 activations are rounded to the weights' type on entry; what is left are the float32 sums (K 2^-24 of the sum of
     magnitudes, below 2^-12 of a row's largest output on these operands) and the bias, added to them unrounded."""
     import mflux_amd
-    from gpu_util import kernel_of
+    from gpu_util import kernel_of, tile_of
     from mflux_amd import _lib, core
 
+    assert tile_of(M, K, N, bits, gs) == (_lib.KERNEL_TWO_KERNELS, 256, 256 if (M, N) in ((2310, 12296), (5632, 3072)) else 192)
     assert kernel_of(M, K, N, bits, gs) == (_lib.KERNEL_TWO_KERNELS, (6 if gs == 128 else 12) if K == 3072 else 1)
     gen = torch.Generator(device="cuda").manual_seed(97)
     packed = mflux_amd.quantize((torch.randn(N, K, generator=gen, device="cuda") * 0.02).to(dtype), gs, bits)
@@ -475,10 +476,10 @@ def test_rounds_of_192_column_tiles(M, K, N, bits, gs, dtype):
     """Against float64 on the weights rounded once: a rounding of the result (at most 2^-8 of it, 2^-11 in float16), the bias add
     once more, the float32 sums (below 2^-12 of a row's largest output here)."""
     import mflux_amd
-    from gpu_util import kernel_of
+    from gpu_util import tile_of
     from mflux_amd import _lib, core
 
-    assert kernel_of(M, K, N, bits, gs)[0] == _lib.KERNEL_TWO_KERNELS
+    assert tile_of(M, K, N, bits, gs) == (_lib.KERNEL_TWO_KERNELS, 256, 192)
     gen = torch.Generator(device="cuda").manual_seed(98)
     packed = mflux_amd.quantize((torch.randn(N, K, generator=gen, device="cuda") * 0.02).to(dtype), gs, bits)
     x = torch.randn(M, K, generator=gen, device="cuda").to(dtype)
@@ -496,3 +497,36 @@ def test_rounds_of_192_column_tiles(M, K, N, bits, gs, dtype):
     close(core.quantized_matmul(x, *packed, True, gs, bits, bias=bias, low_rank=(t, bs)),
           ref + t.double() @ bs.double().t() + bias.double(), 2)
     close(core.quantized_matmul(x.float(), *packed, True, gs, bits), ref, 0)
+
+
+@pytest.mark.parametrize("M,K,N,has_bias", [(6889, 3072, 3072, True), (5711, 6144, 3832, False)])
+def test_192_column_tiles_need_no_planes(M, K, N, has_bias):
+    """The same bits with the workspace of the plan, the copy alone, and with the cut's planes behind it, which are not written; a
+    prepared copy likewise."""
+    import ctypes
+
+    import mflux_amd
+    from gpu_util import tile_of
+    from mflux_amd import _lib
+
+    lib, bits, gs = _lib.load(), 4, 64
+    assert tile_of(M, K, N, bits, gs) == (_lib.KERNEL_TWO_KERNELS, 256, 192)
+    gen = torch.Generator(device="cuda").manual_seed(99)
+    packed = mflux_amd.quantize((torch.randn(N, K, generator=gen, device="cuda") * 0.02).bfloat16(), gs, bits)
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    bias = torch.randn(N, generator=gen, device="cuda").bfloat16() if has_bias else None
+    need = ctypes.c_size_t()
+    lib.mfq_qmm_t_plan(M, K, N, gs, bits, 0, None, None, None, ctypes.byref(need))
+    most = lib.mfq_qmm_t_workspace_bytes(M, K, N, gs, bits)
+    assert need.value == -(-N // 16) * 16 * K * 2 < most
+    ys = [mflux_amd.quantized_matmul(x, *packed, group_size=gs, bits=bits, bias=bias)]
+    for size in (need.value, most):
+        ws = torch.full((most,), 7, dtype=torch.uint8, device="cuda")
+        y = torch.full_like(ys[0], float("nan"))
+        assert _call(lib, "mfq_qmm_t_ws", _lib.BF16, M, K, N, gs, bits, x, *packed, bias, y, ws, size) == 0
+        assert bool((ws[need.value:] == 7).all())
+        ys.append(y)
+    assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
+    copy = mflux_amd.prepare_weights(*packed, gs, bits)
+    assert lib.mfq_qmm_t_prepared_workspace_bytes(M, K, N) == 0
+    assert torch.equal(mflux_amd.quantized_matmul_prepared(x, copy, bias=bias), ys[0])

@@ -1,5 +1,5 @@
 """GPU parity: the GEMM with K sliced over the wavefronts of a workgroup (csrc/qmm_slice.hip), at the edges of its tiles
-(32 and 64 rows; 32, 48, 64 and 96 columns), rings, chunks and windows, and the kernels that take the same call when scales
+(32 and 64 rows; 32, 48, 64, 80 and 96 columns), rings, chunks and windows, and the kernels that take the same call when scales
 and biases lie at odd addresses (the 128-column tiles in their form for those, K whole).
 
 Reference: float64 on the dequantised weights rounded once to the 16-bit type, which is what the kernels multiply.  What
@@ -140,11 +140,15 @@ def test_update_and_swiglu_together():
 # whole and ragged last tiles of columns and rows; K: a wavefront's sub-steps fewer than the ring holds, and more
 @pytest.mark.parametrize("M,K,N,bits,gs,dtype", [
     (449, 1280, 2552, 4, 64, "bf16"), (449, 1280, 2552, 8, 64, "f16"), (449, 1280, 2552, 6, 32, "bf16"), (449, 1280, 2560, 5, 64, "f16"),
-    (300, 1024, 4072, 3, 64, "bf16"), (33, 2560, 19448, 4, 32, "f16"), (64, 2560, 19456, 8, 64, "bf16")])
+    (300, 1024, 4072, 3, 64, "bf16"), (33, 2560, 19448, 4, 32, "f16"), (64, 2560, 19456, 8, 64, "bf16"),
+    (449, 1280, 2560, 4, 64, "bf16"), (449, 1280, 2552, 4, 128, "f16"), (33, 2560, 19456, 8, 128, "bf16")])
 def test_tiles_of_80_columns(M, K, N, bits, gs, dtype):
     import mflux_amd
-    from mflux_amd import core
+    from gpu_util import tile_of
+    from mflux_amd import _lib, core
 
+    for epilogue in (0, _lib.EPILOGUE_SWIGLU) if N % 64 == 0 else (0,):
+        assert tile_of(M, K, N, bits, gs, epilogue) == (_lib.KERNEL_SLICED, 64, 80)
     dtype = DT[dtype]
     x, packed, bias, ref = _operands(M, K, N, bits, gs, dtype)
     y = mflux_amd.quantized_matmul(x, *packed, group_size=gs, bits=bits, bias=bias)

@@ -97,7 +97,7 @@ def test_where_the_wide_kernel_is_taken(M, K, N, bits, gs, wide):
 
 def plan(M, K, N, bits, gs, epilogue):
     ranges, need = ctypes.c_int(), ctypes.c_size_t()
-    kernel = _lib.load().mfq_qmm_t_plan(M, K, N, gs, bits, epilogue, ctypes.byref(ranges), ctypes.byref(need))
+    kernel = _lib.load().mfq_qmm_t_plan(M, K, N, gs, bits, epilogue, ctypes.byref(ranges), None, None, ctypes.byref(need))
     return kernel, ranges.value, need.value
 
 
@@ -157,6 +157,17 @@ def test_whole_192_column_tiles_ask_for_no_planes():
     assert plan(2100, 2048, 7440, 4, 64, 0) == (_lib.KERNEL_TWO_KERNELS, 8, 7440 * 2048 * 2 + 14 * 8 * 256 * 256 * 4)
     assert lib.mfq_qmm_n_workspace_bytes(4700, 1024, 3520, 64, 4) > 3520 * 1024 * 2
     assert lib.mfq_qmm_t_prepared_workspace_bytes(2100, 2048, 7440) > 0
+
+
+@pytest.mark.parametrize("M,K,N,bits,gs,epilogue,tile", [
+    (16, 3072, 64, 4, 64, 0, (0, 0)), (100, 2304, 38016, 4, 64, 0, (128, 256)), (256, 12288, 3072, 4, 64, 0, (256, 128)),
+    (70, 3072, 12288, 4, 64, 0, (64, 96)), (17, 3072, 3072, 4, 64, 0, (32, 32)), (512, 3072, 2560, 4, 64, 0, (64, 80)),
+    (1024, 3072, 21504, 4, 64, 0, (256, 256)), (6889, 3072, 3072, 4, 64, 0, (256, 192)), (6889, 3072, 3072, 4, 64, 2, (256, 256)),
+    (4608, 3072, 21504, 4, 64, 0, (256, 256)), (4096, 3072, 3072, 4, 64, 0, (256, 192))])
+def test_tiles_of_a_plan(M, K, N, bits, gs, epilogue, tile):
+    rows, columns = ctypes.c_int(-1), ctypes.c_int(-1)
+    assert _lib.load().mfq_qmm_t_plan(M, K, N, gs, bits, epilogue, None, ctypes.byref(rows), ctypes.byref(columns), None) > 0
+    assert (rows.value, columns.value) == tile
 
 
 def test_plan_checks_its_arguments():
