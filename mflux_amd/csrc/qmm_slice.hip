@@ -532,13 +532,13 @@ struct SlicePlan {
   float us = 0.f;
 };
 
-inline SlicePlan plan_slice(int64_t M, int64_t N, int64_t K, int bits, bool may_cut, bool with_80 = true) {
+// *without_80 (0 on entry): the time of the best of the other tiles
+inline SlicePlan plan_slice(int64_t M, int64_t N, int64_t K, int bits, bool may_cut, float* without_80) {
   const int64_t cus = compute_units();
   const int gran = bits == 3 || bits == 5 ? 2 : 1, grains = (int)(K / (64 * gran));
   const int width = bits == 3 ? 0 : bits == 4 ? 1 : bits == 5 ? 2 : bits == 6 ? 3 : 4;
   SlicePlan best;
   for (const Tile& t : kTiles) {
-    if (t.columns == 80 && !with_80) continue;
     if (t.rows == 32 && M > 128) continue;  // (every code is then dequantised for five row tiles and more)
     const int64_t tiles = ((M + t.rows - 1) / t.rows) * ((N + t.columns - 1) / t.columns);
     for (int s = 1; s == 1 || (may_cut && t.columns != 80 && s <= 8 && tiles * s <= cus && K / 64 / s >= 8); ++s) {
@@ -546,6 +546,7 @@ inline SlicePlan plan_slice(int64_t M, int64_t N, int64_t K, int bits, bool may_
       const int subs = (grains + kWaves * s - 1) / (kWaves * s) * gran;
       float us = 3.1f + (float)rounds * (t.first + (float)subs * t.step[width]);
       if (s > 1) us += 3.4f + (float)(s * M * N) * (4.f / 1.3e6f);
+      if (t.columns != 80 && (*without_80 == 0.f || us < *without_80)) *without_80 = us;
       if (best.splits == 0 || us < best.us) best = SlicePlan{t.rows, t.columns, s, us};
     }
   }
@@ -568,10 +569,10 @@ inline float others_us(int64_t M, int64_t N, int64_t K, int gs, int bits) {
 inline SlicePlan choose_slice(int64_t M, int64_t N, int64_t K, int gs, int bits, bool may_cut) {
   const int64_t gran = bits == 3 || bits == 5 ? 128 : 64;
   if (M > 1024 || N % 8 || K % gran || (K / gs) % 2 || M * K >= ((int64_t)1 << 31) - 2048 || N * K >= (int64_t)1 << 31) return SlicePlan();
-  const SlicePlan plan = plan_slice(M, N, K, bits, may_cut);
+  float without_80 = 0.f;
+  const SlicePlan plan = plan_slice(M, N, K, bits, may_cut, &without_80);
   // (the 80 columns were measured against the other kernel in groups of 32 and 64: in groups of 128 they take no calls from it)
-  const float us = gs == 128 ? plan_slice(M, N, K, bits, may_cut, false).us : plan.us;
-  return us < 0.9f * others_us(M, N, K, gs, bits) ? plan : SlicePlan();
+  return (gs == 128 ? without_80 : plan.us) < 0.9f * others_us(M, N, K, gs, bits) ? plan : SlicePlan();
 }
 
 template <typename T, int BITS, int kA, int kB>
