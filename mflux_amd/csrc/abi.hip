@@ -91,15 +91,23 @@ int mfq_dequantize_rows(const uint32_t* wq, const void* scales, const void* bias
                                      out, out_dtype, (hipStream_t)stream);
 }
 
-int mfq_qmm_t_kernel(int64_t M, int64_t K, int64_t N, int group_size, int bits, int* k_ranges) {
+// the kernel of a call and what else is asked for, planned once: a plan is a good part of a small call's host time
+static int route_of(int64_t M, int64_t K, int64_t N, int group_size, int bits,
+                    mfq::QmmRoute (*plan)(int64_t M, int64_t N, int64_t K, int gs, int bits), mfq::QmmRoute* route) {
   if (int rc = check_common(group_size, bits)) return rc;
   if (M <= 0 || N <= 0 || K <= 0 || K % group_size || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return MFQ_ESHAPE;
   const bool odd_bits = bits != 4 && bits != 8;
   if (odd_bits && M == 1 && K > 8192) return MFQ_EUNSUPPORTED;  // (a GEMM without the workspace that qmm_route() counts on)
-  mfq::QmmRoute route{MFQ_KERNEL_MATVEC, 1, 0, 0};
-  if (M > (odd_bits ? 1 : 16)) route = mfq::qmm_route(M, N, K, group_size, bits);
-  if (k_ranges) *k_ranges = route.ranges;
-  return route.kernel;
+  *route = mfq::QmmRoute{MFQ_KERNEL_MATVEC, 1, 0, 0};
+  if (M > (odd_bits ? 1 : 16)) *route = plan(M, N, K, group_size, bits);
+  return route->kernel;
+}
+
+int mfq_qmm_t_kernel(int64_t M, int64_t K, int64_t N, int group_size, int bits, int* k_ranges) {
+  mfq::QmmRoute route;
+  const int kernel = route_of(M, K, N, group_size, bits, mfq::qmm_route, &route);
+  if (kernel > 0 && k_ranges) *k_ranges = route.ranges;
+  return kernel;
 }
 
 size_t mfq_qmm_t_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size, int bits) {
@@ -114,14 +122,11 @@ int mfq_qmm_t_plan(int64_t M, int64_t K, int64_t N, int group_size, int bits, in
                    int* tile_columns, size_t* workspace_bytes) {
   if (workspace_bytes) *workspace_bytes = 0;
   if (epilogue < 0 || epilogue > MFQ_EPILOGUE_SWIGLU) return MFQ_ESHAPE;
-  int ranges = 1;
-  const int kernel = mfq_qmm_t_kernel(M, K, N, group_size, bits, &ranges);
+  mfq::QmmRoute route;
+  const int kernel = route_of(M, K, N, group_size, bits, epilogue ? mfq::qmm_epilogue_route : mfq::qmm_linear_route, &route);
   if (kernel < 0) return kernel;
   if (epilogue && (M <= 16 || N % 8)) return MFQ_EUNSUPPORTED;
   if (epilogue == MFQ_EPILOGUE_SWIGLU && N % 64) return MFQ_ESHAPE;
-  mfq::QmmRoute route{kernel, ranges, 0, 0};
-  if (kernel != MFQ_KERNEL_MATVEC)
-    route = epilogue ? mfq::qmm_epilogue_route(M, N, K, group_size, bits) : mfq::qmm_linear_route(M, N, K, group_size, bits);
   if (k_ranges) *k_ranges = route.ranges;
   if (workspace_bytes) *workspace_bytes = route.copy + route.planes;
   if (tile_rows && tile_columns) mfq::qmm_route_tile(route, M, N, K, group_size, bits, !epilogue, tile_rows, tile_columns);
