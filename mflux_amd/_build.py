@@ -47,6 +47,8 @@ def _compile(src: str) -> str:
 ASM_MFMA_KERNELS = {"qmm_frag.hip": "frag_gemm_kernel", "qmm_frag_f32.hip": "frag_gemm_kernel"}
 # Sources whose loads from memory straight into LDS are inline assembly, with the write of m0 (their LDS base) in front.
 ASM_LDS_LOAD_SOURCES = ("qmm_frag.hip", "qmm_frag_f32.hip", "qmm_slice.hip")
+# Kernels that use every register there is, whose k loops must not wait for one that was put away: as above.
+FULL_REGISTER_KERNELS = {"qmm_wide.hip": "qmm_wide_kernel"}
 
 
 def _parse_blocks(body: str):
@@ -236,11 +238,37 @@ def check_listing(text: str, kernel_substring: str, where: str = "listing") -> i
     return checked
 
 
+def check_loop_spills(text: str, kernel_substring: str, where: str = "listing") -> int:
+    """Checks every kernel of the assembly listing `text` whose name contains
+    `kernel_substring`: no k loop (a block of 64 matrix instructions and more
+    that branches back to its own label) may read or write a spilled register.  One such load waits for every
+    request in flight, each time round (5 % of the calls' time when the compiler
+    came to it).  Returns the number of kernels; raises RuntimeError on a finding
+    or if a kernel has no such loop."""
+    import re
+
+    checked = 0
+    for m in re.finditer(r"^(\S*%s\S*):" % re.escape(kernel_substring), text, re.M):
+        loops = []
+        for label, ins in _parse_blocks(text[m.end():text.index(".Lfunc_end", m.end())]):
+            back = [i for i, s in enumerate(ins) if label and re.fullmatch(r"s_c?branch\S*\s+%s" % re.escape(label), s)]
+            if back and sum(s.startswith("v_mfma") for s in ins[:back[-1]]) >= 64:
+                loops.append(ins[:back[-1]])
+        if not loops:
+            raise RuntimeError(f"{where}: {m.group(1)} has no k loop; the check does not see the kernel")
+        if any(s.startswith(("scratch_", "buffer_load", "buffer_store")) for ins in loops for s in ins):
+            raise RuntimeError(f"{where}: {m.group(1)} spills registers inside its k loop")
+        checked += 1
+    if not checked:
+        raise RuntimeError(f"{where}: no kernel named *{kernel_substring}* found")
+    return checked
+
+
 def check_generated_code(src: str) -> int:
     """Compiles `src` to assembly (device side) and runs check_lds_loads (for
-    ASM_LDS_LOAD_SOURCES) and check_listing (over the kernels named in
-    ASM_MFMA_KERNELS).  Returns the number of kernels check_listing checked; raises
-    on a finding."""
+    ASM_LDS_LOAD_SOURCES), check_listing (over the kernels named in
+    ASM_MFMA_KERNELS) and check_loop_spills (those in FULL_REGISTER_KERNELS).
+    Returns the number of kernels the last two checked; raises on a finding."""
     import tempfile
 
     with tempfile.TemporaryDirectory() as tmp:
@@ -252,7 +280,8 @@ def check_generated_code(src: str) -> int:
         text = open(asm).read()
     if src in ASM_LDS_LOAD_SOURCES:
         check_lds_loads(text, src)
-    return check_listing(text, ASM_MFMA_KERNELS[src], src) if src in ASM_MFMA_KERNELS else 0
+    checked = check_listing(text, ASM_MFMA_KERNELS[src], src) if src in ASM_MFMA_KERNELS else 0
+    return checked + (check_loop_spills(text, FULL_REGISTER_KERNELS[src], src) if src in FULL_REGISTER_KERNELS else 0)
 
 
 def build_library(verbose: bool = False) -> str:

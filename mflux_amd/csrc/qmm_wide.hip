@@ -67,7 +67,8 @@ __global__ __launch_bounds__(kThreads, 2) void qmm_wide_kernel(
   const int m0 = (tile % tiles_m) * TM, n0 = (tile / tiles_m) * TN;
   // the first n_long k ranges are one quad longer than the others
   const int steps = 4 * (base_quads + (split < n_long ? 1 : 0));
-  const int kb = (split * base_quads + min(split, n_long)) * 4 * TK;  // first k of the item
+  // first k of the item (by itself the compiler keeps it in a vector register, and the loads' addresses with it)
+  const int kb = __builtin_amdgcn_readfirstlane((split * base_quads + min(split, n_long)) * 4 * TK);
   char* y_item = static_cast<char*>(y) + (size_t)split * M * N * 4;   // split > 0 only with float32 planes
 
   // byte offsets (32 bits, checked by the launcher)
@@ -111,10 +112,12 @@ __global__ __launch_bounds__(kThreads, 2) void qmm_wide_kernel(
   };
   auto load_s = [&](Scales& o, int q, int j) __attribute__((always_inline)) {  // the four steps from q on
     const uint32_t at = (uint32_t)(kb + min(q, steps - 4) * TK) / GS * 2u;
+    uint32_t off = soff[j];
+    asm volatile("" : "+v"(off));  // (or the 64-bit addresses of all columns' scales live through the loop, and are spilled)
 #pragma unroll
     for (int l = 0; l < kSWords; ++l) {
-      o.s[j][l] = reinterpret_cast<const uint32_t*>(sb + (size_t)at + soff[j])[l];
-      o.b[j][l] = reinterpret_cast<const uint32_t*>(bb + (size_t)at + soff[j])[l];
+      o.s[j][l] = reinterpret_cast<const uint32_t*>(sb + (size_t)at + off)[l];
+      o.b[j][l] = reinterpret_cast<const uint32_t*>(bb + (size_t)at + off)[l];
     }
   };
   float sc[2][2], bi[2][2];  // [step & 1][column]
@@ -243,8 +246,8 @@ __global__ __launch_bounds__(kThreads, 2) void qmm_wide_kernel(
     }
   };
   // A tile of at most 64 rows leaves the matrix work of the other half out (its weights are dequantised all the same): 320
-  // rows x 3584 -> 37888 113 -> 107 us, x 18944 -> 3584 67.6 -> 64.8.  A kernel of its own, because both loops in one cost
-  // the whole tiles' up to 1 % (registers; at 8 bits some are spilled in it).
+  // rows x 3584 -> 37888 113 -> 107 us, x 18944 -> 3584 67.6 -> 64.8, at 8 bits 124 -> 117 and level.  A kernel of its own,
+  // because both loops in one cost the whole tiles' up to 1 % (registers).
   if (kShort && M - m0 <= TM / 2) run(std::integral_constant<int, kI / 2>{});
   else run(std::integral_constant<int, kI>{});
 

@@ -281,6 +281,32 @@ def test_generated_code_of_the_assembly_lds_loads():
     assert _build.check_generated_code("qmm_slice.hip") == 0
 
 
+def test_generated_code_of_the_wide_kernels():
+    """The 128 x 256-tile GEMM uses all 256 registers of its two wavefronts per SIMD: two types x 4 bits in three group sizes
+    and 8 bits in two x with and without the loop for a short last tile, none with a spilled register in a k loop."""
+    from mflux_amd import _build
+
+    assert _build.check_generated_code("qmm_wide.hip") == 20
+
+
+def test_listing_check_of_loop_spills():
+    from mflux_amd import _build
+
+    matrix = ["v_mfma_f32_32x32x16_bf16 v[0:15], v[16:19], v[20:23], v[0:15]"] * 32
+    back = ["s_cbranch_scc1 .LBB0_1"]
+    spill = ["scratch_load_dwordx2 v[182:183], off, off"]
+
+    def listing(*loop):
+        return _listing([("", spill), (".LBB0_1", [s for part in loop for s in part]), (".LBB0_9", spill + ["s_endpgm"])])
+
+    assert _build.check_loop_spills(listing(matrix, matrix, back, spill), "demo_gemm") == 1  # behind the loop: nothing waits there
+    for bad in (spill, ["scratch_store_dword off, v1, off"]):
+        with pytest.raises(RuntimeError, match="inside its k loop"):
+            _build.check_loop_spills(listing(matrix, bad, matrix, back), "demo_gemm")
+    with pytest.raises(RuntimeError, match="no k loop"):
+        _build.check_loop_spills(listing(matrix, matrix), "demo_gemm")
+
+
 def test_listing_check_of_lds_loads():
     """A load into LDS directly behind a write of m0 is refused, over a branch and
     through an empty block too; an s_nop or another instruction between the two is
