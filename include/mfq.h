@@ -261,8 +261,8 @@ int mfq_qmm_n_low_rank(const void* x, int x_dtype, int64_t M, int64_t N, const u
  * into its own float32 plane of the workspace, and a second kernel adds the
  * planes, rounds and applies the bias (same two roundings as the fused
  * epilogue).  Large calls -- K a multiple of 128, from 1281 to 2048
- * activation rows on at 4 or 8 bits and 1024 at 3, 5 or 6 (where it starts to
- * pay), e.g. the single-stream
+ * activation rows on at 4 or 8 bits, as their tiles and an epilogue have it, and
+ * 1024 at 3, 5 or 6 (where it starts to pay), e.g. the single-stream
  * linears of FLUX.1 at M = 4608 -- use the workspace first for a 16-bit copy of
  * the dequantised weights (round_up(N, 16) * K * 2 bytes rounded up to 256,
  * written once per call in the order the matrix instructions consume it) and
@@ -329,8 +329,9 @@ int mfq_qmm_t_ws(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_
  * multiple of 128 or below 256, N not a multiple of 8, or more than 2 GiB) --
  * into a buffer the caller keeps, and mfq_qmm_t_prepared multiplies x
  * [M, K] of the same 16-bit type with it into y [M, N] of that type (+ bias):
- * bit-identical to what mfq_qmm_t_ws gives on its two-kernel path, for any M,
- * at 2 bytes per weight of memory held instead of bits / 8 -- on FLUX.1's
+ * bit-identical to what mfq_qmm_t_ws gives on its two-kernel path (a short last
+ * round of tiles that both cut along K apart: into ranges of whole pairs of 64
+ * here, of whole scale periods there), for any M, at 2 bytes per weight of memory held instead of bits / 8 -- on FLUX.1's
  * single-block linears at M = 4608 the copy is 7 % of the call.
  * `workspace` (optional, 16-byte aligned, mfq_qmm_t_prepared_workspace_bytes)
  * takes the float32 planes of a K cut of a short last round of tiles; without

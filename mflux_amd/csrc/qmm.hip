@@ -1200,7 +1200,7 @@ constexpr int64_t kOddBitsFragRows = MFQ_ODD_FRAG_ROWS;
 // the tail of the tile sequence by the same plan as the fused kernel, or takes narrower tiles there.
 // 4 and 8 bits, eight rows of tiles (1793 to 2047 rows): of 35 drawn shapes (all group sizes, float32 results, low-rank updates)
 // 0.60 to 1.01 of the fused kernel's time (1985 x 2560 -> 9216 107 us -> 102, 1951 x 15360 -> 4304 303 -> 248), with an epilogue
-// 0.91 to 0.98 by itself and 0.94 to 0.97 between other kernels (Z-Image's feed-forward, 1850 rows at 8 bits 486 us -> 456; a
+// 0.91 to 0.98 by itself and 0.92 to 0.97 between other kernels (Z-Image's feed-forward, 1850 rows at 8 bits 486 us -> 456; a
 // single-stream block of 2000 rows at 4 489 -> 463).  With seven rows of tiles and six the two are level by themselves, and
 // between other kernels the copy's traffic costs more (a training step at 1536 x 3072 -> 12288 283 us, 293 with the copy), except
 // from 1281 rows on
